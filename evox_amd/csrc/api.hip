@@ -21,6 +21,7 @@
 #include "peel_lds.hpp"
 #include "prefix.hpp"
 #include "radix.hpp"
+#include "spatial.hpp"
 #include "stepped.hpp"
 #include "two.hpp"
 #include "two_small.hpp"
@@ -82,7 +83,7 @@ struct Layout {
   int64_t wstride;
   // byte offsets
   size_t ctrl, fsize, fronts_slot, fronts_orig, hist, zero_end, fstart, xs, key, partials, sortparam, bstart, bcursor,
-      scanflags, tailbuf, records, two_ring, members, member_key, slot_of, xs_sorted, key_sorted, kid_sorted, orig_of, count, witness, total0, witness0, rank, dist, perm, order, rpairs0, rpairs1, rtable, rtotals, pos, scost, dkey, wide, wide_bytes, dom, total;
+      scanflags, tailbuf, records, two_ring, members, member_key, slot_of, xs_sorted, key_sorted, kid_sorted, orig_of, count, witness, total0, witness0, leaf_lo, leaf_hi, group_lo, rank, dist, perm, order, rpairs0, rpairs1, rtable, rtotals, pos, scost, dkey, wide, wide_bytes, dom, total;
 };
 
 static size_t align_up(size_t v) { return (v + 255) / 256 * 256; }
@@ -138,6 +139,11 @@ static bool make_layout(int64_t n, int64_t m, Layout* L) {
   // from count / witness, which the peel consumes, so that the count stage can be repeated)
   L->total0 = o;     o = align_up(o + sizeof(int) * (size_t)n);
   L->witness0 = o;   o = align_up(o + sizeof(int) * (size_t)n);
+  // boxes of the rows in spatial order (spatial.hpp)
+  const size_t box = m <= kSpatialObjectives ? sizeof(float) * (size_t)m : 0;
+  L->leaf_lo = o;    o = align_up(o + box * (size_t)spatial_leaf_stride(n));
+  L->leaf_hi = o;    o = align_up(o + box * (size_t)spatial_leaf_stride(n));
+  L->group_lo = o;   o = align_up(o + box * (size_t)spatial_group_stride(n));
   L->rank = o;       o = align_up(o + sizeof(int) * (size_t)n);
   L->dist = o;       o = align_up(o + sizeof(float) * (size_t)n);
   L->perm = o;       o = align_up(o + sizeof(int) * (size_t)n);
@@ -316,14 +322,6 @@ static void launch_dominance(const Ws& w, int variant, hipStream_t s) {
                          w.at<uint32_t>(L.kid_sorted), w.at<uint64_t>(L.dom), L.n, L.npad, L.wstride, L.nwords, L.m, w.step);
     }
   }
-}
-
-template <int M>
-static void launch_first_front(const Ws& w, uint8_t* mask, hipStream_t s) {
-  const Layout& L = w.L;
-  hipLaunchKernelGGL((first_front_kernel<M>), dim3((L.n + 255) / 256, 1, w.batch), dim3(256), 0, s, w.at<float>(L.xs_sorted),
-                     w.at<uint64_t>(L.key_sorted), w.at<uint32_t>(L.kid_sorted), w.at<int>(L.orig_of), L.n, L.npad, mask,
-                     w.ctrl(), w.at<SortParam>(L.sortparam), w.step);
 }
 
 // Fitness -> structure of arrays + keys, state reset, then the slot sort (order.hpp).
@@ -1535,6 +1533,117 @@ size_t evox_hip_first_front_workspace_bytes(int64_t n, int64_t m) {
 
 }  // extern "C"
 
+// The rows xs[k][.] of which *count are left, if more than `least`, into spatial order: xs_sorted, slot_row, slot_end and the
+// boxes.  The histogram and the flags of its scan must be zero; counted: it holds the buckets' sizes already, and the rows'
+// buckets are known.
+static int spatial_bucket_bits(const Layout& L) {
+  int bits = 10;
+  while ((1 << bits) < L.buckets) ++bits;
+  return bits;
+}
+template <int M>
+static int stage_spatial_order(const Ws& w, const float* xs, float* xs_sorted, const int* count, int least, bool counted, hipStream_t s) {
+  const Layout& L = w.L;
+  int* const bucket = w.at<int>(L.members);
+  int* const slot_row = w.at<int>(L.orig_of);
+  int* const slot_end = w.at<int>(L.kid_sorted);
+  int blocks = (L.npad + 255) / 256;
+  if (blocks > 2048) blocks = 2048;
+  if (!counted) {
+    hipLaunchKernelGGL(spatial_bucket_kernel<M>, dim3(blocks < 1024 ? blocks : 1024, 1, w.batch), dim3(256), 0, s, xs, L.npad, count,
+                       least, spatial_bucket_bits(L), bucket, w.at<int>(L.hist), w.step);
+    EVX_LAUNCH_CHECK();
+  }
+  auto launch_scan = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(L.buckets / 1024, 1, w.batch), dim3(256), 0, s, w.at<int>(L.hist), L.buckets, w.at<int>(L.bstart),
+                       w.at<int>(L.bcursor), w.at<unsigned long long>(L.scanflags), w.ctrl(), w.step);
+  };
+  w.batch > 1 ? launch_scan(bucket_scan_kernel<true>) : launch_scan(bucket_scan_kernel<false>);
+  EVX_LAUNCH_CHECK();
+  hipLaunchKernelGGL(spatial_scatter_kernel<M>, dim3(blocks, 1, w.batch), dim3(256), 0, s, xs, L.npad, count, least, bucket,
+                     w.at<int>(L.bstart), w.at<int>(L.bcursor), xs_sorted, slot_row, slot_end, w.ctrl(), w.step);
+  EVX_LAUNCH_CHECK();
+  const int64_t leaf_stride = spatial_leaf_stride(L.n), group_stride = spatial_group_stride(L.n);
+  hipLaunchKernelGGL(leaf_box_kernel, dim3((unsigned)(leaf_stride / kGroupLeaves), 1, w.batch), dim3(kBoxThreads), 0, s, xs_sorted,
+                     count, least, L.npad, L.m, leaf_stride, group_stride, w.at<float>(L.leaf_lo), w.at<float>(L.leaf_hi),
+                     w.at<float>(L.group_lo), w.ctrl(), w.step);
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
+// The first front of up to kSpatialObjectives objectives (spatial.hpp).
+template <int M>
+static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hipStream_t s) {
+  const Layout& L = w.L;
+  // The rows step 2 leaves stand in xs, those of step 1 in xs_sorted, and the spatial order goes to the other of the two.
+  constexpr bool kGrid = M == 2 || M == 3;
+  const bool grid_step = kGrid && L.n > kFrontGridPopulation;
+  const bool order_step = L.n > kFrontPairsRows;
+  FrontCount* const count = w.at<FrontCount>(L.fstart);
+  const int* const counted = grid_step ? &count->rows_grid : &count->rows;
+  float* const left = w.at<float>(L.xs_sorted);
+  int* const left_of = w.at<int>(L.order);
+  float* const to = grid_step ? w.at<float>(L.xs) : nullptr;
+  int* const to_of = grid_step ? w.at<int>(L.perm) : nullptr;
+  // (the cells before and after the prefix passes: up to 256 KB each, where the radix sort's pairs go)
+  uint32_t* const cells = grid_step ? w.at<uint32_t>(L.rpairs0) : nullptr;
+  uint32_t* const turned = grid_step ? w.at<uint32_t>(L.rpairs1) : nullptr;
+  const bool small_grid = M == 3 && L.n <= kFrontGridSmallRows;
+  const int cell_bits = small_grid ? 7 : 8;
+  const int grid_cells = !grid_step ? 0 : (M == 2 ? 1 << cell_bits : 1 << (2 * cell_bits));
+  hipLaunchKernelGGL(front_reset_kernel, dim3(1, 1, w.batch), dim3(256), 0, s, w.ctrl(), count, w.step);
+  EVX_LAUNCH_CHECK();
+  int blocks = (L.n + 256 * kFrontRowsPerThread - 1) / (256 * kFrontRowsPerThread);
+  if (blocks > 1024) blocks = 1024;
+  hipLaunchKernelGGL(front_filter_kernel<M>, dim3(blocks, 1, w.batch), dim3(256), 0, s, fit.f, fit.sr, fit.sc, fit.step, L.n, L.npad,
+                     left, left_of, mask, count, cells, grid_cells, w.at<uint32_t>(L.hist),
+                     order_step ? (int)((L.tailbuf - L.hist) / 4) : 0, w.step);
+  EVX_LAUNCH_CHECK();
+  if constexpr (kGrid) {
+    if (grid_step) {
+      int build_blocks = (L.n + 255) / 256;
+      if (build_blocks > 1024) build_blocks = 1024;
+      hipLaunchKernelGGL(front_grid_kernel<M>, dim3(build_blocks, 1, w.batch), dim3(256), 0, s, left, L.npad, cell_bits, count, cells,
+                         w.step);
+      EVX_LAUNCH_CHECK();
+      const uint32_t* below = turned;
+      if (small_grid) {
+        if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(front_grid_small_kernel), kFrontGridLds)) return e;
+        hipLaunchKernelGGL(front_grid_small_kernel, dim3(1, 1, w.batch), dim3(kFrontGridThreads), kFrontGridLds, s, cells, turned, count,
+                           w.step);
+        EVX_LAUNCH_CHECK();
+      } else {
+        hipLaunchKernelGGL(front_grid_prefix_kernel, dim3(M == 2 ? 1 : kFrontGrid, 1, w.batch), dim3(kFrontGrid), 0, s, cells, turned,
+                           M == 2 ? 1 : kFrontGrid, count, w.step);
+        EVX_LAUNCH_CHECK();
+        if (M == 3) {
+          below = cells;
+          hipLaunchKernelGGL(front_grid_prefix_kernel, dim3(kFrontGrid, 1, w.batch), dim3(kFrontGrid), 0, s, turned, cells, kFrontGrid,
+                             count, w.step);
+          EVX_LAUNCH_CHECK();
+        }
+      }
+      hipLaunchKernelGGL(front_grid_filter_kernel<M>, dim3(blocks, 1, w.batch), dim3(256), 0, s, left, left_of, L.npad, cell_bits, count,
+                         below, to, to_of, mask, L.n, spatial_bucket_bits(L), w.at<int>(L.members),
+                         order_step ? w.at<int>(L.hist) : (int*)nullptr, w.step);
+      EVX_LAUNCH_CHECK();
+    }
+  }
+  const int pair_rows = L.n < kFrontPairsRows ? L.n : kFrontPairsRows;
+  hipLaunchKernelGGL(front_pairs_kernel<M>, dim3((pair_rows + 255) / 256, kFrontPairsParts, w.batch), dim3(256), 0, s, left, left_of,
+                     to, to_of, L.npad, mask, L.n, count, w.step);
+  EVX_LAUNCH_CHECK();
+  if (!order_step) return 0;
+  float* const sorted = grid_step ? left : w.at<float>(L.xs);
+  if (int e = stage_spatial_order<M>(w, grid_step ? to : left, sorted, counted, kFrontPairsRows, grid_step, s)) return e;
+  hipLaunchKernelGGL((first_front_leaf_kernel<M>), dim3((unsigned)spatial_leaves(L.n), 1, w.batch), dim3(64 * kFrontWaves), 0, s,
+                     sorted, w.at<int>(L.orig_of), w.at<int>(L.kid_sorted), grid_step ? to_of : left_of, count, counted, L.npad,
+                     spatial_leaf_stride(L.n), spatial_group_stride(L.n), w.at<float>(L.leaf_lo), w.at<float>(L.leaf_hi),
+                     w.at<float>(L.group_lo), mask, L.n, w.ctrl(), w.step);
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
 // batch > 1: that many populations of one shape in the same launches, their workspaces (without the matrix) ws_step
 // bytes apart, their masks n bytes.
 static int first_front_rows(const Fitness& fit, int64_t n, int64_t m, uint8_t* mask_out, void* ws, size_t ws_bytes, hipStream_t s,
@@ -1548,25 +1657,26 @@ static int first_front_rows(const Fitness& fit, int64_t n, int64_t m, uint8_t* m
     w.batch = batch;
     w.step = ws_step;
   }
-  if (int e = stage_prepare(w, fit, true, s)) return e;
+  if (fit.f == nullptr) return kErrBadArg;
   switch (L.m) {
-    case 1: launch_first_front<1>(w, mask_out, s); break;
-    case 2: launch_first_front<2>(w, mask_out, s); break;
-    case 3: launch_first_front<3>(w, mask_out, s); break;
-    case 4: launch_first_front<4>(w, mask_out, s); break;
-    case 5: launch_first_front<5>(w, mask_out, s); break;
-    case 6: launch_first_front<6>(w, mask_out, s); break;
-    case 7: launch_first_front<7>(w, mask_out, s); break;
-    case 8: launch_first_front<8>(w, mask_out, s); break;
-    case 9: launch_first_front<9>(w, mask_out, s); break;
-    case 10: launch_first_front<10>(w, mask_out, s); break;
-    case 11: launch_first_front<11>(w, mask_out, s); break;
-    case 12: launch_first_front<12>(w, mask_out, s); break;
-    case 13: launch_first_front<13>(w, mask_out, s); break;
-    case 14: launch_first_front<14>(w, mask_out, s); break;
-    case 15: launch_first_front<15>(w, mask_out, s); break;
-    case 16: launch_first_front<16>(w, mask_out, s); break;
+    case 1: return first_front_steps<1>(w, fit, mask_out, s);
+    case 2: return first_front_steps<2>(w, fit, mask_out, s);
+    case 3: return first_front_steps<3>(w, fit, mask_out, s);
+    case 4: return first_front_steps<4>(w, fit, mask_out, s);
+    case 5: return first_front_steps<5>(w, fit, mask_out, s);
+    case 6: return first_front_steps<6>(w, fit, mask_out, s);
+    case 7: return first_front_steps<7>(w, fit, mask_out, s);
+    case 8: return first_front_steps<8>(w, fit, mask_out, s);
+    case 9: return first_front_steps<9>(w, fit, mask_out, s);
+    case 10: return first_front_steps<10>(w, fit, mask_out, s);
+    case 11: return first_front_steps<11>(w, fit, mask_out, s);
+    case 12: return first_front_steps<12>(w, fit, mask_out, s);
+    case 13: return first_front_steps<13>(w, fit, mask_out, s);
+    case 14: return first_front_steps<14>(w, fit, mask_out, s);
+    case 15: return first_front_steps<15>(w, fit, mask_out, s);
+    case 16: return first_front_steps<16>(w, fit, mask_out, s);
     default:
+      if (int e = stage_prepare(w, fit, true, s)) return e;
       hipLaunchKernelGGL(first_front_any_m_kernel, dim3((L.n + 255) / 256, 1, w.batch), dim3(256), 0, s, w.at<float>(L.xs_sorted),
                          w.at<uint32_t>(L.kid_sorted), w.at<int>(L.orig_of), L.n, L.npad, L.m, mask_out, w.ctrl(), w.step);
   }

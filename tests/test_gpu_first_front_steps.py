@@ -1,0 +1,53 @@
+"""The steps of the first-front mask (sampled champions, grid, pairs, leaves in spatial order) at the sizes where one takes
+over from another, against the C checker: masks are whole numbers and must be equal."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle
+
+pytestmark = pytest.mark.gpu
+
+INF, NAN = float("inf"), float("nan")
+
+
+def population(kind, n, m, seed):
+    g = torch.Generator("cpu").manual_seed(seed)
+    f = torch.rand(n, m, generator=g)
+    if kind == "uniform":
+        return f
+    d = torch.randn(n, m, generator=g).abs()
+    if kind == "one front":
+        return d / d.sum(dim=1, keepdim=True)
+    f = d / d.norm(dim=1, keepdim=True) * (1.0 - 0.1 * torch.log1p(-torch.rand(n, 1, generator=g)))
+    if kind == "ties":  # equal rows and equal values in every objective
+        f = torch.round(f * 32) / 32
+    if kind == "special":  # penalties, infinities, signed zeros, NaN
+        f[: n // 3] = 1e9
+        f[::101, 0] = -0.0
+        f[1::103, m - 1] = 0.0
+        f[2::107, 0] = INF
+        f[3::109, m - 1] = -INF
+        f[4::113, m // 2] = NAN
+    return f
+
+
+@pytest.mark.parametrize("kind", ["uniform", "shell", "one front", "ties", "special"])
+@pytest.mark.parametrize("n,m", [(1, 3), (63, 2), (1025, 3), (1024, 16), (16384, 3), (16385, 2), (16385, 3), (21000, 4), (65536, 3),
+                                 (65537, 2), (65537, 3), (65537, 4), (70001, 7), (131072, 3), (131073, 3)])
+def test_mask_at_the_edges_of_the_steps(n, m, kind):
+    from evox_amd.operators.selection import non_dominated_mask
+
+    f = population(kind, n, m, n + m)
+    got = non_dominated_mask(f.to("cuda")).cpu().numpy()
+    assert np.array_equal(got, c_oracle.first_front(f.numpy()))
+
+
+def test_masks_of_several_large_populations():
+    from evox_amd.operators.selection import non_dominated_mask
+
+    f = torch.stack([population(kind, 66000, 3, 5) for kind in ("uniform", "one front", "special")])
+    got = non_dominated_mask(f.to("cuda")).cpu().numpy()
+    for b in range(3):
+        assert np.array_equal(got[b], c_oracle.first_front(f[b].numpy())), b
