@@ -2812,13 +2812,92 @@ int evox_hip_tournament_pick_keys(const int64_t* parents, int64_t n_round, int64
   return 0;
 }
 
+}  // extern "C"
+
+// What the two uses of the points against the samples keep in their workspace.
+struct HvBytes {
+  size_t packed, partial, alpha, points, extreme, counts;
+};
+static HvBytes hv_bytes(int64_t n, int64_t m, int64_t n_sample) {
+  HvBytes b;
+  const int64_t share = hv_share(n_sample);
+  b.packed = align_up(sizeof(float) * (size_t)hv_packed((int)m) * (size_t)n_sample);
+  b.partial = align_up(sizeof(float) * (size_t)((n_sample + share - 1) / share) * (size_t)n);
+  b.alpha = align_up(sizeof(float) * (size_t)n);
+  b.points = align_up(sizeof(float) * (size_t)n * (size_t)m);
+  b.extreme = align_up(sizeof(float) * (size_t)kHvParts * (size_t)m);
+  b.counts = align_up(sizeof(uint32_t) * (size_t)((n_sample + 63) / 64));
+  return b;
+}
+static bool hv_sizes_fit(int64_t n, int64_t n_sample) { return n >= 1 && n_sample >= 1 && n <= 0x7FFFFF00ll && n_sample <= 0x7FFFFF00ll; }
+
+// Waves that share the points of 64 samples: sixteen until the samples alone bring more than the device holds at a time
+// (1024 workgroups), then four (1001 x 3 against 100 000 samples: see hv.hpp).  Never more than there are steps over the points.
+static unsigned hv_threads(int64_t n, int64_t n_sample) {
+  int64_t waves = n_sample > (1ll << 28) ? 1 : (n_sample > 65536 ? 4 : 16);  // (a grid has less than 2^32 threads)
+  const int64_t steps = (n + kHvStep - 1) / kHvStep;
+  if (waves > steps) waves = steps;
+  return (unsigned)(64 * waves);
+}
+
+// The kernels are built for 1 to 8 objectives, for up to kHvRegs (their number read at run time) and for any number.
+template <typename F>
+static int hv_for_objectives(int64_t m, F&& launch) {
+  switch (m) {
+    case 1: return launch(std::integral_constant<int, 1>());
+    case 2: return launch(std::integral_constant<int, 2>());
+    case 3: return launch(std::integral_constant<int, 3>());
+    case 4: return launch(std::integral_constant<int, 4>());
+    case 5: return launch(std::integral_constant<int, 5>());
+    case 6: return launch(std::integral_constant<int, 6>());
+    case 7: return launch(std::integral_constant<int, 7>());
+    case 8: return launch(std::integral_constant<int, 8>());
+    default: break;
+  }
+  if (m <= kHvRegs) return launch(std::integral_constant<int, kHvRegs>());
+  return launch(std::integral_constant<int, 0>());
+}
+
+template <int kMode>
+static int hv_contribution_launches(const float* points_t, const HvSamples& samples, const float* alpha, int64_t n, int64_t m,
+                                    int64_t n_sample, float scale, float* packed, float* partial, float* out, hipStream_t s) {
+  const int64_t share = hv_share(n_sample);
+  const int shares = (int)((n_sample + share - 1) / share);
+  if (int e = hv_for_objectives(m, [&](auto objectives) {
+        constexpr int M = decltype(objectives)::value;
+        hipLaunchKernelGGL((hv_sample_weight_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, n_sample)), 0,
+                           s, points_t, samples, (int)n, (int)m, (int)n_sample, alpha, packed);
+        EVX_LAUNCH_CHECK();
+        hipLaunchKernelGGL(hv_point_partial_kernel<M>, dim3((unsigned)((n + 255) / 256), (unsigned)shares), dim3(256), 0, s, points_t,
+                           packed, samples, (int)n, (int)m, (int)n_sample, (int)share, partial);
+        EVX_LAUNCH_CHECK();
+        return 0;
+      }))
+    return e;
+  hipLaunchKernelGGL(hv_point_total_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, partial, samples, (int)n, (int)m, shares,
+                     (int)n_sample, scale, out);
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int kMode>
+static int hv_covered_launch(const float* points_t, const HvSamples& samples, int64_t n, int64_t m, int64_t n_sample,
+                             uint32_t* counts, hipStream_t s) {
+  return hv_for_objectives(m, [&](auto objectives) {
+    constexpr int M = decltype(objectives)::value;
+    hipLaunchKernelGGL((hv_covered_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, n_sample)), 0, s,
+                       points_t, samples, (int)n, (int)m, (int)n_sample, counts);
+    EVX_LAUNCH_CHECK();
+    return 0;
+  });
+}
+
+extern "C" {
+
 size_t evox_hip_hv_workspace_bytes(int64_t n, int64_t n_sample) {
-  if (n < 1 || n_sample < 1 || n > 0x7FFFFF00ll || n_sample > 0x7FFFFF00ll) return 0;
-  const int point_chunk = hv_chunk_length(n, kHvPointChunk), sample_chunk = hv_chunk_length(n_sample, kHvChunk);
-  const size_t point_chunks = (size_t)((n + point_chunk - 1) / point_chunk);
-  const size_t sample_chunks = (size_t)((n_sample + sample_chunk - 1) / sample_chunk);
-  return align_up(sizeof(float) * (size_t)n_sample) + align_up(sizeof(int32_t) * point_chunks * (size_t)n_sample) +
-         align_up(sizeof(float) * sample_chunks * (size_t)n);
+  if (!hv_sizes_fit(n, n_sample)) return 0;
+  const HvBytes b = hv_bytes(n, kHvRegs, n_sample);  // (the call's objectives are not known here)
+  return b.packed + b.partial;
 }
 
 int evox_hip_hv_contributions(const float* fit_t, const float* samples_t, const float* alpha, int64_t n, int64_t m,
@@ -2827,28 +2906,39 @@ int evox_hip_hv_contributions(const float* fit_t, const float* samples_t, const 
   const size_t need = evox_hip_hv_workspace_bytes(n, n_sample);
   if (need == 0) return kErrBadArg;
   if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0) return kErrWorkspace;
-  hipStream_t s = (hipStream_t)stream;
-  const int point_chunk = hv_chunk_length(n, kHvPointChunk), sample_chunk = hv_chunk_length(n_sample, kHvChunk);
-  const int point_chunks = (int)((n + point_chunk - 1) / point_chunk);
-  const int sample_chunks = (int)((n_sample + sample_chunk - 1) / sample_chunk);
+  const HvBytes b = hv_bytes(n, kHvRegs, n_sample);
   uint8_t* base = static_cast<uint8_t*>(ws);
-  float* weight = reinterpret_cast<float*>(base);
-  int32_t* cover = reinterpret_cast<int32_t*>(base + align_up(sizeof(float) * (size_t)n_sample));
-  float* partial = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(cover) +
-                                            align_up(sizeof(int32_t) * (size_t)point_chunks * (size_t)n_sample));
-  const unsigned sample_blocks = (unsigned)((n_sample + 255) / 256), point_blocks = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(hv_cover_count_kernel, dim3(sample_blocks, (unsigned)point_chunks), dim3(256), 0, s, fit_t, samples_t, (int)n,
-                     (int)m, (int)n_sample, point_chunk, cover);
+  const HvSamples samples = {samples_t, 1, n_sample, nullptr, nullptr, 0, 0};
+  return hv_contribution_launches<kHvPlain>(fit_t, samples, alpha, n, m, n_sample, scale, reinterpret_cast<float*>(base),
+                                            reinterpret_cast<float*>(base + b.packed), out, (hipStream_t)stream);
+}
+
+size_t evox_hip_hype_workspace_bytes(int64_t n, int64_t m, int64_t n_sample) {
+  if (!hv_sizes_fit(n, n_sample) || m < 1 || m > kHvRegs) return 0;
+  const HvBytes b = hv_bytes(n, m, n_sample);
+  return b.packed + b.partial + b.alpha + b.points + b.extreme;
+}
+
+int evox_hip_hype_contributions(const float* f, int64_t stride_row, int64_t stride_col, int64_t n, int64_t m, const float* ref,
+                                int64_t ref_stride, int64_t pop_size, const float* u, int64_t n_sample, float* out, void* ws,
+                                size_t ws_bytes, void* stream) {
+  const size_t need = evox_hip_hype_workspace_bytes(n, m, n_sample);
+  if (need == 0 || f == nullptr || ref == nullptr || u == nullptr || out == nullptr || pop_size < 1) return kErrBadArg;
+  if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0) return kErrWorkspace;
+  hipStream_t s = (hipStream_t)stream;
+  const HvBytes b = hv_bytes(n, m, n_sample);
+  uint8_t* at = static_cast<uint8_t*>(ws);
+  float* packed = reinterpret_cast<float*>(at);
+  float* partial = reinterpret_cast<float*>(at += b.packed);
+  float* alpha = reinterpret_cast<float*>(at += b.partial);
+  float* points = reinterpret_cast<float*>(at += b.alpha);
+  float* extreme = reinterpret_cast<float*>(at += b.points);
+  const int parts = hv_parts(n);
+  hipLaunchKernelGGL(hv_points_kernel<false>, dim3((unsigned)parts + 1), dim3(256), 0, s, f, stride_row, stride_col, ref, ref_stride,
+                     (int)n, (int)m, parts, points, extreme, alpha, pop_size);
   EVX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(hv_sample_weight_kernel, dim3(sample_blocks), dim3(256), 0, s, cover, alpha, point_chunks, (int)n_sample,
-                     weight);
-  EVX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(hv_point_partial_kernel, dim3(point_blocks, (unsigned)sample_chunks), dim3(256), 0, s, fit_t, samples_t, weight,
-                     (int)n, (int)m, (int)n_sample, sample_chunk, partial);
-  EVX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(hv_point_total_kernel, dim3(point_blocks), dim3(256), 0, s, partial, (int)n, sample_chunks, scale, out);
-  EVX_LAUNCH_CHECK();
-  return 0;
+  const HvSamples samples = {u, m, 1, extreme, ref, ref_stride, parts};
+  return hv_contribution_launches<kHvHype>(points, samples, alpha, n, m, n_sample, 1.0f, packed, partial, out, s);
 }
 
 size_t evox_hip_hv_covered_workspace_bytes(int64_t n_sample) {
@@ -2858,25 +2948,46 @@ size_t evox_hip_hv_covered_workspace_bytes(int64_t n_sample) {
 
 int evox_hip_hv_covered_count(const float* points_t, const float* samples_t, int64_t n, int64_t m, int64_t n_sample,
                               int64_t* out_count, void* ws, size_t ws_bytes, void* stream) {
-  if (points_t == nullptr || samples_t == nullptr || out_count == nullptr || n < 1 || n > 0x7FFFFF00ll || m < 1 || m > 65535)
+  if (points_t == nullptr || samples_t == nullptr || out_count == nullptr || n < 1 || n > 65535ll * 1024 || m < 1 || m > 65535)
     return kErrBadArg;
   const size_t need = evox_hip_hv_covered_workspace_bytes(n_sample);
   if (need == 0) return kErrBadArg;
   if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0) return kErrWorkspace;
-  const int64_t point_chunks = (n + kHvCoverChunk - 1) / kHvCoverChunk;
-  if (point_chunks > 65535) return kErrBadArg;
   hipStream_t s = (hipStream_t)stream;
-  uint32_t* flag = static_cast<uint32_t*>(ws);
-  hipLaunchKernelGGL(reset_state_kernel, dim3(64), dim3(256), 0, s, flag, n_sample);
+  uint32_t* counts = static_cast<uint32_t*>(ws);
+  const HvSamples samples = {samples_t, 1, n_sample, nullptr, nullptr, 0, 0};
+  if (int e = hv_covered_launch<kHvPlain>(points_t, samples, n, m, n_sample, counts, s)) return e;
+  hipLaunchKernelGGL(hv_covered_total_kernel<false>, dim3(1), dim3(1024), 0, s, counts, (int)((n_sample + 63) / 64), samples, (int)m,
+                     (int)n_sample, out_count, (float*)nullptr);
   EVX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(reset_state_kernel, dim3(1), dim3(64), 0, s, reinterpret_cast<uint32_t*>(out_count), (int64_t)2);
+  return 0;
+}
+
+size_t evox_hip_hv_estimate_workspace_bytes(int64_t n, int64_t m, int64_t n_sample) {
+  if (!hv_sizes_fit(n, n_sample) || m < 1 || m > kHvRegs) return 0;
+  const HvBytes b = hv_bytes(n, m, n_sample);
+  return b.points + b.extreme + b.counts;
+}
+
+int evox_hip_hv_estimate(const float* objs, int64_t stride_row, int64_t stride_col, int64_t n, int64_t m, const float* ref,
+                         int64_t ref_stride, const float* u, int64_t n_sample, float* out, void* ws, size_t ws_bytes, void* stream) {
+  const size_t need = evox_hip_hv_estimate_workspace_bytes(n, m, n_sample);
+  if (need == 0 || objs == nullptr || ref == nullptr || u == nullptr || out == nullptr) return kErrBadArg;
+  if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0) return kErrWorkspace;
+  hipStream_t s = (hipStream_t)stream;
+  const HvBytes b = hv_bytes(n, m, n_sample);
+  uint8_t* at = static_cast<uint8_t*>(ws);
+  float* points = reinterpret_cast<float*>(at);
+  float* extreme = reinterpret_cast<float*>(at += b.points);
+  uint32_t* counts = reinterpret_cast<uint32_t*>(at += b.extreme);
+  const int parts = hv_parts(n);
+  hipLaunchKernelGGL(hv_points_kernel<true>, dim3((unsigned)parts), dim3(256), 0, s, objs, stride_row, stride_col, ref, ref_stride,
+                     (int)n, (int)m, parts, points, extreme, (float*)nullptr, (int64_t)0);
   EVX_LAUNCH_CHECK();
-  const unsigned sample_blocks = (unsigned)((n_sample + 255) / 256);
-  hipLaunchKernelGGL(hv_covered_kernel, dim3(sample_blocks, (unsigned)point_chunks), dim3(256), 0, s, points_t, samples_t, (int)n,
-                     (int)m, (int)n_sample, flag);
-  EVX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(hv_covered_total_kernel, dim3(sample_blocks < 64u ? sample_blocks : 64u), dim3(256), 0, s, flag, (int)n_sample,
-                     reinterpret_cast<unsigned long long*>(out_count));
+  const HvSamples samples = {u, m, 1, extreme, ref, ref_stride, parts};
+  if (int e = hv_covered_launch<kHvMetric>(points, samples, n, m, n_sample, counts, s)) return e;
+  hipLaunchKernelGGL(hv_covered_total_kernel<true>, dim3(1), dim3(1024), 0, s, counts, (int)((n_sample + 63) / 64), samples, (int)m,
+                     (int)n_sample, (int64_t*)nullptr, out);
   EVX_LAUNCH_CHECK();
   return 0;
 }

@@ -14,6 +14,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
+from torch.autograd import forward_ad
 from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import _lib, runtime
@@ -813,6 +814,44 @@ def _hv_covered_count_vmap(info, in_dims, points, samples):
 
 
 torch.library.register_vmap(hv_covered_count, _hv_covered_count_vmap)
+
+
+_HV_OBJECTIVES = 16  # most objectives of the whole-call hypervolume kernels
+
+
+def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> bool:
+    """Whether a whole hypervolume estimate runs in the library (hv_estimate, hype_contributions): plain float32 tensors
+    under a float32 default, no derivative asked for and nothing looking at the call; every other call goes through the
+    reference's statements around the operators above, which trace, batch and differentiate."""
+    return (type(points) is torch.Tensor and type(ref) is torch.Tensor and plain_eager() and points.is_cuda and ref.device == points.device
+            and points.dtype is torch.float32 and ref.dtype is torch.float32 and points.dim() == 2 and points.size(0) > 0
+            and 1 <= points.size(1) <= _HV_OBJECTIVES and ref.shape == points.shape[1:] and type(n_sample) is int and n_sample > 0
+            and not points.requires_grad and not ref.requires_grad and torch.get_default_dtype() is torch.float32
+            and forward_ad._current_level < 0)
+
+
+def _hv_whole_call(bytes_query: str, entry: str, points: torch.Tensor, ref: torch.Tensor, extra: tuple, u: torch.Tensor, out: torch.Tensor):
+    n, m = points.shape
+    u = u.contiguous()
+    n_sample = u.size(0)
+    need = int(getattr(_lib.lib(), bytes_query)(n, m, n_sample))
+    with torch.cuda.device(points.device):
+        ws = torch.empty(need, dtype=torch.uint8, device=points.device)
+        _lib.call(entry, points.data_ptr(), points.stride(0), points.stride(1), n, m, ref.data_ptr(), ref.stride(0), *extra, u.data_ptr(),
+                  n_sample, out.data_ptr(), ws.data_ptr(), need, runtime.stream_handle(points.device))
+    return out
+
+
+def hv_estimate(objs: torch.Tensor, ref: torch.Tensor, u: torch.Tensor) -> torch.Tensor:
+    """The hypervolume metric of objs (N, M) and ref (M,) with the random numbers u (S, M), where hv_whole_call_fits."""
+    out = torch.empty((), dtype=torch.float32, device=objs.device)
+    return _hv_whole_call("evox_hip_hv_estimate_workspace_bytes", "evox_hip_hv_estimate", objs, ref, (), u, out)
+
+
+def hype_contributions(fit: torch.Tensor, ref: torch.Tensor, pop_size: int, u: torch.Tensor) -> torch.Tensor:
+    """HypE's contributions of fit (N, M) with the random numbers u (S, M), where hv_whole_call_fits."""
+    out = torch.empty(fit.size(0), dtype=torch.float32, device=fit.device)
+    return _hv_whole_call("evox_hip_hype_workspace_bytes", "evox_hip_hype_contributions", fit, ref, (pop_size,), u, out)
 
 
 @torch.library.custom_op("evox_amd::tournament_pick", mutates_args=())

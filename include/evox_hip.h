@@ -294,6 +294,15 @@ int evox_hip_hv_contributions(const float* fit_t, const float* samples_t, const 
                               int64_t n_sample, float scale, float* out, void* workspace, size_t workspace_bytes,
                               void* stream);
 
+/* The whole of cal_hv (hype.py:12-39) for up to 16 objectives, given its random numbers: u is (n_sample, m) uniform in
+ * [0, 1), row-major; the samples are u * (ref - f_min) + f_min with f_min the smallest of each objective (:26-28), the weights
+ * those of pop_size >= 1 points to be kept (:14-24).  f[i][k] at i * stride_row + k * stride_col, ref[k] at k * ref_stride
+ * (elements).  Workspace: evox_hip_hype_workspace_bytes (0: sizes that are not taken). */
+size_t evox_hip_hype_workspace_bytes(int64_t n, int64_t m, int64_t n_sample);
+int evox_hip_hype_contributions(const float* f, int64_t stride_row, int64_t stride_col, int64_t n, int64_t m, const float* ref,
+                                int64_t ref_stride, int64_t pop_size, const float* u, int64_t n_sample, float* out,
+                                void* workspace, size_t workspace_bytes, void* stream);
+
 /* Monte-Carlo hypervolume metric (src/evox/metrics/hv.py:18, the sample-against-points test after the samples
  * are drawn): out_count[0] = the number of samples s with some point i strictly greater in every objective
  * (all_k samples[s,k] < points[i,k]; a NaN on either side compares false).  points_t is (m, n) row-major,
@@ -302,6 +311,14 @@ int evox_hip_hv_contributions(const float* fit_t, const float* samples_t, const 
 size_t evox_hip_hv_covered_workspace_bytes(int64_t n_sample);
 int evox_hip_hv_covered_count(const float* points_t, const float* samples_t, int64_t n, int64_t m, int64_t n_sample,
                               int64_t* out_count, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The whole of hv (hv.py:13-20) for up to 16 objectives, given its random numbers: u is (n_sample, m) uniform in [0, 1),
+ * row-major; the points are |objs - ref|, the samples u * bound with bound the largest of each objective, out[0] =
+ * covered / n_sample * prod(bound).  Strides in elements as above.  Workspace: evox_hip_hv_estimate_workspace_bytes. */
+size_t evox_hip_hv_estimate_workspace_bytes(int64_t n, int64_t m, int64_t n_sample);
+int evox_hip_hv_estimate(const float* objs, int64_t stride_row, int64_t stride_col, int64_t n, int64_t m, const float* ref,
+                         int64_t ref_stride, const float* u, int64_t n_sample, float* out, void* workspace,
+                         size_t workspace_bytes, void* stream);
 
 /* No counterpart in the reference: launches `blocks` workgroups of 256 threads that issue, `iterations` times,
  * 16 independent v_add_f32 (kind 0), 16 independent v_cmp_le_f32 with SGPR results (kind 1), twice the

@@ -1,0 +1,78 @@
+"""The hypervolume functions as whole calls in the library against the same functions around the operators, at the edges of
+their kernels: eights of points, workgroups of 64 samples, shares and tiles of samples, objectives held in registers, the
+number of samples from which fewer waves share the points, strided inputs, values that are not finite."""
+
+import pytest
+import torch
+
+from evox_amd import hype, ops
+from evox_amd.metrics import hv
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+SIZES = [
+    (1, 1, 1), (2, 3, 63), (7, 3, 64), (8, 2, 65), (9, 4, 127), (64, 5, 128), (65, 6, 129), (255, 7, 1000), (257, 8, 1025),
+    (300, 9, 4097), (1000, 16, 2000), (2000, 3, 10000), (5003, 3, 20001), (130, 3, 65536), (1001, 3, 65537), (20000, 2, 300),
+]
+
+
+def _both(monkeypatch, call):
+    out = []
+    for whole in (True, False):
+        with monkeypatch.context() as patch:
+            if not whole:
+                patch.setattr(ops, "hv_whole_call_fits", lambda *a: False)
+            torch.manual_seed(5)
+            with torch.device(DEV):
+                out.append(call())
+    return out
+
+
+def _close(got, want, rtol):
+    assert got.shape == want.shape and got.dtype == want.dtype and got.device == want.device
+    assert torch.allclose(got, want, rtol=rtol, atol=0.0, equal_nan=True), (got, want)
+
+
+@pytest.mark.parametrize("n, m, n_sample", SIZES)
+def test_whole_calls_match_the_operators(monkeypatch, n, m, n_sample):
+    g = torch.Generator().manual_seed(n + m)
+    wide = torch.rand(n, 2 * m, generator=g).to(DEV)
+    for objs in (wide[:, :m].contiguous(), wide[:, ::2], wide[:, :m].t().contiguous().t()):
+        ref = (objs.max(dim=0).values * 1.1)
+        assert ops.hv_whole_call_fits(objs, ref, n_sample)
+        # the counts are equal; the quotient and the product of m sides are rounded m + 1 times on either side
+        _close(*_both(monkeypatch, lambda: hv(objs, ref, n_sample)), rtol=2 * (m + 1) * 2.0**-24)
+        # the sums have one order; a weight is a product of up to n rounded quotients on the operators' side
+        _close(*_both(monkeypatch, lambda: hype.cal_hv(objs, ref, max(1, n // 2), n_sample)), rtol=(2 * n + 2 * m + 8) * 2.0**-24)
+
+
+def test_values_that_are_not_finite(monkeypatch):
+    base = torch.rand(200, 3, generator=torch.Generator().manual_seed(3)).to(DEV)
+    ref = torch.full((3,), 1.2, device=DEV)
+    for value in (float("nan"), float("inf"), -float("inf")):
+        objs = base.clone()
+        objs[17, 1] = value
+        _close(*_both(monkeypatch, lambda: hv(objs, ref, 3000)), rtol=1e-6)
+        _close(*_both(monkeypatch, lambda: hype.cal_hv(objs, ref, 100, 3000)), rtol=4e-5)
+
+
+def test_calls_that_keep_to_the_operators():
+    objs, ref = torch.rand(20, 3, device=DEV), torch.ones(3, device=DEV)
+    assert ops.hv_whole_call_fits(objs, ref, 100)
+    assert not ops.hv_whole_call_fits(objs.double(), ref, 100)
+    assert not ops.hv_whole_call_fits(objs.clone().requires_grad_(), ref, 100)
+    assert not ops.hv_whole_call_fits(objs, ref[:1], 100)
+    assert not ops.hv_whole_call_fits(objs[:0], ref, 100)
+    assert not ops.hv_whole_call_fits(torch.rand(20, 17, device=DEV), torch.ones(17, device=DEV), 100)
+    seen = []
+    torch.vmap(lambda f: seen.append(ops.hv_whole_call_fits(f, ref, 100)) or f)(objs.view(2, 10, 3))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(ops.hv_whole_call_fits(objs, ref, 100))
+    assert seen == [False, False]
+    # a gradient still reaches the points (through the volume of the box)
+    leaf = objs.clone().requires_grad_()
+    torch.manual_seed(2)
+    with torch.device(DEV):
+        hv(leaf, ref, 1000).backward()
+    assert float(leaf.grad.abs().sum()) > 0.0
