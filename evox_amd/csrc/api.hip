@@ -2532,6 +2532,14 @@ int evox_hip_many_nd_environmental_selection(const void* x, int64_t x_row_bytes,
 
 }  // extern "C"
 
+// Parts of a sorted row of n values in dense_rank_kernel, `rows` rows in the launch: as many as there are compute units
+// for each row, none smaller than one value per thread.  Every part reads all values before it, so more parts than
+// compute units would only add reads.
+static int dense_rank_parts(int64_t rows, int64_t n) {
+  const int64_t most = (n + kDenseRankThreads - 1) / kDenseRankThreads, share = device_cus() / rows;
+  return (int)(share < 1 ? 1 : share < most ? share : most);
+}
+
 extern "C" {
 
 int evox_hip_dense_rank_rows(const void* sorted, int kind, const int64_t* index, int64_t batch, int64_t n, int64_t m, float* out,
@@ -2539,12 +2547,15 @@ int evox_hip_dense_rank_rows(const void* sorted, int kind, const int64_t* index,
   if (sorted == nullptr || index == nullptr || out == nullptr || (kind != kWideFloat64 && kind != kWideInt64)) return kErrBadArg;
   if (batch < 1 || n < 1 || m < 1 || n >= (1ll << 24) || batch * m > 0x7FFFFFFFll) return kErrBadArg;
   hipStream_t s = (hipStream_t)stream;
+  const int parts = dense_rank_parts(batch * m, n);
+  const int per = (int)round_up((n + parts - 1) / parts, kDenseRankThreads);
+  const dim3 grid((unsigned)(batch * m), (unsigned)((n + per - 1) / per));
   if (kind == kWideFloat64)
-    hipLaunchKernelGGL(dense_rank_kernel<double>, dim3((unsigned)(batch * m)), dim3(kDenseRankThreads), 0, s,
-                       static_cast<const double*>(sorted), index, (int)n, (int)m, out);
+    hipLaunchKernelGGL(dense_rank_kernel<double>, grid, dim3(kDenseRankThreads), 0, s, static_cast<const double*>(sorted), index,
+                       (int)n, (int)m, per, out);
   else
-    hipLaunchKernelGGL(dense_rank_kernel<long long>, dim3((unsigned)(batch * m)), dim3(kDenseRankThreads), 0, s,
-                       static_cast<const long long*>(sorted), index, (int)n, (int)m, out);
+    hipLaunchKernelGGL(dense_rank_kernel<long long>, grid, dim3(kDenseRankThreads), 0, s, static_cast<const long long*>(sorted), index,
+                       (int)n, (int)m, per, out);
   EVX_LAUNCH_CHECK();
   return 0;
 }

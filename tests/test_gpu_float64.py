@@ -227,6 +227,27 @@ def test_dense_rank_image(dtype):
                 assert np.array_equal(got.reshape(cols.shape)[b][:, k], want, equal_nan=True), (shape, b, k)
 
 
+@pytest.mark.parametrize("shape", [(1023, 1), (1024, 2), (1025, 3), (4096, 1), (20001, 3), (300000, 2), (300, 1500, 1), (100, 3000, 2), (7, 5001, 3)])
+def test_dense_rank_parts(shape):
+    """The same image where a sorted row is one part, one part per workgroup of values and a remainder, parts of several
+    passes, and where rows outnumber the compute units: runs of equal values across the ends of parts, NaN at the end."""
+    from evox_amd import ops
+
+    g = torch.Generator("cpu").manual_seed(71)
+    f = torch.rand(*shape, generator=g, dtype=torch.float64)
+    f.view(-1)[::2] = (f.view(-1)[::2] * 9).round() / 9 - 0.5  # long runs, among them -0.0
+    f.view(-1)[5::701] = float("nan")
+    got = ops._order_preserving_f32(f.to(DEV), "fitness").cpu()
+    cols = f.reshape(-1, *shape[-2:])
+    for b in range(cols.size(0)):
+        for k in range(shape[-1]):
+            col = cols[b, :, k]
+            ok = ~torch.isnan(col)
+            want = torch.full(col.shape, float("nan"))
+            want[ok] = torch.unique(col[ok] + 0.0, return_inverse=True)[1].float()
+            assert torch.equal(got.reshape(cols.shape)[b, :, k].nan_to_num(-1.0), want.nan_to_num(-1.0)), (shape, b, k)
+
+
 def test_batches_of_8_byte_fitness_share_their_launches(float64_default):
     """Several populations of float64 or int64 fitness in one call: the same as one population at a time."""
     g = torch.Generator("cpu").manual_seed(70)
