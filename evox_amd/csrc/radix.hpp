@@ -368,6 +368,7 @@ constexpr int kMidArgsortThreads = 1024;
 // of 1536 (28 KB), so that 32768 keys still fit beside them (20 000 keys: 15 us slower with the small tables).
 constexpr int kMidArgsortWideRows = 24576;
 constexpr int kMidArgsortIndexBits = 15;
+constexpr uint32_t kMidArgsortLast = 0xFFFFFFFFu;
 
 // Exclusive scan, in place, of the BUCKETS counts in `hist` by the whole workgroup; returns their sum.
 template <int BUCKETS>
@@ -446,7 +447,8 @@ __device__ inline MidSortLds mid_sort_lds(void* lds) {  // (16-byte aligned)
 // position e (read once), emit(slot, e) = position e belongs in `slot`.  The keys go into BUCKETS buckets
 // by value; the buckets that hold the wanted slots are collected (a bucket too large for the list is cut into buckets
 // of its own range first) and their members placed by counting.  Every thread of the workgroup calls it.
-template <int BUCKETS, int LIST, int TRACE, class KeyOf, class Emit>
+// LAST: thousands of positions may hold the largest image there is (below).
+template <int BUCKETS, int LIST, int TRACE, bool LAST, class KeyOf, class Emit>
 __device__ inline void mid_argsort_slice_sized(void* lds, int n, int s0, int s1_wanted, KeyOf key_of, Emit emit) {
   constexpr int kMidArgsortBuckets = BUCKETS, kMidArgsortList = LIST;
   const MidSortLds T = mid_sort_lds<BUCKETS, LIST>(lds);
@@ -465,7 +467,7 @@ __device__ inline void mid_argsort_slice_sized(void* lds, int n, int s0, int s1_
     const uint32_t k = key_of(e);
     mid_keys[e] = k;
     kmin = k < kmin ? k : kmin;
-    kmax = k > kmax ? k : kmax;
+    kmax = k > kmax && (!LAST || k != kMidArgsortLast) ? k : kmax;
   }
   EVX_TRACE(TRACE, 0);
   for (int b = tid; b < kMidArgsortBuckets; b += kMidArgsortThreads) top_hist[b] = 0;
@@ -487,6 +489,17 @@ __device__ inline void mid_argsort_slice_sized(void* lds, int n, int s0, int s1_
     kmin = T.red[w] < kmin ? T.red[w] : kmin;
     kmax = T.red[kWaves + w] > kmax ? T.red[kWaves + w] : kmax;
   }
+  // The largest image there is (the rank of the rows behind a cut: thousands of them) moves next to the largest other
+  // one: left where it is, all ranks that a selection wants shared the lowest of the buckets, and every workgroup had to
+  // cut that one up (20 000 ranks, half of them behind the cut: 74 us, 31 with this).  Equal keys stay
+  // equal and the order stays the order; where no other image is, all keys are equal as they are.  The sorts of crowding
+  // distances and objectives, which meet no such crowd, go without (the look at every key cost a front of 20 001 rows
+  // 2.6 us).
+  uint32_t last = kMidArgsortLast;
+  if constexpr (LAST) {
+    if (kmin != kMidArgsortLast) last = kmax + 1u;  // (kmax < kMidArgsortLast here: no overflow)
+    kmax = last;
+  }
   auto composite = [&](int e) { return ((unsigned long long)mid_keys[e] << kMidArgsortIndexBits) | (unsigned long long)e; };
   auto shift_for = [](unsigned long long span) {
     int shift = 0;
@@ -496,7 +509,12 @@ __device__ inline void mid_argsort_slice_sized(void* lds, int n, int s0, int s1_
   const unsigned long long top_lo = (unsigned long long)kmin << kMidArgsortIndexBits;
   const unsigned long long top_hi = ((unsigned long long)kmax << kMidArgsortIndexBits) | kIndexMask;
   const int top_shift = shift_for(top_hi - top_lo);
-  for (int e = tid; e < n; e += kMidArgsortThreads) atomicAdd(&top_hist[(int)((composite(e) - top_lo) >> top_shift)], 1);
+  for (int e = tid; e < n; e += kMidArgsortThreads) {  // (the positions whose keys this thread stored above)
+    if constexpr (LAST) {
+      if (mid_keys[e] == kMidArgsortLast) mid_keys[e] = last;
+    }
+    atomicAdd(&top_hist[(int)((composite(e) - top_lo) >> top_shift)], 1);
+  }
   __syncthreads();
   mid_argsort_scan<BUCKETS>(top_hist, wave_tot);  // (the total is n)
   EVX_TRACE(TRACE, 1);
@@ -639,12 +657,12 @@ __device__ inline void mid_argsort_slice_sized(void* lds, int n, int s0, int s1_
 
 // WIDE: the large tables (at most kMidArgsortWideRows keys).  `lds` = mid_sort_lds_bytes(most keys the launch may
 // meet) bytes, 16-byte aligned: the host picks WIDE by that number, so that a kernel holds one size of the code.
-template <bool WIDE, int TRACE = 51, class KeyOf, class Emit>
+template <bool WIDE, int TRACE = 51, bool LAST = false, class KeyOf, class Emit>
 __device__ inline void mid_argsort_slice(void* lds, int n, int s0, int s1_wanted, KeyOf key_of, Emit emit) {
   if constexpr (WIDE)
-    mid_argsort_slice_sized<4096, 2048, TRACE>(lds, n, s0, s1_wanted, key_of, emit);
+    mid_argsort_slice_sized<4096, 2048, TRACE, LAST>(lds, n, s0, s1_wanted, key_of, emit);
   else
-    mid_argsort_slice_sized<2048, 1536, TRACE>(lds, n, s0, s1_wanted, key_of, emit);
+    mid_argsort_slice_sized<2048, 1536, TRACE, LAST>(lds, n, s0, s1_wanted, key_of, emit);
 }
 
 // One step of a lexsort of n <= kMidArgsortRows positions: a workgroup per `slots_per_block` slots of the order.
@@ -666,7 +684,8 @@ __global__ __launch_bounds__(kMidArgsortThreads) void mid_argsort_kernel(const v
     return static_cast<const uint32_t*>(key)[(int64_t)idx * stride];
   };
   const int s0 = (int)blockIdx.x * slots_per_block;
-  mid_argsort_slice<WIDE>(mid_lds, n, s0, s0 + slots_per_block, key_of, [&](int slot, int e) { order_out[slot] = prev ? prev[e] : e; });
+  mid_argsort_slice<WIDE, 51, true>(mid_lds, n, s0, s0 + slots_per_block, key_of,
+                                    [&](int slot, int e) { order_out[slot] = prev ? prev[e] : e; });
 }
 
 // Many independent steps at once: `batch` sorts of n <= kSmallArgsortRows positions each, sort b reading
