@@ -11,6 +11,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "deal.hpp"
 #include "order.hpp"
 
 namespace evx {
@@ -754,20 +755,14 @@ __global__ __launch_bounds__(64 * kFrontWaves) void first_front_leaf_kernel(
   }
   if (__syncthreads_or(few)) {
     // (a wave that left early has not asked its share of the leaves: what is open now is open to the whole workgroup)
-    const uint64_t still = rows & ~decided;
-    int turn_row = wave;
-    for (uint64_t todo = still; todo != 0ull; todo &= todo - 1) {
-      if (turn_row != 0) {
-        --turn_row;
-        continue;
-      }
-      turn_row = kFrontWaves - 1;
-      const int r = __ffsll((unsigned long long)todo) - 1;
-      float x[M];
+    deal_open_rows(
+        wave, kFrontWaves, [&] { return rows & ~decided; }, [] { __syncthreads(); },
+        [&](int r) {
+          float x[M];
 #pragma unroll
-      for (int k = 0; k < M; ++k) x[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(xj[k]), r));
-      if (front_row_beaten<M>(x, last, xs, npad, leaf_stride, group_stride, leaf_lo, group_lo) && lane == 0) atomicOr(&decided, 1ull << r);
-    }
+          for (int k = 0; k < M; ++k) x[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(xj[k]), r));
+          if (front_row_beaten<M>(x, last, xs, npad, leaf_stride, group_stride, leaf_lo, group_lo) && lane == 0) atomicOr(&decided, 1ull << r);
+        });
     __syncthreads();
   }
   if (wave == 0 && j < n && ((decided >> lane) & 1ull) != 0ull) mask[left_of[slot_row[j]]] = 0;

@@ -51,3 +51,19 @@ def test_masks_of_several_large_populations():
     got = non_dominated_mask(f.to("cuda")).cpu().numpy()
     for b in range(3):
         assert np.array_equal(got[b], c_oracle.first_front(f[b].numpy())), b
+
+
+@pytest.mark.parametrize("n,m", [(120001, 2), (120001, 3), (90001, 4), (70003, 5)])
+def test_rows_that_a_leaf_asks_one_by_one(n, m):
+    """Three rows in four are slightly worse copies of a row of the front, by steps from below a leaf's extent to well above
+    it: after a leaf's nearest neighbours a few of its rows are open, some of which only a distant row dominates."""
+    from evox_amd.operators.selection import non_dominated_mask
+
+    g = torch.Generator("cpu").manual_seed(n + m)
+    f = population("one front", n, m, n - m)
+    copies = n * 3 // 4
+    step = 10.0 ** (-5.5 + 4.0 * torch.rand(copies, 1, generator=g))
+    f[:copies] = f[torch.randint(copies, n, (copies,), generator=g)] + step * torch.rand(copies, m, generator=g)
+    f = f[torch.randperm(n, generator=g)]
+    got = non_dominated_mask(f.to("cuda")).cpu().numpy()
+    assert np.array_equal(got, c_oracle.first_front(f.numpy()))
