@@ -17,9 +17,9 @@ def _plain(op, *tensors):
     """``op`` itself, or -- for plain tensors with no transform, tracer or dispatch mode looking at the call
     (``ops.plain_eager``) -- the function that the custom operator wraps: what the operator would run after four
     layers of dispatch, a fifth of the time of a selection of 200 rows.  Tensor subclasses (fake tensors, functional
-    wrappers) and tensors that require a gradient keep to the operator."""
+    wrappers), tensors that require a gradient and views with a negative or conjugate bit keep to the operator."""
     for t in tensors:
-        if type(t) is not torch.Tensor or t.requires_grad:
+        if type(t) is not torch.Tensor or t.requires_grad or not ops.holds_its_values(t):
             return op
     return getattr(op, "_init_fn", op) if ops.plain_eager() else op  # (another torch may not keep it there: the operator then)
 

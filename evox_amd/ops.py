@@ -827,7 +827,7 @@ def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> boo
             and points.dtype is torch.float32 and ref.dtype is torch.float32 and points.dim() == 2 and points.size(0) > 0
             and 1 <= points.size(1) <= _HV_OBJECTIVES and ref.shape == points.shape[1:] and type(n_sample) is int and n_sample > 0
             and not points.requires_grad and not ref.requires_grad and torch.get_default_dtype() is torch.float32
-            and forward_ad._current_level < 0)
+            and forward_ad._current_level < 0 and holds_its_values(points) and holds_its_values(ref))
 
 
 def _hv_whole_call(bytes_query: str, entry: str, points: torch.Tensor, ref: torch.Tensor, extra: tuple, u: torch.Tensor, out: torch.Tensor):
@@ -908,6 +908,12 @@ def plain_eager() -> bool:
                 and _get_current_dispatch_mode() is None)
     except AttributeError:  # another torch: take the dispatcher
         return False
+
+
+def holds_its_values(t: torch.Tensor) -> bool:
+    """False for a view whose memory holds other bytes than its values (a negative or conjugate bit: ``z.conj().imag``).
+    The dispatcher resolves such a tensor before an operator sees it; a function called past it reads the memory as it is."""
+    return not (t.is_neg() or t.is_conj())
 
 
 def tournament_pick_keys_direct(parents: torch.Tensor, keys: List[torch.Tensor]) -> torch.Tensor:
