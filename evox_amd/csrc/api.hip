@@ -2844,9 +2844,9 @@ static bool hv_sizes_fit(int64_t n, int64_t n_sample) { return n >= 1 && n_sampl
 
 // Waves that share the points of 64 samples: sixteen until the samples alone bring more than the device holds at a time
 // (1024 workgroups), then four (1001 x 3 against 100 000 samples: see hv.hpp).  Never more than there are steps over the points.
-static unsigned hv_threads(int64_t n, int64_t n_sample) {
+static unsigned hv_threads(int64_t n, int64_t m, int64_t n_sample) {
   int64_t waves = n_sample > (1ll << 28) ? 1 : (n_sample > 65536 ? 4 : 16);  // (a grid has less than 2^32 threads)
-  const int64_t steps = (n + kHvStep - 1) / kHvStep;
+  const int64_t steps = (n + hv_step((int)m) - 1) / hv_step((int)m);
   if (waves > steps) waves = steps;
   return (unsigned)(64 * waves);
 }
@@ -2876,7 +2876,7 @@ static int hv_contribution_launches(const float* points_t, const HvSamples& samp
   const int shares = (int)((n_sample + share - 1) / share);
   if (int e = hv_for_objectives(m, [&](auto objectives) {
         constexpr int M = decltype(objectives)::value;
-        hipLaunchKernelGGL((hv_sample_weight_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, n_sample)), 0,
+        hipLaunchKernelGGL((hv_sample_weight_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, m, n_sample)), 0,
                            s, points_t, samples, (int)n, (int)m, (int)n_sample, alpha, packed);
         EVX_LAUNCH_CHECK();
         hipLaunchKernelGGL(hv_point_partial_kernel<M>, dim3((unsigned)((n + 255) / 256), (unsigned)shares), dim3(256), 0, s, points_t,
@@ -2896,7 +2896,7 @@ static int hv_covered_launch(const float* points_t, const HvSamples& samples, in
                              uint32_t* counts, hipStream_t s) {
   return hv_for_objectives(m, [&](auto objectives) {
     constexpr int M = decltype(objectives)::value;
-    hipLaunchKernelGGL((hv_covered_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, n_sample)), 0, s,
+    hipLaunchKernelGGL((hv_covered_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, m, n_sample)), 0, s,
                        points_t, samples, (int)n, (int)m, (int)n_sample, counts);
     EVX_LAUNCH_CHECK();
     return 0;

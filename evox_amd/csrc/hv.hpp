@@ -11,7 +11,7 @@
 // Bound by vector issue: a test costs M compares, and a few thousand points against a hundred thousand samples are
 // 10^8 tests, some 5 us of the device.  What the kernels have to see to is that enough waves are there to hide the
 // loads of the other side.  Whether a sample is covered, and by how many points, is decided by ONE workgroup that holds 64
-// samples, one to a lane, in each of its waves; the waves take the points in turn, kHvStep at a time, as scalar operands.
+// samples, one to a lane, in each of its waves; the waves take the points in turn, hv_step at a time, as scalar operands.
 // (A wave that took all the points of its samples was alone with the latency of every scalar load: 129 us for 1001 x 3
 // against 100 000 samples, 27 us this way; counts and weights of 2000 x 3 against 10 000, 25 us before, 15 now.)  The sums
 // over the samples have the points in the lanes and read the samples, packed with their weights, from LDS, eight reads in
@@ -28,8 +28,12 @@ constexpr int kHvParts = 64;         // workgroups that look for the box of the 
 constexpr int kHvRegs = 16;          // objectives held in registers; more are re-read from memory
 constexpr int kHvPacked = 20;        // floats per packed sample, at most (16 objectives, the weight, whole 16-byte pieces)
 constexpr int kHvAlphaShare = 14;    // weights that one thread computes in ascending order, at least
-constexpr int kHvStep = 16;          // points that a wave takes at a time, as scalar operands
 constexpr int kHvMeet = 32;          // steps after which the waves of a workgroup tell each other what is covered
+
+// Points that a wave takes at a time, as scalar operands.  (A step's values are in registers together: 8 objectives times
+// 16 points no longer fit the 128 registers of a workgroup of 1024 threads, and went through scratch memory: 5000 x 8 against
+// 20 000 samples, 1861 us, 78 with eight points.  From 9 objectives on the values are read objective by objective.)
+constexpr int hv_step(int m) { return m == 8 ? 8 : 16; }
 
 __host__ __device__ constexpr int hv_packed(int m) { return (m + 1 + 3) & ~3; }
 
@@ -161,10 +165,11 @@ __global__ __launch_bounds__(256) void hv_points_kernel(const float* __restrict_
 
 // ---------------------------------------------------------------- HypE's contributions
 
-// The number of points of [0, n) that pass the test against the lane's sample, over the steps of kHvStep points that this
+// The number of points of [0, n) that pass the test against the lane's sample, over the steps of points that this
 // wave takes: wave, wave + waves, ...; of the last step, which is moved back to end with the points, those not yet counted.
 template <int M, bool kFinite>
 __device__ inline int hv_count_points(const float* __restrict__ points_t, int n, int m, const float (&sv)[M], int wave, int waves) {
+  constexpr int kHvStep = hv_step(M);
   int count = 0;
   const int steps = n < kHvStep ? 0 : (n + kHvStep - 1) / kHvStep;
 #pragma unroll 1
@@ -373,6 +378,7 @@ __global__ __launch_bounds__(1024) void hv_covered_kernel(const float* __restric
   __syncthreads();
   bool cov = !live;
   if constexpr (M > 0) {
+    constexpr int kHvStep = hv_step(M);
     float sv[M];
 #pragma unroll
     for (int k = 0; k < M; ++k) {

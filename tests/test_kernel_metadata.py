@@ -74,6 +74,13 @@ def test_the_one_workgroup_kernels_spill_nothing(kernels):
     assert {k[".name"]: k[".private_segment_fixed_size"] for k in small if k[".private_segment_fixed_size"]} == {}
 
 
+def test_the_hypervolume_kernels_have_no_scratch(kernels):
+    """Their loops over the points hold a step of points in registers, for every number of objectives."""
+    hypervolume = [k for k in kernels if "evx" in k[".name"] and "hv_" in k[".name"]]
+    assert len(hypervolume) > 40
+    assert {k[".name"]: k[".private_segment_fixed_size"] for k in hypervolume if k[".private_segment_fixed_size"]} == {}
+
+
 def test_every_kernel_is_built_for_wave64(kernels):
     assert len(kernels) > 100
     assert all(k[".wavefront_size"] == 64 for k in kernels)
