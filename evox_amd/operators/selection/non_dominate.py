@@ -19,7 +19,7 @@ def _plain(op, *tensors):
     layers of dispatch, a fifth of the time of a selection of 200 rows.  Tensor subclasses (fake tensors, functional
     wrappers), tensors that require a gradient and views with a negative or conjugate bit keep to the operator."""
     for t in tensors:
-        if type(t) is not torch.Tensor or t.requires_grad or not ops.holds_its_values(t):
+        if type(t) is not torch.Tensor or t.requires_grad or t.is_neg() or t.is_conj():
             return op
     return getattr(op, "_init_fn", op) if ops.plain_eager() else op  # (another torch may not keep it there: the operator then)
 
