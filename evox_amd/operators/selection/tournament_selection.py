@@ -23,7 +23,7 @@ def tournament_selection_multifit(n_round: int, fitnesses: List[torch.Tensor], t
         # float32 and int32 vectors -- the crowding distances and ranks that NSGA-II passes: read where they lie
         # (the stacked copy with its type promotion is two or three more launches than the tournaments themselves)
         parents = torch.randint(0, fitnesses[0].size(0), (n_round, tournament_size), device=fitnesses[0].device)
-        pick = ops.tournament_pick_keys_direct if ops.plain_eager() and all(map(ops.holds_its_values, fitnesses)) else ops.tournament_pick_keys
+        pick = ops.tournament_pick_keys_direct if ops.plain_eager() and not any(t.is_neg() for t in fitnesses) else ops.tournament_pick_keys
         return pick(parents, list(fitnesses)).squeeze()
     fitness_tensor = torch.stack(fitnesses, dim=1)
     num_candidates = fitness_tensor.size(0)

@@ -823,11 +823,14 @@ def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> boo
     """Whether a whole hypervolume estimate runs in the library (hv_estimate, hype_contributions): plain float32 tensors
     under a float32 default, no derivative asked for and nothing looking at the call; every other call goes through the
     reference's statements around the operators above, which trace, batch and differentiate."""
-    return (type(points) is torch.Tensor and type(ref) is torch.Tensor and plain_eager() and points.is_cuda and ref.device == points.device
-            and points.dtype is torch.float32 and ref.dtype is torch.float32 and points.dim() == 2 and points.size(0) > 0
-            and 1 <= points.size(1) <= _HV_OBJECTIVES and ref.shape == points.shape[1:] and type(n_sample) is int and n_sample > 0
-            and not points.requires_grad and not ref.requires_grad and torch.get_default_dtype() is torch.float32
-            and forward_ad._current_level < 0 and holds_its_values(points) and holds_its_values(ref))
+    if type(points) is not torch.Tensor or type(ref) is not torch.Tensor or not plain_eager():
+        return False
+    shape, device = points.shape, points.device  # (under a default device every look at a tensor costs half a microsecond)
+    return (device.type == "cuda" and ref.device == device and points.dtype is torch.float32 and ref.dtype is torch.float32
+            and len(shape) == 2 and shape[0] > 0 and 1 <= shape[1] <= _HV_OBJECTIVES and ref.shape == shape[1:]
+            and type(n_sample) is int and n_sample > 0 and not points.requires_grad and not ref.requires_grad
+            and torch.get_default_dtype() is torch.float32 and forward_ad._current_level < 0
+            and not points.is_neg() and not ref.is_neg())
 
 
 def _hv_whole_call(bytes_query: str, entry: str, points: torch.Tensor, ref: torch.Tensor, extra: tuple, u: torch.Tensor, out: torch.Tensor):
@@ -902,18 +905,13 @@ def tournament_keys_fit(keys) -> bool:
 def plain_eager() -> bool:
     """True when no transform (vmap, grad), tracer (torch.compile, make_fx) or dispatch mode is looking at the call,
     so that an operator's implementation may be called as the Python function it is: the dispatcher's way to the same
-    function costs about 10 us, a third of a host-bound call like a tournament selection."""
+    function costs about 10 us, a third of a host-bound call like a tournament selection.  It also resolves tensors whose memory
+    holds other bytes than their values (a negative or conjugate bit: ``z.conj().imag``), which a caller must look for itself."""
     try:
         return (not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
                 and _get_current_dispatch_mode() is None)
     except AttributeError:  # another torch: take the dispatcher
         return False
-
-
-def holds_its_values(t: torch.Tensor) -> bool:
-    """False for a view whose memory holds other bytes than its values (a negative or conjugate bit: ``z.conj().imag``).
-    The dispatcher resolves such a tensor before an operator sees it; a function called past it reads the memory as it is."""
-    return not (t.is_neg() or t.is_conj())
 
 
 def tournament_pick_keys_direct(parents: torch.Tensor, keys: List[torch.Tensor]) -> torch.Tensor:
