@@ -2827,7 +2827,7 @@ int evox_hip_tournament_pick_keys(const int64_t* parents, int64_t n_round, int64
 
 // What the two uses of the points against the samples keep in their workspace.
 struct HvBytes {
-  size_t packed, partial, alpha, points, extreme, counts;
+  size_t packed, partial, alpha, points, extreme, covered, cover;
 };
 static HvBytes hv_bytes(int64_t n, int64_t m, int64_t n_sample) {
   HvBytes b;
@@ -2837,19 +2837,11 @@ static HvBytes hv_bytes(int64_t n, int64_t m, int64_t n_sample) {
   b.alpha = align_up(sizeof(float) * (size_t)n);
   b.points = align_up(sizeof(float) * (size_t)n * (size_t)m);
   b.extreme = align_up(sizeof(float) * (size_t)kHvParts * (size_t)m);
-  b.counts = align_up(sizeof(uint32_t) * (size_t)((n_sample + 63) / 64));
+  b.covered = align_up(sizeof(uint64_t) * (size_t)((n_sample + 63) / 64));
+  b.cover = align_up(sizeof(int) * (size_t)n_sample);
   return b;
 }
 static bool hv_sizes_fit(int64_t n, int64_t n_sample) { return n >= 1 && n_sample >= 1 && n <= 0x7FFFFF00ll && n_sample <= 0x7FFFFF00ll; }
-
-// Waves that share the points of 64 samples: sixteen until the samples alone bring more than the device holds at a time
-// (1024 workgroups), then four (1001 x 3 against 100 000 samples: see hv.hpp).  Never more than there are steps over the points.
-static unsigned hv_threads(int64_t n, int64_t m, int64_t n_sample) {
-  int64_t waves = n_sample > (1ll << 28) ? 1 : (n_sample > 65536 ? 4 : 16);  // (a grid has less than 2^32 threads)
-  const int64_t steps = (n + hv_step((int)m) - 1) / hv_step((int)m);
-  if (waves > steps) waves = steps;
-  return (unsigned)(64 * waves);
-}
 
 // The kernels are built for 1 to 8 objectives, for up to kHvRegs (their number read at run time) and for any number.
 template <typename F>
@@ -2869,16 +2861,25 @@ static int hv_for_objectives(int64_t m, F&& launch) {
   return launch(std::integral_constant<int, 0>());
 }
 
+static HvSplit hv_split_for(int64_t n, int64_t m, int64_t n_sample) { return hv_split(n, n_sample, hv_step((int)m), device_cus()); }
+
+// cover: zero where the split has several parts.
 template <int kMode>
 static int hv_contribution_launches(const float* points_t, const HvSamples& samples, const float* alpha, int64_t n, int64_t m,
-                                    int64_t n_sample, float scale, float* packed, float* partial, float* out, hipStream_t s) {
+                                    int64_t n_sample, float scale, const HvSplit& split, float* packed, int* cover, float* partial,
+                                    float* out, hipStream_t s) {
   const int64_t share = hv_share(n_sample);
   const int shares = (int)((n_sample + share - 1) / share);
+  const unsigned blocks = (unsigned)((n_sample + 63) / 64);
   if (int e = hv_for_objectives(m, [&](auto objectives) {
         constexpr int M = decltype(objectives)::value;
-        hipLaunchKernelGGL((hv_sample_weight_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, m, n_sample)), 0,
-                           s, points_t, samples, (int)n, (int)m, (int)n_sample, alpha, packed);
+        hipLaunchKernelGGL((hv_sample_weight_kernel<M, kMode>), dim3(blocks, split.parts), dim3(split.threads), 0, s, points_t, samples,
+                           (int)n, (int)m, (int)n_sample, alpha, packed, cover);
         EVX_LAUNCH_CHECK();
+        if (split.parts > 1) {
+          hipLaunchKernelGGL((hv_weight_kernel<M, kMode>), dim3(blocks), dim3(64), 0, s, samples, (int)m, (int)n_sample, cover, alpha, packed);
+          EVX_LAUNCH_CHECK();
+        }
         hipLaunchKernelGGL(hv_point_partial_kernel<M>, dim3((unsigned)((n + 255) / 256), (unsigned)shares), dim3(256), 0, s, points_t,
                            packed, samples, (int)n, (int)m, (int)n_sample, (int)share, partial);
         EVX_LAUNCH_CHECK();
@@ -2891,16 +2892,24 @@ static int hv_contribution_launches(const float* points_t, const HvSamples& samp
   return 0;
 }
 
+// covered: zero where the split has several parts.
 template <int kMode>
 static int hv_covered_launch(const float* points_t, const HvSamples& samples, int64_t n, int64_t m, int64_t n_sample,
-                             uint32_t* counts, hipStream_t s) {
+                             const HvSplit& split, unsigned long long* covered, hipStream_t s) {
   return hv_for_objectives(m, [&](auto objectives) {
     constexpr int M = decltype(objectives)::value;
-    hipLaunchKernelGGL((hv_covered_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64)), dim3(hv_threads(n, m, n_sample)), 0, s,
-                       points_t, samples, (int)n, (int)m, (int)n_sample, counts);
+    hipLaunchKernelGGL((hv_covered_kernel<M, kMode>), dim3((unsigned)((n_sample + 63) / 64), split.parts), dim3(split.threads), 0, s,
+                       points_t, samples, (int)n, (int)m, (int)n_sample, covered);
     EVX_LAUNCH_CHECK();
     return 0;
   });
+}
+
+static int hv_clear(void* words, int64_t n_words, hipStream_t s) {
+  const int64_t blocks = (n_words + 255) / 256;
+  hipLaunchKernelGGL(reset_state_kernel, dim3((unsigned)(blocks < 64 ? blocks : 64)), dim3(256), 0, s, static_cast<uint32_t*>(words), n_words);
+  EVX_LAUNCH_CHECK();
+  return 0;
 }
 
 extern "C" {
@@ -2908,7 +2917,7 @@ extern "C" {
 size_t evox_hip_hv_workspace_bytes(int64_t n, int64_t n_sample) {
   if (!hv_sizes_fit(n, n_sample)) return 0;
   const HvBytes b = hv_bytes(n, kHvRegs, n_sample);  // (the call's objectives are not known here)
-  return b.packed + b.partial;
+  return b.packed + b.partial + b.cover;
 }
 
 int evox_hip_hv_contributions(const float* fit_t, const float* samples_t, const float* alpha, int64_t n, int64_t m,
@@ -2919,15 +2928,20 @@ int evox_hip_hv_contributions(const float* fit_t, const float* samples_t, const 
   if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0) return kErrWorkspace;
   const HvBytes b = hv_bytes(n, kHvRegs, n_sample);
   uint8_t* base = static_cast<uint8_t*>(ws);
+  int* cover = reinterpret_cast<int*>(base + b.packed + b.partial);
+  const HvSplit split = hv_split_for(n, m, n_sample);
+  if (split.parts > 1) {
+    if (int e = hv_clear(cover, n_sample, (hipStream_t)stream)) return e;
+  }
   const HvSamples samples = {samples_t, 1, n_sample, nullptr, nullptr, 0, 0};
-  return hv_contribution_launches<kHvPlain>(fit_t, samples, alpha, n, m, n_sample, scale, reinterpret_cast<float*>(base),
+  return hv_contribution_launches<kHvPlain>(fit_t, samples, alpha, n, m, n_sample, scale, split, reinterpret_cast<float*>(base), cover,
                                             reinterpret_cast<float*>(base + b.packed), out, (hipStream_t)stream);
 }
 
 size_t evox_hip_hype_workspace_bytes(int64_t n, int64_t m, int64_t n_sample) {
   if (!hv_sizes_fit(n, n_sample) || m < 1 || m > kHvRegs) return 0;
   const HvBytes b = hv_bytes(n, m, n_sample);
-  return b.packed + b.partial + b.alpha + b.points + b.extreme;
+  return b.packed + b.partial + b.alpha + b.points + b.extreme + b.cover;
 }
 
 int evox_hip_hype_contributions(const float* f, int64_t stride_row, int64_t stride_col, int64_t n, int64_t m, const float* ref,
@@ -2944,17 +2958,20 @@ int evox_hip_hype_contributions(const float* f, int64_t stride_row, int64_t stri
   float* alpha = reinterpret_cast<float*>(at += b.partial);
   float* points = reinterpret_cast<float*>(at += b.alpha);
   float* extreme = reinterpret_cast<float*>(at += b.points);
+  int* cover = reinterpret_cast<int*>(at += b.extreme);
   const int parts = hv_parts(n);
+  const HvSplit split = hv_split_for(n, m, n_sample);
   hipLaunchKernelGGL(hv_points_kernel<false>, dim3((unsigned)parts + 1), dim3(256), 0, s, f, stride_row, stride_col, ref, ref_stride,
-                     (int)n, (int)m, parts, points, extreme, alpha, pop_size);
+                     (int)n, (int)m, parts, points, extreme, alpha, pop_size, reinterpret_cast<uint32_t*>(cover),
+                     split.parts > 1 ? n_sample : 0);
   EVX_LAUNCH_CHECK();
   const HvSamples samples = {u, m, 1, extreme, ref, ref_stride, parts};
-  return hv_contribution_launches<kHvHype>(points, samples, alpha, n, m, n_sample, 1.0f, packed, partial, out, s);
+  return hv_contribution_launches<kHvHype>(points, samples, alpha, n, m, n_sample, 1.0f, split, packed, cover, partial, out, s);
 }
 
 size_t evox_hip_hv_covered_workspace_bytes(int64_t n_sample) {
   if (n_sample < 1 || n_sample > 0x7FFFFF00ll) return 0;
-  return align_up(sizeof(uint32_t) * (size_t)n_sample);
+  return hv_bytes(1, 1, n_sample).covered;
 }
 
 int evox_hip_hv_covered_count(const float* points_t, const float* samples_t, int64_t n, int64_t m, int64_t n_sample,
@@ -2965,10 +2982,14 @@ int evox_hip_hv_covered_count(const float* points_t, const float* samples_t, int
   if (need == 0) return kErrBadArg;
   if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0) return kErrWorkspace;
   hipStream_t s = (hipStream_t)stream;
-  uint32_t* counts = static_cast<uint32_t*>(ws);
+  unsigned long long* covered = static_cast<unsigned long long*>(ws);
+  const HvSplit split = hv_split_for(n, m, n_sample);
+  if (split.parts > 1) {
+    if (int e = hv_clear(covered, 2 * ((n_sample + 63) / 64), s)) return e;
+  }
   const HvSamples samples = {samples_t, 1, n_sample, nullptr, nullptr, 0, 0};
-  if (int e = hv_covered_launch<kHvPlain>(points_t, samples, n, m, n_sample, counts, s)) return e;
-  hipLaunchKernelGGL(hv_covered_total_kernel<false>, dim3(1), dim3(1024), 0, s, counts, (int)((n_sample + 63) / 64), samples, (int)m,
+  if (int e = hv_covered_launch<kHvPlain>(points_t, samples, n, m, n_sample, split, covered, s)) return e;
+  hipLaunchKernelGGL(hv_covered_total_kernel<false>, dim3(1), dim3(1024), 0, s, covered, (int)((n_sample + 63) / 64), samples, (int)m,
                      (int)n_sample, out_count, (float*)nullptr);
   EVX_LAUNCH_CHECK();
   return 0;
@@ -2977,7 +2998,7 @@ int evox_hip_hv_covered_count(const float* points_t, const float* samples_t, int
 size_t evox_hip_hv_estimate_workspace_bytes(int64_t n, int64_t m, int64_t n_sample) {
   if (!hv_sizes_fit(n, n_sample) || m < 1 || m > kHvRegs) return 0;
   const HvBytes b = hv_bytes(n, m, n_sample);
-  return b.points + b.extreme + b.counts;
+  return b.points + b.extreme + b.covered;
 }
 
 int evox_hip_hv_estimate(const float* objs, int64_t stride_row, int64_t stride_col, int64_t n, int64_t m, const float* ref,
@@ -2990,14 +3011,16 @@ int evox_hip_hv_estimate(const float* objs, int64_t stride_row, int64_t stride_c
   uint8_t* at = static_cast<uint8_t*>(ws);
   float* points = reinterpret_cast<float*>(at);
   float* extreme = reinterpret_cast<float*>(at += b.points);
-  uint32_t* counts = reinterpret_cast<uint32_t*>(at += b.extreme);
+  unsigned long long* covered = reinterpret_cast<unsigned long long*>(at += b.extreme);
   const int parts = hv_parts(n);
+  const HvSplit split = hv_split_for(n, m, n_sample);
   hipLaunchKernelGGL(hv_points_kernel<true>, dim3((unsigned)parts), dim3(256), 0, s, objs, stride_row, stride_col, ref, ref_stride,
-                     (int)n, (int)m, parts, points, extreme, (float*)nullptr, (int64_t)0);
+                     (int)n, (int)m, parts, points, extreme, (float*)nullptr, (int64_t)0, reinterpret_cast<uint32_t*>(covered),
+                     split.parts > 1 ? 2 * ((n_sample + 63) / 64) : 0);
   EVX_LAUNCH_CHECK();
   const HvSamples samples = {u, m, 1, extreme, ref, ref_stride, parts};
-  if (int e = hv_covered_launch<kHvMetric>(points, samples, n, m, n_sample, counts, s)) return e;
-  hipLaunchKernelGGL(hv_covered_total_kernel<true>, dim3(1), dim3(1024), 0, s, counts, (int)((n_sample + 63) / 64), samples, (int)m,
+  if (int e = hv_covered_launch<kHvMetric>(points, samples, n, m, n_sample, split, covered, s)) return e;
+  hipLaunchKernelGGL(hv_covered_total_kernel<true>, dim3(1), dim3(1024), 0, s, covered, (int)((n_sample + 63) / 64), samples, (int)m,
                      (int)n_sample, (int64_t*)nullptr, out);
   EVX_LAUNCH_CHECK();
   return 0;

@@ -10,8 +10,9 @@
 //
 // Bound by vector issue: a test costs M compares, and a few thousand points against a hundred thousand samples are
 // 10^8 tests, some 5 us of the device.  What the kernels have to see to is that enough waves are there to hide the
-// loads of the other side.  Whether a sample is covered, and by how many points, is decided by ONE workgroup that holds 64
+// loads of the other side.  Whether a sample is covered, and by how many points, is decided by a workgroup that holds 64
 // samples, one to a lane, in each of its waves; the waves take the points in turn, hv_step at a time, as scalar operands.
+// Where the samples are too few to fill the device, several workgroups have the same samples and share the points.
 // (A wave that took all the points of its samples was alone with the latency of every scalar load: 129 us for 1001 x 3
 // against 100 000 samples, 27 us this way; counts and weights of 2000 x 3 against 10 000, 25 us before, 15 now.)  The sums
 // over the samples have the points in the lanes and read the samples, packed with their weights, from LDS, eight reads in
@@ -19,6 +20,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "hv_split.hpp"
 
 namespace evx {
 
@@ -29,11 +31,6 @@ constexpr int kHvRegs = 16;          // objectives held in registers; more are r
 constexpr int kHvPacked = 20;        // floats per packed sample, at most (16 objectives, the weight, whole 16-byte pieces)
 constexpr int kHvAlphaShare = 14;    // weights that one thread computes in ascending order, at least
 constexpr int kHvMeet = 32;          // steps after which the waves of a workgroup tell each other what is covered
-
-// Points that a wave takes at a time, as scalar operands.  (A step's values are in registers together: 8 objectives times
-// 16 points no longer fit the 128 registers of a workgroup of 1024 threads, and went through scratch memory: 5000 x 8 against
-// 20 000 samples, 1861 us, 78 with eight points.  From 9 objectives on the values are read objective by objective.)
-constexpr int hv_step(int m) { return m == 8 ? 8 : 16; }
 
 __host__ __device__ constexpr int hv_packed(int m) { return (m + 1 + 3) & ~3; }
 
@@ -108,11 +105,14 @@ __device__ inline bool hv_finite(float v) { return fabsf(v) <= 3.402823466385288
 // j + 1 points, alpha[j] = prod_{1 <= i <= j} (pop - i) / (n - i) / (j + 1), infinities as the largest numbers and NaN as
 // zero (hype.py:14-24), rounded at every step as the reference's statements are; a thread has kHvAlphaShare of them or
 // more, so that the first weights, which decide between points that cover a few samples, are products in ascending order.
+// zero: what the workgroups that share samples add up in, cleared here.
 template <bool kMetric>
 __global__ __launch_bounds__(256) void hv_points_kernel(const float* __restrict__ f, int64_t row, int64_t col,
                                                         const float* __restrict__ ref, int64_t ref_stride, int n, int m, int parts,
                                                         float* __restrict__ points_t, float* __restrict__ extreme,
-                                                        float* __restrict__ alpha, int64_t pop) {
+                                                        float* __restrict__ alpha, int64_t pop, uint32_t* __restrict__ zero,
+                                                        int64_t zero_words) {
+  for (int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x; w < zero_words; w += (int64_t)gridDim.x * 256) zero[w] = 0u;
   __shared__ float wave_extreme[4];
   __shared__ float product[256];
   const int t = threadIdx.x;
@@ -165,8 +165,8 @@ __global__ __launch_bounds__(256) void hv_points_kernel(const float* __restrict_
 
 // ---------------------------------------------------------------- HypE's contributions
 
-// The number of points of [0, n) that pass the test against the lane's sample, over the steps of points that this
-// wave takes: wave, wave + waves, ...; of the last step, which is moved back to end with the points, those not yet counted.
+// The number of points of [0, n) that pass the test against the lane's sample, over the steps of points that this wave
+// takes: wave, wave + waves, ...; of the last step, which is moved back to end with the points, those not yet counted.
 template <int M, bool kFinite>
 __device__ inline int hv_count_points(const float* __restrict__ points_t, int n, int m, const float (&sv)[M], int wave, int waves) {
   constexpr int kHvStep = hv_step(M);
@@ -200,16 +200,34 @@ __device__ inline int hv_count_points(const float* __restrict__ points_t, int n,
   return count;
 }
 
-// weight[s] = alpha[max(ds[s], 0)], ds[s] = points that cover sample s, minus one.  A workgroup of up to 16 waves has 64
-// samples.  Up to kHvRegs objectives (M > 0) the weight goes behind the sample's coordinates in `packed`, hv_packed(m)
-// floats a sample; for more (M == 0) `packed` holds the weights alone.
+// weight[s] = alpha[max(ds[s], 0)], ds[s] = points that cover sample s, minus one.  Up to kHvRegs objectives (M > 0) the weight
+// goes behind the sample's coordinates in `packed`, hv_packed(m) floats a sample; for more (M == 0) `packed` holds the
+// weights alone.
+template <int M, int R>
+__device__ inline void hv_store_weight(int64_t s, int m, int covered, const float (&sv)[R], const float* __restrict__ alpha,
+                                       float* __restrict__ packed) {
+  const float w = alpha[covered == 0 ? 0 : covered - 1];
+  if constexpr (M > 0) {
+    float* const at = packed + s * hv_packed(m);
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+      if (M <= 8 || k < m) at[k] = sv[k];
+    at[m] = w;
+  } else {
+    packed[s] = w;
+  }
+}
+
+// A workgroup of up to 16 waves has 64 samples and, where gridDim.y workgroups have the same ones, a share of the points:
+// these add to cover[s], which must be zero, and hv_weight_kernel takes it from there.
 template <int M, int kMode>
 __global__ __launch_bounds__(1024) void hv_sample_weight_kernel(const float* __restrict__ points_t, HvSamples samples, int n, int m,
                                                                 int n_sample, const float* __restrict__ alpha,
-                                                                float* __restrict__ packed) {
+                                                                float* __restrict__ packed, int* __restrict__ cover) {
   __shared__ int part[64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int turn = (int)blockIdx.y * waves + wave, turns = (int)gridDim.y * waves;
   const int64_t s = (int64_t)blockIdx.x * 64 + lane;
   const int64_t sc = s < n_sample ? s : n_sample - 1;
   if (threadIdx.x < 64) part[lane] = 0;
@@ -224,10 +242,10 @@ __global__ __launch_bounds__(1024) void hv_sample_weight_kernel(const float* __r
       if (M <= 8 || k < m) sv[k] = hv_sample<kMode>(samples, m, sc, k);
       finite &= hv_finite(sv[k]);
     }
-    count = __builtin_amdgcn_ballot_w64(!finite) == 0ull ? hv_count_points<M, true>(points_t, n, m, sv, wave, waves)
-                                                         : hv_count_points<M, false>(points_t, n, m, sv, wave, waves);
+    count = __builtin_amdgcn_ballot_w64(!finite) == 0ull ? hv_count_points<M, true>(points_t, n, m, sv, turn, turns)
+                                                         : hv_count_points<M, false>(points_t, n, m, sv, turn, turns);
   } else {
-    for (int i = wave; i < n; i += waves) {
+    for (int64_t i = turn; i < n; i += turns) {
       bool c = true;
       for (int k = 0; k < m; ++k) c &= hv_no_worse<false>(points_t[(int64_t)k * n + i], samples.u[sc * samples.row + k * samples.col]);
       count += c ? 1 : 0;
@@ -237,17 +255,27 @@ __global__ __launch_bounds__(1024) void hv_sample_weight_kernel(const float* __r
   if (count != 0) atomicAdd(&part[lane], count);
   __syncthreads();
   if (wave != 0 || s >= n_sample) return;
-  const int covered = part[lane];
-  const float w = alpha[covered == 0 ? 0 : covered - 1];
-  if constexpr (M > 0) {
-    float* const at = packed + s * hv_packed(m);
-#pragma unroll
-    for (int k = 0; k < M; ++k)
-      if (M <= 8 || k < m) at[k] = sv[k];
-    at[m] = w;
-  } else {
-    packed[s] = w;
+  if (gridDim.y > 1) {
+    if (part[lane] != 0) atomicAdd(&cover[s], part[lane]);
+    return;
   }
+  hv_store_weight<M>(s, m, part[lane], sv, alpha, packed);
+}
+
+// The weights of samples whose points were shared: cover[s] points cover sample s.
+template <int M, int kMode>
+__global__ __launch_bounds__(64) void hv_weight_kernel(HvSamples samples, int m, int n_sample, const int* __restrict__ cover,
+                                                       const float* __restrict__ alpha, float* __restrict__ packed) {
+  const int64_t s = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  const int64_t sc = s < n_sample ? s : n_sample - 1;  // (hv_sample needs every lane)
+  constexpr int R = M > 0 ? M : 1;
+  float sv[R];
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    sv[k] = 0.0f;
+    if (M <= 8 || k < m) sv[k] = hv_sample<kMode>(samples, m, sc, k);
+  }
+  if (s < n_sample) hv_store_weight<M>(s, m, cover[s], sv, alpha, packed);
 }
 
 // The sum goes on over `count` samples of the tile, a multiple of eight (the tile is filled up with weights of zero).
@@ -362,21 +390,24 @@ __global__ __launch_bounds__(64) void hv_point_total_kernel(const float* __restr
 
 // ---------------------------------------------------------------- the metric
 
-// block_count[b] = number of the 64 samples of workgroup b that some point exceeds strictly in every objective (a NaN on
-// either side compares false).  A wave stops as soon as all of its samples are covered; every kHvMeet steps the waves of
-// the workgroup tell each other which are.  points_t is (m, n), row-major.
+// covered[b]: which of the 64 samples of workgroup b some point exceeds strictly in every objective (a NaN on either side
+// compares false).  A wave stops as soon as all of its samples are covered; every kHvMeet steps the waves of the workgroup
+// tell each other which are.  points_t is (m, n), row-major.  Where gridDim.y workgroups have the same samples, each with
+// a share of the points, covered[b] must be zero, and one that starts late does not look for what it already holds.
 template <int M, int kMode>
 __global__ __launch_bounds__(1024) void hv_covered_kernel(const float* __restrict__ points_t, HvSamples samples, int n, int m,
-                                                          int n_sample, uint32_t* __restrict__ block_count) {
+                                                          int n_sample, unsigned long long* __restrict__ covered) {
   __shared__ unsigned long long met;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int turn = (int)blockIdx.y * waves + wave, turns = (int)gridDim.y * waves;
   const int64_t s = (int64_t)blockIdx.x * 64 + lane;
   const bool live = s < n_sample;
   const int64_t sc = live ? s : n_sample - 1;
-  if (threadIdx.x == 0) met = 0ull;
+  if (threadIdx.x == 0)
+    met = gridDim.y > 1 ? __hip_atomic_load(&covered[blockIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
   __syncthreads();
-  bool cov = !live;
+  bool cov = !live || ((met >> lane) & 1ull) != 0ull;
   if constexpr (M > 0) {
     constexpr int kHvStep = hv_step(M);
     float sv[M];
@@ -386,10 +417,10 @@ __global__ __launch_bounds__(1024) void hv_covered_kernel(const float* __restric
       if (M <= 8 || k < m) sv[k] = hv_sample<kMode>(samples, m, sc, k);
     }
     // (the last points once more where they are no whole step: a test may be repeated)
-    const int steps = n < kHvStep ? 0 : (n + kHvStep - 1) / kHvStep;
+    const int steps = n < kHvStep || __builtin_amdgcn_ballot_w64(!cov) == 0ull ? 0 : (n + kHvStep - 1) / kHvStep;
     int since = 0;
 #pragma unroll 1
-    for (int step = wave; step < steps; step += waves) {
+    for (int step = turn; step < steps; step += turns) {
       const int i = min(step * kHvStep, n - kHvStep);
       bool c[kHvStep];
 #pragma unroll
@@ -414,7 +445,7 @@ __global__ __launch_bounds__(1024) void hv_covered_kernel(const float* __restric
       }
       if (__builtin_amdgcn_ballot_w64(!cov) == 0ull) break;
     }
-    for (int i = wave; n < kHvStep && i < n; i += waves) {
+    for (int i = turn; n < kHvStep && i < n; i += turns) {
       bool c = true;
 #pragma unroll
       for (int k = 0; k < M; ++k)
@@ -422,7 +453,7 @@ __global__ __launch_bounds__(1024) void hv_covered_kernel(const float* __restric
       cov |= c;
     }
   } else {
-    for (int i = wave; i < n && __builtin_amdgcn_ballot_w64(!cov) != 0ull; i += waves) {
+    for (int64_t i = turn; i < n && __builtin_amdgcn_ballot_w64(!cov) != 0ull; i += turns) {
       bool c = true;
       for (int k = 0; k < m; ++k) c &= samples.u[sc * samples.row + k * samples.col] < points_t[(int64_t)k * n + i];
       cov |= c;
@@ -432,17 +463,21 @@ __global__ __launch_bounds__(1024) void hv_covered_kernel(const float* __restric
   const unsigned long long mine = __builtin_amdgcn_ballot_w64(cov && live);
   if (lane == 0 && mine != 0ull) atomicOr(&met, mine);
   __syncthreads();
-  if (threadIdx.x == 0) block_count[blockIdx.x] = (uint32_t)__popcll(met & lives);
+  if (threadIdx.x != 0) return;
+  if (gridDim.y == 1)
+    covered[blockIdx.x] = met & lives;
+  else if ((met & lives) != 0ull)
+    atomicOr(&covered[blockIdx.x], met & lives);
 }
 
-// The sum of the blocks' counts: out_count[0], or out[0] = sum / n_sample * (product of the box's sides).
+// The number of covered samples: out_count[0], or out[0] = sum / n_sample * (product of the box's sides).
 template <bool kEstimate>
-__global__ __launch_bounds__(1024) void hv_covered_total_kernel(const uint32_t* __restrict__ block_count, int blocks, HvSamples box, int m,
-                                                                int n_sample, int64_t* __restrict__ out_count, float* __restrict__ out) {
+__global__ __launch_bounds__(1024) void hv_covered_total_kernel(const unsigned long long* __restrict__ covered, int blocks, HvSamples box,
+                                                                int m, int n_sample, int64_t* __restrict__ out_count, float* __restrict__ out) {
   __shared__ int part[16];
   int acc = 0;
 #pragma unroll 2
-  for (int b = threadIdx.x; b < blocks; b += 1024) acc += (int)block_count[b];
+  for (int b = threadIdx.x; b < blocks; b += 1024) acc += __popcll(covered[b]);
   for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
   float volume = 1.0f;

@@ -76,3 +76,28 @@ def test_calls_that_keep_to_the_operators():
     with torch.device(DEV):
         hv(leaf, ref, 1000).backward()
     assert float(leaf.grad.abs().sum()) > 0.0
+
+
+@pytest.mark.parametrize("n, m, n_sample", [(100003, 3, 64), (70000, 3, 1), (65537, 8, 130), (40001, 17, 65), (30011, 5, 1000),
+                                            (300000, 1, 100), (20000, 16, 63), (20001, 8, 2000)])
+def test_points_shared_by_several_workgroups(n, m, n_sample):
+    """Few samples against many points, where several workgroups have the same samples, against counts made on the CPU.
+    Some samples are covered by no point, some only by points of the last steps."""
+    g = torch.Generator().manual_seed(n + m)
+    fit = torch.randn(n, m, generator=g).abs()
+    fit = fit / fit.norm(dim=1, keepdim=True) + 0.3
+    fit[-5:] *= 0.9
+    samples = 0.25 + 1.1 * torch.rand(n_sample, m, generator=g)
+    samples[::3] = fit[torch.randint(n - 16, n, (len(samples[::3]),), generator=g)]
+    covers = torch.stack([(fit <= s).all(dim=1) for s in samples])
+    count = covers.sum(dim=1)
+    alpha = torch.rand(n, generator=g)
+    weight = alpha[(count - 1).clamp(min=0)].double()
+    got = ops.hv_contributions(fit.to(DEV), samples.to(DEV), alpha.to(DEV), 1.0).cpu().double()
+    want = covers.double().t() @ weight
+    assert torch.allclose(got, want, rtol=(n_sample + 2) * 2.0**-24, atol=0.0)
+    # the metric: points above the samples
+    points, below = fit.to(DEV), samples.to(DEV)
+    exceeded = torch.stack([(s < fit).all(dim=1).any() for s in samples]).sum()
+    for _ in range(2):
+        assert int(ops.hv_covered_count(points, below)) == int(exceeded)
