@@ -18,10 +18,12 @@ def _plain(op, *tensors):
     (``ops.plain_eager``) -- the function that the custom operator wraps: what the operator would run after four
     layers of dispatch, a fifth of the time of a selection of 200 rows.  Tensor subclasses (fake tensors, functional
     wrappers), tensors that require a gradient and views with a negative or conjugate bit keep to the operator."""
+    if not ops.plain_eager():  # (first: a tracer stumbles over the questions below)
+        return op
     for t in tensors:
         if type(t) is not torch.Tensor or t.requires_grad or t.is_neg() or t.is_conj():
             return op
-    return getattr(op, "_init_fn", op) if ops.plain_eager() else op  # (another torch may not keep it there: the operator then)
+    return getattr(op, "_init_fn", op)  # (another torch may not keep it there: the operator then)
 
 
 def non_dominate_rank(x: torch.Tensor) -> torch.Tensor:

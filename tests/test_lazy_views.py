@@ -27,6 +27,14 @@ def test_lazy_views_keep_to_the_operator():
     assert non_dominate._plain(ops.nd_select, x.conj(), f) is ops.nd_select
 
 
+def test_the_choice_can_be_traced():
+    @torch.compile(fullgraph=True, backend="eager")
+    def kept(f):
+        return f + 1.0 if non_dominate._plain(ops.nd_rank, f) is ops.nd_rank else f
+
+    assert torch.equal(kept(torch.zeros(3)), torch.ones(3))
+
+
 CALLS = {
     "rank": lambda f: selection.non_dominate_rank(f),
     "rank until": lambda f: selection.non_dominate_rank_until(f, f.size(0) // 2),
