@@ -1571,10 +1571,26 @@ static int stage_spatial_order(const Ws& w, const float* xs, float* xs_sorted, c
   return 0;
 }
 
+// Whether front_small_kernel takes a population, or `batch` of them.  One population around a sphere, it / the steps, us a call:
+// 4096 x 3 13 / 21, 6000 x 3 17 / 21, 4096 x 5 18 / 27, 1000 x 8 15 / 19, 2000 x 8 24 / 19, 512 x 12 13 / 20, 1000 x 12 22 / 22,
+// 512 x 16 20 / 25, 1000 x 16 34 / 29.  Where the workgroups no longer fit the device at once (two on a compute unit) the pairs
+// are paid in full: 256 x 700 x 3 25 / 44, 1000 x 3 57 / 50; 256 x 700 x 8 96 / 140, 1000 x 8 147 / 116; 64 x 2000 x 2 36 / 26.
+static bool front_small_fits(int n, int m, int batch) {
+  if (n > 4096 || (int64_t)n * m > (m <= 8 ? 12288 : 8192)) return false;
+  return n <= 768 || (int64_t)batch * ((n + 63) / 64) <= 2 * device_cus();
+}
+
 // The first front of up to kSpatialObjectives objectives (spatial.hpp).
 template <int M>
 static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hipStream_t s) {
   const Layout& L = w.L;
+  if (front_small_fits(L.n, M, w.batch)) {
+    const int tiles = (L.n + 63) / 64, waves = tiles < front_small_waves(M) ? tiles : front_small_waves(M);
+    hipLaunchKernelGGL(front_small_kernel<M>, dim3((unsigned)tiles, 1, w.batch), dim3(64 * waves), 0, s, fit.f, fit.sr, fit.sc, fit.step,
+                       L.n, mask, w.ctrl(), w.step);
+    EVX_LAUNCH_CHECK();
+    return 0;
+  }
   // The rows step 2 leaves stand in xs, those of step 1 in xs_sorted, and the spatial order goes to the other of the two.
   constexpr bool kGrid = M == 2 || M == 3;
   const bool grid_step = kGrid && L.n > kFrontGridPopulation;

@@ -276,6 +276,77 @@ __device__ inline int dominance_sign(const float (&a)[M], const float (&b)[M]) {
   return (int)o;
 }
 
+// A whole small population in one launch.  A workgroup has 64 rows, one to a lane, in each of its waves; the waves take all
+// rows in turn, 64 at a time, through LDS.  Every pair is compared, so it serves where the three launches of the steps below
+// cost more than that.
+constexpr int front_small_waves(int m) { return m <= 8 ? 16 : 8; }  // (of 64 * m values in LDS each)
+template <int M>
+__global__ __launch_bounds__(1024) void front_small_kernel(const float* __restrict__ f, int64_t stride_row, int64_t stride_col,
+                                                           int64_t f_step, int n, uint8_t* __restrict__ mask, Ctrl* __restrict__ ctrl,
+                                                           int64_t ws_step) {
+  f += (int64_t)blockIdx.z * f_step;
+  mask += (int64_t)blockIdx.z * n;
+  to_population(ws_step, ctrl);
+  __shared__ __attribute__((aligned(16))) float tiles[front_small_waves(M)][M][64];
+  __shared__ unsigned long long dominated;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = (int)(blockDim.x >> 6);
+  if (blockIdx.x == 0)  // (no wait here, so no error either)
+    for (int i = threadIdx.x; i < (int)(sizeof(Ctrl) / 4); i += (int)blockDim.x) reinterpret_cast<uint32_t*>(ctrl)[i] = 0u;
+  if (threadIdx.x == 0) dominated = 0ull;
+  const int j = (int)blockIdx.x * 64 + lane;
+  auto row = [&](int i, float pad, float (&x)[M]) {
+    bool finite = true;
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      x[k] = i < n ? f[i * stride_row + k * stride_col] + 0.0f : pad;  // (-0.0 as +0.0)
+      finite &= fabsf(x[k]) <= 3.4028234663852886e38f;
+    }
+    return __builtin_amdgcn_ballot_w64(!finite) == 0ull;
+  };
+  float x[M];
+  const bool own_finite = row(j, 0.0f, x);
+  int beaten = 0;
+  for (int c0 = 0; c0 < n; c0 += 64 * waves) {
+    const int first = c0 + 64 * wave;
+    float(&tile)[M][64] = tiles[wave];
+    float mine[M];
+    // (a row of the largest numbers exceeds no finite row in the differences below)
+    const bool all_finite = row(first + lane, 3.4028234663852886e38f, mine) && own_finite;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < M; ++k) tile[k][lane] = mine[k];
+    __syncthreads();
+    const int count = min(64, n - first);
+    if (all_finite) {
+      for (int e = 0; e < count; e += 4) {
+        uint32_t o[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          const float4 t = *reinterpret_cast<const float4*>(&tile[k][e]);
+          o[0] |= __float_as_uint(x[k] - t.x);
+          o[1] |= __float_as_uint(x[k] - t.y);
+          o[2] |= __float_as_uint(x[k] - t.z);
+          o[3] |= __float_as_uint(x[k] - t.w);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) beaten = max(beaten, (int)o[u]);  // (dominance_sign)
+      }
+    } else {
+      for (int e = 0; e < count; ++e) {
+        float t[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) t[k] = tile[k][e];
+        if (row_dominates<M>(t, x)) beaten = 1;
+      }
+    }
+  }
+  const uint64_t found = __builtin_amdgcn_ballot_w64(beaten > 0);
+  if (lane == 0 && found != 0ull) atomicOr(&dominated, found);
+  __syncthreads();
+  if (wave == 0 && j < n) mask[j] = ((dominated >> lane) & 1ull) != 0ull ? 0 : 1;
+}
+
 // Copies the rows of a stretch of 256 * kFrontRowsPerThread rows that are kept to the next free places of `to` (any order):
 // one addition to the counter per stretch.  bucket / to_bucket: null, or what else goes along with a row.
 template <int M>

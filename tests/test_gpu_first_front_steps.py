@@ -34,7 +34,8 @@ def population(kind, n, m, seed):
 
 
 @pytest.mark.parametrize("kind", ["uniform", "shell", "one front", "ties", "special"])
-@pytest.mark.parametrize("n,m", [(1, 3), (63, 2), (1025, 3), (1024, 16), (16384, 3), (16385, 2), (16385, 3), (21000, 4), (65536, 3),
+@pytest.mark.parametrize("n,m", [(1, 3), (63, 2), (64, 1), (65, 16), (100, 3), (513, 9), (1025, 3), (1024, 16), (512, 16), (1536, 8),
+                                 (1537, 8), (2457, 5), (2458, 5), (4096, 3), (4097, 3), (4097, 16), (16384, 3), (16385, 2), (16385, 3), (21000, 4), (65536, 3),
                                  (65537, 2), (65537, 3), (65537, 4), (70001, 7), (131072, 3), (131073, 3)])
 def test_mask_at_the_edges_of_the_steps(n, m, kind):
     from evox_amd.operators.selection import non_dominated_mask
@@ -42,6 +43,19 @@ def test_mask_at_the_edges_of_the_steps(n, m, kind):
     f = population(kind, n, m, n + m)
     got = non_dominated_mask(f.to("cuda")).cpu().numpy()
     assert np.array_equal(got, c_oracle.first_front(f.numpy()))
+
+
+@pytest.mark.parametrize("n,m", [(5, 3), (100, 2), (130, 9), (1024, 3), (4096, 2), (4100, 3)])
+def test_masks_of_several_small_populations(n, m):
+    from evox_amd.operators.selection import non_dominated_mask
+
+    f = torch.stack([population(kind, n, m, n + b) for b, kind in enumerate(("uniform", "one front", "special", "ties"))])
+    wide = torch.full((4, n, m + 2), -1.0)
+    wide[:, :, 1 : m + 1] = f
+    for view in (f.to("cuda"), wide.to("cuda")[:, :, 1 : m + 1], f.transpose(1, 2).contiguous().to("cuda").transpose(1, 2)):
+        got = non_dominated_mask(view).cpu().numpy()
+        for b in range(4):
+            assert np.array_equal(got[b], c_oracle.first_front(f[b].numpy())), b
 
 
 def test_masks_of_several_large_populations():
