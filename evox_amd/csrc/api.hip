@@ -1646,7 +1646,8 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
     }
   }
   const int pair_rows = L.n < kFrontPairsRows ? L.n : kFrontPairsRows;
-  hipLaunchKernelGGL(front_pairs_kernel<M>, dim3((pair_rows + 255) / 256, kFrontPairsParts, w.batch), dim3(256), 0, s, left, left_of,
+  const int pair_parts = (pair_rows + 63) / 64 < kFrontPairsParts ? (pair_rows + 63) / 64 : kFrontPairsParts;  // (a part has 64 rows or more)
+  hipLaunchKernelGGL(front_pairs_kernel<M>, dim3((pair_rows + 255) / 256, pair_parts, w.batch), dim3(256), 0, s, left, left_of,
                      to, to_of, L.npad, mask, L.n, count, w.step);
   EVX_LAUNCH_CHECK();
   if (!order_step) return 0;
