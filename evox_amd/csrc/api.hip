@@ -1607,12 +1607,28 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
   const bool small_grid = M == 3 && L.n <= kFrontGridSmallRows;
   const int cell_bits = small_grid ? 7 : 8;
   const int grid_cells = !grid_step ? 0 : (M == 2 ? 1 << cell_bits : 1 << (2 * cell_bits));
-  hipLaunchKernelGGL(front_reset_kernel, dim3(1, 1, w.batch), dim3(256), 0, s, w.ctrl(), count, w.step);
+  // The rows of low sums cost a pass over the rows (and a launch that is needed anyway).  Without them, a population that a
+  // few rows dominate which no sample holds goes on whole: pairs of up to 65 536 rows of four objectives take some 35 us then,
+  // of 60 000 x 6 315, and 200 000 x 4 took 145 us where the rows of low sums leave 36.  (An entry per stretch of 256 rows or
+  // more fits the 4 bytes that each of them has there.)
+  const bool with_lowest = M > 4 || order_step;
+  unsigned long long* const lowest = with_lowest ? w.at<unsigned long long>(L.witness) : nullptr;
+  if (with_lowest) {
+    const int stretches = (L.n + front_stretch_rows(L.n) - 1) / front_stretch_rows(L.n);
+    hipLaunchKernelGGL(front_lowest_kernel<M>, dim3((unsigned)stretches, 1, w.batch), dim3(256), 0, s, fit.f, fit.sr, fit.sc, fit.step,
+                       L.n, lowest, w.ctrl(), count, w.step);
+  } else {
+    hipLaunchKernelGGL(front_reset_kernel, dim3(1, 1, w.batch), dim3(256), 0, s, w.ctrl(), count, w.step);
+  }
   EVX_LAUNCH_CHECK();
+  // (fewer rows per thread as long as every workgroup, which finds the champions first, has a compute unit of its own)
   int blocks = (L.n + 256 * kFrontRowsPerThread - 1) / (256 * kFrontRowsPerThread);
   if (blocks > 1024) blocks = 1024;
-  hipLaunchKernelGGL(front_filter_kernel<M>, dim3(blocks, 1, w.batch), dim3(256), 0, s, fit.f, fit.sr, fit.sc, fit.step, L.n, L.npad,
-                     left, left_of, mask, count, cells, grid_cells, w.at<uint32_t>(L.hist),
+  int per = kFrontRowsPerThread;
+  while (per > 1 && (int64_t)w.batch * ((L.n + 128 * per - 1) / (128 * per)) <= device_cus()) per /= 2;
+  const int filter_blocks = per < kFrontRowsPerThread ? (L.n + 256 * per - 1) / (256 * per) : blocks;
+  hipLaunchKernelGGL(front_filter_kernel<M>, dim3(filter_blocks, 1, w.batch), dim3(256), 0, s, fit.f, fit.sr, fit.sc, fit.step, L.n, L.npad, per,
+                     lowest, left, left_of, mask, count, cells, grid_cells, w.at<uint32_t>(L.hist),
                      order_step ? (int)((L.tailbuf - L.hist) / 4) : 0, w.step);
   EVX_LAUNCH_CHECK();
   if constexpr (kGrid) {

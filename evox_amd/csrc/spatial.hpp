@@ -233,7 +233,16 @@ constexpr int kFrontPairsRows = 65536;
 constexpr int kFrontSamples = 256;      // sampled rows; those that no other sample dominates serve as champions
 constexpr int kFrontChampions = 64;     // of which at most this many
 constexpr int kFrontFilterObjectives = 6;  // (with more objectives hardly any row is dominated by a sample)
+// Champions besides: rows of low sums.  Where a few rows dominate the rest, these are among them.  A few where samples serve
+// too (each champion costs every row a comparison), more where they stand alone.
+constexpr int front_lowest(int m) { return m <= kFrontFilterObjectives ? 4 : 16; }
 constexpr int kFrontRowsPerThread = 4;
+constexpr int kFrontStretchRows = 256;  // rows of which the lowest is found, at least,
+constexpr int kFrontStretches = 1024;   // and how many such stretches, at most
+__host__ __device__ inline int front_stretch_rows(int n) {
+  const int rows = (n + kFrontStretches - 1) / kFrontStretches;
+  return rows < kFrontStretchRows ? kFrontStretchRows : rows;
+}
 constexpr int kFrontGridPopulation = 16384;  // step 2 is launched for populations of more rows,
 constexpr int kFrontGridLeast = 20480;       // and has work when step 1 leaves more than these (compared pair by pair in 45 us)
 constexpr int kFrontGrid = 256;       // cells of the grid of step 2 along an objective,
@@ -247,12 +256,52 @@ struct FrontCount {
   int nonfinite;
 };
 
-// Clears the control block and the counters.
+// Clears the control block and the counters, where front_lowest_kernel is not launched.
 __global__ __launch_bounds__(256) void front_reset_kernel(Ctrl* __restrict__ ctrl, FrontCount* __restrict__ count, int64_t ws_step) {
   to_population(ws_step, ctrl, count);
   uint32_t* words = reinterpret_cast<uint32_t*>(ctrl);
   for (int i = threadIdx.x; i < (int)(sizeof(Ctrl) / 4); i += 256) words[i] = 0u;
   if (threadIdx.x == 0) *count = FrontCount{0, 0, 0};
+}
+
+// lowest[b]: the row of the lowest sum in stretch b of the rows, its sum before it (as an ordered key; all ones where every
+// sum of the stretch is infinite or NaN).  A row of a low sum lies near the front, and in a population that a few rows dominate
+// it is one of them, which a sample by position may well miss: 60 000 x 8, one row dominates all others, 850 us without these
+// rows, 19 with.  Also clears the control block and the counters.
+template <int M>
+__global__ __launch_bounds__(256) void front_lowest_kernel(const float* __restrict__ f, int64_t stride_row, int64_t stride_col,
+                                                           int64_t f_step, int n, unsigned long long* __restrict__ lowest,
+                                                           Ctrl* __restrict__ ctrl, FrontCount* __restrict__ count, int64_t ws_step) {
+  f += (int64_t)blockIdx.z * f_step;
+  to_population(ws_step, lowest, ctrl, count);
+  if (blockIdx.x == 0) {
+    uint32_t* words = reinterpret_cast<uint32_t*>(ctrl);
+    for (int i = threadIdx.x; i < (int)(sizeof(Ctrl) / 4); i += 256) words[i] = 0u;
+    if (threadIdx.x == 0) *count = FrontCount{0, 0, 0};
+  }
+  __shared__ unsigned long long part[4];
+  const int64_t rows = front_stretch_rows(n), first = (int64_t)blockIdx.x * rows;
+  const int64_t end = first + rows < n ? first + rows : n;
+  unsigned long long best = ~0ull;
+#pragma unroll 4
+  for (int64_t i = first + threadIdx.x; i < end; i += 256) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < M; ++k) sum += f[i * stride_row + k * stride_col];
+    const unsigned long long own = ((unsigned long long)ordered_key(sum) << 32) | (unsigned long long)i;
+    if (fabsf(sum) <= 3.4028234663852886e38f && own < best) best = own;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long other = __shfl_xor(best, off);
+    best = other < best ? other : best;
+  }
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) best = part[w] < best ? part[w] : best;
+  lowest[blockIdx.x] = best;
 }
 
 template <int M>
@@ -347,8 +396,8 @@ __global__ __launch_bounds__(1024) void front_small_kernel(const float* __restri
   if (wave == 0 && j < n) mask[j] = ((dominated >> lane) & 1ull) != 0ull ? 0 : 1;
 }
 
-// Copies the rows of a stretch of 256 * kFrontRowsPerThread rows that are kept to the next free places of `to` (any order):
-// one addition to the counter per stretch.  bucket / to_bucket: null, or what else goes along with a row.
+// Copies those of a workgroup's 256 * kFrontRowsPerThread rows that are kept to the next free places of `to` (any order): one
+// addition to the counter for all of them.  bucket / to_bucket: null, or what else goes along with a row.
 template <int M>
 __device__ inline void front_keep(const float (&x)[kFrontRowsPerThread][M], const int (&number)[kFrontRowsPerThread],
                                   const bool (&keep)[kFrontRowsPerThread], int* counter, float* __restrict__ to,
@@ -382,83 +431,125 @@ __device__ inline void front_keep(const float (&x)[kFrontRowsPerThread][M], cons
   __syncthreads();  // scratch is used again
 }
 
-// Step 1.  Every workgroup finds the champions for itself (256 sampled rows compared in LDS) and takes stretches of 1024
-// rows.  left[k][p] / left_of[p]: the rows kept, in any order, and their numbers; mask: 1 for them, 0 for the others.
-// grid: null or the grid_cells cells of step 2, set to "empty" here; zero: what step 4 needs cleared.
+// Step 1.  Every workgroup finds the champions for itself (with `lowest` front_lowest of the stretches' lowest rows, each of its
+// share of them, and up to kFrontFilterObjectives objectives those of 256 sampled rows that no other dominates) and takes per
+// rows per thread at a time.  left[k][p] / left_of[p]: the rows kept, in any order, and their numbers; mask: 1 for them, 0 for the
+// others.  grid: null or the grid_cells cells of step 2, set to "empty" here; zero: what step 4 needs cleared.
 template <int M>
 __global__ __launch_bounds__(256) void front_filter_kernel(const float* __restrict__ f, int64_t stride_row, int64_t stride_col,
-                                                           int64_t f_step, int n, int npad, float* __restrict__ left,
+                                                           int64_t f_step, int n, int npad, int per,
+                                                           const unsigned long long* __restrict__ lowest, float* __restrict__ left,
                                                            int* __restrict__ left_of, uint8_t* __restrict__ mask,
                                                            FrontCount* __restrict__ count, uint32_t* __restrict__ grid,
                                                            int grid_cells, uint32_t* __restrict__ zero, int zero_words,
                                                            int64_t ws_step) {
   f += (int64_t)blockIdx.z * f_step;
   mask += (int64_t)blockIdx.z * n;
-  to_population(ws_step, left, left_of, count, grid, zero);
+  to_population(ws_step, lowest, left, left_of, count, grid, zero);
   for (int c = blockIdx.x * 256 + threadIdx.x; c < grid_cells; c += gridDim.x * 256) grid[c] = ~0u;
   for (int c = blockIdx.x * 256 + threadIdx.x; c < zero_words; c += gridDim.x * 256) zero[c] = 0u;
-  constexpr bool kFilter = M <= kFrontFilterObjectives;
-  __shared__ __attribute__((aligned(16))) float sample[kFilter ? M : 1][kFrontSamples];
-  __shared__ __attribute__((aligned(16))) float champion[kFilter ? kFrontChampions : 1][(M + 3) / 4 * 4];
+  constexpr bool kSampled = M <= kFrontFilterObjectives;
+  constexpr int kLowest = front_lowest(M), kMost = (kSampled ? kFrontChampions : 0) + kLowest;
+  static_assert(kFrontSamples == 256 && kMost % 4 == 0 && 256 % kLowest == 0, "one sample per thread; champions in fours");
+  __shared__ __attribute__((aligned(16))) float sample[kSampled ? M : 1][kFrontSamples];
+  __shared__ __attribute__((aligned(16))) float champion[kMost][(M + 3) / 4 * 4];
   __shared__ int champions;
   __shared__ int scratch[5];
-  if constexpr (kFilter) {
-    const int64_t i = (int64_t)threadIdx.x * n / kFrontSamples;
-    float mine[M];
-    bool finite = true;
+  {
+    auto read = [&](int64_t i, float (&x)[M]) {
+      bool finite = true;
 #pragma unroll
-    for (int k = 0; k < M; ++k) {
-      mine[k] = f[i * stride_row + k * stride_col] + 0.0f;
-      finite &= fabsf(mine[k]) <= 3.4028234663852886e38f;
-      sample[k][threadIdx.x] = mine[k];
+      for (int k = 0; k < M; ++k) {
+        x[k] = f[i * stride_row + k * stride_col] + 0.0f;
+        finite &= fabsf(x[k]) <= 3.4028234663852886e38f;
+      }
+      return finite;
+    };
+    auto enter = [&](const float (&x)[M]) {
+      const int c = atomicAdd(&champions, 1);
+#pragma unroll
+      for (int k = 0; k < M; ++k) champion[c][k] = x[k];
+    };
+    float mine[M];
+    bool finite = false;
+    if constexpr (kSampled) {
+      finite = read((int64_t)threadIdx.x * n / kFrontSamples, mine);
+#pragma unroll
+      for (int k = 0; k < M; ++k) sample[k][threadIdx.x] = mine[k];
     }
     if (threadIdx.x == 0) champions = 0;
     __syncthreads();
-    // (a sample that is not finite is no champion, and may wrongly keep another from being one: neither does harm)
-    int beaten = 0;
-    for (int e = 0; e < kFrontSamples; e += 4) {
-      float4 o[M];
+    if (lowest != nullptr) {
+      const int stretches = (n + front_stretch_rows(n) - 1) / front_stretch_rows(n);
+      unsigned long long best = ~0ull;
+      for (int e = threadIdx.x; e < stretches; e += 256) best = lowest[e] < best ? lowest[e] : best;
 #pragma unroll
-      for (int k = 0; k < M; ++k) o[k] = *reinterpret_cast<const float4*>(&sample[k][e]);
-      float a[4][M];
-#pragma unroll
-      for (int k = 0; k < M; ++k) {
-        a[0][k] = o[k].x;
-        a[1][k] = o[k].y;
-        a[2][k] = o[k].z;
-        a[3][k] = o[k].w;
+      for (int off = 128 / kLowest; off > 0; off >>= 1) {
+        const unsigned long long other = __shfl_xor(best, off);
+        best = other < best ? other : best;
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) beaten = max(beaten, dominance_sign<M>(a[u], mine));
+      float low[M];
+      if (threadIdx.x % (256 / kLowest) == 0 && best != ~0ull && read((int64_t)(uint32_t)best, low)) enter(low);
     }
-    if (finite && beaten <= 0) {
-      const int c = atomicAdd(&champions, 1);
-      if (c < kFrontChampions)
+    // (a sample that is not finite is no champion, and may wrongly keep another from being one: neither does harm)
+    if constexpr (kSampled) {
+      int beaten = 0;
+#pragma unroll 2
+      for (int e = 0; e < kFrontSamples; e += 4) {
+        float4 o[M];
 #pragma unroll
-        for (int k = 0; k < M; ++k) champion[c][k] = mine[k];
+        for (int k = 0; k < M; ++k) o[k] = *reinterpret_cast<const float4*>(&sample[k][e]);
+        float a[4][M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          a[0][k] = o[k].x;
+          a[1][k] = o[k].y;
+          a[2][k] = o[k].z;
+          a[3][k] = o[k].w;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) beaten = max(beaten, dominance_sign<M>(a[u], mine));
+      }
+      __syncthreads();  // (the rows of low sums are in)
+      if (finite && beaten <= 0) {
+        const int c = atomicAdd(&champions, 1);
+        if (c < kMost)
+#pragma unroll
+          for (int k = 0; k < M; ++k) champion[c][k] = mine[k];
+      }
     }
     __syncthreads();
   }
-  const int nc = kFilter ? min(champions, kFrontChampions) : 0;
+  const int nc = min(champions, kMost);
+  if (threadIdx.x < 4 && nc + threadIdx.x < kMost) {  // (up to a whole four with rows that dominate nothing finite)
+#pragma unroll
+    for (int k = 0; k < M; ++k) champion[nc + threadIdx.x][k] = 3.4028234663852886e38f;
+  }
+  __syncthreads();
   bool bad = false;
-  for (int64_t i0 = (int64_t)blockIdx.x * 256 * kFrontRowsPerThread; i0 < n; i0 += (int64_t)gridDim.x * 256 * kFrontRowsPerThread) {
+  for (int64_t i0 = (int64_t)blockIdx.x * 256 * per; i0 < n; i0 += (int64_t)gridDim.x * 256 * per) {
     float x[kFrontRowsPerThread][M];
     int number[kFrontRowsPerThread], beaten[kFrontRowsPerThread];
     bool keep[kFrontRowsPerThread];
 #pragma unroll
     for (int r = 0; r < kFrontRowsPerThread; ++r) {
-      const int64_t i = i0 + r * 256 + threadIdx.x;
-      number[r] = (int)i;
+      const int64_t i = r < per ? i0 + r * 256 + threadIdx.x : n;
+      number[r] = i < n ? (int)i : n;
       beaten[r] = 0;
 #pragma unroll
       for (int k = 0; k < M; ++k) x[r][k] = i < n ? f[i * stride_row + k * stride_col] + 0.0f : 0.0f;  // (-0.0 as +0.0)
     }
-    for (int c = 0; c < nc; ++c) {
-      float champ[M];
+    for (int c = 0; c < nc; c += 4) {
+      float champ[4][M];
 #pragma unroll
-      for (int k = 0; k < M; ++k) champ[k] = champion[c][k];
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int r = 0; r < kFrontRowsPerThread; ++r) beaten[r] = max(beaten[r], dominance_sign<M>(champ, x[r]));
+        for (int k = 0; k < M; ++k) champ[u][k] = champion[c + u][k];
+#pragma unroll
+      for (int r = 0; r < kFrontRowsPerThread; ++r)
+        if (r < per)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) beaten[r] = max(beaten[r], dominance_sign<M>(champ[u], x[r]));
     }
 #pragma unroll
     for (int r = 0; r < kFrontRowsPerThread; ++r) {
@@ -626,10 +717,12 @@ __global__ __launch_bounds__(256) void front_grid_filter_kernel(const float* __r
 }
 
 // Whether a row of xs[.][first .. first + 31] dominates the lane's row x; rows >= n are padding.  The rows are scalar
-// operands, in vector arithmetic where the population is finite.
+// operands, in vector arithmetic where the population is finite: the last 32 rows once more where fewer are left (one by one
+// they were a third of the pair step at 4090 x 8).
 template <int M>
 __device__ inline bool half_leaf_dominates(const float* __restrict__ xs, int npad, int first, int n, const float (&x)[M], bool all_finite) {
-  if (all_finite && first + 32 <= n) {
+  if (all_finite && n >= 32) {
+    first = min(first, n - 32);
     int worst = 0;
     constexpr int G = M <= 3 ? 32 : (M <= 5 ? 8 : (M <= 8 ? 4 : 2));  // rows whose values sit in scalar registers at once
 #pragma unroll 1

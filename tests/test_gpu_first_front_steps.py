@@ -58,6 +58,23 @@ def test_masks_of_several_small_populations(n, m):
             assert np.array_equal(got[b], c_oracle.first_front(f[b].numpy())), b
 
 
+@pytest.mark.parametrize("n,m", [(4097, 3), (5000, 16), (20000, 7), (70001, 2), (66000, 8), (300001, 3)])
+@pytest.mark.parametrize("good", [1, 17])
+def test_few_rows_that_dominate_the_rest(n, m, good):
+    """At places that no sample by position holds; among the others infinities and sums that overflow."""
+    from evox_amd.operators.selection import non_dominated_mask
+
+    g = torch.Generator("cpu").manual_seed(n + m)
+    f = torch.rand(n, m, generator=g) + 1.0
+    f[::1009, 0] = INF
+    f[5::1013] = 3e38
+    f[7::1019, m - 1] = -3e38
+    at = torch.randint(n // 3, n, (good,), generator=g)
+    f[at] = 0.9 * torch.rand(good, m, generator=g)
+    got = non_dominated_mask(f.to("cuda")).cpu().numpy()
+    assert np.array_equal(got, c_oracle.first_front(f.numpy()))
+
+
 def test_masks_of_several_large_populations():
     from evox_amd.operators.selection import non_dominated_mask
 
