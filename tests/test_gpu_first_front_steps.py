@@ -45,6 +45,24 @@ def test_mask_at_the_edges_of_the_steps(n, m, kind):
     assert np.array_equal(got, c_oracle.first_front(f.numpy()))
 
 
+@pytest.mark.parametrize("finite", [True, False])
+@pytest.mark.parametrize("n,m", [(65601, 5), (65601, 6), (65601, 9), (65700, 12), (65601, 16)])
+def test_leaves_of_more_objectives(n, m, finite):
+    """Rows on one front, more of them than are compared pair by pair."""
+    from evox_amd.operators.selection import non_dominated_mask
+
+    f = population("one front", n if finite else n + n // 4, m, n + m)
+    if not finite:
+        f[2::1007, 0] = INF
+        f[4::1013, m // 2] = NAN
+        f[3::40001, m - 1] = -INF
+        f[7] = INF
+    want = c_oracle.first_front(f.numpy())
+    assert 65536 < want.sum()
+    got = non_dominated_mask(f.to("cuda")).cpu().numpy()
+    assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("n,m", [(5, 3), (100, 2), (130, 9), (1024, 3), (4096, 2), (4100, 3)])
 def test_masks_of_several_small_populations(n, m):
     from evox_amd.operators.selection import non_dominated_mask

@@ -1,12 +1,14 @@
-"""The hypervolume functions as whole calls in the library against the same functions around the operators, at the edges of
-their kernels: eights of points, workgroups of 64 samples, shares and tiles of samples, objectives held in registers, the
-number of samples from which fewer waves share the points, strided inputs, values that are not finite."""
+"""The hypervolume functions as whole calls in the library, at the edges of their kernels: steps of points, workgroups of 64
+samples, shares and tiles of samples, objectives held in registers, the number of samples from which fewer waves share the
+points, strided inputs, values that are not finite -- against the restatement on the CPU, which shares no kernel with them,
+and against the same functions around the operators."""
 
 import pytest
 import torch
 
 from evox_amd import hype, ops
 from evox_amd.metrics import hv
+from oracle import eager_restatement as er
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -32,6 +34,58 @@ def _both(monkeypatch, call):
 def _close(got, want, rtol):
     assert got.shape == want.shape and got.dtype == want.dtype and got.device == want.device
     assert torch.allclose(got, want, rtol=rtol, atol=0.0, equal_nan=True), (got, want)
+
+
+def _against_the_restatement(objs, ref, n_sample, seed):
+    u = torch.rand(n_sample, objs.size(1), generator=torch.Generator().manual_seed(seed))
+    n, m = objs.shape
+    pop = max(1, n // 2)
+    assert ops.hv_whole_call_fits(objs.to(DEV), ref.to(DEV), n_sample)
+    # the counts are equal; the quotient and the product of m sides are rounded m + 1 times on either side
+    got = ops.hv_estimate(objs.to(DEV), ref.to(DEV), u.to(DEV)).cpu()
+    _close(got, er.hv_estimate(objs, ref, u), rtol=2 * (m + 1) * 2.0**-24)
+    # weights, none of them negative, are products of up to n rounded quotients, and n_sample of them are added up
+    got = ops.hype_contributions(objs.to(DEV), ref.to(DEV), pop, u.to(DEV)).cpu()
+    _close(got, er.hv_contributions(objs, ref, pop, u), rtol=(n_sample + 2 * n + 2 * m + 8) * 2.0**-24)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 255, 257])
+@pytest.mark.parametrize("m", range(1, 17))
+def test_whole_calls_against_the_restatement(n, m):
+    g = torch.Generator().manual_seed(100 * n + m)
+    objs = torch.randn(n, m, generator=g).abs()
+    objs = objs / objs.sum(dim=1, keepdim=True)
+    _against_the_restatement(objs, objs.max(dim=0).values * 1.1 + 0.05, 641, n + m)
+
+
+@pytest.mark.parametrize("m", [1, 3, 8, 9, 16])
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan")])
+def test_values_that_are_not_finite_against_the_restatement(m, value):
+    """A point of infinite cost leaves everything else finite; the others make the box and with it every result infinite or NaN."""
+    objs = torch.rand(300, m, generator=torch.Generator().manual_seed(m))
+    objs[17, m // 2] = value
+    objs[290, m - 1] = value
+    _against_the_restatement(objs, torch.full((m,), 1.2), 1500, m)
+
+
+@pytest.mark.parametrize("m", [1, 4, 8, 13, 17])
+def test_samples_that_are_not_finite(m):
+    """The operators, whose samples may be anything, against the tests written out: differences for the contributions, in
+    which infinity minus itself is no cover, comparisons for the metric."""
+    g = torch.Generator().manual_seed(m)
+    fit, samples = torch.rand(400, m, generator=g), 0.4 + torch.rand(700, m, generator=g)
+    for t in (fit, samples):
+        t[::7, 0] = float("inf")
+        t[3::11, m // 2] = -float("inf")
+        t[5::13, m - 1] = float("nan")
+    covers = torch.stack([(fit - s <= 0).all(dim=1) for s in samples])
+    assert not torch.equal(covers, torch.stack([(fit <= s).all(dim=1) for s in samples]))
+    alpha = torch.rand(400, generator=g)
+    want = covers.double().t() @ alpha[(covers.sum(dim=1) - 1).clamp(min=0)].double()
+    got = ops.hv_contributions(fit.to(DEV), samples.to(DEV), alpha.to(DEV), 1.0).cpu().double()
+    assert torch.allclose(got, want, rtol=702 * 2.0**-24, atol=0.0)
+    exceeded = torch.stack([(s < fit).all(dim=1).any() for s in samples]).sum()
+    assert int(ops.hv_covered_count(fit.to(DEV), samples.to(DEV))) == int(exceeded)
 
 
 @pytest.mark.parametrize("n, m, n_sample", SIZES)
