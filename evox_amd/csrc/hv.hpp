@@ -29,8 +29,13 @@ constexpr int kHvMaxShares = 64;     // shares of the samples in the sums, at mo
 constexpr int kHvParts = 64;         // workgroups that look for the box of the points, at most
 constexpr int kHvRegs = 16;          // objectives held in registers; more are re-read from memory
 constexpr int kHvPacked = 20;        // floats per packed sample, at most (16 objectives, the weight, whole 16-byte pieces)
-constexpr int kHvAlphaShare = 14;    // weights that one thread computes in ascending order, at least
-constexpr int kHvMeet = 32;          // steps after which the waves of a workgroup tell each other what is covered
+// Weights that one thread computes in ascending order, at least: those of a sample that up to 14 points cover, which decide
+// between the points, are the plain products.  (A HypE call on 2000 x 3 against 10 000 samples takes 47 us with 4, 14 or 32, on
+// 5000 x 3 against 20 000 80, 80 or 83.)
+constexpr int kHvAlphaShare = 14;
+// Steps after which the waves of a workgroup tell each other what is covered.  8 / 32 / 128, us a call: uniform 100 000 x 3
+// against 10 000 samples 137 / 155 / 180, 20 000 x 3 against 100 000 279 / 282 / 315, up to 5000 points 3 % apart at most.
+constexpr int kHvMeet = 32;
 
 __host__ __device__ constexpr int hv_packed(int m) { return (m + 1 + 3) & ~3; }
 
@@ -103,8 +108,9 @@ __device__ inline bool hv_finite(float v) { return fabsf(v) <= 3.402823466385288
 // points_t[k][i] = value of row i in objective k: |f - ref| for the metric, f for HypE; extreme[part][k] = the largest
 // (smallest for HypE) of the part's rows.  With alpha, one more workgroup writes the weights of a sample covered by
 // j + 1 points, alpha[j] = prod_{1 <= i <= j} (pop - i) / (n - i) / (j + 1), infinities as the largest numbers and NaN as
-// zero (hype.py:14-24), rounded at every step as the reference's statements are; a thread has kHvAlphaShare of them or
-// more, so that the first weights, which decide between points that cover a few samples, are products in ascending order.
+// zero (hype.py:14-24), in the precision of the reference's statements, whose cumprod is a scan too: a thread has
+// kHvAlphaShare of them or more in ascending order, the threads' products are scanned.  Largest relative error against 64
+// bits over n = 50 to 5000 with half of them kept: 5.0e-7, that of the cumprod on the same device 5.4e-7.
 // zero: what the workgroups that share samples add up in, cleared here.
 template <bool kMetric>
 __global__ __launch_bounds__(256) void hv_points_kernel(const float* __restrict__ f, int64_t row, int64_t col,

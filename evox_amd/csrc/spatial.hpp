@@ -5,9 +5,7 @@
 // corner -- the smallest value per objective among its rows -- then rules whole leaves out at once: no row of a leaf whose
 // low corner exceeds a row in some objective dominates that row.  A dominator has no larger quantile in any objective, so
 // its cell comes no later on the curve (at the first interleaved bit that differs it has the 0): nothing behind the end of a
-// row's own cell can dominate it, and the leaves nearest below are the likeliest.  For 200 000 uniform rows of three
-// objectives a fifth of the leaves can hold a dominator of a leaf's rows, and one of the first eight does for most leaves;
-// of 200 000 rows around a sphere in eight objectives, most of which nothing dominates, a row has to look at a twentieth.
+// row's own cell can dominate it, and the leaves nearest below are the likeliest.
 #pragma once
 
 #include "common.hpp"
@@ -20,7 +18,6 @@ constexpr int kLeafRows = 64;
 constexpr int kGroupLeaves = 64;         // leaves under one box of the second level (4096 rows)
 constexpr int kSpatialSamples = 256;     // rows whose values cut an objective into quantiles
 constexpr int kSpatialObjectives = 16;   // the most objectives that take this way
-constexpr int kSpatialBucketBits = 16;   // at most this many buckets (bits of the curve) tell cells apart
 
 // Boxes of a population of up to `rows` slots: leaves and groups, as rows of a structure of arrays.
 __host__ __device__ inline int64_t spatial_leaves(int64_t rows) { return (rows + kLeafRows - 1) / kLeafRows; }
@@ -223,16 +220,20 @@ __global__ __launch_bounds__(kBoxThreads) void leaf_box_kernel(const float* __re
 // ---------------------------------------------------------------- first front only
 //
 // mask[i] = 1 when no row dominates row i: `non_dominate_rank(f) == 0`, the only thing that
-// src/evox/workflows/eval_monitor.py:301-302 and :333-335 keep of the ranks.  Four steps, none of which waits for another
-// workgroup: (1) rows that some sampled row dominates are dropped and the rest is copied together; (2) with two or three
+// src/evox/workflows/eval_monitor.py:301-302 and :333-335 keep of the ranks.  Four steps: (1) rows that a champion, one of some
+// sampled rows and rows of low sums, dominates are dropped and the rest is copied together; (2) with two or three
 // objectives, where more than kFrontGridLeast are left, so are the rows that a row of a smaller cell of a grid dominates;
 // (3) up to kFrontPairsRows rows left are compared pair by pair; (4) more are put in spatial order and compared by leaves.
 // Which of the steps have work is decided on the device, by the number of rows left (a kernel with nothing to do takes
-// 1.6 us).
+// 1.6 us).  Only the scan of the buckets in (4) waits for other workgroups, those before its own, and not forever: where the
+// wait runs out no row is reported, and the status says so.
 constexpr int kFrontPairsRows = 65536;
 constexpr int kFrontSamples = 256;      // sampled rows; those that no other sample dominates serve as champions
-constexpr int kFrontChampions = 64;     // of which at most this many
-constexpr int kFrontFilterObjectives = 6;  // (with more objectives hardly any row is dominated by a sample)
+// Of these at most this many.  32 / 64 / 128, us a call: 1 000 003 x 3 around a sphere 247 / 238 / 232, 30 000 x 4 111 / 104 / 96;
+// uniform 30 000 x 5, where the few that matter are among any 32, 25.5 / 26.6 / 27.0.
+constexpr int kFrontChampions = 64;
+// With more objectives hardly any row is dominated by a sample (uniform 30 000 x 7 32 us, 73 with samples; x 8 55 and 105).
+constexpr int kFrontFilterObjectives = 6;
 // Champions besides: rows of low sums.  Where a few rows dominate the rest, these are among them.  A few where samples serve
 // too (each champion costs every row a comparison), more where they stand alone.
 constexpr int front_lowest(int m) { return m <= kFrontFilterObjectives ? 4 : 16; }
@@ -799,8 +800,11 @@ __global__ __launch_bounds__(256) void front_pairs_kernel(const float* __restric
 // of them rows of the front: if they are few, the waves take them one by one (front_row_beaten), which asks a leaf 64 rows
 // at a time and only the leaves whose low corner is no worse than the one row.
 constexpr int kFrontWaves = 4;
-constexpr int kFrontBulkLeaves = 3;  // leaves per wave before that
-constexpr int kFrontFewRows = 24;    // and the most rows it is done for
+// Leaves per wave before that: 1 / 3 / 6, us a call around a sphere, 1 000 003 x 3 234 / 238 / 251, 100 000 x 8, where the rows
+// seldom get few, 2490 / 2496 / 2363.
+constexpr int kFrontBulkLeaves = 3;
+// And the most rows it is done for: 8 / 24 / 48, 1 000 003 x 3 241 / 238 / 248, 100 000 x 5 503 / 454 / 545.
+constexpr int kFrontFewRows = 24;
 
 // Whether some row of the leaves up to `last` dominates the row x (the same in every lane); wave-cooperative.
 template <int M>
