@@ -540,17 +540,18 @@ __global__ __launch_bounds__(256) void front_filter_kernel(const float* __restri
 #pragma unroll
       for (int k = 0; k < M; ++k) x[r][k] = i < n ? f[i * stride_row + k * stride_col] + 0.0f : 0.0f;  // (-0.0 as +0.0)
     }
-    for (int c = 0; c < nc; c += 4) {
-      float champ[4][M];
+    constexpr int kTogether = M <= 8 ? 4 : 1;  // champions whose LDS reads are in flight together, as far as registers go
+    for (int c = 0; c < nc; c += kTogether) {
+      float champ[kTogether][M];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < kTogether; ++u)
 #pragma unroll
         for (int k = 0; k < M; ++k) champ[u][k] = champion[c + u][k];
 #pragma unroll
       for (int r = 0; r < kFrontRowsPerThread; ++r)
         if (r < per)
 #pragma unroll
-          for (int u = 0; u < 4; ++u) beaten[r] = max(beaten[r], dominance_sign<M>(champ[u], x[r]));
+          for (int u = 0; u < kTogether; ++u) beaten[r] = max(beaten[r], dominance_sign<M>(champ[u], x[r]));
     }
 #pragma unroll
     for (int r = 0; r < kFrontRowsPerThread; ++r) {
