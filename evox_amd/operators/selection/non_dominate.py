@@ -13,6 +13,9 @@ import torch
 from ... import ops
 
 
+_Tensor = torch.Tensor
+
+
 def _plain(op, *tensors):
     """``op`` itself, or -- for plain tensors with no transform, tracer or dispatch mode looking at the call
     (``ops.plain_eager``) -- the function that the custom operator wraps: what the operator would run after four
@@ -21,7 +24,7 @@ def _plain(op, *tensors):
     if not ops.plain_eager():  # (first: a tracer stumbles over the questions below)
         return op
     for t in tensors:
-        if type(t) is not torch.Tensor or t.requires_grad or t.is_neg() or t.is_conj():
+        if type(t) is not _Tensor or t.requires_grad or t.is_neg() or t.is_conj():
             return op
     return getattr(op, "_init_fn", op)  # (another torch may not keep it there: the operator then)
 

@@ -20,6 +20,10 @@ from torch.utils._python_dispatch import _get_current_dispatch_mode
 from . import _lib, runtime
 
 
+# (the raw query: it is asked with a tensor on a GPU at hand, so the device layer is up)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def _batched_first(info, dims, tensors):
     """The tensors of a vmap rule with the mapped dimension in front; those that are not mapped are expanded."""
     out = []
@@ -462,7 +466,7 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
         raise IndexError(f"topk must be at least 1; got {topk}")
     if m == 0:
         raise ValueError("fitness must have at least one objective")
-    if bd == 0 and f.dtype is torch.float32 and x.is_contiguous() and f.device.index == torch.cuda.current_device():
+    if bd == 0 and f.dtype is torch.float32 and x.is_contiguous() and f.device.index == _current_device():
         # One population of float32 fitness on the current device -- what an algorithm's step passes: the same call
         # without the views and the device guard of the general path below (a third of the time of a selection of
         # 200 rows is spent on this side of the C ABI).
@@ -570,7 +574,8 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
         raise ValueError("the decision vectors of the two parts differ in row shape or dtype")
     if x_a.size(0) != f_a.size(0) or x_b.size(0) != f_b.size(0):
         raise ValueError("decision vectors and fitness disagree on the number of rows")
-    if len({x_a.device, x_b.device, f_a.device, f_b.device}) != 1:
+    device = f_a.device
+    if x_a.device != device or x_b.device != device or f_b.device != device:
         raise RuntimeError("the parts are on different devices")
     if f_a.dtype != f_b.dtype:
         raise TypeError("the fitness parts differ in dtype")
@@ -583,7 +588,7 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
     if m == 0:
         raise ValueError("fitness must have at least one objective")
     if (n_a > 0 and n_b > 0 and f_a.dtype is torch.float32 and f_a.stride() == f_b.stride() and x_a.is_contiguous()
-            and x_b.is_contiguous() and f_a.device.index == torch.cuda.current_device()
+            and x_b.is_contiguous() and f_a.device.index == _current_device()
             and runtime.small_population_kernel_fits(n, m, 1)):
         # parents and offspring of a run with a few hundred individuals: one launch of the one-workgroup kernel,
         # which reads both parts where they lie (the pipeline's four launches took half as long again)
@@ -902,16 +907,20 @@ def tournament_keys_fit(keys) -> bool:
                and t.device == first.device and t.size(0) == first.size(0) for t in keys) and first.size(0) > 0
 
 
+_is_compiling = torch.compiler.is_compiling
+try:
+    _interpreter = torch._C._functorch.peek_interpreter_stack
+except AttributeError:  # another torch: take the dispatcher
+    def _interpreter():
+        return "unknown"
+
+
 def plain_eager() -> bool:
     """True when no transform (vmap, grad), tracer (torch.compile, make_fx) or dispatch mode is looking at the call,
     so that an operator's implementation may be called as the Python function it is: the dispatcher's way to the same
     function costs about 10 us, a third of a host-bound call like a tournament selection.  It also resolves tensors whose memory
-    holds other bytes than their values (a negative or conjugate bit: ``z.conj().imag``), which a caller must look for itself."""
-    try:
-        return (not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
-                and _get_current_dispatch_mode() is None)
-    except AttributeError:  # another torch: take the dispatcher
-        return False
+    holds other bytes than their values (a negative or conjugate bit: ``z.conj().imag``), for which a caller has to look itself."""
+    return not _is_compiling() and _interpreter() is None and _get_current_dispatch_mode() is None
 
 
 def tournament_pick_keys_direct(parents: torch.Tensor, keys: List[torch.Tensor]) -> torch.Tensor:
