@@ -116,3 +116,29 @@ def test_rows_that_a_leaf_asks_one_by_one(n, m):
     f = f[torch.randperm(n, generator=g)]
     got = non_dominated_mask(f.to("cuda")).cpu().numpy()
     assert np.array_equal(got, c_oracle.first_front(f.numpy()))
+
+
+@pytest.mark.parametrize("n,m", [(1000, 3), (3000, 5), (20000, 3), (66000, 8), (70001, 2), (70001, 3)])
+def test_masks_in_a_graph(n, m):
+    """One capture, replayed on other populations with eager calls in between: nothing is left over from a replay."""
+    from evox_amd import runtime
+    from evox_amd.operators.selection import non_dominated_mask
+
+    static = population("shell", n, m, n).to("cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        non_dominated_mask(static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = non_dominated_mask(static)
+    for seed, kind in enumerate(("shell", "one front", "uniform", "special", "one front")):
+        f = population(kind, n, m, n + seed).to("cuda")
+        static.copy_(f)
+        graph.replay()
+        eager = non_dominated_mask(f)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), kind
+    del graph
+    runtime.release_workspaces()  # (those of the capture's stream among them)

@@ -155,3 +155,38 @@ def test_points_shared_by_several_workgroups(n, m, n_sample):
     exceeded = torch.stack([(s < fit).all(dim=1).any() for s in samples]).sum()
     for _ in range(2):
         assert int(ops.hv_covered_count(points, below)) == int(exceeded)
+
+
+@pytest.mark.parametrize("n, m, n_sample", [(500, 3, 5000), (30011, 3, 300), (20001, 8, 130)])
+def test_hypervolume_in_a_graph(n, m, n_sample):
+    """One capture, replayed on other points with eager calls in between; the counts of workgroups that share samples start
+    from zero in every replay."""
+    g = torch.Generator().manual_seed(n)
+
+    def draw():
+        return torch.rand(n, m, generator=g).to(DEV), torch.rand(n_sample, m, generator=g).to(DEV)
+
+    objs, u = draw()
+    ref, alpha = torch.full((m,), 1.2, device=DEV), torch.rand(n, generator=g).to(DEV)
+
+    def calls(objs, u):
+        return (ops.hv_estimate(objs, ref, u), ops.hype_contributions(objs, ref, n // 2, u), ops.hv_covered_count(objs, u),
+                ops.hv_contributions(objs, u, alpha, 1.0))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        calls(objs, u)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = calls(objs, u)
+    for _ in range(4):
+        new = draw()
+        objs.copy_(new[0])
+        u.copy_(new[1])
+        graph.replay()
+        eager = calls(*new)
+        torch.cuda.synchronize()
+        for got, want in zip(out, eager):
+            assert torch.equal(got, want)
