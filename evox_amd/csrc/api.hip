@@ -21,6 +21,7 @@
 #include "peel_lds.hpp"
 #include "prefix.hpp"
 #include "radix.hpp"
+#include "runs.hpp"
 #include "spatial.hpp"
 #include "stepped.hpp"
 #include "two.hpp"
@@ -868,18 +869,18 @@ static int radix_grid(const Layout& L) {
   return workers + kFirstSweeper;
 }
 
-// Grid of the two kernels that order the last front (finish.hpp): the radix grid when a front of this
-// population can exceed kRadixMinCandidates rows (they then synchronise across blocks), else one block
-// per 256 candidates and objective.
-// A last front of more than kMidSortMinCandidates rows in a population of at most kMidArgsortRows: its orders come from
-// workgroups that sort in LDS without waiting for each other (finish.hpp), one per compute unit.
+// The last front of a population of at most kMidArgsortRows rows goes through the kernels with the sorted runs (finish.hpp),
+// whose workgroups hold all its keys in LDS.
 static bool crowd_mid_sort(const Layout& L) { return opt().mid_argsort != 0 && L.n > kMidSortMinCandidates && L.n <= kMidArgsortRows; }
-// A larger population: such a front gets a launch of its own (its kernels have kMidArgsortThreads threads, the radix
-// sort of a larger front kRadixThreads); each of the two returns at once from a front that is the other's.
+// A larger population: a front of more than kMidSortMinCandidates and at most that many rows does; the other kernels return at
+// once from it, and these from any other.
 static bool crowd_mid_split(const Layout& L) { return opt().mid_argsort != 0 && L.n > kMidArgsortRows; }
 
+// Grid of crowd_gather_kernel, crowd_sort_kernel and crowd_finish_kernel (finish.hpp): the radix grid when a front of this
+// population can exceed kRadixMinCandidates rows (they then synchronise across blocks), else one block
+// per 256 candidates and objective.
 static int finish_grid(const Layout& L, int per_candidate_block) {
-  if (crowd_mid_sort(L)) return device_cus();  // (their LDS leaves room for one workgroup per compute unit: all resident)
+  if (crowd_mid_sort(L)) return device_cus();  // (crowd_gather_kernel with the LDS sorter: its LDS leaves room for one workgroup per compute unit: all resident)
   if (L.n > kRadixMinCandidates) {
     // The kernels choose on the device: a front of at most kRadixMinCandidates rows is still ordered by counting,
     // one work item per 256 candidates (and objective), and wants as many blocks as it has items -- a population
@@ -902,6 +903,13 @@ static int shared_grid(int grid, int resident, int batch) {
   if (batch <= 1) return grid;
   const int cap = resident / batch < 1 ? 1 : resident / batch;
   return grid < cap ? grid : cap;
+}
+
+// Workgroups of one population that place its candidates by searching the runs: one per compute unit, fewer where
+// several populations share the launch (none waits for another: at least sixteen).
+static int run_share_grid(const Ws& w) {
+  const int share = device_cus() / w.batch;
+  return share < 16 ? 16 : share;
 }
 
 // phase 0: totals and matrix in one launch (or what the tunable prefix_mode asks for); 1: the totals alone, and the
@@ -1064,10 +1072,11 @@ static CrowdArgs crowd_args(const Ws& w, const int* list, bool use_orders, int f
   a.param = w.at<SortParam>(L.sortparam);
   a.use_orders = use_orders ? 1 : 0;
   a.fused = fused;
-  a.mid_sort = crowd_mid_sort(L) ? 1 : (crowd_mid_split(L) ? 3 : 0);
+  a.mid_sort = crowd_mid_sort(L) ? 1 : (crowd_mid_split(L) ? 2 : 0);
   a.dist = w.at<float>(L.dist);
   a.dkey = w.at<uint32_t>(L.dkey);
   a.order = w.at<int>(L.order);
+  a.runs = w.at<uint32_t>(L.xs_sorted);
   a.ws_step = w.step;
   return a;
 }
@@ -1080,14 +1089,15 @@ static int stage_front_orders(const Ws& w, const int* list, hipStream_t s) {
     const int spans = (L.n + kFrontOrderSpan - 1) / kFrontOrderSpan;
     int* const number = reinterpret_cast<int*>(w.at<uint32_t>(L.dkey));  // free until the distances are known
     int* const per_span = b.table;
+    const int above = crowd_mid_split(L) ? kMidArgsortRows : kRadixMinCandidates;  // (smaller ones: the sorted runs)
     hipLaunchKernelGGL(front_number_kernel, dim3((L.n + 1023) / 1024), dim3(256), 0, s, list, w.ctrl(),
-                       w.at<SortParam>(L.sortparam), number);
+                       w.at<SortParam>(L.sortparam), above, number);
     EVX_LAUNCH_CHECK();
     hipLaunchKernelGGL(front_order_count_kernel, dim3(spans, L.m), dim3(256), 0, s, b.pairs[0], b.kstride, L.n, w.at<int>(L.rank),
-                       w.ctrl(), w.at<SortParam>(L.sortparam), per_span);
+                       w.ctrl(), w.at<SortParam>(L.sortparam), above, per_span);
     EVX_LAUNCH_CHECK();
     hipLaunchKernelGGL(front_order_place_kernel, dim3(spans, L.m), dim3(256), 0, s, b.pairs[0], b.kstride, L.n,
-                       w.at<int>(L.rank), w.ctrl(), w.at<SortParam>(L.sortparam), per_span, number, w.at<float>(L.xs), L.npad,
+                       w.at<int>(L.rank), w.ctrl(), w.at<SortParam>(L.sortparam), above, per_span, number, w.at<float>(L.xs), L.npad,
                        w.at<int>(L.pos), w.at<float>(L.scost));
     EVX_LAUNCH_CHECK();
   }
@@ -1102,92 +1112,114 @@ static size_t crowd_lds_bytes(const Layout& L, int fused) {
   return lds;
 }
 
+// The first two of the launches that order a front from sorted runs (finish.hpp).
+static int launch_crowd_runs(const Ws& w, const CrowdArgs& a, int tail_flag, hipStream_t s) {
+  const Layout& L = w.L;
+  const int most = L.n < kRunMaxRows ? L.n : kRunMaxRows;
+  const size_t runs_lds = a.mid_sort == 1 && a.fused != 0 ? kFusedFrontLdsBytes : sizeof(uint32_t) * 2 * kRunRows;
+  // (a small front: up to 64 workgroups of it, which wait for each other, are resident at once)
+  const int small_blocks = shared_grid(kFusedFrontRows * 16 / kRunRows, device_cus(), w.batch);
+  int grid = (most + kRunRows - 1) / kRunRows * L.m;
+  if (grid < small_blocks) grid = small_blocks;
+  if (grid > 65536) grid = 65536;
+  const void* const runs_kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_runs_kernel<true>) : reinterpret_cast<const void*>(crowd_runs_kernel<false>);
+  if (int e = grant_dynamic_lds(runs_kernel, runs_lds)) return e;
+  if (w.batch > 1)
+    hipLaunchKernelGGL(crowd_runs_kernel<true>, dim3(grid, 1, w.batch), dim3(kRunRows), runs_lds, s, a, tail_flag, small_blocks);
+  else
+    hipLaunchKernelGGL(crowd_runs_kernel<false>, dim3(grid), dim3(kRunRows), runs_lds, s, a, tail_flag, small_blocks);
+  EVX_LAUNCH_CHECK();
+  const size_t lds = run_rank_lds_bytes(most);
+  const void* const terms_kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_terms_kernel<true>) : reinterpret_cast<const void*>(crowd_terms_kernel<false>);
+  if (int e = grant_dynamic_lds(terms_kernel, lds)) return e;
+  if (w.batch > 1)
+    hipLaunchKernelGGL(crowd_terms_kernel<true>, dim3(run_share_grid(w), 1, w.batch), dim3(kRunRankThreads), lds, s, a, tail_flag);
+  else
+    hipLaunchKernelGGL(crowd_terms_kernel<false>, dim3(run_share_grid(w)), dim3(kRunRankThreads), lds, s, a, tail_flag);
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
+// The distances, and with `want_order` the selection order; `gather`: and the selected rows.
+static int launch_crowd_pick(const Ws& w, const CrowdArgs& a, bool want_order, const GatherArgs* gather, int tail_flag, hipStream_t s) {
+  const Layout& L = w.L;
+  const int most = L.n < kRunMaxRows ? L.n : kRunMaxRows;
+  const int runs = (most + kRunRows - 1) / kRunRows;
+  if (w.batch > 1)
+    hipLaunchKernelGGL(crowd_distances_kernel<true>, dim3(runs, 1, w.batch), dim3(kRunRows), 0, s, a, want_order ? 1 : 0, tail_flag);
+  else
+    hipLaunchKernelGGL(crowd_distances_kernel<false>, dim3(runs), dim3(kRunRows), 0, s, a, want_order ? 1 : 0, tail_flag);
+  EVX_LAUNCH_CHECK();
+  if (!want_order) return 0;
+  const int grid = run_share_grid(w);
+  const size_t picks_at = run_rank_lds_bytes(most);  // (a multiple of 16)
+  const size_t lds = picks_at + (gather != nullptr ? sizeof(int2) * (size_t)((most + grid - 1) / grid) : 0);
+  const GatherArgs g = gather != nullptr ? *gather : GatherArgs{};
+  auto launch = [&](auto kernel) {
+    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return e;
+    hipLaunchKernelGGL(kernel, dim3(grid, 1, w.batch), dim3(kRunRankThreads), lds, s, a, g, tail_flag, (int)picks_at);
+    return 0;
+  };
+  int e = 0;
+  if (w.batch > 1)
+    e = gather != nullptr ? launch(crowd_pick_kernel<true, true>) : launch(crowd_pick_kernel<true, false>);
+  else
+    e = gather != nullptr ? launch(crowd_pick_kernel<false, true>) : launch(crowd_pick_kernel<false, false>);
+  if (e) return e;
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
 static int stage_crowd_sort(const Ws& w, const int* list, bool use_orders, int fused, hipStream_t s, bool after_peel_tail = false) {
   const Layout& L = w.L;
+  const int tail_flag = after_peel_tail ? 1 : 0;
+  if (crowd_mid_sort(L)) return launch_crowd_runs(w, crowd_args(w, list, false, fused), tail_flag, s);
   use_orders = use_orders && prefix_dominance_applies(L) && w.batch == 1;
   // a large front of a population whose matrix came from the per-objective orders: its own orders are read off
-  // those (finish.hpp); the three kernels and the one below choose on the device which of them has work
+  // those (finish.hpp); the three kernels and those below choose on the device which of them has work
   if (use_orders)
     if (int e = stage_front_orders(w, list, s)) return e;
-  if (crowd_mid_split(L)) {
-    const size_t mid_lds = mid_sort_lds_bytes(kMidArgsortRows);
-    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(crowd_sort_kernel<kMidArgsortThreads, 2>), mid_lds)) return e;
-    CrowdArgs a = crowd_args(w, list, use_orders, fused);
-    a.mid_sort = 2;
-    hipLaunchKernelGGL((crowd_sort_kernel<kMidArgsortThreads, 2>), dim3(device_cus()), dim3(kMidArgsortThreads), mid_lds, s, a,
-                       after_peel_tail ? 1 : 0);
-    EVX_LAUNCH_CHECK();
-  }
+  const CrowdArgs a = crowd_args(w, list, use_orders, fused);
+  if (crowd_mid_split(L))
+    if (int e = launch_crowd_runs(w, a, tail_flag, s)) return e;
   const size_t lds = crowd_lds_bytes(L, fused);
-  const bool mid = crowd_mid_sort(L);
-  const bool wide = L.n <= kMidArgsortWideRows;  // (which tables of the LDS sorter the population leaves room for)
-  const bool many = w.batch > 1;
-  auto instance = [&](auto one, auto several) { return many ? reinterpret_cast<const void*>(several) : reinterpret_cast<const void*>(one); };
-  const void* const kernel = !mid   ? instance(crowd_sort_kernel<kRadixThreads, 0, false>, crowd_sort_kernel<kRadixThreads, 0, true>)
-                             : wide ? instance(crowd_sort_kernel<kMidArgsortThreads, 1, false>, crowd_sort_kernel<kMidArgsortThreads, 1, true>)
-                                    : instance(crowd_sort_kernel<kMidArgsortThreads, 2, false>, crowd_sort_kernel<kMidArgsortThreads, 2, true>);
+  const void* const kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_sort_kernel<true>) : reinterpret_cast<const void*>(crowd_sort_kernel<false>);
   if (int e = grant_dynamic_lds(kernel, lds)) return e;
   // (the fused path ends with a barrier between all blocks: the grid must be resident at once, which a grid of at
   // most two blocks of 256 threads per compute unit is)
   int grid = finish_grid(L, L.m);
   if (fused != 0 && grid > device_cus() * 2) grid = device_cus() * 2;
-  grid = shared_grid(grid, mid ? device_cus() : device_cus() * 2, w.batch);
-  const CrowdArgs ca = crowd_args(w, list, use_orders, fused);
-  const int tail_flag = after_peel_tail ? 1 : 0;
-  if (mid && wide && many)
-    hipLaunchKernelGGL((crowd_sort_kernel<kMidArgsortThreads, 1, true>), dim3(grid, 1, w.batch), dim3(kMidArgsortThreads), lds, s, ca, tail_flag);
-  else if (mid && wide)
-    hipLaunchKernelGGL((crowd_sort_kernel<kMidArgsortThreads, 1, false>), dim3(grid), dim3(kMidArgsortThreads), lds, s, ca, tail_flag);
-  else if (mid && many)
-    hipLaunchKernelGGL((crowd_sort_kernel<kMidArgsortThreads, 2, true>), dim3(grid, 1, w.batch), dim3(kMidArgsortThreads), lds, s, ca, tail_flag);
-  else if (mid)
-    hipLaunchKernelGGL((crowd_sort_kernel<kMidArgsortThreads, 2, false>), dim3(grid), dim3(kMidArgsortThreads), lds, s, ca, tail_flag);
-  else if (many)
-    hipLaunchKernelGGL((crowd_sort_kernel<kRadixThreads, 0, true>), dim3(grid, 1, w.batch), dim3(kRadixThreads), lds, s, ca, tail_flag);
+  grid = shared_grid(grid, device_cus() * 2, w.batch);
+  if (w.batch > 1)
+    hipLaunchKernelGGL(crowd_sort_kernel<true>, dim3(grid, 1, w.batch), dim3(kRadixThreads), lds, s, a, tail_flag);
   else
-    hipLaunchKernelGGL((crowd_sort_kernel<kRadixThreads, 0, false>), dim3(grid), dim3(kRadixThreads), lds, s, ca, tail_flag);
+    hipLaunchKernelGGL(crowd_sort_kernel<false>, dim3(grid), dim3(kRadixThreads), lds, s, a, tail_flag);
   EVX_LAUNCH_CHECK();
   return 0;
 }
 
-// Crowding distances of those candidates and, with want_order, the selection order.
-static int stage_crowd_finish(const Ws& w, const int* list, bool want_order, int fused, hipStream_t s, bool after_peel_tail = false) {
+// Crowding distances of those candidates and, with want_order, the selection order; gather, where it is given: the
+// selected rows too, behind the order (crowd_mid_sort populations only).
+static int stage_crowd_finish(const Ws& w, const int* list, bool want_order, int fused, hipStream_t s, bool after_peel_tail = false,
+                              const GatherArgs* gather = nullptr) {
   const Layout& L = w.L;
-  // (no front of this population is too large for the fused path of crowd_sort_kernel: nothing is left to do)
-  if (fused != 0 && L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives) return 0;
-  if (crowd_mid_split(L)) {
-    const size_t mid_lds = mid_sort_lds_bytes(kMidArgsortRows);
-    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(crowd_finish_kernel<kMidArgsortThreads, 2>), mid_lds)) return e;
-    CrowdArgs a = crowd_args(w, list, false, fused);
-    a.mid_sort = 2;
-    hipLaunchKernelGGL((crowd_finish_kernel<kMidArgsortThreads, 2>), dim3(device_cus()), dim3(kMidArgsortThreads), mid_lds, s, a,
-                       want_order ? 1 : 0, after_peel_tail ? 1 : 0);
-    EVX_LAUNCH_CHECK();
-  }
+  const int tail_flag = after_peel_tail ? 1 : 0;
+  const CrowdArgs a = crowd_args(w, list, false, fused);
+  if (gather == nullptr && fused != 0 && L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives)
+    return 0;  // (no front of this population is too large for crowd_small_front: nothing is left to do)
+  if (crowd_mid_sort(L)) return launch_crowd_pick(w, a, want_order, gather, tail_flag, s);
+  if (gather != nullptr) return kErrBadArg;
+  if (crowd_mid_split(L))
+    if (int e = launch_crowd_pick(w, a, want_order, nullptr, tail_flag, s)) return e;
   const size_t lds = crowd_lds_bytes(L, 0);
-  const bool mid = crowd_mid_sort(L);
-  const bool wide = L.n <= kMidArgsortWideRows;
-  const bool many = w.batch > 1;
-  auto instance = [&](auto one, auto several) { return many ? reinterpret_cast<const void*>(several) : reinterpret_cast<const void*>(one); };
-  const void* const kernel = !mid   ? instance(crowd_finish_kernel<kRadixThreads, 0, false>, crowd_finish_kernel<kRadixThreads, 0, true>)
-                             : wide ? instance(crowd_finish_kernel<kMidArgsortThreads, 1, false>, crowd_finish_kernel<kMidArgsortThreads, 1, true>)
-                                    : instance(crowd_finish_kernel<kMidArgsortThreads, 2, false>, crowd_finish_kernel<kMidArgsortThreads, 2, true>);
+  const void* const kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_finish_kernel<true>) : reinterpret_cast<const void*>(crowd_finish_kernel<false>);
   if (int e = grant_dynamic_lds(kernel, lds)) return e;
-  const int grid = shared_grid(finish_grid(L, 1), mid ? device_cus() : device_cus() * 2, w.batch);
-  const CrowdArgs ca = crowd_args(w, list, false, fused);
-  const int order_flag = want_order ? 1 : 0, tail_flag = after_peel_tail ? 1 : 0;
-  if (mid && wide && many)
-    hipLaunchKernelGGL((crowd_finish_kernel<kMidArgsortThreads, 1, true>), dim3(grid, 1, w.batch), dim3(kMidArgsortThreads), lds, s, ca, order_flag, tail_flag);
-  else if (mid && wide)
-    hipLaunchKernelGGL((crowd_finish_kernel<kMidArgsortThreads, 1, false>), dim3(grid), dim3(kMidArgsortThreads), lds, s, ca, order_flag, tail_flag);
-  else if (mid && many)
-    hipLaunchKernelGGL((crowd_finish_kernel<kMidArgsortThreads, 2, true>), dim3(grid, 1, w.batch), dim3(kMidArgsortThreads), lds, s, ca, order_flag, tail_flag);
-  else if (mid)
-    hipLaunchKernelGGL((crowd_finish_kernel<kMidArgsortThreads, 2, false>), dim3(grid), dim3(kMidArgsortThreads), lds, s, ca, order_flag, tail_flag);
-  else if (many)
-    hipLaunchKernelGGL((crowd_finish_kernel<kRadixThreads, 0, true>), dim3(grid, 1, w.batch), dim3(kRadixThreads), lds, s, ca, order_flag, tail_flag);
+  const int grid = shared_grid(finish_grid(L, 1), device_cus() * 2, w.batch);
+  const int order_flag = want_order ? 1 : 0;
+  if (w.batch > 1)
+    hipLaunchKernelGGL(crowd_finish_kernel<true>, dim3(grid, 1, w.batch), dim3(kRadixThreads), lds, s, a, order_flag, tail_flag);
   else
-    hipLaunchKernelGGL((crowd_finish_kernel<kRadixThreads, 0, false>), dim3(grid), dim3(kRadixThreads), lds, s, ca, order_flag, tail_flag);
+    hipLaunchKernelGGL(crowd_finish_kernel<false>, dim3(grid), dim3(kRadixThreads), lds, s, a, order_flag, tail_flag);
   EVX_LAUNCH_CHECK();
   return 0;
 }
@@ -2327,6 +2359,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
       if (e) return e == kErrNotResident ? kErrBadArg : e;
       // the last front by the ordering kernels, then the gather, as after a peel that leaves the last front alone
       if (int c = stage_crowd_sort(w, w.at<int>(L.perm), false, 2, s, false)) return c;
+      if (crowd_mid_sort(L)) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, false, &g);
       if (int c = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, false)) return c;
       launch_gather(false);
       EVX_LAUNCH_CHECK();
@@ -2358,15 +2391,16 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   g.outcome = batch == 1 && peel_orders && !peel_always_orders && opt().launch_memory ? outcome_slot(n, m, may_allocate, s) : nullptr;
   const int last_outcome = g.outcome != nullptr ? __atomic_load_n(g.outcome, __ATOMIC_RELAXED) : 0;
   // Where the peel kernel may have ordered the last front, the kernels that would order it look at Ctrl.tail_done and
-  // return at once.  A launch that does nothing still costs about 4.7 us, so with up to three objectives -- last
-  // fronts of a few hundred rows, which the peel kernel orders -- the two ordering stages and the gather share one
+  // return at once.  A launch that does nothing still costs 2 to 4.7 us, so with up to three objectives -- last
+  // fronts of a few hundred rows, which the peel kernel orders -- all ordering stages and the gather share one
   // launch (crowd_gather_kernel); with more objectives the last front is usually too large for the peel kernel, and
-  // the two stages as kernels of their own, each on the grid that suits it, order it faster than the shared launch does
-  // (20 000 x 5, a front of 2532 rows: 245 against 261 us per selection; 20 000 x 8, 7481 rows: 457 against 493).
+  // the stages as kernels of their own order it faster than the shared launch does (20 000 x 5, a front of 2532 rows:
+  // 138 us per selection).
   // What the last selection of this shape found decides where it is known: a population that has converged keeps
-  // last fronts of thousands of rows, which the kernels of their own order 20-30 us faster (20 000 x 3, one front: 166
-  // against 194 us), and a last front that the peel ordered will mostly be followed by another.
-  const bool one_ordering_launch = peel_orders && opt().tail_merged && L.m <= 3 && last_outcome != 2;
+  // last fronts of thousands of rows, which the kernels of their own order 40 us faster (20 001 x 3, one front: 114
+  // against 155 us), and a last front that the peel ordered will mostly be followed by another (2000 x 5: 55 -> 52.7 us
+  // in the one launch, 57 in the four).
+  const bool one_ordering_launch = peel_orders && opt().tail_merged && (L.m <= 3 ? last_outcome != 2 : last_outcome == 1);
   if (stepped) {
     // distances of the rows of the last front (the mask rank == worst), the order by (rank, distance descending, index)
     // from three stable argsort steps, the gather: the fitness is read from its structure-of-arrays copy
@@ -2405,6 +2439,8 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   }
   if (!one_ordering_launch) {
     if (int e = stage_crowd_sort(w, w.at<int>(L.perm), true, 2, s, peel_orders)) return e;
+    const bool never_large = L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives;
+    if (crowd_mid_sort(L) && !never_large) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, &g);
     if (int e = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders)) return e;
     if (peel_orders)
       launch_gather(true);

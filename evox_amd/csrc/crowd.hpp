@@ -169,33 +169,8 @@ __device__ __forceinline__ void to_population(GatherArgs& g) {
   if (g.out_order != nullptr) g.out_order += b * g.topk;
 }
 
-// Called by every thread of `blocks` blocks of 256 threads (`block` = the caller's index among them).
-// listed_until: positions below it take their row from a.listed instead of a.order.
-__device__ inline void gather_body(const GatherArgs& a, int block, int blocks, int listed_until) {
-  const int topk = a.topk, m = a.m, unit = a.unit, n_first = a.n_first;
-  const uint8_t* __restrict__ x = a.x;
-  const uint8_t* __restrict__ x2 = a.x2;
-  uint8_t* __restrict__ out_x = a.out_x;
-  const int64_t x_row_bytes = a.x_row_bytes;
-  float* __restrict__ out_f = a.out_f;
-  int* __restrict__ out_rank = a.out_rank;
-  float* __restrict__ out_dist = a.out_dist;
-  int* __restrict__ out_order = a.out_order;
-  if (a.ctrl->err != 0 || (a.order_from_peel != 0 && a.ctrl->tail_done == 0)) {
-    // a device-side wait ran out and `order` was not produced: no partial result leaves the call -- rank -1,
-    // distance and fitness NaN, order -1, decision vectors all-ones bytes (NaN as floats)
-    const int64_t threads = (int64_t)blocks * blockDim.x, t0 = (int64_t)block * blockDim.x + threadIdx.x;
-    for (int64_t p = t0; p < topk; p += threads) {
-      out_rank[p] = -1;
-      out_dist[p] = __uint_as_float(0x7FC00000u);
-      if (out_order) out_order[p] = -1;
-    }
-    for (int64_t e = t0; e < (int64_t)topk * m; e += threads) out_f[e] = __uint_as_float(0x7FC00000u);
-    if (x)
-      for (int64_t b = t0; b < (int64_t)topk * x_row_bytes; b += threads) out_x[b] = 0xFF;
-    return;
-  }
-  // (for the host's choice of launches at its next call; it reads the word without waiting for anything)
+// What the host's choice of launches at its next call goes by (it reads the words without waiting for anything).
+__device__ __forceinline__ void gather_notes(const GatherArgs& a, int block) {
   if (a.outcome != nullptr && block == 0 && threadIdx.x == 0)
     __hip_atomic_store(a.outcome, a.ctrl->tail_done != 0 ? 1 : 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (a.front0_note != nullptr && block == 0 && threadIdx.x == 0) {
@@ -203,51 +178,83 @@ __device__ inline void gather_body(const GatherArgs& a, int block, int blocks, i
     const int now = *a.front0_size >= a.front0_enough ? (before == 1 || before == 3 ? 3 : 1) : 2;
     __hip_atomic_store(a.front0_note, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  // A row is copied by g lanes, g = the smallest power of two (4 .. 64) that holds the row's units and its m
-  // fitness values: short rows share a wave (a row of 400 bytes in 16-byte units took 25 of 64 lanes).
-  const int64_t units = (x ? x_row_bytes : 0) / unit;
+}
+
+// A row is copied by g lanes, g = the smallest power of two (4 .. 64) that holds the row's units and its m
+// fitness values: short rows share a wave (a row of 400 bytes in 16-byte units took 25 of 64 lanes).
+__device__ __forceinline__ int gather_lanes(const GatherArgs& a) {
+  const int64_t units = (a.x ? a.x_row_bytes : 0) / a.unit;
   int g = 64;
-  while (g > 4 && (g >> 1) >= units && (g >> 1) >= m) g >>= 1;
+  while (g > 4 && (g >> 1) >= units && (g >> 1) >= a.m) g >>= 1;
+  return g;
+}
+
+// Row `src` of the population becomes row p of the results, by `g` lanes.
+__device__ __forceinline__ void gather_row(const GatherArgs& a, int64_t p, int64_t src, int lane, int g) {
+  const int m = a.m, unit = a.unit;
+  const int64_t x_row_bytes = a.x_row_bytes;
+  if (src < 0) {  // an order that a failed sort has poisoned: no row is read through it, the outputs say so
+    if (a.x)
+      for (int64_t b = lane; b < x_row_bytes; b += g) a.out_x[p * x_row_bytes + b] = 0xFF;
+    for (int k = lane; k < m; k += g) a.out_f[p * m + k] = __uint_as_float(0x7FC00000u);
+    if (lane == 0) {
+      a.out_rank[p] = -1;
+      a.out_dist[p] = __uint_as_float(0x7FC00000u);
+      if (a.out_order) a.out_order[p] = -1;
+    }
+    return;
+  }
+  const bool second = src >= a.n_first;  // rows of the second part of a two-part population
+  if (a.x) {
+    const uint8_t* __restrict__ s = second ? a.x2 + (src - a.n_first) * a.x2_row_stride : a.x + src * a.x_row_stride;
+    uint8_t* __restrict__ d = a.out_x + p * x_row_bytes;
+    if (unit == 16) {
+      for (int64_t b = lane * 16; b < x_row_bytes; b += g * 16)
+        *reinterpret_cast<uint4*>(d + b) = *reinterpret_cast<const uint4*>(s + b);
+    } else if (unit == 4) {
+      for (int64_t b = lane * 4; b < x_row_bytes; b += g * 4)
+        *reinterpret_cast<uint32_t*>(d + b) = *reinterpret_cast<const uint32_t*>(s + b);
+    } else {
+      for (int64_t b = lane; b < x_row_bytes; b += g) d[b] = s[b];
+    }
+  }
+  for (int k = lane; k < m; k += g)
+    a.out_f[p * m + k] = second ? a.f2[(src - a.n_first) * a.f2_stride_row + k * a.f2_stride_col]
+                                : a.f[src * a.f_stride_row + k * a.f_stride_col];
+  if (lane == 0) {
+    a.out_rank[p] = a.rank[src];
+    a.out_dist[p] = a.dist[src];
+    if (a.out_order) a.out_order[p] = (int)src;
+  }
+}
+
+// Called by every thread of `blocks` blocks (`block` = the caller's index among them).
+// listed_until: positions below it take their row from a.listed instead of a.order.
+__device__ inline void gather_body(const GatherArgs& a, int block, int blocks, int listed_until) {
+  const int topk = a.topk, m = a.m;
+  const int64_t x_row_bytes = a.x_row_bytes;
+  if (a.ctrl->err != 0 || (a.order_from_peel != 0 && a.ctrl->tail_done == 0)) {
+    // a device-side wait ran out and `order` was not produced: no partial result leaves the call -- rank -1,
+    // distance and fitness NaN, order -1, decision vectors all-ones bytes (NaN as floats)
+    const int64_t threads = (int64_t)blocks * blockDim.x, t0 = (int64_t)block * blockDim.x + threadIdx.x;
+    for (int64_t p = t0; p < topk; p += threads) {
+      a.out_rank[p] = -1;
+      a.out_dist[p] = __uint_as_float(0x7FC00000u);
+      if (a.out_order) a.out_order[p] = -1;
+    }
+    for (int64_t e = t0; e < (int64_t)topk * m; e += threads) a.out_f[e] = __uint_as_float(0x7FC00000u);
+    if (a.x)
+      for (int64_t b = t0; b < (int64_t)topk * x_row_bytes; b += threads) a.out_x[b] = 0xFF;
+    return;
+  }
+  gather_notes(a, block);
+  const int g = gather_lanes(a);
   const int per_wave = 64 / g;
   const int lane = (threadIdx.x & 63) % g, sub = (threadIdx.x & 63) / g;
   const int64_t waves = (int64_t)blocks * (blockDim.x >> 6);
   for (int64_t p = ((int64_t)block * (blockDim.x >> 6) + (threadIdx.x >> 6)) * per_wave + sub; p < topk;
-       p += waves * per_wave) {
-    const int64_t src = p < listed_until ? a.listed[p] : a.order[p];
-    if (src < 0) {  // an order that a failed sort has poisoned: no row is read through it, the outputs say so
-      if (x)
-        for (int64_t b = lane; b < x_row_bytes; b += g) out_x[p * x_row_bytes + b] = 0xFF;
-      for (int k = lane; k < m; k += g) out_f[p * m + k] = __uint_as_float(0x7FC00000u);
-      if (lane == 0) {
-        out_rank[p] = -1;
-        out_dist[p] = __uint_as_float(0x7FC00000u);
-        if (out_order) out_order[p] = -1;
-      }
-      continue;
-    }
-    const bool second = src >= n_first;  // rows of the second part of a two-part population
-    if (x) {
-      const uint8_t* __restrict__ s = second ? x2 + (src - n_first) * a.x2_row_stride : x + src * a.x_row_stride;
-      uint8_t* __restrict__ d = out_x + p * x_row_bytes;
-      if (unit == 16) {
-        for (int64_t b = lane * 16; b < x_row_bytes; b += g * 16)
-          *reinterpret_cast<uint4*>(d + b) = *reinterpret_cast<const uint4*>(s + b);
-      } else if (unit == 4) {
-        for (int64_t b = lane * 4; b < x_row_bytes; b += g * 4)
-          *reinterpret_cast<uint32_t*>(d + b) = *reinterpret_cast<const uint32_t*>(s + b);
-      } else {
-        for (int64_t b = lane; b < x_row_bytes; b += g) d[b] = s[b];
-      }
-    }
-    for (int k = lane; k < m; k += g)
-      out_f[p * m + k] = second ? a.f2[(src - n_first) * a.f2_stride_row + k * a.f2_stride_col]
-                                : a.f[src * a.f_stride_row + k * a.f_stride_col];
-    if (lane == 0) {
-      out_rank[p] = a.rank[src];
-      out_dist[p] = a.dist[src];
-      if (out_order) out_order[p] = (int)src;
-    }
-  }
+       p += waves * per_wave)
+    gather_row(a, p, p < listed_until ? a.listed[p] : a.order[p], lane, g);
 }
 
 // Winner of every tournament: the candidate that comes first when the tournament's candidates are

@@ -1,21 +1,21 @@
-// The two kernels that follow the peeling: the per-objective ordering of the last front, and its
-// crowding distances together with the index-stable top-k.
+// The kernels that follow the peeling: the crowding distances of the last front and the index-stable top-k.
 //
 // Reference semantics:
 //   crowding_distance            src/evox/operators/selection/non_dominate.py:198-231
 //   lexsort (stable, last key primary)   src/evox/utils/jit_fix_operator.py:246-252
 //   nd_environmental_selection   non_dominate.py:250-254
 //
-// The size of the last front is only known on the device, and two orderings exist for it: ranking by
-// counting (crowd.hpp: one pass, no dependent steps) for fronts of at most kRadixMinCandidates rows and
-// the segmented radix sort (radix.hpp: persistent, grid barriers) above.  Each kernel here holds both
-// and picks one when it runs, so that a selection costs two launches after the peeling instead of one
-// launch per variant and stage.
+// The size of the last front is only known on the device.  Populations of at most kMidArgsortRows rows take four launches
+// that never wait (crowd_runs_kernel and those after it; a small front is done in the first of them).  Larger ones have
+// these for fronts of that size, and beside them crowd_sort_kernel and crowd_finish_kernel, which hold ranking by counting
+// (crowd.hpp: one pass, no dependent steps, for fronts of at most kRadixMinCandidates rows) and the segmented radix sort
+// (radix.hpp: persistent, grid barriers) above and pick one when they run.
 #pragma once
 
 #include "crowd.hpp"
 #include "order.hpp"
 #include "radix.hpp"
+#include "runs.hpp"
 
 namespace evx {
 
@@ -62,11 +62,13 @@ __device__ inline bool fused_front_applies(int nv, int m) {
   return nv <= kFusedFrontRows && (int64_t)nv * m <= kFusedFrontValues && m <= kFusedFrontObjectives;
 }
 
-// mode 1: distances only; mode 2: distances and the selection order.  Called by every thread of every block;
-// blockDim.x == kRadixThreads.  lds: kFusedFrontLdsBytes.
+// mode 1: distances only; mode 2: distances and the selection order.  Called by every thread of every block (blockDim.x
+// a multiple of 64); at most `most_blocks` of them, which are resident at once, wait for each other.  lds:
+// kFusedFrontLdsBytes.
 __device__ inline void crowd_small_front(const float* __restrict__ xs, int npad, const int* __restrict__ list_base,
                                          Ctrl* __restrict__ ctrl, int m, float* __restrict__ dist, uint32_t* __restrict__ dkey,
-                                         int* __restrict__ order, unsigned spin_limit, int mode, uint64_t* lds, int* scratch) {
+                                         int* __restrict__ order, unsigned spin_limit, int mode, int most_blocks, uint64_t* lds,
+                                         int* scratch) {
   const int nv = ctrl->nv, start = ctrl->worst_start, need = ctrl->need;
   const int* __restrict__ list = list_base + start;
   const int tid = threadIdx.x, sub = tid & 15;
@@ -80,7 +82,7 @@ __device__ inline void crowd_small_front(const float* __restrict__ xs, int npad,
   // ... and a front of up to kFusedFrontRows rows that of as many workgroups as have sixteen candidates each: the
   // barrier below costs every workgroup that arrives a write-back and an invalidation of its die's cache (the 512
   // workgroups of the grid of a population of 200 000 rows: 100 us for a front of 600 rows)
-  const int active = solo ? 1 : min((int)gridDim.x, (nv + (int)(blockDim.x >> 4) - 1) / (int)(blockDim.x >> 4));
+  const int active = solo ? 1 : min(most_blocks, (nv + (int)(blockDim.x >> 4) - 1) / (int)(blockDim.x >> 4));
   if (mode == 2)  // the better fronts keep the order in which they are listed
     for (int i = blockIdx.x * blockDim.x + tid; i < start; i += gridDim.x * blockDim.x) order[i] = list_base[i];
   if ((int)blockIdx.x >= active) return;
@@ -198,20 +200,21 @@ struct CrowdArgs {
   unsigned spin_limit;
   SortParam* param;
   int use_orders, fused;
-  // The LDS sorter (mid_argsort_slice) for fronts of kMidSortMinCandidates + 1 to kMidArgsortRows rows: 0 = not used;
-  // 1 = this launch has it beside everything else (kMidArgsortThreads threads, populations up to kMidArgsortRows);
-  // larger populations get two launches: 2 = this one (kMidArgsortThreads threads) orders such a front and nothing
-  // else, 3 = this one (kRadixThreads threads) leaves such a front to the other.
+  // Who orders a front that is too large for crowd_small_front: 0 = counting up to kRadixMinCandidates rows, above them
+  // the radix sort; 1 = a population of at most kMidArgsortRows rows: the sorted runs below (crowd_gather_kernel, which
+  // has it all in one launch: the LDS sorter mid_argsort_slice); 2 = a larger population: the sorted runs take a front of
+  // kMidSortMinCandidates + 1 to kMidArgsortRows rows, and the other launches leave it alone.
   int mid_sort;
   float* dist;
   uint32_t* dkey;
   int* order;
+  uint32_t* runs;  // sorted runs of the candidates' keys, objectives npad apart (the slot-ordered fitness, dead by now)
   int64_t ws_step;  // several populations in one launch: bytes from one population's buffers to the next one's
 };
 
 __device__ __forceinline__ void to_population(CrowdArgs& a) {
   to_population(a.ws_step, a.xs, a.list_base, a.ctrl, a.pos, a.sorted_cost, a.buf.pairs[0], a.buf.pairs[1], a.buf.table, a.buf.totals,
-                a.param, a.dist, a.dkey, a.order);
+                a.param, a.dist, a.dkey, a.order, a.runs);
 }
 
 // Whether a last front of nv rows is ordered by workgroups that sort in LDS (the same answer in every workgroup).
@@ -219,17 +222,13 @@ __device__ __forceinline__ void to_population(CrowdArgs& a) {
 // the 24 workgroups that the counting keeps busy.
 constexpr int kMidSortMinCandidates = 1024;
 __device__ inline bool crowd_mid_applies(const CrowdArgs& a, int nv) {
-  return (a.mid_sort == 1 || a.mid_sort == 2) && nv > kMidSortMinCandidates && nv <= kMidArgsortRows &&
-         blockDim.x == kMidArgsortThreads;
+  return a.mid_sort == 1 && nv > kMidSortMinCandidates && nv <= kMidArgsortRows && blockDim.x == kMidArgsortThreads;
 }
-// Where the work is split over two launches (mid_sort 2 and 3): whether the one with the LDS sorter orders the front
-// by objective (`by_objective`) or by distance.  A front that crowd_small_front takes, or whose per-objective orders
-// are read off those of the population, is not the LDS sorter's.
-__device__ inline bool crowd_mid_takes(const CrowdArgs& a, int nv, bool by_objective) {
-  if (nv <= kMidSortMinCandidates || nv > kMidArgsortRows) return false;
+// Whether the kernels with the sorted runs order the front.  A front that crowd_small_front takes is not theirs.
+static_assert(kRunMaxRows == kMidArgsortRows, "the runs of a front must fit the LDS of a workgroup");
+__device__ inline bool crowd_runs_take(const CrowdArgs& a, int nv) {
   if (a.fused != 0 && fused_front_applies(nv, a.m)) return false;
-  if (by_objective && nv > kRadixMinCandidates && a.use_orders != 0 && a.param->orders_valid != 0) return false;
-  return true;
+  return a.mid_sort == 1 || (a.mid_sort == 2 && nv > kMidSortMinCandidates && nv <= kMidArgsortRows);
 }
 
 // `epochs`: how many epochs of radix barrier generations the control block's counter moves on when the radix path
@@ -252,9 +251,9 @@ __device__ inline void crowd_sort_body(const CrowdArgs& a, unsigned gen0, int ep
   int* __restrict__ order = a.order;
   if (coherent_load(&ctrl->err) != 0) return;
   const int nv = ctrl->nv;
-  if (a.mid_sort >= 2 && (a.mid_sort == 2) != crowd_mid_takes(a, nv, true)) return;  // the other launch's front
+  if (a.mid_sort == 2 && crowd_runs_take(a, nv)) return;  // another launch's front
   if (fused != 0 && fused_front_applies(nv, m)) {  // a small front: distances (and order) right here
-    crowd_small_front(xs, npad, list_base, ctrl, m, dist, dkey, order, spin_limit, fused, finish_lds, scratch);
+    crowd_small_front(xs, npad, list_base, ctrl, m, dist, dkey, order, spin_limit, fused, (int)gridDim.x, finish_lds, scratch);
     return;
   }
   const int* __restrict__ list = list_base + ctrl->worst_start;
@@ -322,16 +321,14 @@ __device__ inline void crowd_sort_body(const CrowdArgs& a, unsigned gen0, int ep
 }
 
 // after_peel_tail: the peel kernel may have ordered the last front already (Ctrl.tail_done).
-// T threads: kRadixThreads, or kMidArgsortThreads where CrowdArgs.mid_sort is set (the radix sort, which is written for
-// kRadixThreads, does not run then).
-template <int T, int TABLES, bool MANY = false>
-__global__ __launch_bounds__(T) void crowd_sort_kernel(CrowdArgs a, int after_peel_tail) {
+template <bool MANY>
+__global__ __launch_bounds__(kRadixThreads) void crowd_sort_kernel(CrowdArgs a, int after_peel_tail) {
   extern __shared__ __attribute__((aligned(16))) uint64_t finish_lds[];
   __shared__ int base[256];
   __shared__ int scratch[kRadixThreads];
   if constexpr (MANY) to_population(a);  // several populations in the launch, one per blockIdx.z
   if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
-  crowd_sort_body<TABLES>(a, radix_generation_base(a.ctrl), 1, finish_lds, base, scratch);
+  crowd_sort_body<0>(a, radix_generation_base(a.ctrl), 1, finish_lds, base, scratch);
 }
 
 // ---- The same per-objective order of a large last front, taken from the orders of the whole population that
@@ -341,14 +338,15 @@ __global__ __launch_bounds__(T) void crowd_sort_kernel(CrowdArgs a, int after_pe
 // dependence between workgroups inside a launch; each does nothing unless the front is large and the orders are valid.
 constexpr int kFrontOrderSpan = 1024;  // positions per workgroup
 
-__device__ inline bool front_orders_apply(const Ctrl* ctrl, const SortParam* param) {
-  return ctrl->err == 0 && param->orders_valid != 0 && ctrl->nv > kRadixMinCandidates;
+// above: fronts of at most this many rows are ordered otherwise.
+__device__ inline bool front_orders_apply(const Ctrl* ctrl, const SortParam* param, int above) {
+  return ctrl->err == 0 && param->orders_valid != 0 && ctrl->nv > above;
 }
 
 // number[list[q]] = q: the candidate number of every row of the front.
 __global__ __launch_bounds__(256) void front_number_kernel(const int* __restrict__ list_base, const Ctrl* __restrict__ ctrl,
-                                                           const SortParam* __restrict__ param, int* __restrict__ number) {
-  if (!front_orders_apply(ctrl, param)) return;
+                                                           const SortParam* __restrict__ param, int above, int* __restrict__ number) {
+  if (!front_orders_apply(ctrl, param, above)) return;
   const int nv = ctrl->nv;
   const int* __restrict__ list = list_base + ctrl->worst_start;
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nv; q += gridDim.x * blockDim.x) number[list[q]] = q;
@@ -357,9 +355,9 @@ __global__ __launch_bounds__(256) void front_number_kernel(const int* __restrict
 // per_span[k * gridDim.x + b] = candidates among positions b * kFrontOrderSpan ... of objective k = blockIdx.y.
 __global__ __launch_bounds__(256) void front_order_count_kernel(const unsigned long long* __restrict__ sorted, int kstride, int n,
                                                                 const int* __restrict__ rank, const Ctrl* __restrict__ ctrl,
-                                                                const SortParam* __restrict__ param, int* __restrict__ per_span) {
+                                                                const SortParam* __restrict__ param, int above, int* __restrict__ per_span) {
   __shared__ int total;
-  if (!front_orders_apply(ctrl, param)) return;
+  if (!front_orders_apply(ctrl, param, above)) return;
   const int worst = ctrl->worst;
   const int k = blockIdx.y;
   if (threadIdx.x == 0) total = 0;
@@ -379,13 +377,13 @@ __global__ __launch_bounds__(256) void front_order_count_kernel(const unsigned l
 // pos[k][number] and sorted_cost[k][position] of the candidates among the positions of this workgroup.
 __global__ __launch_bounds__(256) void front_order_place_kernel(const unsigned long long* __restrict__ sorted, int kstride, int n,
                                                                 const int* __restrict__ rank, const Ctrl* __restrict__ ctrl,
-                                                                const SortParam* __restrict__ param,
+                                                                const SortParam* __restrict__ param, int above,
                                                                 const int* __restrict__ per_span, const int* __restrict__ number,
                                                                 const float* __restrict__ xs, int npad, int* __restrict__ pos,
                                                                 float* __restrict__ sorted_cost) {
   __shared__ int before_span;
   __shared__ int wave_count[kFrontOrderSpan / 256][4];
-  if (!front_orders_apply(ctrl, param)) return;
+  if (!front_orders_apply(ctrl, param, above)) return;
   const int worst = ctrl->worst;
   const int k = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -455,7 +453,7 @@ __device__ inline void crowd_finish_body(const CrowdArgs& a, int want_order, uns
   int* __restrict__ order = a.order;
   if (coherent_load(&ctrl->err) != 0) return;
   const int nv = ctrl->nv;
-  if (a.mid_sort >= 2 && (a.mid_sort == 2) != crowd_mid_takes(a, nv, false)) return;  // the other launch's front
+  if (a.mid_sort == 2 && crowd_runs_take(a, nv)) return;  // another launch's front
   if (fused != 0 && fused_front_applies(nv, m)) return;  // crowd_sort_kernel has done it all
   const int start = ctrl->worst_start;
   const int need = ctrl->need;
@@ -549,14 +547,187 @@ __device__ inline void crowd_finish_body(const CrowdArgs& a, int want_order, uns
   }
 }
 
-template <int T, int TABLES, bool MANY = false>
-__global__ __launch_bounds__(T) void crowd_finish_kernel(CrowdArgs a, int want_order, int after_peel_tail) {
+template <bool MANY>
+__global__ __launch_bounds__(kRadixThreads) void crowd_finish_kernel(CrowdArgs a, int want_order, int after_peel_tail) {
   extern __shared__ __attribute__((aligned(16))) uint64_t finish_lds[];
   __shared__ int base[256];
   __shared__ int scratch[kRadixThreads];
   if constexpr (MANY) to_population(a);
   if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
-  crowd_finish_body<TABLES>(a, want_order, radix_generation_base(a.ctrl), 1, finish_lds, base, scratch);
+  crowd_finish_body<0>(a, want_order, radix_generation_base(a.ctrl), 1, finish_lds, base, scratch);
+}
+
+// ---- The same for a front of up to kMidArgsortRows rows in four launches whose workgroups never wait for each other
+// (but for a front that crowd_small_front takes): the sorted runs of every objective's keys, each objective's terms of
+// the distances, the distances with the sorted runs of their keys, and the places by distance, where the selected rows are
+// gathered at once.
+// Measured on 20 001 x 3, one front, us by kernel trace: 6.7 + 11 + 6.5 + 11.5; as two kernels around the LDS sorter, the
+// second with a barrier of all workgroups inside, 28 + 45, and 5 for the gather.  Per selection, us: 2000 x 3 58 -> 46,
+// 8000 x 3 95 -> 74, 16 000 x 8 167 -> 133, 20 001 x 3 156 -> 114, twenty populations of 4000 x 5 293 -> 206.
+template <bool MANY>
+__global__ __launch_bounds__(kRunRows) void crowd_runs_kernel(CrowdArgs a, int after_peel_tail, int small_blocks) {
+  extern __shared__ __attribute__((aligned(16))) uint64_t finish_lds[];  // 2 * kRunRows keys, or what crowd_small_front needs
+  __shared__ int scratch[1];
+  if constexpr (MANY) to_population(a);
+  if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
+  if (coherent_load(&a.ctrl->err) != 0) return;
+  const int nv = a.ctrl->nv, m = a.m;
+  if (a.mid_sort == 1 && a.fused != 0 && fused_front_applies(nv, m)) {
+    crowd_small_front(a.xs, a.npad, a.list_base, a.ctrl, m, a.dist, a.dkey, a.order, a.spin_limit, a.fused, small_blocks, finish_lds, scratch);
+    return;
+  }
+  if (!crowd_runs_take(a, nv)) return;
+  const int* __restrict__ list = a.list_base + a.ctrl->worst_start;
+  const int runs = (nv + kRunRows - 1) / kRunRows;
+  for (int item = blockIdx.x; item < runs * m; item += gridDim.x) {
+    const int k = item / runs, r = item - k * runs;
+    const int q = r * kRunRows + (int)threadIdx.x;
+    const uint32_t key = q < nv ? ordered_key(a.xs[(int64_t)k * a.npad + list[q]]) : 0xFFFFFFFFu;
+    const int at = run_position(key, reinterpret_cast<uint32_t*>(finish_lds));
+    if (q < nv) {
+      a.runs[(int64_t)k * a.npad + r * kRunRows + at] = key;
+      a.pos[(int64_t)k * a.kstride + r * kRunRows + at] = q;  // (whose key it is)
+    }
+    __syncthreads();
+  }
+}
+
+// terms[k][q]: what objective k adds to the distance of candidate q, (next - previous) / (last - first) in the objective's
+// order, or kBoundaryTerm where the candidate is its first or last.  The neighbours are found by the searches that count
+// the candidates before q: neither the order nor the sorted costs are written.  (The costs are those of the keys: a
+// difference of two zeros of either sign is +0.0.)  Dynamic LDS: run_rank_lds_bytes(most candidates).
+constexpr uint32_t kBoundaryTerm = 0x7F800001u;  // (a signalling NaN, which no arithmetic gives)
+template <bool MANY>
+__global__ __launch_bounds__(kRunRankThreads) void crowd_terms_kernel(CrowdArgs a, int after_peel_tail) {
+  extern __shared__ __attribute__((aligned(16))) uint64_t finish_lds[];
+  uint32_t* const lds = reinterpret_cast<uint32_t*>(finish_lds);
+  if constexpr (MANY) to_population(a);
+  if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
+  if (coherent_load(&a.ctrl->err) != 0) return;
+  const int nv = a.ctrl->nv, m = a.m;
+  if (!crowd_runs_take(a, nv)) return;
+  const int runs = (nv + kRunRows - 1) / kRunRows;
+  const int shares = (int)gridDim.x >= m ? (int)gridDim.x / m : 1;  // workgroups of one objective
+  const int share = (nv + shares - 1) / shares;
+  constexpr int groups = kRunRankThreads / kRunLanes;
+  for (int item = blockIdx.x; item < shares * m; item += gridDim.x) {
+    const int k = item % m, e0 = (item / m) * share, e1 = min(nv, e0 + share);
+    if (e0 >= nv) continue;
+    const int* __restrict__ candidate = a.pos + (int64_t)k * a.kstride;
+    uint32_t* __restrict__ terms = reinterpret_cast<uint32_t*>(a.sorted_cost) + (int64_t)k * a.kstride;
+    runs_to_lds(a.runs + (int64_t)k * a.npad, nv, lds);
+    __syncthreads();
+    uint32_t first = 0xFFFFFFFFu, last = 0u;
+    for (int r = threadIdx.x & 15; r < runs; r += 16) {
+      first = min(first, lds[r * kRunLdsStride]);
+      last = max(last, lds[r * kRunLdsStride + min(kRunRows, nv - r * kRunRows) - 1]);
+    }
+    const float span = ordered_value(group16_max(last)) - ordered_value(group16_min(first));
+    for (int base = e0; base < e1; base += groups) {
+      if (base + (int)(threadIdx.x & ~63u) / kRunLanes >= e1) break;  // (none left for this wave)
+      const int entry = base + (int)threadIdx.x / kRunLanes;
+      const int e = min(entry, e1 - 1);
+      const int q = candidate[e];
+      RunNeighbours next_to;
+      const int p = run_place<true>(lds, runs, e, &next_to);
+      if (entry < e1 && (threadIdx.x & (kRunLanes - 1)) == 0)
+        terms[q] = p == 0 || p == nv - 1
+                       ? kBoundaryTerm
+                       : __float_as_uint((ordered_value(next_to.behind) - ordered_value(next_to.before)) / span);
+    }
+    __syncthreads();
+  }
+}
+
+template <bool MANY>
+__global__ __launch_bounds__(kRunRows) void crowd_distances_kernel(CrowdArgs a, int want_order, int after_peel_tail) {
+  __shared__ uint32_t lds[2 * kRunRows];
+  if constexpr (MANY) to_population(a);
+  if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
+  if (coherent_load(&a.ctrl->err) != 0) return;
+  const int nv = a.ctrl->nv;
+  if (!crowd_runs_take(a, nv)) return;
+  const int* __restrict__ list = a.list_base + a.ctrl->worst_start;
+  for (int r = blockIdx.x; r * kRunRows < nv; r += gridDim.x) {
+    const int q = r * kRunRows + (int)threadIdx.x;
+    uint32_t key = 0xFFFFFFFFu;
+    if (q < nv) {
+      // (added in column order from the first term on, as crowding_distance_of does)
+      bool boundary = false;
+      float sum = 0.0f;
+#pragma unroll 4
+      for (int k = 0; k < a.m; ++k) {
+        const float term = a.sorted_cost[(int64_t)k * a.kstride + q];
+        boundary |= __float_as_uint(term) == kBoundaryTerm;
+        sum = k == 0 ? term : sum + term;
+      }
+      const float d = boundary ? INFINITY : sum;
+      a.dist[list[q]] = d;
+      key = ordered_key(-d);
+    }
+    if (want_order == 0) continue;
+    const int at = run_position(key, lds);
+    if (q < nv) {
+      a.runs[r * kRunRows + at] = key;
+      a.dkey[r * kRunRows + at] = (uint32_t)q;  // (whose key it is)
+    }
+    __syncthreads();
+  }
+}
+
+// The selection order of the last front; GATHER: and the selected rows of all fronts, whichever kernel has ordered the
+// last one -- the gather launch behind it is saved.  Dynamic LDS: run_rank_lds_bytes(most candidates) and, with GATHER,
+// 8 bytes per candidate of a workgroup (ceil(most candidates / workgroups)).
+template <bool MANY, bool GATHER>
+__global__ __launch_bounds__(kRunRankThreads) void crowd_pick_kernel(CrowdArgs a, GatherArgs g, int after_peel_tail, int picks_at) {
+  extern __shared__ __attribute__((aligned(16))) uint64_t finish_lds[];
+  uint32_t* const lds = reinterpret_cast<uint32_t*>(finish_lds);
+  if constexpr (MANY) {
+    to_population(a);
+    to_population(g);
+  }
+  const bool failed = coherent_load(&a.ctrl->err) != 0;
+  const bool done = after_peel_tail != 0 && a.ctrl->tail_done != 0;
+  const int nv = a.ctrl->nv, start = a.ctrl->worst_start, need = a.ctrl->need;
+  if (failed || done || !crowd_runs_take(a, nv)) {
+    if constexpr (GATHER) gather_body(g, blockIdx.x, gridDim.x, !failed && done ? start : 0);
+    return;
+  }
+  const int* __restrict__ list = a.list_base + start;
+  const int share = (nv + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int e0 = (int)blockIdx.x * share, e1 = min(nv, e0 + share);  // (keys of the sorted runs)
+  int2* const picks = reinterpret_cast<int2*>(reinterpret_cast<char*>(finish_lds) + picks_at);  // (place, row), place -1: not selected
+  if constexpr (!GATHER)
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < start; i += gridDim.x * blockDim.x) a.order[i] = a.list_base[i];
+  if (e0 < nv) runs_to_lds(a.runs, nv, lds);
+  __syncthreads();
+  const int runs = (nv + kRunRows - 1) / kRunRows;
+  constexpr int groups = kRunRankThreads / kRunLanes;
+  for (int base = e0; base < e1; base += groups) {
+    if (base + (int)(threadIdx.x & ~63u) / kRunLanes >= e1) break;  // (none left for this wave)
+    const int entry = base + (int)threadIdx.x / kRunLanes;
+    const int e = min(entry, e1 - 1);
+    const int row = list[a.dkey[e]];
+    const int p = run_place<false>(lds, runs, e, nullptr);
+    if (entry >= e1 || (threadIdx.x & (kRunLanes - 1)) != 0) continue;
+    if constexpr (GATHER) {
+      picks[entry - e0] = p < need ? make_int2(start + p, row) : make_int2(-1, 0);
+    } else {
+      if (p < need) a.order[start + p] = row;
+    }
+  }
+  if constexpr (GATHER) {
+    __syncthreads();
+    gather_notes(g, blockIdx.x);
+    const int lanes = gather_lanes(g);
+    const int per_wave = 64 / lanes;
+    const int lane = (threadIdx.x & 63) % lanes, sub = (threadIdx.x & 63) / lanes;
+    const int waves = blockDim.x >> 6, wave = threadIdx.x >> 6;
+    for (int i = wave * per_wave + sub; i < e1 - e0; i += waves * per_wave)
+      if (picks[i].x >= 0) gather_row(g, picks[i].x, picks[i].y, lane, lanes);
+    for (int p = ((int)blockIdx.x * waves + wave) * per_wave + sub; p < start; p += (int)gridDim.x * waves * per_wave)
+      gather_row(g, p, a.list_base[p], lane, lanes);
+  }
 }
 
 // ---- The ordering of the last front in one launch (crowd_gather_kernel below), for populations whose peel kernel
