@@ -41,6 +41,9 @@ _SIGNATURES = {
     "evox_hip_nd_environmental_selection_wide": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int,
                                                          c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
                                                          c_void_p, c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
+    "evox_hip_nd_environmental_selection_wide_whole": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int,
+                                                               c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+                                                               c_void_p, c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
     "evox_hip_nd_environmental_selection": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                                     c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                                     c_size_t, c_void_p]),

@@ -2728,6 +2728,110 @@ int evox_hip_many_nd_environmental_selection_wide(const void* x, int64_t x_row_b
 
 }  // extern "C"
 
+extern "C" {
+
+int evox_hip_nd_environmental_selection_wide_whole(const void* x, int64_t x_row_bytes, int64_t x_row_stride_bytes, const void* f_rows,
+                                                   int64_t f_row_bytes, int64_t f_row_stride_bytes, const void* costs, int kind,
+                                                   int64_t n, int64_t m, int64_t sr, int64_t sc, int64_t topk, void* out_x, void* out_f,
+                                                   int32_t* out_rank, void* out_dist, int out_kind, void* ws, size_t ws_bytes,
+                                                   void* stream) {
+  Ws w;
+  if (costs == nullptr || f_rows == nullptr || out_f == nullptr || out_rank == nullptr || out_dist == nullptr) return kErrBadArg;
+  if ((kind != kWideFloat64 && kind != kWideInt64) || (out_kind != 0 && out_kind != 1)) return kErrBadArg;
+  if ((x == nullptr) != (out_x == nullptr) || x_row_bytes < 0 || x_row_stride_bytes < 0 || f_row_bytes < 1 || f_row_stride_bytes < 0)
+    return kErrBadArg;
+  if (n > kRunMaxRows || topk < 1 || topk > n) return kErrBadArg;
+  if (int e = open_ws(n, m, ws, ws_bytes, &w)) return e;
+  const Layout& L = w.L;
+  WideLayout WL;
+  if (!make_wide_layout(n, m, &WL) || WL.total > L.wide_bytes) return kErrWorkspace;
+  uint8_t* const wb = w.base + L.wide;
+  hipStream_t s = (hipStream_t)stream;
+  // (regions of the 8-byte kernels' part of the workspace: the two halves of the keys lie side by side and hold whole
+  // images, the image that is ranked lies where the terms go later)
+  uint64_t* const runs = reinterpret_cast<uint64_t*>(wb + WL.key_lo);
+  int* const whose = reinterpret_cast<int*>(wb + WL.ord_a);
+  float* const images = reinterpret_cast<float*>(wb + WL.terms);
+  const int all_runs = runs_of((int)n), most_shares = (int)((n + kWideShare - 1) / kWideShare);
+  const size_t lds = run_rank8_lds_bytes((int)n);
+  if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(value_images_kernel), lds)) return e;
+  hipLaunchKernelGGL(value_runs_kernel, dim3(all_runs, (unsigned)m), dim3(kRunRows), 0, s, costs, kind, sr, sc, (int)n, runs, whose);
+  EVX_LAUNCH_CHECK();
+  hipLaunchKernelGGL(value_images_kernel, dim3(most_shares, (unsigned)m), dim3(kRunRankThreads), lds, s, runs, whose, kind, (int)n, (int)m,
+                     images);
+  EVX_LAUNCH_CHECK();
+  const Fitness fit = one_part(images, n, m, 1);
+  bool stepped = false;
+  int ranked = kErrNotResident;
+  if (two_applies(L, topk)) ranked = stage_rank_two(w, fit, topk, false, nullptr, s);
+  if (ranked == kErrNotResident) {
+    if (int e = stage_prepare(w, fit, true, s)) return e;
+    if (int e = stage_dominance(w, kDomAuto, s)) return e;
+    ranked = count_and_peel(w, topk, true, false, s, false, nullptr, nullptr, &stepped);
+  }
+  if (ranked) return ranked;
+  if (stepped) {  // (its fronts have no listing: the order from the ranks alone)
+    if (int e = copy_out(w.ctrl(), w.at<int>(L.order), w.at<int>(L.rank), n, kPoisonIndex, s)) return e;
+    return evox_hip_nd_environmental_selection_wide(x, x_row_bytes, x_row_stride_bytes, f_rows, f_row_bytes, f_row_stride_bytes, costs,
+                                                    kind, n, m, sr, sc, w.at<int>(L.order), topk, out_x, out_f, out_rank, out_dist,
+                                                    out_kind, wb, L.wide_bytes, stream);
+  }
+  WideFront a = {};
+  a.costs = costs;
+  a.kind = kind;
+  a.stride_row = sr;
+  a.stride_col = sc;
+  a.n = (int)n;
+  a.m = (int)m;
+  a.list_base = w.at<int>(L.perm);
+  a.ctrl = w.ctrl();
+  a.runs = runs;
+  a.whose = whose;
+  a.terms = wb + WL.terms;
+  a.dist = wb + WL.dist;
+  a.dist_runs = reinterpret_cast<uint64_t*>(wb + WL.front_dkey);
+  a.dist_whose = reinterpret_cast<int*>(wb + WL.order_a);
+  a.topk = (int)topk;
+  auto unit_of = [](const void* src, const void* dst, int64_t row_bytes, int64_t stride) {
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst) | (uintptr_t)row_bytes | (uintptr_t)stride;
+    return bits % 16 == 0 ? 16 : bits % 8 == 0 ? 8 : bits % 4 == 0 ? 4 : 1;
+  };
+  a.x = static_cast<const uint8_t*>(x);
+  a.x_row_bytes = x_row_bytes;
+  a.x_row_stride = x_row_stride_bytes;
+  a.x_unit = unit_of(x, out_x, x_row_bytes, x_row_stride_bytes);
+  a.out_x = static_cast<uint8_t*>(out_x);
+  a.f = static_cast<const uint8_t*>(f_rows);
+  a.f_row_bytes = f_row_bytes;
+  a.f_row_stride = f_row_stride_bytes;
+  a.f_unit = unit_of(f_rows, out_f, f_row_bytes, f_row_stride_bytes);
+  a.out_f = static_cast<uint8_t*>(out_f);
+  a.rank = w.at<int>(L.rank);
+  a.out_rank = out_rank;
+  a.out_dist = out_dist;
+  int runs_grid = all_runs * (int)m;
+  if (runs_grid > 65536) runs_grid = 65536;
+  const int shares = device_cus() / (int)m > most_shares ? device_cus() / (int)m : most_shares;  // workgroups of one objective
+  const int picks = device_cus() > most_shares ? device_cus() : most_shares;
+  auto launch = [&](auto terms_kernel, auto distances_kernel, auto pick_kernel) -> int {
+    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(terms_kernel), lds)) return e;
+    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(pick_kernel), lds)) return e;
+    hipLaunchKernelGGL(wide_front_runs_kernel, dim3(runs_grid), dim3(kRunRows), 0, s, a);
+    EVX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(terms_kernel, dim3(shares * (int)m), dim3(kRunRankThreads), lds, s, a);
+    EVX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(distances_kernel, dim3(all_runs), dim3(kRunRows), 0, s, a);
+    EVX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(pick_kernel, dim3(picks), dim3(kRunRankThreads), lds, s, a);
+    EVX_LAUNCH_CHECK();
+    return 0;
+  };
+  if (out_kind == 0) return launch(wide_front_terms_kernel<double>, wide_front_distances_kernel<double>, wide_front_pick_kernel<double>);
+  return launch(wide_front_terms_kernel<float>, wide_front_distances_kernel<float>, wide_front_pick_kernel<float>);
+}
+
+}  // extern "C"
+
 // Scratch memory of the entry point that allocates nothing: part of the device image, one copy per GPU.  In host
 // code the array's name stands for the symbol, not for device memory: its address on the current GPU comes from
 // hipGetSymbolAddress, looked up once per device and kept.

@@ -578,7 +578,7 @@ __global__ __launch_bounds__(kRunRows) void crowd_runs_kernel(CrowdArgs a, int a
   }
   if (!crowd_runs_take(a, nv)) return;
   const int* __restrict__ list = a.list_base + a.ctrl->worst_start;
-  const int runs = (nv + kRunRows - 1) / kRunRows;
+  const int runs = runs_of(nv);
   for (int item = blockIdx.x; item < runs * m; item += gridDim.x) {
     const int k = item / runs, r = item - k * runs;
     const int q = r * kRunRows + (int)threadIdx.x;
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(kRunRankThreads) void crowd_terms_kernel(CrowdArgs 
   if (coherent_load(&a.ctrl->err) != 0) return;
   const int nv = a.ctrl->nv, m = a.m;
   if (!crowd_runs_take(a, nv)) return;
-  const int runs = (nv + kRunRows - 1) / kRunRows;
+  const int runs = runs_of(nv);
   const int shares = (int)gridDim.x >= m ? (int)gridDim.x / m : 1;  // workgroups of one objective
   const int share = (nv + shares - 1) / shares;
   constexpr int groups = kRunRankThreads / kRunLanes;
@@ -615,12 +615,12 @@ __global__ __launch_bounds__(kRunRankThreads) void crowd_terms_kernel(CrowdArgs 
     if (e0 >= nv) continue;
     const int* __restrict__ candidate = a.pos + (int64_t)k * a.kstride;
     uint32_t* __restrict__ terms = reinterpret_cast<uint32_t*>(a.sorted_cost) + (int64_t)k * a.kstride;
-    runs_to_lds(a.runs + (int64_t)k * a.npad, nv, lds);
+    runs_to_lds(a.runs + (int64_t)k * a.npad, nv, 0, runs, lds);
     __syncthreads();
     uint32_t first = 0xFFFFFFFFu, last = 0u;
     for (int r = threadIdx.x & 15; r < runs; r += 16) {
-      first = min(first, lds[r * kRunLdsStride]);
-      last = max(last, lds[r * kRunLdsStride + min(kRunRows, nv - r * kRunRows) - 1]);
+      first = min(first, lds[r * RunLds<uint32_t>::kStride]);
+      last = max(last, lds[r * RunLds<uint32_t>::kStride + min(kRunRows, nv - r * kRunRows) - 1]);
     }
     const float span = ordered_value(group16_max(last)) - ordered_value(group16_min(first));
     for (int base = e0; base < e1; base += groups) {
@@ -628,12 +628,17 @@ __global__ __launch_bounds__(kRunRankThreads) void crowd_terms_kernel(CrowdArgs 
       const int entry = base + (int)threadIdx.x / kRunLanes;
       const int e = min(entry, e1 - 1);
       const int q = candidate[e];
-      RunNeighbours next_to;
-      const int p = run_place<true>(lds, runs, e, &next_to);
+      RunSearch<uint32_t> s;
+      s.own = e / kRunRows;
+      s.at = e % kRunRows;
+      s.key = lds[s.own * RunLds<uint32_t>::kStride + s.at];
+      run_search_all<kRunNeighbours>(lds, 0, runs, s);
+      run_search_end<kRunNeighbours>(s);
+      const int p = (int)s.smaller;
       if (entry < e1 && (threadIdx.x & (kRunLanes - 1)) == 0)
         terms[q] = p == 0 || p == nv - 1
                        ? kBoundaryTerm
-                       : __float_as_uint((ordered_value(next_to.behind) - ordered_value(next_to.before)) / span);
+                       : __float_as_uint((ordered_value(s.behind) - ordered_value(s.before)) / span);
     }
     __syncthreads();
   }
@@ -699,16 +704,22 @@ __global__ __launch_bounds__(kRunRankThreads) void crowd_pick_kernel(CrowdArgs a
   int2* const picks = reinterpret_cast<int2*>(reinterpret_cast<char*>(finish_lds) + picks_at);  // (place, row), place -1: not selected
   if constexpr (!GATHER)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < start; i += gridDim.x * blockDim.x) a.order[i] = a.list_base[i];
-  if (e0 < nv) runs_to_lds(a.runs, nv, lds);
+  const int runs = runs_of(nv);
+  if (e0 < nv) runs_to_lds(a.runs, nv, 0, runs, lds);
   __syncthreads();
-  const int runs = (nv + kRunRows - 1) / kRunRows;
   constexpr int groups = kRunRankThreads / kRunLanes;
   for (int base = e0; base < e1; base += groups) {
     if (base + (int)(threadIdx.x & ~63u) / kRunLanes >= e1) break;  // (none left for this wave)
     const int entry = base + (int)threadIdx.x / kRunLanes;
     const int e = min(entry, e1 - 1);
     const int row = list[a.dkey[e]];
-    const int p = run_place<false>(lds, runs, e, nullptr);
+    RunSearch<uint32_t> s;
+    s.own = e / kRunRows;
+    s.at = e % kRunRows;
+    s.key = lds[s.own * RunLds<uint32_t>::kStride + s.at];
+    run_search_all<kRunTies>(lds, 0, runs, s);
+    run_search_end<kRunTies>(s);
+    const int p = (int)s.smaller;
     if (entry >= e1 || (threadIdx.x & (kRunLanes - 1)) != 0) continue;
     if constexpr (GATHER) {
       picks[entry - e0] = p < need ? make_int2(start + p, row) : make_int2(-1, 0);

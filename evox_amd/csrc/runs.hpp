@@ -14,16 +14,25 @@
 // us of it (80 KB per workgroup, the same for all).
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace evx {
 
 constexpr int kRunRows = 512;          // keys per run = threads that sort it
 constexpr int kRunMaxRows = 32768;     // 4-byte keys that one workgroup's LDS holds
-constexpr int kRunLdsStride = kRunRows + 4;  // keys from one run to the next in LDS: sixteen runs' same entries fall into different banks
+constexpr int kRunTile8 = 32;          // runs of 8-byte keys that it holds
 constexpr int kRunRankThreads = 1024;  // threads of a workgroup that searches
-__host__ __device__ inline size_t run_rank_lds_bytes(int n) {
-  return sizeof(uint32_t) * (size_t)kRunLdsStride * (size_t)((n + kRunRows - 1) / kRunRows);
+// Keys from one run to the next in LDS: sixteen bytes more than a run, so that the runs' same entries fall into different banks.
+template <class K>
+struct RunLds {
+  static constexpr int kStride = kRunRows + 16 / (int)sizeof(K);
+};
+__host__ __device__ inline int runs_of(int n) { return (n + kRunRows - 1) / kRunRows; }
+__host__ __device__ inline size_t run_rank_lds_bytes(int n) { return sizeof(uint32_t) * RunLds<uint32_t>::kStride * (size_t)runs_of(n); }
+__host__ __device__ inline size_t run_rank8_lds_bytes(int n) {  // (more keys: a tile after the other)
+  return sizeof(uint64_t) * RunLds<uint64_t>::kStride * (size_t)(runs_of(n) < kRunTile8 ? runs_of(n) : kRunTile8);
 }
 
 // Does a key `other` precede the key `mine`: smaller, or equal where `first` says that its position is the earlier one?
@@ -42,6 +51,9 @@ __device__ __forceinline__ int run_search(const K* run, K mine, bool first) {
 }
 
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int lane) {
+  return ((uint64_t)lane_value((uint32_t)(v >> 32), lane) << 32) | lane_value((uint32_t)v, lane);
+}
 
 // The position of every thread's key among the keys of its workgroup of kRunRows threads (ascending, equal keys by
 // thread): 64 keys of a wave by counting (the other lanes' keys come through scalar registers), then the sorted 64s of
@@ -71,54 +83,69 @@ __device__ __forceinline__ int run_position(K key, K* lds) {
   return at;
 }
 
-// The sorted runs of nv keys (run r at sorted + r * kRunRows, 16-byte aligned) into LDS; the last run is filled up with the
-// largest key.  Called by every thread; the caller puts a barrier behind it.
-__device__ __forceinline__ void runs_to_lds(const uint32_t* __restrict__ sorted, int nv, uint32_t* lds) {
-  const int whole = nv & ~3;
+// The sorted runs first .. first + runs - 1 of nv keys (run r at sorted + r * kRunRows) into LDS, in pieces of sixteen bytes
+// where they are aligned so; the last run of all is filled up with the largest key.  Called by every thread; the caller puts a barrier behind it.
+template <class K>
+__device__ __forceinline__ void runs_to_lds(const K* __restrict__ sorted, int nv, int first, int runs, K* lds) {
+  constexpr int kVec = 16 / (int)sizeof(K);
+  sorted += (int64_t)first * kRunRows;
+  const int count = min(nv - first * kRunRows, runs * kRunRows);
+  const int whole = (reinterpret_cast<uintptr_t>(sorted) & 15u) == 0 ? count & ~(kVec - 1) : 0;
 #pragma unroll 4
-  for (int e = threadIdx.x * 4; e < whole; e += blockDim.x * 4)
-    *reinterpret_cast<uint4*>(lds + (e / kRunRows) * kRunLdsStride + (e % kRunRows)) = *reinterpret_cast<const uint4*>(sorted + e);
-  const int padded = (nv + kRunRows - 1) / kRunRows * kRunRows;
-  for (int e = whole + threadIdx.x; e < padded; e += blockDim.x)
-    lds[(e / kRunRows) * kRunLdsStride + (e % kRunRows)] = e < nv ? sorted[e] : 0xFFFFFFFFu;
+  for (int e = threadIdx.x * kVec; e < whole; e += blockDim.x * kVec)
+    *reinterpret_cast<uint4*>(lds + (e / kRunRows) * RunLds<K>::kStride + (e % kRunRows)) = *reinterpret_cast<const uint4*>(sorted + e);
+#pragma unroll 4
+  for (int e = whole + threadIdx.x; e < runs * kRunRows; e += blockDim.x)
+    lds[(e / kRunRows) * RunLds<K>::kStride + (e % kRunRows)] = e < count ? sorted[e] : ~(K)0;
 }
 
-// Neighbours of a key among all keys: the largest key before it and the smallest behind it.
-struct RunNeighbours {
-  uint32_t before, behind;
-};
-
-// The sum / maximum / minimum over the G (4 or 8) consecutive lanes of a group, the same in all of them.
-template <int G, class Op>
+// The sum / maximum / minimum over the kRunLanes consecutive lanes of a group, the same in all of them.
+constexpr int kRunLanes = 4;
+template <class Op>
 __device__ __forceinline__ uint32_t run_group(uint32_t v, Op op) {
-  static_assert(G == 4 || G == 8, "rotations inside a row of sixteen lanes");
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));  // lanes 1 0 3 2
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));  // lanes 2 3 0 1
-  if constexpr (G == 8) v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));  // the other four
-  return v;
+  static_assert(kRunLanes == 4, "permutations of four lanes");
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));     // lanes 1 0 3 2
+  return op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));  // lanes 2 3 0 1
+}
+template <class Op>
+__device__ __forceinline__ uint64_t run_group(uint64_t v, Op op) {
+  auto permuted = [&](auto control) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, control.value, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), control.value, 0xf, 0xf, false);
+    return ((uint64_t)hi << 32) | lo;
+  };
+  v = op(v, permuted(std::integral_constant<int, 0xB1>{}));
+  return op(v, permuted(std::integral_constant<int, 0x4E>{}));
 }
 
 // A key whose place is being looked for, and what its searches have found so far.
+template <class K>
 struct RunSearch {
-  uint32_t key;
+  K key;
   int own, at;  // its run, and its place in that
-  uint32_t smaller, before, behind;
+  uint32_t smaller = 0;
+  K before = 0, behind = ~(K)0;  // the largest key before it (0 where there is none) and the smallest behind it (meaningless at the last place)
 };
 
-// U searches side by side: runs r0, r0 + G, ... (those below `runs`).
-template <int G, int U, bool NEIGHBOURS>
-__device__ __forceinline__ void run_search_some(const uint32_t* lds, int runs, int r0, RunSearch& q) {
-  const uint32_t* c[U];  // (an address in LDS: a step is one read, one comparison, one selection and one addition)
-  uint32_t bound[U];
+// What a search looks for besides the number of keys that precede the key.
+constexpr int kRunTies = 0;        // (equal keys of earlier positions precede it)
+constexpr int kRunNeighbours = 1;  // ... and its neighbours
+constexpr int kRunSmaller = 2;     // (only smaller keys precede it)
+
+// U searches side by side in the runs `first` + r0, r0 + kRunLanes, ... of which LDS holds `runs`.
+template <int U, int MODE, class K>
+__device__ __forceinline__ void run_search_some(const K* lds, int first, int runs, int r0, RunSearch<K>& q) {
+  const K* c[U];  // (an address in LDS: a step is one read, one comparison, one selection and one addition)
+  K bound[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int r = r0 + G * u;
-    c[u] = lds + (r < runs ? r : 0) * kRunLdsStride;
-    bound[u] = r < q.own ? q.key : q.key - 1u;
+    const int r = r0 + kRunLanes * u;
+    c[u] = lds + (r < runs ? r : 0) * RunLds<K>::kStride;
+    bound[u] = MODE != kRunSmaller && first + r < q.own ? q.key : q.key - (K)1;
   }
 #pragma unroll
   for (int s = kRunRows / 2; s >= 1; s >>= 1) {
-    uint32_t v[U];
+    K v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = c[u][s - 1];
 #pragma unroll
@@ -126,49 +153,45 @@ __device__ __forceinline__ void run_search_some(const uint32_t* lds, int runs, i
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int r = r0 + G * u;
-    const uint32_t* const run = lds + (r < runs ? r : 0) * kRunLdsStride;
+    const int r = r0 + kRunLanes * u;
+    const bool own = MODE != kRunSmaller && first + r == q.own;
+    const K* const run = lds + (r < runs ? r : 0) * RunLds<K>::kStride;
     int n = (int)(c[u] - run) + (*c[u] <= bound[u] ? 1 : 0);
-    if (q.key == 0u && r > q.own) n = 0;
-    if (r == q.own) n = q.at;
+    if (q.key == (K)0 && (MODE == kRunSmaller || first + r > q.own)) n = 0;
+    if (own) n = q.at;
     q.smaller += r < runs ? (uint32_t)n : 0u;
-    if constexpr (NEIGHBOURS) {  // (read whether or not there is one: branches would put the reads one after the other)
-      const uint32_t lower = run[n > 0 ? n - 1 : 0], upper = run[min(r == q.own ? n + 1 : n, kRunRows - 1)];
-      if (r < runs && n > 0) q.before = max(q.before, lower);
-      if (r < runs && n + (r == q.own ? 1 : 0) < kRunRows) q.behind = min(q.behind, upper);
+    if constexpr (MODE == kRunNeighbours) {  // (read whether or not there is one: branches would put the reads one after the other)
+      const K lower = run[n > 0 ? n - 1 : 0], upper = run[min(own ? n + 1 : n, kRunRows - 1)];
+      if (r < runs && n > 0) q.before = lower > q.before ? lower : q.before;
+      if (r < runs && n + (own ? 1 : 0) < kRunRows) q.behind = upper < q.behind ? upper : q.behind;
     }
   }
 }
 
-// The place of a key among all keys, whose runs lie in LDS: the key at entry e (run e / kRunRows, place e % kRunRows in it),
-// the same in the kRunLanes lanes that call it together, each with its share of the runs, four of them at a time (a search
-// is a chain of ten LDS round trips).  The keys of a wave should be neighbours in their run: their searches then read the
-// same words mostly, and four lanes per key mean four different words of a wave's read in the LDS banks instead of
-// sixteen (terms of 20 001 x 3, forty runs, us: sixteen lanes per key 11.6, eight 12.0, four 9.3).
+// The searches for one key in the runs first .. first + runs - 1, which lie in LDS: q is the same in the kRunLanes lanes that
+// call it together, each with its share of the runs, four of them at a time (a search is a chain of ten LDS round trips).
+// The keys of a wave should be neighbours in their run: their searches then read the same words mostly, and four lanes
+// per key mean four different words of a wave's read in the LDS banks instead of sixteen (terms of 20 001 x 3, forty
+// runs, us: sixteen lanes per key 11.6, eight 12.0, four 9.3).
 // The comparison `v precedes key` is v <= bound, the bound being the key or one less: one instruction per step.  A key
 // of zero that no equal key precedes has no such bound; nothing precedes it.
-// NEIGHBOURS: also the keys next to it (before: 0 where there is none; behind: meaningless at the last place).
-constexpr int kRunLanes = 4;
-template <bool NEIGHBOURS>
-__device__ __forceinline__ int run_place(const uint32_t* lds, int runs, int e, RunNeighbours* next_to) {
-  RunSearch q;
-  q.own = e / kRunRows;
-  q.at = e % kRunRows;
-  q.key = lds[q.own * kRunLdsStride + q.at];
-  q.smaller = 0u;
-  q.before = 0u;
-  q.behind = 0xFFFFFFFFu;
+template <int MODE, class K>
+__device__ __forceinline__ void run_search_all(const K* lds, int first, int runs, RunSearch<K>& q) {
   int r0 = threadIdx.x & (kRunLanes - 1), left = runs;
-  for (; left > 2 * kRunLanes; left -= 4 * kRunLanes, r0 += 4 * kRunLanes) run_search_some<kRunLanes, 4, NEIGHBOURS>(lds, runs, r0, q);
+  for (; left > 2 * kRunLanes; left -= 4 * kRunLanes, r0 += 4 * kRunLanes) run_search_some<4, MODE>(lds, first, runs, r0, q);
   if (left > kRunLanes)
-    run_search_some<kRunLanes, 2, NEIGHBOURS>(lds, runs, r0, q);
+    run_search_some<2, MODE>(lds, first, runs, r0, q);
   else if (left > 0)
-    run_search_some<kRunLanes, 1, NEIGHBOURS>(lds, runs, r0, q);
-  if constexpr (NEIGHBOURS) {
-    next_to->before = run_group<kRunLanes>(q.before, [](uint32_t a, uint32_t b) { return max(a, b); });
-    next_to->behind = run_group<kRunLanes>(q.behind, [](uint32_t a, uint32_t b) { return min(a, b); });
+    run_search_some<1, MODE>(lds, first, runs, r0, q);
+}
+// Once all runs have been searched: the sums over the group.  The key's place is q.smaller then.
+template <int MODE, class K>
+__device__ __forceinline__ void run_search_end(RunSearch<K>& q) {
+  q.smaller = run_group(q.smaller, [](uint32_t a, uint32_t b) { return a + b; });
+  if constexpr (MODE == kRunNeighbours) {
+    q.before = run_group(q.before, [](K a, K b) { return a > b ? a : b; });
+    q.behind = run_group(q.behind, [](K a, K b) { return a < b ? a : b; });
   }
-  return (int)run_group<kRunLanes>(q.smaller, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 }  // namespace evx

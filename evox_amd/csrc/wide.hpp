@@ -14,6 +14,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "runs.hpp"
 
 namespace evx {
 
@@ -517,6 +518,282 @@ __global__ __launch_bounds__(256) void gather_parts_kernel(GatherParts g, const 
       *reinterpret_cast<uint32_t*>(to) = *reinterpret_cast<const uint32_t*>(from);
     else
       *to = *from;
+  }
+}
+
+// ---- 8-byte values by sorted runs (runs.hpp), for populations of up to kRunMaxRows rows: the float32 image that the ranking
+// kernels read, and the order of the last front.
+
+__device__ inline double wide_value(double, uint64_t image) {
+  if (image == ~0ull) return __longlong_as_double(0x7FF8000000000000ll);
+  return __longlong_as_double((long long)((image >> 63) ? image & 0x7FFFFFFFFFFFFFFFull : ~image));
+}
+__device__ inline long long wide_value(long long, uint64_t image) { return (long long)(image ^ 0x8000000000000000ull); }
+
+// Run blockIdx.x of objective blockIdx.y: the images of its values in ascending order (rows of n), and whose they are.
+__global__ __launch_bounds__(kRunRows) void value_runs_kernel(const void* __restrict__ costs, int kind, int64_t stride_row,
+                                                              int64_t stride_col, int n, uint64_t* __restrict__ sorted,
+                                                              int* __restrict__ whose) {
+  __shared__ uint64_t lds[2 * kRunRows];
+  const int i = (int)blockIdx.x * kRunRows + (int)threadIdx.x, k = blockIdx.y;
+  const uint64_t key = i < n ? wide_image(costs, kind, (int64_t)i * stride_row + (int64_t)k * stride_col) : ~0ull;
+  const int64_t at = (int64_t)k * n + (int)blockIdx.x * kRunRows + run_position(key, lds);
+  if (i < n) {
+    sorted[at] = key;
+    whose[at] = i;
+  }
+}
+
+// out[i * m + k] = how many values of objective k are smaller than that of row i, as a float (exact below 2^24), NaN where
+// the value is NaN: equal values get equal images, so every `<=` and `<` inside an objective stays what it is.
+// Bound by the searches (as in runs.hpp, with 8-byte reads).  20 000 x 3 float64, us: 6.4 + 9.1 for the two kernels; a copy by
+// objective, the library's sort and the dense ranks of its result 120.
+constexpr int kWideShare = kRunRankThreads / kRunLanes;  // keys that a workgroup looks for at once
+__global__ __launch_bounds__(kRunRankThreads) void value_images_kernel(const uint64_t* __restrict__ sorted, const int* __restrict__ whose,
+                                                                       int kind, int n, int m, float* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) uint64_t wide_lds[];
+  const int k = blockIdx.y, runs = runs_of(n);
+  sorted += (int64_t)k * n;
+  const int e0 = (int)blockIdx.x * kWideShare;
+  const int entry = e0 + (int)threadIdx.x / kRunLanes, e = min(entry, n - 1);
+  const bool work = e0 + (int)(threadIdx.x & ~63u) / kRunLanes < n;  // (of the wave)
+  RunSearch<uint64_t> s;
+  s.own = e / kRunRows;
+  s.at = e % kRunRows;
+  s.key = sorted[e];
+  const int i = whose[(int64_t)k * n + e];
+  for (int first = 0; first < runs; first += kRunTile8) {
+    const int here = min(kRunTile8, runs - first);
+    __syncthreads();
+    runs_to_lds(sorted, n, first, here, wide_lds);
+    __syncthreads();
+    if (work) run_search_all<kRunSmaller>(wide_lds, first, here, s);
+  }
+  run_search_end<kRunSmaller>(s);
+  if (entry < n && (threadIdx.x & (kRunLanes - 1)) == 0)
+    out[(int64_t)i * m + k] = kind == kWideFloat64 && s.key == ~0ull ? NAN : (float)s.smaller;
+}
+
+// The last front in four launches, as crowd_runs_kernel and those after it (finish.hpp) order one of 4-byte costs.
+// 20 000 x 3 float64, a front of some 900 rows, us: 7.3 + 4.6 + 6.8 + 7.0, against 104 for the copy of the ranks, their argsort,
+// a search among all candidates and the gathers; the selection 336 -> 169, with one front of all rows 618 -> 158,
+// 20 000 x 8 1197 -> 210, 100 x 3 106 -> 53.
+// Its rows are list_base[ctrl->worst_start ...], ctrl->nv of them, as the peel left them.
+struct WideFront {
+  const void* costs;
+  int kind;
+  int64_t stride_row, stride_col;
+  int n, m;
+  const int* list_base;
+  const Ctrl* ctrl;
+  uint64_t* runs;  // [m][n] sorted runs of the candidates' images
+  int* whose;      // [m][n] whose they are
+  void* terms;     // [m][n] by candidate
+  void* dist;      // [n] by candidate
+  uint64_t* dist_runs;
+  int* dist_whose;
+  // the selection
+  int topk;
+  const uint8_t *x, *f;  // decision vectors (or null), fitness rows
+  int64_t x_row_bytes, x_row_stride, f_row_bytes, f_row_stride;
+  int x_unit, f_unit;
+  const int* rank;
+  uint8_t *out_x, *out_f;
+  int* out_rank;
+  void* out_dist;
+};
+
+__global__ __launch_bounds__(kRunRows) void wide_front_runs_kernel(WideFront a) {
+  __shared__ uint64_t lds[2 * kRunRows];
+  if (a.ctrl->err != 0) return;
+  const int nv = a.ctrl->nv, runs = runs_of(nv);
+  const int* __restrict__ list = a.list_base + a.ctrl->worst_start;
+  for (int item = blockIdx.x; item < runs * a.m; item += gridDim.x) {
+    const int k = item / runs, r = item - k * runs;
+    const int q = r * kRunRows + (int)threadIdx.x;
+    const uint64_t key = q < nv ? wide_image(a.costs, a.kind, (int64_t)list[q] * a.stride_row + (int64_t)k * a.stride_col) : ~0ull;
+    const int at = run_position(key, lds);
+    if (q < nv) {
+      a.runs[(int64_t)k * a.n + r * kRunRows + at] = key;
+      a.whose[(int64_t)k * a.n + r * kRunRows + at] = q;
+    }
+    __syncthreads();
+  }
+}
+
+// A term that says "first or last of its objective": a signalling NaN, which no arithmetic gives.
+__device__ __forceinline__ void wide_store_boundary(double* term) { *reinterpret_cast<uint64_t*>(term) = 0x7FF0000000000001ull; }
+__device__ __forceinline__ void wide_store_boundary(float* term) { *reinterpret_cast<uint32_t*>(term) = 0x7F800001u; }
+__device__ __forceinline__ bool wide_is_boundary(const double* term) { return *reinterpret_cast<const uint64_t*>(term) == 0x7FF0000000000001ull; }
+__device__ __forceinline__ bool wide_is_boundary(const float* term) { return *reinterpret_cast<const uint32_t*>(term) == 0x7F800001u; }
+
+// (differences and quotients as wide_term computes them)
+template <class Out>
+__device__ inline Out wide_term_of(int kind, uint64_t next, uint64_t prev, uint64_t last, uint64_t first) {
+  if (kind == kWideFloat64) {
+    const double t = 0.0;
+    return (Out)((wide_value(t, next) - wide_value(t, prev)) / (wide_value(t, last) - wide_value(t, first)));
+  }
+  return (Out)(long long)(next - prev) / (Out)(long long)(last - first);  // (the images differ as the integers do, wrapping)
+}
+
+// Grid: any number of workgroups from m * ceil(n / kWideShare) on.  Dynamic LDS: run_rank8_lds_bytes(n).
+template <class Out>
+__global__ __launch_bounds__(kRunRankThreads) void wide_front_terms_kernel(WideFront a) {
+  extern __shared__ __attribute__((aligned(16))) uint64_t wide_lds[];
+  __shared__ uint64_t ends[2];
+  if (a.ctrl->err != 0) return;
+  const int nv = a.ctrl->nv, runs = runs_of(nv), m = a.m;
+  const int shares = (int)gridDim.x / m;  // workgroups of one objective
+  const int share = (nv + shares - 1) / shares;  // at most kWideShare
+  const int k = (int)blockIdx.x % m, e0 = ((int)blockIdx.x / m) * share, e1 = min(nv, e0 + share);
+  if (e0 >= nv || (int)blockIdx.x >= shares * m) return;
+  const uint64_t* __restrict__ sorted = a.runs + (int64_t)k * a.n;
+  const int entry = e0 + (int)threadIdx.x / kRunLanes, e = min(entry, e1 - 1);
+  const bool work = e0 + (int)(threadIdx.x & ~63u) / kRunLanes < e1;  // (of the wave)
+  RunSearch<uint64_t> s;
+  s.own = e / kRunRows;
+  s.at = e % kRunRows;
+  s.key = sorted[e];
+  const int q = a.whose[(int64_t)k * a.n + e];
+  if (threadIdx.x < 64) {
+    uint64_t first = ~0ull, last = 0ull;
+    for (int r = threadIdx.x; r < runs; r += 64) {
+      const uint64_t lo = sorted[r * kRunRows], hi = sorted[min(nv, (r + 1) * kRunRows) - 1];
+      first = lo < first ? lo : first;
+      last = hi > last ? hi : last;
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint64_t lo = __shfl_xor((unsigned long long)first, off), hi = __shfl_xor((unsigned long long)last, off);
+      first = lo < first ? lo : first;
+      last = hi > last ? hi : last;
+    }
+    if (threadIdx.x == 0) {
+      ends[0] = first;
+      ends[1] = last;
+    }
+  }
+  for (int first = 0; first < runs; first += kRunTile8) {
+    const int here = min(kRunTile8, runs - first);
+    __syncthreads();
+    runs_to_lds(sorted, nv, first, here, wide_lds);
+    __syncthreads();
+    if (work) run_search_all<kRunNeighbours>(wide_lds, first, here, s);
+  }
+  run_search_end<kRunNeighbours>(s);
+  if (entry < e1 && (threadIdx.x & (kRunLanes - 1)) == 0) {
+    Out* const term = static_cast<Out*>(a.terms) + (int64_t)k * a.n + q;
+    if (s.smaller == 0u || (int)s.smaller == nv - 1)
+      wide_store_boundary(term);
+    else
+      *term = wide_term_of<Out>(a.kind, s.behind, s.before, ends[1], ends[0]);
+  }
+}
+
+template <class Out>
+__global__ __launch_bounds__(kRunRows) void wide_front_distances_kernel(WideFront a) {
+  __shared__ uint64_t lds[2 * kRunRows];
+  if (a.ctrl->err != 0) return;
+  const int nv = a.ctrl->nv;
+  for (int r = blockIdx.x; r * kRunRows < nv; r += gridDim.x) {
+    const int q = r * kRunRows + (int)threadIdx.x;
+    uint64_t key = ~0ull;
+    if (q < nv) {  // (terms added in column order from the first one on)
+      bool boundary = false;
+      Out sum = (Out)0;
+      for (int k = 0; k < a.m; ++k) {
+        const Out* const term = static_cast<const Out*>(a.terms) + (int64_t)k * a.n + q;
+        boundary |= wide_is_boundary(term);
+        sum = k == 0 ? *term : sum + *term;
+      }
+      const Out d = boundary ? (Out)INFINITY : sum;
+      static_cast<Out*>(a.dist)[q] = d;
+      key = ordered_key64(-(double)d);  // (float -> double keeps order, infinities and NaN)
+    }
+    const int at = run_position(key, lds);
+    if (q < nv) {
+      a.dist_runs[r * kRunRows + at] = key;
+      a.dist_whose[r * kRunRows + at] = q;
+    }
+    __syncthreads();
+  }
+}
+
+__device__ __forceinline__ void wide_copy_row(uint8_t* __restrict__ to, const uint8_t* __restrict__ from, int64_t bytes, int unit, int lane, int lanes) {
+  if (unit == 16) {
+    for (int64_t b = lane * 16; b < bytes; b += lanes * 16) *reinterpret_cast<uint4*>(to + b) = *reinterpret_cast<const uint4*>(from + b);
+  } else if (unit == 8) {
+    for (int64_t b = lane * 8; b < bytes; b += lanes * 8) *reinterpret_cast<uint2*>(to + b) = *reinterpret_cast<const uint2*>(from + b);
+  } else if (unit == 4) {
+    for (int64_t b = lane * 4; b < bytes; b += lanes * 4) *reinterpret_cast<uint32_t*>(to + b) = *reinterpret_cast<const uint32_t*>(from + b);
+  } else {
+    for (int64_t b = lane; b < bytes; b += lanes) to[b] = from[b];
+  }
+}
+
+// The rows of the better fronts as listed, then the candidates by (distance descending, NaN last, row index), as far as
+// topk rows.  Grid: any number of workgroups from ceil(n / kWideShare) on.  Dynamic LDS: run_rank8_lds_bytes(n).
+template <class Out>
+__global__ __launch_bounds__(kRunRankThreads) void wide_front_pick_kernel(WideFront a) {
+  extern __shared__ __attribute__((aligned(16))) uint64_t wide_lds[];
+  __shared__ int pick_place[kWideShare], pick_of[kWideShare];
+  Out* const out_dist = static_cast<Out*>(a.out_dist);
+  const int64_t thread = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, threads = (int64_t)gridDim.x * blockDim.x;
+  if (a.ctrl->err != 0) {  // a device-side wait ran out: no partial result leaves the call
+    for (int64_t p = thread; p < a.topk; p += threads) {
+      a.out_rank[p] = -1;
+      out_dist[p] = (Out)NAN;
+    }
+    for (int64_t b = thread; b < (int64_t)a.topk * a.f_row_bytes; b += threads) a.out_f[b] = 0xFF;
+    if (a.x != nullptr)
+      for (int64_t b = thread; b < (int64_t)a.topk * a.x_row_bytes; b += threads) a.out_x[b] = 0xFF;
+    return;
+  }
+  const int nv = a.ctrl->nv, runs = runs_of(nv), start = a.ctrl->worst_start, need = a.ctrl->need, worst = a.ctrl->worst;
+  const int* __restrict__ list = a.list_base + start;
+  const int share = (nv + (int)gridDim.x - 1) / (int)gridDim.x;  // at most kWideShare
+  const int e0 = (int)blockIdx.x * share, e1 = min(nv, e0 + share);
+  if (e0 < nv) {  // (the whole workgroup)
+    const int entry = e0 + (int)threadIdx.x / kRunLanes, e = min(entry, e1 - 1);
+    const bool work = e0 + (int)(threadIdx.x & ~63u) / kRunLanes < e1;  // (of the wave)
+    RunSearch<uint64_t> s;
+    s.own = e / kRunRows;
+    s.at = e % kRunRows;
+    s.key = a.dist_runs[e];
+    const int q = a.dist_whose[e];
+    for (int first = 0; first < runs; first += kRunTile8) {
+      const int here = min(kRunTile8, runs - first);
+      __syncthreads();
+      runs_to_lds(a.dist_runs, nv, first, here, wide_lds);
+      __syncthreads();
+      if (work) run_search_all<kRunTies>(wide_lds, first, here, s);
+    }
+    run_search_end<kRunTies>(s);
+    if (entry < e1 && (threadIdx.x & (kRunLanes - 1)) == 0) {
+      pick_place[entry - e0] = (int)s.smaller < need ? start + (int)s.smaller : -1;
+      pick_of[entry - e0] = q;
+    }
+    __syncthreads();
+  }
+  int lanes = 64;  // of a row: the smallest power of two that holds its units
+  while (lanes > 4 && (lanes >> 1) >= (a.x != nullptr ? a.x_row_bytes / a.x_unit : 0) && (lanes >> 1) >= a.f_row_bytes / a.f_unit) lanes >>= 1;
+  const int per_wave = 64 / lanes, lane = (threadIdx.x & 63) % lanes;
+  const int slot = (int)(threadIdx.x >> 6) * per_wave + (int)(threadIdx.x & 63) / lanes, slots = (int)(blockDim.x >> 6) * per_wave;
+  auto copy = [&](int p, int row, int rank, Out d) {
+    if (a.x != nullptr)
+      wide_copy_row(a.out_x + (int64_t)p * a.x_row_bytes, a.x + (int64_t)row * a.x_row_stride, a.x_row_bytes, a.x_unit, lane, lanes);
+    wide_copy_row(a.out_f + (int64_t)p * a.f_row_bytes, a.f + (int64_t)row * a.f_row_stride, a.f_row_bytes, a.f_unit, lane, lanes);
+    if (lane == 0) {
+      a.out_rank[p] = rank;
+      out_dist[p] = d;
+    }
+  };
+  for (int i = slot; i < e1 - e0; i += slots)
+    if (pick_place[i] >= 0) copy(pick_place[i], list[pick_of[i]], worst, static_cast<const Out*>(a.dist)[pick_of[i]]);
+  for (int p = (int)blockIdx.x * slots + slot; p < start; p += (int)gridDim.x * slots) {
+    const int row = a.list_base[p];
+    copy(p, row, a.rank[row], (Out)(-INFINITY));
   }
 }
 

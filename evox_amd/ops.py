@@ -358,6 +358,9 @@ def _crowding_wide_vmap(info, in_dims, costs, mask):
 torch.library.register_vmap(crowding_wide, _crowding_wide_vmap)
 
 
+_WIDE_WHOLE_MAX = 32768  # rows of a population of 8-byte fitness whose orders come from sorted runs in LDS
+
+
 @torch.library.custom_op("evox_amd::nd_select_wide", mutates_args=())
 def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """nd_select for float64 or integer fitness: x (..., N, *D), f (..., N, M), topk -> (x, f, rank, crowding distance)
@@ -385,6 +388,26 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
     out_rank = torch.empty(*batch, topk, dtype=torch.int32, device=f.device)
     out_dist = torch.empty(*batch, topk, dtype=out_dtype, device=f.device)
     if out_rank.numel() == 0:
+        return out_x, out_f, out_rank, out_dist
+    if out_rank.numel() == topk and n <= _WIDE_WHOLE_MAX:
+        # one population: the whole selection in one call of the library
+        with torch.cuda.device(f.device):
+            wb = wide.reshape(n, m)
+            rows_f = f.reshape(n, m).contiguous()
+            rows_x = x.reshape(n, -1).contiguous()
+            row_bytes, f_row_bytes = rows_x.size(-1) * rows_x.element_size(), m * rows_f.element_size()
+            has_x = row_bytes > 0
+            ws = runtime.workspace(n, m, f.device)
+            stream = runtime.stream_handle(f.device)
+
+            def issue():
+                _lib.call("evox_hip_nd_environmental_selection_wide_whole", rows_x.data_ptr() if has_x else None, row_bytes, row_bytes,
+                          rows_f.data_ptr(), f_row_bytes, f_row_bytes, wb.data_ptr(), kind, n, m, wb.stride(0), wb.stride(1), topk,
+                          out_x.data_ptr() if has_x else None, out_f.data_ptr(), out_rank.data_ptr(), out_dist.data_ptr(),
+                          0 if out_dtype == torch.float64 else 1, ws.data_ptr(), ws.numel(), stream)
+                runtime.note_call(ws, stream)
+
+            runtime.checked(issue)
         return out_x, out_f, out_rank, out_dist
     # the ranks, as far as the front that holds the topk-th row, from the ranking kernels on a float32 image of the
     # fitness that keeps every comparison (the rows behind that front are marked unset)

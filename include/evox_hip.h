@@ -121,6 +121,15 @@ int evox_hip_nd_environmental_selection_wide(const void* x, int64_t x_row_bytes,
                                              int64_t topk, void* out_x, void* out_f, int32_t* out_rank, void* out_dist,
                                              int out_kind, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The whole selection of one population of at most 32 768 rows in one call: the ranks are found on a float32 image of the
+ * costs, the last front is ordered by the costs themselves.  workspace: evox_hip_workspace_bytes(n, m), with the control
+ * block that evox_hip_read_status reads. */
+int evox_hip_nd_environmental_selection_wide_whole(const void* x, int64_t x_row_bytes, int64_t x_row_stride_bytes, const void* f_rows,
+                                                   int64_t f_row_bytes, int64_t f_row_stride_bytes, const void* costs, int kind,
+                                                   int64_t n, int64_t m, int64_t stride_row, int64_t stride_col, int64_t topk,
+                                                   void* out_x, void* out_f, int32_t* out_rank, void* out_dist, int out_kind,
+                                                   void* workspace, size_t workspace_bytes, void* stream);
+
 /* The same for `batch` populations of one shape in the same launches (what a vmapped caller of the reference's
  * nd_environmental_selection gets, utils/op_register.py:26-51): x, f_rows and costs of population b lie
  * x_batch_stride_bytes, f_batch_stride_bytes and stride_batch elements further; rank is (batch, n), the outputs are
