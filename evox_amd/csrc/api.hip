@@ -22,6 +22,7 @@
 #include "prefix.hpp"
 #include "radix.hpp"
 #include "runs.hpp"
+#include "slots.hpp"
 #include "spatial.hpp"
 #include "stepped.hpp"
 #include "two.hpp"
@@ -340,6 +341,21 @@ static Fitness one_part(const float* f, int64_t n, int64_t sr, int64_t sc, int64
   return Fitness{f, sr, sc, n, f, sr, sc, step, step};
 }
 
+static int grant_dynamic_lds(const void* kernel, size_t lds);
+
+// Workgroups of one population that place its rows or candidates by searching the runs: one per compute unit, fewer where
+// several populations share the launch (none waits for another: at least sixteen).
+static int run_share_grid(const Ws& w) {
+  const int share = device_cus() / w.batch;
+  return share < 16 ? 16 : share;
+}
+
+// Up to this many rows the slot order comes from sorted runs: its searches grow with the square of the rows, the bucket sort's
+// five launches hardly.  Whole calls, us, buckets / runs: rank 4097 x 3 109 / 99, 5000 x 9 85 / 74, 10 007 x 5 85.5 / 77.9, 20 000 x 3
+// 213 / 209, 32 768 x 3 422 / 421, 40 000 x 3 540 / 542, 60 000 x 3 473 / 488; where keys crowd, 20 001 x 3 one front 112 / 104,
+// 16 populations of 4000 x 8 in a launch 311 / 169.
+constexpr int kSlotRunsRows = kRunMaxRows;
+
 static int stage_prepare(const Ws& w, const Fitness& src, bool with_sort, hipStream_t s, bool lexicographic = false) {
   const Layout& L = w.L;
   if (src.f == nullptr || src.f2 == nullptr || src.n_first < 0 || src.n_first > L.n) return kErrBadArg;
@@ -363,6 +379,33 @@ static int stage_prepare(const Ws& w, const Fitness& src, bool with_sort, hipStr
       launch(small_sort_kernel<false>);
     EVX_LAUNCH_CHECK();
     return 0;
+  }
+  if (with_sort && L.n <= kSlotRunsRows) {
+    const int runs = (L.npad + kRunRows - 1) / kRunRows;
+    // (about as many workgroups as there are compute units share the clearing)
+    const int grid = runs > device_cus() / w.batch ? runs : device_cus() / w.batch;
+    const size_t lds = run_rank8_lds_bytes(L.n);
+    int share = (int)round_up((L.n + run_share_grid(w) - 1) / run_share_grid(w), 16);  // (whole waves of sixteen keys)
+    if (share > kRunRankThreads / kRunLanes) share = kRunRankThreads / kRunLanes;
+    auto launch = [&](auto runs_kernel, auto places_kernel, auto* key_type) -> int {
+      using Key = std::remove_pointer_t<decltype(key_type)>;
+      hipLaunchKernelGGL(runs_kernel, dim3(grid, 1, w.batch), dim3(kRunRows), 0, s, src.f, src.sr, src.sc, (int)src.n_first, src.f2, src.sr2,
+                         src.sc2, L.n, L.m, L.npad, w.at<float>(L.xs), w.at<Key>(L.key), w.at<int>(L.members),
+                         w.at<unsigned long long>(L.partials), w.at<uint32_t>(L.ctrl), zero_words, runs, src.step, src.step2, w.step);
+      EVX_LAUNCH_CHECK();
+      if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(places_kernel), lds)) return e;
+      hipLaunchKernelGGL(places_kernel, dim3((L.n + share - 1) / share, 1, w.batch), dim3(kRunRankThreads), lds, s, w.at<Key>(L.key),
+                         w.at<int>(L.members), w.at<unsigned long long>(L.partials), L.n, L.m, L.npad, share, w.at<float>(L.xs),
+                         w.at<uint64_t>(L.key_sorted), w.at<uint32_t>(L.kid_sorted), w.at<float>(L.xs_sorted), w.at<int>(L.orig_of),
+                         w.at<int>(L.slot_of), w.at<SortParam>(L.sortparam), w.step);
+      EVX_LAUNCH_CHECK();
+      return 0;
+    };
+    if (lexicographic)
+      return many ? launch(slot_runs_kernel<true, true>, slot_places_kernel<true, true>, (uint64_t*)nullptr)
+                  : launch(slot_runs_kernel<false, true>, slot_places_kernel<false, true>, (uint64_t*)nullptr);
+    return many ? launch(slot_runs_kernel<true, false>, slot_places_kernel<true, false>, (double*)nullptr)
+                : launch(slot_runs_kernel<false, false>, slot_places_kernel<false, false>, (double*)nullptr);
   }
   auto launch_prepare = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(L.prep_blocks, 1, w.batch), dim3(256), 0, s, src.f, src.sr, src.sc, (int)src.n_first, src.f2,
@@ -903,13 +946,6 @@ static int shared_grid(int grid, int resident, int batch) {
   if (batch <= 1) return grid;
   const int cap = resident / batch < 1 ? 1 : resident / batch;
   return grid < cap ? grid : cap;
-}
-
-// Workgroups of one population that place its candidates by searching the runs: one per compute unit, fewer where
-// several populations share the launch (none waits for another: at least sixteen).
-static int run_share_grid(const Ws& w) {
-  const int share = device_cus() / w.batch;
-  return share < 16 ? 16 : share;
 }
 
 // phase 0: totals and matrix in one launch (or what the tunable prefix_mode asks for); 1: the totals alone, and the

@@ -8,7 +8,7 @@
 // (rows of large key lie in deep fronts).  Results never depend on the labelling: ranks are written
 // back by original index and fronts are listed in original-index order.
 //
-// The sort is an exact bucket sort in four small kernels: histogram of a monotone quantisation of the
+// Above kSlotRunsRows rows (below: slots.hpp) the sort is an exact bucket sort in four small kernels: histogram of a monotone quantisation of the
 // key, exclusive scan of the histogram, unordered scatter of the rows into their bucket ranges
 // (atomics), and an exact placement inside each bucket by counting the members that precede the row in
 // (key, original index) order.  The outcome is deterministic although the scatter is not.

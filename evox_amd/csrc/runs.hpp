@@ -35,6 +35,15 @@ __host__ __device__ inline size_t run_rank8_lds_bytes(int n) {  // (more keys: a
   return sizeof(uint64_t) * RunLds<uint64_t>::kStride * (size_t)(runs_of(n) < kRunTile8 ? runs_of(n) : kRunTile8);
 }
 
+// The key behind all others (no key of a row is larger; equal ones go by position).
+template <class K>
+__device__ __forceinline__ constexpr K run_last_key() {
+  if constexpr (std::is_same_v<K, double>)
+    return (double)INFINITY;
+  else
+    return ~(K)0;
+}
+
 // Does a key `other` precede the key `mine`: smaller, or equal where `first` says that its position is the earlier one?
 template <class K>
 __device__ __forceinline__ bool run_precedes(K other, K mine, bool first) {
@@ -53,6 +62,11 @@ __device__ __forceinline__ int run_search(const K* run, K mine, bool first) {
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ uint64_t lane_value(uint64_t v, int lane) {
   return ((uint64_t)lane_value((uint32_t)(v >> 32), lane) << 32) | lane_value((uint32_t)v, lane);
+}
+
+// (integers below 2^53: the hardware compares doubles at the rate of 32-bit values, 64-bit integers several times slower)
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __longlong_as_double((long long)lane_value((uint64_t)__double_as_longlong(v), lane));
 }
 
 // The position of every thread's key among the keys of its workgroup of kRunRows threads (ascending, equal keys by
@@ -96,7 +110,7 @@ __device__ __forceinline__ void runs_to_lds(const K* __restrict__ sorted, int nv
     *reinterpret_cast<uint4*>(lds + (e / kRunRows) * RunLds<K>::kStride + (e % kRunRows)) = *reinterpret_cast<const uint4*>(sorted + e);
 #pragma unroll 4
   for (int e = whole + threadIdx.x; e < runs * kRunRows; e += blockDim.x)
-    lds[(e / kRunRows) * RunLds<K>::kStride + (e % kRunRows)] = e < count ? sorted[e] : ~(K)0;
+    lds[(e / kRunRows) * RunLds<K>::kStride + (e % kRunRows)] = e < count ? sorted[e] : run_last_key<K>();
 }
 
 // The sum / maximum / minimum over the kRunLanes consecutive lanes of a group, the same in all of them.
@@ -123,14 +137,16 @@ template <class K>
 struct RunSearch {
   K key;
   int own, at;  // its run, and its place in that
-  uint32_t smaller = 0;
-  K before = 0, behind = ~(K)0;  // the largest key before it (0 where there is none) and the smallest behind it (meaningless at the last place)
+  uint32_t smaller = 0;   // how many keys precede it
+  uint32_t equal = 0;     // kRunEqual: how many of them are equal to it
+  K before = 0, behind = run_last_key<K>();  // the largest key before it (0 where there is none) and the smallest behind it (meaningless at the last place)
 };
 
 // What a search looks for besides the number of keys that precede the key.
 constexpr int kRunTies = 0;        // (equal keys of earlier positions precede it)
 constexpr int kRunNeighbours = 1;  // ... and its neighbours
 constexpr int kRunSmaller = 2;     // (only smaller keys precede it)
+constexpr int kRunEqual = 3;       // as kRunTies, and how many of the keys that precede it are equal to it
 
 // U searches side by side in the runs `first` + r0, r0 + kRunLanes, ... of which LDS holds `runs`.
 template <int U, int MODE, class K>
@@ -160,6 +176,9 @@ __device__ __forceinline__ void run_search_some(const K* lds, int first, int run
     if (q.key == (K)0 && (MODE == kRunSmaller || first + r > q.own)) n = 0;
     if (own) n = q.at;
     q.smaller += r < runs ? (uint32_t)n : 0u;
+    if constexpr (MODE == kRunEqual) {  // (seldom any: a second search only where the last key that precedes it is equal)
+      if (r < runs && n > 0 && run[n - 1] == q.key) q.equal += (uint32_t)(n - run_search<kRunRows>(run, q.key, false));
+    }
     if constexpr (MODE == kRunNeighbours) {  // (read whether or not there is one: branches would put the reads one after the other)
       const K lower = run[n > 0 ? n - 1 : 0], upper = run[min(own ? n + 1 : n, kRunRows - 1)];
       if (r < runs && n > 0) q.before = lower > q.before ? lower : q.before;
@@ -188,6 +207,7 @@ __device__ __forceinline__ void run_search_all(const K* lds, int first, int runs
 template <int MODE, class K>
 __device__ __forceinline__ void run_search_end(RunSearch<K>& q) {
   q.smaller = run_group(q.smaller, [](uint32_t a, uint32_t b) { return a + b; });
+  if constexpr (MODE == kRunEqual) q.equal = run_group(q.equal, [](uint32_t a, uint32_t b) { return a + b; });
   if constexpr (MODE == kRunNeighbours) {
     q.before = run_group(q.before, [](K a, K b) { return a > b ? a : b; });
     q.behind = run_group(q.behind, [](K a, K b) { return a < b ? a : b; });
