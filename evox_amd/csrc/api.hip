@@ -948,6 +948,10 @@ static int shared_grid(int grid, int resident, int batch) {
   return grid < cap ? grid : cap;
 }
 
+constexpr int kNearbyMaxObjectives = 15;  // (the order of the slots is one more)
+template <int M>
+static int launch_nearby_totals(const Ws& w, hipStream_t s);
+
 // phase 0: totals and matrix in one launch (or what the tunable prefix_mode asks for); 1: the totals alone, and the
 // pairwise kernel for a population that is not finite; 2: the matrix alone, unless front 0 holds w.matrix_unless rows.
 template <int M>
@@ -972,12 +976,19 @@ static int launch_dominance_prefix(const Ws& w, hipStream_t s, int phase) {
     hipLaunchKernelGGL(kernel, dim3(tiles, stretches), dim3(kPrefixThreads), lds, s, w.at<int>(L.pos), w.at<int>(L.scost),
                        w.at<uint32_t>(L.kid_sorted), w.at<uint64_t>(L.dom), L.n, L.kstride, L.wstride, L.nwords, shift, buckets,
                        chunk, bands, phase == 0 ? opt().prefix_mode : phase, w.at<int>(L.total0), w.at<int>(L.witness0),
-                       w.at<SortParam>(L.sortparam), phase == 2 ? w.at<int>(L.fsize) : (const int*)nullptr, (int)w.matrix_unless);
+                       w.at<SortParam>(L.sortparam), phase == 2 ? w.at<int>(L.fsize) : (const int*)nullptr, (int)w.matrix_unless,
+                       NearbyWork{});
     EVX_LAUNCH_CHECK();
     return 0;
   };
   // (200 000 x 3: 957 -> 769 us, x 4: 972 -> 797; 100 000 x 3: 319 -> 317; 65536 x 3: 184 -> 220: half as many workgroups)
-  if (TT == 2 && opt().prefix_double_tile > 0 && L.n >= opt().prefix_double_tile) {
+  // The totals alone in spatial order or in slot order, whole selections in us where front 0 holds what is kept, slot /
+  // spatial: x 3 70 000 298 / 302, 100 000 366 / 355;  x 5 50 000 274 / 293, 60 000 311 / 309, 150 000 630 / 520;  x 8 50 000
+  // 322 / 331, 60 000 401 / 369, 200 000 1176 / 743;  x 12 60 000 495 / 440;  x 15 40 000 381 / 405.
+  if (M <= kNearbyMaxObjectives && phase == 1 && L.n >= (M <= 4 ? 90112 : 57344)) {
+    if constexpr (M <= kNearbyMaxObjectives)
+      if (int e = launch_nearby_totals<M>(w, s)) return e;
+  } else if (TT == 2 && opt().prefix_double_tile > 0 && L.n >= opt().prefix_double_tile) {
     if (int e = launch(dominance_prefix_kernel<M, WW, TT>, TT)) return e;
   } else {
     if (int e = launch(dominance_prefix_kernel<M, WW, 1>, 1)) return e;
@@ -987,6 +998,70 @@ static int launch_dominance_prefix(const Ws& w, hipStream_t s, int phase) {
   hipLaunchKernelGGL(dominance_nonfinite_kernel<M>, dim3(device_cus() * 8), dim3(256), 0, s, w.at<float>(L.xs_sorted),
                      w.at<uint64_t>(L.key_sorted), w.at<uint32_t>(L.kid_sorted), w.at<uint64_t>(L.dom), L.n, L.npad, L.wstride,
                      L.nwords, w.at<SortParam>(L.sortparam));
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
+// The row totals alone (phase 1) from the rows in spatial order.  What it needs besides the orders lies where the matrix
+// would: nobody reads that before a second launch builds it.
+template <int M>
+static int launch_nearby_totals(const Ws& w, hipStream_t s) {
+  const Layout& L = w.L;
+  constexpr int MO = M + 1;
+  constexpr int WW = MO <= kPrefixWideObjectives ? 8 : 4;
+  const int stride = (int)round_up(L.n, 64), groups = stride / 64;
+  size_t o = L.dom;
+  auto take = [&](size_t bytes) {
+    const size_t at = o;
+    o = align_up(o + bytes);
+    return at;
+  };
+  const int tiles = (groups + WW - 1) / WW;
+  // (parts small enough that the last ones end together, large enough to be worth a tile's tables: 10 us against 0.3 per group)
+  int cap = groups / 16;
+  if (cap > kPrefixNearbyGroups) cap = kPrefixNearbyGroups;
+  if (cap < 32) cap = 32;
+  const size_t most_full = (size_t)tiles * (size_t)(groups / cap + 1);
+  const size_t hist = take(sizeof(int) * kNearbyCells), flags = take(sizeof(unsigned long long) * 64), queue = take(sizeof(int) * 4);
+  const size_t starts = take(sizeof(int) * (kNearbyCells + 1)), cursor = take(sizeof(int) * kNearbyCells);
+  const size_t cell = take(sizeof(uint16_t) * (size_t)L.n), place = take(sizeof(int) * (size_t)L.n), slot_at = take(sizeof(int) * (size_t)L.n);
+  const size_t pos_at = take(sizeof(int) * MO * (size_t)stride), upper_at = take(sizeof(int) * MO * (size_t)stride);
+  const size_t lo = take(sizeof(int) * MO * (size_t)groups), top = take(sizeof(int) * MO * (size_t)groups),
+               hi = take(sizeof(int) * MO * (size_t)groups);
+  const size_t box = take(sizeof(int) * 2 * MO * (size_t)tiles), near_list = take(sizeof(uint16_t) * (size_t)tiles * (size_t)groups);
+  const size_t near_count = take(sizeof(int) * (size_t)tiles), full = take(sizeof(int2) * most_full), rest = take(sizeof(int2) * (size_t)tiles);
+  if (o > L.dom + sizeof(uint64_t) * (size_t)L.n * (size_t)L.wstride || groups > 65536) return kErrWorkspace;
+  SortParam* const param = w.at<SortParam>(L.sortparam);
+  hipLaunchKernelGGL(reset_state_kernel, dim3(16), dim3(256), 0, s, w.at<uint32_t>(hist), (int64_t)((queue - hist) / 4 + 4));
+  EVX_LAUNCH_CHECK();
+  const int cell_rows = kNearbyCellThreads * kNearbyCellRows;
+  hipLaunchKernelGGL(nearby_cells_kernel, dim3((L.n + cell_rows - 1) / cell_rows), dim3(kNearbyCellThreads), 0, s, w.at<int>(L.pos), L.n,
+                     L.kstride, M, param, w.at<uint16_t>(cell), w.at<int>(place), w.at<int>(hist));
+  EVX_LAUNCH_CHECK();
+  hipLaunchKernelGGL(bucket_scan_kernel<false>, dim3(kNearbyCells / 1024), dim3(256), 0, s, w.at<int>(hist), kNearbyCells, w.at<int>(starts),
+                     w.at<int>(cursor), w.at<unsigned long long>(flags), w.ctrl(), (int64_t)0);
+  EVX_LAUNCH_CHECK();
+  int blocks = (L.n + 255) / 256;
+  if (blocks > 2048) blocks = 2048;
+  hipLaunchKernelGGL(nearby_scatter_kernel, dim3(blocks), dim3(256), 0, s, w.at<uint16_t>(cell), w.at<int>(place), L.n, param, w.ctrl(),
+                     w.at<int>(starts), w.at<int>(slot_at));
+  EVX_LAUNCH_CHECK();
+  hipLaunchKernelGGL(nearby_gather_kernel, dim3((L.n + 255) / 256, MO), dim3(256), 0, s, w.at<int>(L.pos), w.at<int>(L.scost),
+                     w.at<uint32_t>(L.kid_sorted), L.n, L.kstride, M, param, w.ctrl(), w.at<int>(slot_at), stride, w.at<int>(pos_at),
+                     w.at<int>(upper_at), groups, w.at<int>(lo), w.at<int>(top), w.at<int>(hi));
+  EVX_LAUNCH_CHECK();
+  hipLaunchKernelGGL(nearby_pairs_kernel<MO>, dim3(tiles), dim3(256), 0, s, w.at<int>(lo), w.at<int>(top), w.at<int>(hi), groups, WW, cap, param,
+                     w.ctrl(), w.at<int>(box), w.at<uint16_t>(near_list), w.at<int>(near_count), w.at<int2>(full), w.at<int2>(rest),
+                     w.at<int>(queue));
+  EVX_LAUNCH_CHECK();
+  const auto kernel = dominance_prefix_kernel<MO, WW, 1, true>;
+  const size_t lds = prefix_lds_bytes(MO, WW, kPrefixBuckets);
+  if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return e;
+  const int grid = device_cus() * (lds <= 76 * 1024 ? 2 : 1);  // (what a compute unit holds at once)
+  const NearbyWork work = {w.at<int>(box), w.at<uint16_t>(near_list), w.at<int>(near_count), w.at<int2>(full), w.at<int2>(rest), w.at<int>(queue), cap};
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kPrefixThreads), lds, s, w.at<int>(pos_at), w.at<int>(upper_at), (const uint32_t*)nullptr,
+                     (uint64_t*)nullptr, L.n, stride, (int64_t)0, groups, 0, kPrefixBuckets, 0, 0, 1, w.at<int>(L.total0), w.at<int>(L.witness0),
+                     param, &w.ctrl()->err, 0, work);
   EVX_LAUNCH_CHECK();
   return 0;
 }
@@ -1117,15 +1192,15 @@ static CrowdArgs crowd_args(const Ws& w, const int* list, bool use_orders, int f
   return a;
 }
 
-// The three launches that read the orders of a large last front off the orders of the whole population.
-static int stage_front_orders(const Ws& w, const int* list, hipStream_t s) {
+// The three launches that read the orders of a large last front (of more than `above` rows) off the orders of the whole
+// population.
+static int stage_front_orders(const Ws& w, const int* list, int above, hipStream_t s) {
   const Layout& L = w.L;
   {
     const RadixBuffers b = radix_buffers(w);
     const int spans = (L.n + kFrontOrderSpan - 1) / kFrontOrderSpan;
     int* const number = reinterpret_cast<int*>(w.at<uint32_t>(L.dkey));  // free until the distances are known
     int* const per_span = b.table;
-    const int above = crowd_mid_split(L) ? kMidArgsortRows : kRadixMinCandidates;  // (smaller ones: the sorted runs)
     hipLaunchKernelGGL(front_number_kernel, dim3((L.n + 1023) / 1024), dim3(256), 0, s, list, w.ctrl(),
                        w.at<SortParam>(L.sortparam), above, number);
     EVX_LAUNCH_CHECK();
@@ -1206,17 +1281,21 @@ static int launch_crowd_pick(const Ws& w, const CrowdArgs& a, bool want_order, c
   return 0;
 }
 
-static int stage_crowd_sort(const Ws& w, const int* list, bool use_orders, int fused, hipStream_t s, bool after_peel_tail = false) {
+// without_runs, here and below: the launches with the sorted runs are left out where a larger population has them beside the
+// others, which then take a front of any size.
+static int stage_crowd_sort(const Ws& w, const int* list, bool use_orders, int fused, hipStream_t s, bool after_peel_tail = false,
+                            bool without_runs = false) {
   const Layout& L = w.L;
   const int tail_flag = after_peel_tail ? 1 : 0;
   if (crowd_mid_sort(L)) return launch_crowd_runs(w, crowd_args(w, list, false, fused), tail_flag, s);
   use_orders = use_orders && prefix_dominance_applies(L) && w.batch == 1;
   // a large front of a population whose matrix came from the per-objective orders: its own orders are read off
   // those (finish.hpp); the three kernels and those below choose on the device which of them has work
+  CrowdArgs a = crowd_args(w, list, use_orders, fused);
+  if (without_runs) a.mid_sort = 0;
   if (use_orders)
-    if (int e = stage_front_orders(w, list, s)) return e;
-  const CrowdArgs a = crowd_args(w, list, use_orders, fused);
-  if (crowd_mid_split(L))
+    if (int e = stage_front_orders(w, list, a.mid_sort == 2 ? kMidArgsortRows : kRadixMinCandidates, s)) return e;
+  if (a.mid_sort == 2)
     if (int e = launch_crowd_runs(w, a, tail_flag, s)) return e;
   const size_t lds = crowd_lds_bytes(L, fused);
   const void* const kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_sort_kernel<true>) : reinterpret_cast<const void*>(crowd_sort_kernel<false>);
@@ -1237,15 +1316,16 @@ static int stage_crowd_sort(const Ws& w, const int* list, bool use_orders, int f
 // Crowding distances of those candidates and, with want_order, the selection order; gather, where it is given: the
 // selected rows too, behind the order (crowd_mid_sort populations only).
 static int stage_crowd_finish(const Ws& w, const int* list, bool want_order, int fused, hipStream_t s, bool after_peel_tail = false,
-                              const GatherArgs* gather = nullptr) {
+                              const GatherArgs* gather = nullptr, bool without_runs = false) {
   const Layout& L = w.L;
   const int tail_flag = after_peel_tail ? 1 : 0;
-  const CrowdArgs a = crowd_args(w, list, false, fused);
+  CrowdArgs a = crowd_args(w, list, false, fused);
+  if (without_runs && a.mid_sort == 2) a.mid_sort = 0;
   if (gather == nullptr && fused != 0 && L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives)
     return 0;  // (no front of this population is too large for crowd_small_front: nothing is left to do)
   if (crowd_mid_sort(L)) return launch_crowd_pick(w, a, want_order, gather, tail_flag, s);
   if (gather != nullptr) return kErrBadArg;
-  if (crowd_mid_split(L))
+  if (a.mid_sort == 2)
     if (int e = launch_crowd_pick(w, a, want_order, nullptr, tail_flag, s)) return e;
   const size_t lds = crowd_lds_bytes(L, 0);
   const void* const kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_finish_kernel<true>) : reinterpret_cast<const void*>(crowd_finish_kernel<false>);
@@ -2389,14 +2469,25 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
     else
       hipLaunchKernelGGL(gather_kernel<false>, gather_grid, dim3(256), 0, s, g);
   };
+  // Above kMidArgsortRows rows the launches with the sorted runs stand beside those for other fronts.  What the last
+  // selection of the shape found says whether they are worth their four launches (a converged population's front is larger:
+  // 70 000 x 3 on a plane 304 -> 288 us).
+  bool without_runs = false;
+  if (batch == 1 && crowd_mid_split(L) && opt().launch_memory) {
+    g.outcome = outcome_slot(n, m, may_allocate, s, 3);
+    const int small = L.m <= kFusedFrontObjectives ? (kFusedFrontValues / L.m < kFusedFrontRows ? kFusedFrontValues / L.m : kFusedFrontRows) : 0;
+    g.outcome_from = small > kMidSortMinCandidates ? small : kMidSortMinCandidates;
+    g.outcome_to = kMidArgsortRows;
+    without_runs = g.outcome != nullptr && __atomic_load_n(g.outcome, __ATOMIC_RELAXED) == 2;
+  }
   if (batch == 1 ? two_applies(L, topk) : many_two_share(L, batch, topk) >= batch) {
     const int e = stage_rank_two(w, fit, topk, true, nullptr, s);
     if (e != kErrNotResident || batch > 1) {
       if (e) return e == kErrNotResident ? kErrBadArg : e;
       // the last front by the ordering kernels, then the gather, as after a peel that leaves the last front alone
-      if (int c = stage_crowd_sort(w, w.at<int>(L.perm), false, 2, s, false)) return c;
+      if (int c = stage_crowd_sort(w, w.at<int>(L.perm), false, 2, s, false, without_runs)) return c;
       if (crowd_mid_sort(L)) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, false, &g);
-      if (int c = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, false)) return c;
+      if (int c = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, false, nullptr, without_runs)) return c;
       launch_gather(false);
       EVX_LAUNCH_CHECK();
       return 0;
@@ -2424,8 +2515,9 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
     return e;
   }
   g.order_from_peel = peel_always_orders ? 1 : 0;
-  g.outcome = batch == 1 && peel_orders && !peel_always_orders && opt().launch_memory ? outcome_slot(n, m, may_allocate, s) : nullptr;
-  const int last_outcome = g.outcome != nullptr ? __atomic_load_n(g.outcome, __ATOMIC_RELAXED) : 0;
+  if (!crowd_mid_split(L))
+    g.outcome = batch == 1 && peel_orders && !peel_always_orders && opt().launch_memory ? outcome_slot(n, m, may_allocate, s) : nullptr;
+  const int last_outcome = g.outcome != nullptr && g.outcome_to == 0 ? __atomic_load_n(g.outcome, __ATOMIC_RELAXED) : 0;
   // Where the peel kernel may have ordered the last front, the kernels that would order it look at Ctrl.tail_done and
   // return at once.  A launch that does nothing still costs 2 to 4.7 us, so with up to three objectives -- last
   // fronts of a few hundred rows, which the peel kernel orders -- all ordering stages and the gather share one
@@ -2474,10 +2566,10 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
     return 0;
   }
   if (!one_ordering_launch) {
-    if (int e = stage_crowd_sort(w, w.at<int>(L.perm), true, 2, s, peel_orders)) return e;
+    if (int e = stage_crowd_sort(w, w.at<int>(L.perm), true, 2, s, peel_orders, without_runs)) return e;
     const bool never_large = L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives;
     if (crowd_mid_sort(L) && !never_large) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, &g);
-    if (int e = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders)) return e;
+    if (int e = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, nullptr, without_runs)) return e;
     if (peel_orders)
       launch_gather(true);
     else

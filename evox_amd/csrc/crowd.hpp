@@ -144,7 +144,10 @@ struct GatherArgs {
   int* out_order;
   const Ctrl* ctrl;
   int order_from_peel;  // the host launched nothing that orders the last front: the peel kernel must have (Ctrl.tail_done)
-  int* outcome;  // pinned host memory or null: 1 when the peel kernel has ordered the last front of this call, else 2
+  // pinned host memory or null: 1 when the peel kernel has ordered the last front of this call, else 2; with outcome_to > 0:
+  // 1 when that front has more than outcome_from and at most outcome_to rows, else 2
+  int* outcome;
+  int outcome_from, outcome_to;
   // pinned host memory or null: whether front 0 (front0_size rows) held the front0_enough rows that this call keeps --
   // 2: no, 1: yes, 3: yes, and at the call that wrote the word before as well
   int* front0_note;
@@ -172,7 +175,8 @@ __device__ __forceinline__ void to_population(GatherArgs& g) {
 // What the host's choice of launches at its next call goes by (it reads the words without waiting for anything).
 __device__ __forceinline__ void gather_notes(const GatherArgs& a, int block) {
   if (a.outcome != nullptr && block == 0 && threadIdx.x == 0)
-    __hip_atomic_store(a.outcome, a.ctrl->tail_done != 0 ? 1 : 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(a.outcome, (a.outcome_to > 0 ? a.ctrl->nv > a.outcome_from && a.ctrl->nv <= a.outcome_to : a.ctrl->tail_done != 0) ? 1 : 2,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (a.front0_note != nullptr && block == 0 && threadIdx.x == 0) {
     const int before = __hip_atomic_load(a.front0_note, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const int now = *a.front0_size >= a.front0_enough ? (before == 1 || before == 3 ? 3 : 1) : 2;

@@ -37,6 +37,7 @@ constexpr int kPrefixWideObjectives = 10;  // up to here tiles of 8 words (14.4 
 constexpr int kPrefixBuckets = 1024;       // entries of the coarse index per objective, at most (plus two)
 constexpr int kPrefixThreads = 1024;
 constexpr int kPrefixRowChunk = 32768;     // rows per workgroup, at most (`chunk`, a multiple of 64)
+constexpr int kPrefixNearbyGroups = 256;  // groups of 64 rows in a part of the work on rows in spatial order, at most
 constexpr int kPrefixMaxRows = 1 << 22;    // a position and a slot of the tile share one int
 
 // LDS of dominance_prefix_kernel<M, WW>, per objective: bit sets and counts (the scratch of the build lies over
@@ -389,48 +390,260 @@ __device__ inline void quad_transpose_pieces(uint64_t (&d)[8], int lane) {
   for (int w = 0; w < 8; ++w) d[w] = (uint64_t)(uint32_t)v[2 * w] | ((uint64_t)(uint32_t)v[2 * w + 1] << 32);
 }
 
+// ---- The row totals alone, without the matrix: nothing is written where a tile's words would lie, so the rows need not be
+// in slot order.  In spatial order -- by the leading bits of their positions, an objective's after the other's -- a tile of
+// 512 rows and a group of 64 rows lie in boxes of their own, and a tile whose box does not lie below the group's in
+// every objective holds no dominator of its rows: of the pairs of tile and group 13 % are left at 200 000 x 8 (directions
+// on a sphere), 17 % for uniform fitness, where the triangle of the slot order is 50 %.  The order of the slots is one
+// more objective: a dominator's slot lies before the first slot with the row's key, which leaves out the row itself and
+// its equals.
+// 200 000 x 8, us: the order 68 (cells 16, gather 22, pairs 16), the totals 251 -- LDS look-ups as before, a quarter as many --
+// against 760 in slot order; the selection 1176 -> 743.
+constexpr int kNearbyCodeBits = 12;
+constexpr int kNearbyCells = 1 << kNearbyCodeBits;
+
+// cell[slot] = the row's cell, place[slot] = its place among the rows of that cell, hist = the number of rows in every cell.
+// A workgroup counts its rows in LDS and takes its places of a cell with one addition (an addition per row, and another one
+// for its place: 19 us each at 200 000 rows).
+constexpr int kNearbyCellThreads = 1024, kNearbyCellRows = 4;  // rows per thread
+__global__ __launch_bounds__(kNearbyCellThreads) void nearby_cells_kernel(const int* __restrict__ pos, int n, int kstride, int m,
+                                                                          const SortParam* __restrict__ param, uint16_t* __restrict__ cell,
+                                                                          int* __restrict__ place, int* __restrict__ hist) {
+  __shared__ int count[kNearbyCells];
+  if (param->nonfinite != 0) return;
+  for (int c = threadIdx.x; c < kNearbyCells; c += kNearbyCellThreads) count[c] = 0;
+  __syncthreads();
+  const float scale = 4096.0f / (float)n;
+  const int j0 = (int)blockIdx.x * kNearbyCellThreads * kNearbyCellRows + (int)threadIdx.x;
+  uint32_t code[kNearbyCellRows] = {};
+  int at[kNearbyCellRows];
+  int bits = 0;
+  for (int level = 11; bits < kNearbyCodeBits; --level)
+    for (int k = 0; k < m && bits < kNearbyCodeBits; ++k, ++bits)
+#pragma unroll
+      for (int u = 0; u < kNearbyCellRows; ++u) {
+        const int j = j0 + u * kNearbyCellThreads;
+        const uint32_t q = j < n ? (uint32_t)((float)pos[(int64_t)k * kstride + j] * scale) : 0u;
+        code[u] = (code[u] << 1) | ((q >> level) & 1u);
+      }
+#pragma unroll
+  for (int u = 0; u < kNearbyCellRows; ++u) at[u] = j0 + u * kNearbyCellThreads < n ? atomicAdd(&count[code[u]], 1) : 0;
+  __syncthreads();
+  for (int c = threadIdx.x; c < kNearbyCells; c += kNearbyCellThreads) {
+    const int mine = count[c];
+    if (mine != 0) count[c] = atomicAdd(&hist[c], mine);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kNearbyCellRows; ++u) {
+    const int j = j0 + u * kNearbyCellThreads;
+    if (j < n) {
+      cell[j] = (uint16_t)code[u];
+      place[j] = count[code[u]] + at[u];
+    }
+  }
+}
+
+// slot_at[i] = the slot at place i of the spatial order (any order inside a cell: the totals do not depend on it).
+__global__ __launch_bounds__(256) void nearby_scatter_kernel(const uint16_t* __restrict__ cell, const int* __restrict__ place, int n,
+                                                             const SortParam* __restrict__ param, const Ctrl* __restrict__ ctrl,
+                                                             const int* __restrict__ start, int* __restrict__ slot_at) {
+  if (param->nonfinite != 0 || ctrl->err != 0) return;
+  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) slot_at[start[cell[j]] + place[j]] = j;
+}
+
+// Order blockIdx.y (below m: that of an objective; m: that of the slots) of the rows at 256 places: positions and
+// bounds by place (columns `stride` apart), and the box of every 64 places: smallest and
+// largest position, largest bound.
+__global__ __launch_bounds__(256) void nearby_gather_kernel(const int* __restrict__ pos, const int* __restrict__ upper,
+                                                            const uint32_t* __restrict__ kid, int n, int kstride, int m,
+                                                            const SortParam* __restrict__ param, const Ctrl* __restrict__ ctrl,
+                                                            const int* __restrict__ slot_at, int stride, int* __restrict__ pos_at, int* __restrict__ upper_at, int group_stride,
+                                                            int* __restrict__ group_lo, int* __restrict__ group_top,
+                                                            int* __restrict__ group_hi) {
+  if (param->nonfinite != 0 || ctrl->err != 0) return;
+  const int k = blockIdx.y, i = blockIdx.x * 256 + (int)threadIdx.x;
+  int p = 0x7FFFFFFF, top = 0, u = 0;
+  if (i < n) {
+    const int slot = slot_at[i];
+    p = k < m ? pos[(int64_t)k * kstride + slot] : slot;
+    u = k < m ? upper[(int64_t)k * kstride + slot] : (int)kid[slot];
+    top = p;
+    pos_at[(int64_t)k * stride + i] = p;
+    upper_at[(int64_t)k * stride + i] = u;
+  }
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    p = min(p, __shfl_xor(p, off));
+    top = max(top, __shfl_xor(top, off));
+    u = max(u, __shfl_xor(u, off));
+  }
+  const int group = i >> 6;
+  if ((threadIdx.x & 63) == 0 && group < group_stride) {
+    group_lo[(int64_t)k * group_stride + group] = p;
+    group_top[(int64_t)k * group_stride + group] = top;
+    group_hi[(int64_t)k * group_stride + group] = u;
+  }
+}
+
+// The box of every tile, the groups that it can have dominators of (near[tile * groups ...]: the smallest position of the
+// tile lies below the largest bound of the group in every objective), and the work: parts of `cap` groups of a tile's list in
+// `full`, what is left of the lists in `rest`, counted in queue[0] and queue[1].  The tiles differ by a factor of fifty (a
+// tile at the foot of the population is near to all groups): a workgroup per tile and quarter of the groups ended 200 us
+// after the average one at 200 000 x 8.  A workgroup per tile.
+template <int M>
+__global__ __launch_bounds__(256) void nearby_pairs_kernel(const int* __restrict__ group_lo, const int* __restrict__ group_top,
+                                                           const int* __restrict__ group_hi, int groups, int tile_groups, int cap,
+                                                           const SortParam* __restrict__ param, const Ctrl* __restrict__ ctrl,
+                                                           int* __restrict__ box, uint16_t* __restrict__ near_list, int* __restrict__ near_count,
+                                                           int2* __restrict__ full, int2* __restrict__ rest, int* __restrict__ queue) {
+  __shared__ int lo[M];
+  __shared__ int found, first_item;
+  if (param->nonfinite != 0 || ctrl->err != 0) return;
+  const int tile = blockIdx.x, lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) found = 0;
+  if ((int)threadIdx.x < M * 8) {  // (up to eight groups to a tile)
+    const int k = (int)threadIdx.x >> 3, u = (int)threadIdx.x & 7, g = tile * tile_groups + u;
+    const bool have = u < tile_groups && g < groups;
+    int low = have ? group_lo[(int64_t)k * groups + g] : 0x7FFFFFFF;
+    int top = have ? group_top[(int64_t)k * groups + g] : 0;
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) {
+      low = min(low, __shfl_xor(low, off));
+      top = max(top, __shfl_xor(top, off));
+    }
+    if (u == 0) {
+      lo[k] = low;
+      box[(tile * M + k) * 2] = low;
+      box[(tile * M + k) * 2 + 1] = top;
+    }
+  }
+  __syncthreads();
+  uint16_t* const list = near_list + (int64_t)tile * groups;
+  for (int g0 = 0; g0 < groups; g0 += blockDim.x) {
+    const int g = g0 + (int)threadIdx.x;
+    int hi[M];  // (all loads before any use)
+#pragma unroll
+    for (int k = 0; k < M; ++k) hi[k] = group_hi[(int64_t)k * groups + (g < groups ? g : 0)];
+    bool near = g < groups;
+#pragma unroll
+    for (int k = 0; k < M; ++k) near &= lo[k] < hi[k];
+    const uint64_t members = __builtin_amdgcn_ballot_w64(near);
+    int at = 0;
+    if (lane == 0 && members != 0ull) at = atomicAdd(&found, __popcll(members));
+    at = __shfl(at, 0);
+    if (near) list[at + __popcll(members & ((1ull << lane) - 1ull))] = (uint16_t)g;
+  }
+  __syncthreads();
+  const int parts = found / cap;
+  if (threadIdx.x == 0) {
+    near_count[tile] = found;
+    if (parts > 0) first_item = atomicAdd(&queue[0], parts);
+    if (found > parts * cap) rest[atomicAdd(&queue[1], 1)] = make_int2(tile, parts);
+  }
+  __syncthreads();
+  for (int p = threadIdx.x; p < parts; p += blockDim.x) full[first_item + p] = make_int2(tile, p);
+}
+
+// Inclusive scan over the 64 lanes of a wave: shifts inside the DPP rows of sixteen lanes, then a row's last lane to the
+// rows behind it -- six vector instructions, where a permute through LDS is a round trip each.  op(0, v) == v.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, Op op) {
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr 1, 2, 4, 8
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));         // row_bcast 15: into rows 1 and 3
+  return op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));      // row_bcast 31: into rows 2 and 3
+}
+template <class Op>
+__device__ __forceinline__ uint64_t wave_scan_halves(uint64_t v, Op op) {  // (nothing passes from the lower half to the upper)
+  return (uint64_t)wave_scan((uint32_t)v, op) | ((uint64_t)wave_scan((uint32_t)(v >> 32), op) << 32);
+}
+
 // A workgroup takes TT neighbouring tiles of WW words (TT = 2 with WW = 8: the whole 128-byte line of every row).
 // grid.x = the ceil(nwords / (WW * TT)) tile groups of dominator slots, rounded up to a multiple of 128 / (WW * TT),
 // grid.y = stretches of `chunk` rows, counted from the first row of the tile or (bands) from row 0 (rows above the
 // tile have no word there).  Dynamic LDS: TT * prefix_lds_bytes(M, WW, buckets).  Writes the words of its tiles in
 // every row of the stretch and adds their popcount to total0[row]; witness0[row] = the highest non-empty word so far
 // (both start from objective_order_kernel's 0 and -1).  Sets param->totals_valid.  mode: bit 0 = the row totals,
-// bit 1 = the matrix.  unless_front0 (null: always run): the size of front 0, known from a launch with mode 1 and the
+// bit 1 = the matrix.  NEARBY: the totals alone, of rows in spatial order, by workgroups that take parts of
+// the work until none is left (unless_front0: the error word).  unless_front0 (null: always run): the size of front 0, known from a launch with mode 1 and the
 // count stage; when it holds `enough` rows nobody will read the matrix, and the launch (mode 2) does nothing.
-template <int M, int WW, int TT>
+struct NearbyWork {
+  const int* box;         // [tile][objective]: smallest and largest position
+  const uint16_t* near_list;  // [tile][groups]
+  const int* near_count;
+  const int2 *full, *rest;  // (tile, part of its list)
+  int* queue;             // how many of either, and the next one to take
+  int cap;                // groups per part, at most kPrefixNearbyGroups
+};
+template <int M, int WW, int TT, bool NEARBY = false>
 __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const int* __restrict__ pos, const int* __restrict__ upper,
                                                                           const uint32_t* __restrict__ kid,
                                                                           uint64_t* __restrict__ dom, int n, int kstride,
                                                                           int64_t wstride, int nwords, int shift, int buckets,
                                                                           int chunk, int bands, int mode, int* __restrict__ total0,
                                                                           int* __restrict__ witness0, SortParam* __restrict__ param,
-                                                                          const int* __restrict__ unless_front0, int enough) {
+                                                                          const int* __restrict__ unless_front0, int enough, NearbyWork work) {
+  static_assert(!NEARBY || TT == 1, "a tile of rows in spatial order");
   constexpr int TS = 64 * WW, T = kPrefixThreads;
   constexpr int TPL = 16 / (WW * TT);  // workgroups that share a 128-byte line of the matrix
   constexpr int MPL = TS / 64;  // members of the tile per lane when a wave walks through them
   extern __shared__ uint64_t prefix_lds[];
   if (param->nonfinite != 0) return;
-  if (unless_front0 != nullptr && *unless_front0 >= enough) return;
+  if (unless_front0 != nullptr && (NEARBY ? *unless_front0 != 0 : *unless_front0 >= enough)) return;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) param->totals_valid = 1;  // for the count stage
-  // Workgroups go to the eight dies in turn (linear index modulo 8), and a die has its own L2.  The tiles
-  // that share the 128-byte lines of the matrix are given to consecutive workgroups of one die, which run
-  // side by side over the same rows: their pieces of a line then meet in that L2 and leave as one line.
-  const int64_t linear = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-  const int die = (int)(linear & 7);
-  const int seq = (int)blockIdx.x >> 3;  // this workgroup among those of its die in this row of the grid
-  const int tile = TPL * ((seq / TPL) * 8 + die) + seq % TPL;
-  if (tile * WW * TT >= nwords) return;
+  __shared__ uint16_t nearby[NEARBY ? kPrefixNearbyGroups : 1];
+  __shared__ int nearby_item;
+  __shared__ int tile_lo[M], tile_span[M], tile_shift[M];
+  for (;;) {
+  int tid = (int)threadIdx.x;
+  // (what hangs on the thread alone is computed anew for every part: kept across them it took 128 registers and spilled)
+  if constexpr (NEARBY) asm volatile("" : "+v"(tid));
+  const int lane = tid & 63, wave = tid >> 6;
+  int tile, r0 = 0, r1 = n, nearby_count = 0;
+  if constexpr (NEARBY) {
+    // the next part of the work; the grid ends when none is left
+    __syncthreads();  // (the tables of the part before are no longer read)
+    if (tid == 0) nearby_item = atomicAdd(&work.queue[2], 1);
+    __syncthreads();
+    const int item = nearby_item, fulls = work.queue[0];
+    if (item >= fulls + work.queue[1]) return;
+    const int2 part = item < fulls ? work.full[item] : work.rest[item - fulls];
+    tile = part.x;
+    nearby_count = min(work.cap, work.near_count[tile] - part.y * work.cap);
+    for (int g = tid; g < nearby_count; g += T) nearby[g] = work.near_list[(int64_t)tile * nwords + part.y * work.cap + g];
+    if (tid < M) {  // (positions of such a tile lie close together: its coarse index covers those only)
+      const int low = work.box[(tile * M + tid) * 2], high = work.box[(tile * M + tid) * 2 + 1];
+      int wide = 0;
+      while (((high - low) >> wide) >= kPrefixBuckets) ++wide;
+      tile_lo[tid] = low;
+      tile_span[tid] = high - low + 1;  // (the bucket of every bound above the tile)
+      tile_shift[tid] = wide;
+    }
+  } else {
+    // Workgroups go to the eight dies in turn (linear index modulo 8), and a die has its own L2.  The tiles
+    // that share the 128-byte lines of the matrix are given to consecutive workgroups of one die, which run
+    // side by side over the same rows: their pieces of a line then meet in that L2 and leave as one line.
+    const int64_t linear = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    const int die = (int)(linear & 7);
+    const int seq = (int)blockIdx.x >> 3;  // this workgroup among those of its die in this row of the grid
+    tile = TPL * ((seq / TPL) * 8 + die) + seq % TPL;
+    if (tile * WW * TT >= nwords) return;
+    const int first_slot = tile * WW * TT * 64;
+    int64_t first_row = (int64_t)first_slot + (int64_t)blockIdx.y * chunk, end_row = first_row + chunk;
+    if (bands) {  // the same rows for all tiles of a grid row: the tiles left of the diagonal in rows y * chunk ...
+      first_row = (int64_t)blockIdx.y * chunk;
+      end_row = first_row + chunk;
+      if (first_row < first_slot) first_row = first_slot;
+    }
+    if (first_row >= n || first_row >= end_row) return;
+    r0 = (int)first_row;
+    r1 = (int)(end_row < n ? end_row : n);
+  }
   const int w0 = tile * WW * TT;  // the first word of the workgroup's TT tiles (tile `sub` starts WW * sub words on)
   const int slot0 = w0 * 64;
-  int64_t first_row = (int64_t)slot0 + (int64_t)blockIdx.y * chunk, end_row = first_row + chunk;
-  if (bands) {  // the same rows for all tiles of a grid row: the tiles left of the diagonal in rows y * chunk ...
-    first_row = (int64_t)blockIdx.y * chunk;
-    end_row = first_row + chunk;
-    if (first_row < slot0) first_row = slot0;
-  }
-  if (first_row >= n || first_row >= end_row) return;
-  const int r0 = (int)first_row;
-  const int r1 = (int)(end_row < n ? end_row : n);
   const int HB = buckets + 2;  // entries of the coarse index per objective
   // per objective k (all arrays [M][...]):
   constexpr int kSetWords = WW * 65;                 // sets[k][w][c]: the slots of the first c members of word w
@@ -460,50 +673,56 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
   };
   auto hist_of = [&](int k) { return reinterpret_cast<int*>(tile_lds + (size_t)k * over); };  // [HB]
   auto claimed_of = [&](int k) { return hist_of(k) + HB; };                                      // [TS]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int index_stride = (HB + 3) & ~3;
+  auto bucket_of_bound = [&](int k, int e) {  // the bucket of a bound; of a position p likewise
+    if constexpr (!NEARBY) return e >> shift;
+    const int past = e - tile_lo[k];
+    return min(past > 0 ? past : 0, tile_span[k]) >> tile_shift[k];
+  };
 
   for (int sub = 0; sub < TT; ++sub) {
   select_tile(sub);
   // ---- the tile's slots by position, objective by objective
-  for (int t = threadIdx.x; t < M * HB; t += T) hist_of(t / HB)[t % HB] = 0;
-  for (int t = threadIdx.x; t < M * (TS + 8); t += T) mp[t] = 0x7FFFFFFF;
+  for (int t = tid; t < M * HB; t += T) hist_of(t / HB)[t % HB] = 0;
+  for (int t = tid; t < M * (TS + 8); t += T) mp[t] = 0x7FFFFFFF;
   __syncthreads();
   constexpr int PER = (M * TS + T - 1) / T;
   int mine[PER];
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int item = threadIdx.x + u * T;
+    const int item = tid + u * T;
     const int k = item / TS, i = item - k * TS;
     mine[u] = -1;
     if (item < M * TS && i < live) {
       const int p = pos[(int64_t)k * kstride + tile_slot0 + i];
       mine[u] = (p << 9) | i;
-      atomicAdd(&hist_of(k)[p >> shift], 1);
+      atomicAdd(&hist_of(k)[bucket_of_bound(k, p)], 1);
     }
   }
   __syncthreads();
-  if (wave < M) {  // exclusive prefix of the bucket counts of objective `wave`
-    int carry = 0;
-    for (int b0 = 0; b0 < HB; b0 += 64) {
-      const int b = b0 + lane;
-      const int v = b < HB ? hist_of(wave)[b] : 0;
-      int incl = v;
+  if (wave < M) {  // exclusive prefix of the bucket counts of objective `wave`: a lane adds up kPer consecutive buckets
+    constexpr int kPer = (kPrefixBuckets + 2 + 63) / 64;  // (odd: the lanes' reads fall into different banks)
+    int count[kPer], sum = 0;
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int up = __shfl_up(incl, off);
-        if (lane >= off) incl += up;
-      }
-      if (b < HB) index[wave * index_stride + b] = (uint16_t)(carry + incl - v);
-      carry += __shfl(incl, 63);
+    for (int c = 0; c < kPer; ++c) {
+      const int b = lane * kPer + c;
+      count[c] = b < HB ? hist_of(wave)[b] : 0;
+      sum += count[c];
+    }
+    int before = (int)wave_scan((uint32_t)sum, [](uint32_t a, uint32_t b) { return a + b; }) - sum;
+#pragma unroll
+    for (int c = 0; c < kPer; ++c) {
+      const int b = lane * kPer + c;
+      if (b < HB) index[wave * index_stride + b] = (uint16_t)before;
+      before += count[c];
     }
   }
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     if (mine[u] >= 0) {
-      const int k = (threadIdx.x + u * T) / TS;
-      const int b = (mine[u] >> 9) >> shift;
+      const int k = (tid + u * T) / TS;
+      const int b = bucket_of_bound(k, mine[u] >> 9);
       const int r = atomicSub(&hist_of(k)[b], 1) - 1;
       claimed_of(k)[(int)index[k * index_stride + b] + r] = mine[u];
     }
@@ -512,8 +731,8 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     if (mine[u] >= 0) {
-      const int k = (threadIdx.x + u * T) / TS;
-      const int b = (mine[u] >> 9) >> shift;
+      const int k = (tid + u * T) / TS;
+      const int b = bucket_of_bound(k, mine[u] >> 9);
       const int t0 = index[k * index_stride + b], t1 = index[k * index_stride + b + 1];
       int before = 0;
       for (int t = t0; t < t1; ++t) before += claimed_of(k)[t] < mine[u] ? 1 : 0;
@@ -523,7 +742,7 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
   }
   __syncthreads();
   // ---- counts[k][t] and the single bits of sets[k][w][c + 1]; a wave per objective, a lane per MPL members
-  for (int t = threadIdx.x; t < M * kSetWords; t += T) sets[(size_t)(t / kSetWords) * over + t % kSetWords] = 0ull;
+  for (int t = tid; t < M * kSetWords; t += T) sets[(size_t)(t / kSetWords) * over + t % kSetWords] = 0ull;
   __syncthreads();
   for (int k = wave; k < M; k += T / 64) {
     uint64_t one[MPL];
@@ -534,12 +753,8 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
       one[c] = t < live ? 1ull << (8 * ((sorted[k * TS + t] & (TS - 1)) >> 6)) : 0ull;
       sum += one[c];
     }
-    uint64_t incl = sum;  // byte-wise counts: at most 64 per byte, no carry between bytes
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint64_t up = __shfl_up(incl, off);
-      if (lane >= off) incl += up;
-    }
+    // byte-wise counts: at most 64 per byte, no carry between bytes
+    const uint64_t incl = wave_scan_halves(sum, [](uint32_t a, uint32_t b) { return a + b; });
     uint64_t run = incl - sum;  // members before this lane's eight
     uint64_t* const cnt = counts + (size_t)k * over;
     uint64_t* const set = sets + (size_t)k * over;
@@ -562,12 +777,7 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
   for (int item = wave; item < M * WW; item += T / 64) {
     const int k = item / WW, w = item - k * WW;
     uint64_t* const col = sets + (size_t)k * over + w * 65;
-    uint64_t incl = col[lane + 1];
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint64_t up = __shfl_up(incl, off);
-      if (lane >= off) incl |= up;
-    }
+    const uint64_t incl = wave_scan_halves(col[lane + 1], [](uint32_t a, uint32_t b) { return a | b; });
     col[lane + 1] = ~incl;  // kept complemented: a row ORs the complements of its M sets (three-input ORs) and
     if (lane == 0) col[0] = ~0ull;  // complements once
   }
@@ -577,19 +787,20 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
 
   // ---- the rows of the stretch, 64 at a time per wave; the inputs of a wave's next rows are fetched while it
   // works on the present ones
-  const int groups = (r1 - r0 + 63) / 64;
+  const int groups = NEARBY ? nearby_count : (r1 - r0 + 63) / 64;
   int e_next[M];
   int same_next = 0;
+  auto row_of = [&](int g) { return r0 + (NEARBY ? (int)nearby[g] : g) * 64 + lane; };
   auto fetch = [&](int g) {
-    const int j = r0 + g * 64 + lane;
+    const int j = row_of(g);
     const int jc = j < n ? j : n - 1;
 #pragma unroll
     for (int k = 0; k < M; ++k) e_next[k] = upper[(int64_t)k * kstride + jc];
-    same_next = (int)kid[jc];
+    same_next = NEARBY ? pos[(int64_t)(M - 1) * kstride + jc] : (int)kid[jc];  // (NEARBY: its place in the order of the slots)
   };
   if (wave < groups) fetch(wave);
   for (int g = wave; g < groups; g += T / 64) {
-    const int j = r0 + g * 64 + lane;
+    const int j = row_of(g);
     int e[M];
 #pragma unroll
     for (int k = 0; k < M; ++k) e[k] = e_next[k];
@@ -607,7 +818,7 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
       int t[M];
       bool more = false;
 #pragma unroll
-      for (int k = 0; k < M; ++k) t[k] = index[k * index_stride + (e[k] >> shift)];
+      for (int k = 0; k < M; ++k) t[k] = index[k * index_stride + bucket_of_bound(k, e[k])];
 #pragma unroll
       for (int k = 0; k < M; ++k) {
         const int m0 = mp[k * (TS + 8) + t[k]], m1 = mp[k * (TS + 8) + t[k] + 1];
@@ -631,8 +842,9 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
       }
 #pragma unroll
       for (int w = 0; w < WW; ++w) d[w] = ~d[w];
-      // rows identical to j and everything after them: only near the diagonal (wave-uniform test)
-      if (__builtin_amdgcn_ballot_w64(same_from < tile_slot0 + TS) != 0ull) {
+      // rows identical to j and everything after them: only near the diagonal (wave-uniform test; NEARBY: the last
+      // of its orders, that of the slots, has left them out)
+      if (!NEARBY && __builtin_amdgcn_ballot_w64(same_from < tile_slot0 + TS) != 0ull) {
 #pragma unroll
         for (int w = 0; w < WW; ++w) {
           const int first = (tw0 + w) * 64;
@@ -648,6 +860,13 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
         dominators += __popcll(d[w]);
         highest = d[w] != 0ull ? tw0 + w : highest;
       }
+    }
+    if constexpr (NEARBY) {
+      if (j < n && dominators != 0) {
+        atomicAdd(&total0[same_from], dominators);
+        witness0[same_from] = same_from >> 6;  // (no word above this one: where a peel of the matrix would begin to look)
+      }
+      continue;
     }
     if (j < n && (mode & 1) && dominators != 0) {
       atomicAdd(&total0[j], dominators);
@@ -714,6 +933,8 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
       }
     }
   }
+  if constexpr (!NEARBY) break;
+  }  // parts of the work (NEARBY)
 }
 
 }  // namespace evx
