@@ -823,8 +823,10 @@ static int stage_peel(const Ws& w, int64_t stop_count, bool want_perm, hipStream
   if (use_witness && opt().peel_records && L.n <= kRecordsMaxRowsWide) {
     // all-to-all records: 1 lister + a power of two of sweeping blocks, all resident at once
     // by size: 64 blocks up to 32768 rows, 128 above (measured at 20000 rows: 221 us per selection with 64
-    // blocks, 225 with 128, 228 with 32, 238 with 192; between 1200 and 6000 rows the count hardly matters)
-    const int by_size = L.n <= 32768 ? 64 : 128;
+    // blocks, 225 with 128, 228 with 32, 238 with 192; between 1200 and 6000 rows the count hardly matters), 160 above
+    // five times that, where more waves for the rescans outweigh the longer exchange (128 / 160 blocks, us per selection:
+    // 60 000 x 3 477 / 550, 150 000 x 4 882 / 898, 200 003 x 3 1494 / 1398)
+    const int by_size = L.n <= 32768 ? 64 : L.n <= 163840 ? 128 : 160;
     const int sweepers = cus >= 64 ? (opt().peel_record_blocks ? opt().peel_record_blocks : by_size) : 16;
     const int wpb = kRecThreads / 64;
     const int list_capacity = wpb * ((L.n + sweepers * wpb - 1) / (sweepers * wpb));
