@@ -1741,7 +1741,8 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
     EVX_LAUNCH_CHECK();
     return 0;
   }
-  // The rows step 2 leaves stand in xs, those of step 1 in xs_sorted, and the spatial order goes to the other of the two.
+  // The rows step 1 leaves stand in xs_sorted, those between the passes of step 2 in xs, those it leaves in xs_sorted again,
+  // and the spatial order goes to xs.
   constexpr bool kGrid = M == 2 || M == 3;
   const bool grid_step = kGrid && L.n > kFrontGridPopulation;
   const bool order_step = L.n > kFrontPairsRows;
@@ -1751,12 +1752,16 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
   int* const left_of = w.at<int>(L.order);
   float* const to = grid_step ? w.at<float>(L.xs) : nullptr;
   int* const to_of = grid_step ? w.at<int>(L.perm) : nullptr;
-  // (the cells before and after the prefix passes: up to 256 KB each, where the radix sort's pairs go)
+  // (the cells before and after the prefix passes, where the radix sort's pairs go)
   uint32_t* const cells = grid_step ? w.at<uint32_t>(L.rpairs0) : nullptr;
   uint32_t* const turned = grid_step ? w.at<uint32_t>(L.rpairs1) : nullptr;
   const bool small_grid = M == 3 && L.n <= kFrontGridSmallRows;
   const int cell_bits = small_grid ? 7 : 8;
   const int grid_cells = !grid_step ? 0 : (M == 2 ? 1 << cell_bits : 1 << (2 * cell_bits));
+  // (A cell to every 64 bytes, where they fit; side by side where one workgroup reads them all, which from 16 384 lines of
+  // memory costs more than the minima save: 100 000 x 3 around a sphere took 112 us.)
+  int spread = small_grid ? 0 : 4;
+  while (spread > 0 && sizeof(uint32_t) * ((size_t)grid_cells << spread) > sizeof(unsigned long long) * (size_t)L.m * (size_t)L.kstride) --spread;
   // The rows of low sums cost a pass over the rows (and a launch that is needed anyway).  Without them, a population that a
   // few rows dominate which no sample holds goes on whole: pairs of up to 65 536 rows of four objectives take some 35 us then,
   // of 60 000 x 6 315, and 200 000 x 4 took 145 us where the rows of low sums leave 36.  (An entry per stretch of 256 rows or
@@ -1778,15 +1783,19 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
   while (per > 1 && (int64_t)w.batch * ((L.n + 128 * per - 1) / (128 * per)) <= device_cus()) per /= 2;
   const int filter_blocks = per < kFrontRowsPerThread ? (L.n + 256 * per - 1) / (256 * per) : blocks;
   hipLaunchKernelGGL(front_filter_kernel<M>, dim3(filter_blocks, 1, w.batch), dim3(256), 0, s, fit.f, fit.sr, fit.sc, fit.step, L.n, L.npad, per,
-                     lowest, left, left_of, mask, count, cells, grid_cells, w.at<uint32_t>(L.hist),
+                     lowest, left, left_of, mask, count, cells, grid_cells << spread, w.at<uint32_t>(L.hist),
                      order_step ? (int)((L.tailbuf - L.hist) / 4) : 0, w.step);
   EVX_LAUNCH_CHECK();
   if constexpr (kGrid) {
     if (grid_step) {
-      int build_blocks = (L.n + 255) / 256;
-      if (build_blocks > 1024) build_blocks = 1024;
-      hipLaunchKernelGGL(front_grid_kernel<M>, dim3(build_blocks, 1, w.batch), dim3(256), 0, s, left, L.npad, cell_bits, count, cells,
-                         w.step);
+      // (as many rows to a workgroup, up to four per thread, as leave every compute unit one: a workgroup drops what its own
+      // rows dominate, 44 % of 1024 rows around a sphere and 58 % of 4096)
+      uint32_t* const tables = w.at<uint32_t>(L.key);
+      int grid_per = (int)(((int64_t)L.n * w.batch + (int64_t)kFrontGridBlock * device_cus() - 1) / ((int64_t)kFrontGridBlock * device_cus()));
+      if (grid_per > kFrontRowsPerThread) grid_per = kFrontRowsPerThread;
+      const int build_blocks = (L.n + kFrontGridBlock * grid_per - 1) / (kFrontGridBlock * grid_per);
+      hipLaunchKernelGGL(front_grid_kernel<M>, dim3(build_blocks, 1, w.batch), dim3(kFrontGridBlock), 0, s, left, left_of, L.npad, grid_per,
+                         cell_bits, count, to, to_of, mask, L.n, tables, cells, spread, w.step);
       EVX_LAUNCH_CHECK();
       const uint32_t* below = turned;
       if (small_grid) {
@@ -1795,18 +1804,18 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
                            w.step);
         EVX_LAUNCH_CHECK();
       } else {
-        hipLaunchKernelGGL(front_grid_prefix_kernel, dim3(M == 2 ? 1 : kFrontGrid, 1, w.batch), dim3(kFrontGrid), 0, s, cells, turned,
+        hipLaunchKernelGGL(front_grid_prefix_kernel, dim3(M == 2 ? 1 : kFrontGrid, 1, w.batch), dim3(kFrontGrid), 0, s, cells, spread, turned,
                            M == 2 ? 1 : kFrontGrid, count, w.step);
         EVX_LAUNCH_CHECK();
         if (M == 3) {
           below = cells;
-          hipLaunchKernelGGL(front_grid_prefix_kernel, dim3(kFrontGrid, 1, w.batch), dim3(kFrontGrid), 0, s, turned, cells, kFrontGrid,
+          hipLaunchKernelGGL(front_grid_prefix_kernel, dim3(kFrontGrid, 1, w.batch), dim3(kFrontGrid), 0, s, turned, 0, cells, kFrontGrid,
                              count, w.step);
           EVX_LAUNCH_CHECK();
         }
       }
-      hipLaunchKernelGGL(front_grid_filter_kernel<M>, dim3(blocks, 1, w.batch), dim3(256), 0, s, left, left_of, L.npad, cell_bits, count,
-                         below, to, to_of, mask, L.n, spatial_bucket_bits(L), w.at<int>(L.members),
+      hipLaunchKernelGGL(front_grid_filter_kernel<M>, dim3(blocks, 1, w.batch), dim3(256), 0, s, to, to_of, L.npad, cell_bits, count,
+                         tables, below, left, left_of, mask, L.n, spatial_bucket_bits(L), w.at<int>(L.members),
                          order_step ? w.at<int>(L.hist) : (int*)nullptr, w.step);
       EVX_LAUNCH_CHECK();
     }
@@ -1814,13 +1823,13 @@ static int first_front_steps(const Ws& w, const Fitness& fit, uint8_t* mask, hip
   const int pair_rows = L.n < kFrontPairsRows ? L.n : kFrontPairsRows;
   const int pair_parts = (pair_rows + 63) / 64 < kFrontPairsParts ? (pair_rows + 63) / 64 : kFrontPairsParts;  // (a part has 64 rows or more)
   hipLaunchKernelGGL(front_pairs_kernel<M>, dim3((pair_rows + 255) / 256, pair_parts, w.batch), dim3(256), 0, s, left, left_of,
-                     to, to_of, L.npad, mask, L.n, count, w.step);
+                     L.npad, mask, L.n, count, grid_step ? 1 : 0, w.step);
   EVX_LAUNCH_CHECK();
   if (!order_step) return 0;
-  float* const sorted = grid_step ? left : w.at<float>(L.xs);
-  if (int e = stage_spatial_order<M>(w, grid_step ? to : left, sorted, counted, kFrontPairsRows, grid_step, s)) return e;
+  float* const sorted = w.at<float>(L.xs);
+  if (int e = stage_spatial_order<M>(w, left, sorted, counted, kFrontPairsRows, grid_step, s)) return e;
   hipLaunchKernelGGL((first_front_leaf_kernel<M>), dim3((unsigned)spatial_leaves(L.n), 1, w.batch), dim3(64 * kFrontWaves), 0, s,
-                     sorted, w.at<int>(L.orig_of), w.at<int>(L.kid_sorted), grid_step ? to_of : left_of, count, counted, L.npad,
+                     sorted, w.at<int>(L.orig_of), w.at<int>(L.kid_sorted), left_of, count, counted, L.npad,
                      spatial_leaf_stride(L.n), spatial_group_stride(L.n), w.at<float>(L.leaf_lo), w.at<float>(L.leaf_hi),
                      w.at<float>(L.group_lo), mask, L.n, w.ctrl(), w.step);
   EVX_LAUNCH_CHECK();

@@ -25,23 +25,20 @@ __host__ __device__ inline int64_t spatial_leaf_stride(int64_t rows) { return (s
 __host__ __device__ inline int64_t spatial_group_stride(int64_t rows) { return (spatial_leaf_stride(rows) / kGroupLeaves + 63) / 64 * 64; }
 
 // The workgroup's table of ascending sample values of every objective (kSpatialSamples of them, as ordered keys): each
-// workgroup of 256 threads ranks the same samples by counting, 1.2 us an objective, less than a launch of its own would cost.
+// workgroup ranks the same samples by counting, 1.2 us an objective per 256 threads, less than a launch of its own would cost.
 // The low eight bits of a sample give way to its thread, which makes the samples distinct: one comparison each, and any
 // ascending values will do for a table.
 template <int M>
 __device__ inline void spatial_quantiles(const float* __restrict__ xs, int npad, int n, uint32_t* table) {
   static_assert(kSpatialSamples == 256, "one sample per thread, eight bits to tell them apart");
   __shared__ __attribute__((aligned(16))) uint32_t sample[M][kSpatialSamples];
-  const int i = (int)((int64_t)threadIdx.x * n / kSpatialSamples);
-  uint32_t mine[M];
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    mine[k] = (ordered_key(xs[(int64_t)k * npad + i]) & ~255u) | threadIdx.x;
-    sample[k][threadIdx.x] = mine[k];
-  }
+  // (each 256 threads of a larger workgroup take the next objective)
+  const int t = threadIdx.x & (kSpatialSamples - 1), first = threadIdx.x / kSpatialSamples, step = blockDim.x / kSpatialSamples;
+  const int i = (int)((int64_t)t * n / kSpatialSamples);
+  for (int k = first; k < M; k += step) sample[k][t] = (ordered_key(xs[(int64_t)k * npad + i]) & ~255u) | t;
   __syncthreads();
-  for (int k = 0; k < M; ++k) {
-    const uint32_t own = sample[k][threadIdx.x];
+  for (int k = first; k < M; k += step) {
+    const uint32_t own = sample[k][t];
     int before = 0;
 #pragma unroll 8
     for (int e = 0; e < kSpatialSamples; e += 4) {
@@ -250,11 +247,13 @@ constexpr int kFrontGrid = 256;       // cells of the grid of step 2 along an ob
 constexpr int kFrontGridSmall = 128;  // and in three objectives up to kFrontGridSmallRows rows, where both passes over its
 constexpr int kFrontGridSmallRows = 131072;  // cells fit one workgroup (a launch costs 4 us of host time)
 
-// Rows left after step 1 and after step 2, and whether any row of the population holds a NaN or an infinity.
+// Rows left after step 1, after step 2 and between its two passes over the rows, and whether any row of the population
+// holds a NaN or an infinity.
 struct FrontCount {
   int rows;
   int rows_grid;
   int nonfinite;
+  int rows_between;
 };
 
 // Clears the control block and the counters, where front_lowest_kernel is not launched.
@@ -572,8 +571,8 @@ __global__ __launch_bounds__(256) void front_filter_kernel(const float* __restri
 // Step 2, for two and three objectives.  All objectives but the last are cut into 2^bits quantiles; a cell keeps the
 // smallest value of the last objective among its rows (front_grid_kernel), then the smallest of all cells that are smaller
 // in every cut objective (front_grid_prefix_kernel, one objective after the other): a row no better than that is dominated
-// (front_grid_filter_kernel, which also counts the rows it leaves per bucket of the spatial order).  What it leaves are the rows within about a cell of the front: 1 000 003 rows around a sphere,
-// 35 000 of them on the front, go down to 134 000.
+// (front_grid_filter_kernel, which also counts the rows it leaves per bucket of the spatial order).  What it leaves are the
+// rows within about a cell of the front: 1 000 003 rows around a sphere, 35 000 of them on the front, go down to 134 000.
 template <int M>
 __device__ inline int front_cell(const float (&x)[M], const uint32_t* table, int bits) {
   const int c0 = (int)spatial_quantile(table, ordered_key(x[0]), bits);
@@ -581,40 +580,132 @@ __device__ inline int front_cell(const float (&x)[M], const uint32_t* table, int
   return (c0 << bits) + (int)spatial_quantile(table + kSpatialSamples, ordered_key(x[1]), bits);
 }
 
+// Minimum over the lanes up to this one (shifts inside the DPP rows, then from row to row).
+__device__ __forceinline__ uint32_t lanes_prefix_min(uint32_t v) {
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false));
+  return min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false));
+}
+__device__ __forceinline__ uint32_t lanes_before(uint32_t prefix) {  // ... up to the lane before it
+  const uint32_t up = __shfl_up(prefix, 1);
+  return (threadIdx.x & 63) == 0 ? ~0u : up;
+}
+
+// The workgroup goes through its own rows first, `per` to a thread, on a grid of 64 cells along an objective in LDS: a row
+// that one of these rows dominates there is dropped -- what it would have told the grid, its dominator tells at least as
+// well -- and comes neither to the grid in memory nor to the second pass over the rows.  Of 630 000 rows left by step 1
+// (1 000 003 x 3 around a sphere) some 260 000 go on.  The grid's cells lie 2^spread words apart: minima in one line of memory
+// follow one another, some 55 ns each, and up to 900 of them fell on the 32 cells of a line.  Both together, with 1024 threads
+// to a workgroup and each 256 of them ranking the samples of one objective: 38 us for 60, and 17 for 31 in
+// front_grid_filter_kernel (a call 206 us for 241; 1 000 000 x 2 146 for 175, 100 000 x 3 97 for 102).  The minima are bound
+// by the lines they meet in; all but 21 us of this kernel.
+// to / to_of: the rows that go on; tables: the quantiles, for the pass that follows.
+constexpr int kFrontGridBlock = 1024, kFrontLocal = 64;
 template <int M>
-__global__ __launch_bounds__(256) void front_grid_kernel(const float* __restrict__ left, int npad, int bits,
-                                                         const FrontCount* __restrict__ count, uint32_t* __restrict__ grid,
-                                                         int64_t ws_step) {
-  to_population(ws_step, left, count, grid);
+__global__ __launch_bounds__(kFrontGridBlock) void front_grid_kernel(const float* __restrict__ left, const int* __restrict__ left_of,
+                                                                     int npad, int per, int bits, FrontCount* __restrict__ count,
+                                                                     float* __restrict__ to, int* __restrict__ to_of,
+                                                                     uint8_t* __restrict__ mask, int population,
+                                                                     uint32_t* __restrict__ tables, uint32_t* __restrict__ grid,
+                                                                     int spread, int64_t ws_step) {
+  mask += (int64_t)blockIdx.z * population;
+  to_population(ws_step, left, left_of, count, to, to_of, tables, grid);
   const int rows = count->rows;
   if (rows <= kFrontGridLeast) return;
-  __shared__ uint32_t table[kSpatialSamples * (M - 1)];
-  spatial_quantiles<M - 1>(left, npad, rows, table);
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < rows; i += gridDim.x * 256) {
-    float x[M];
-    bool nan = false;
+  constexpr int kStride = kFrontLocal + 1, kLines = M == 2 ? 1 : kFrontLocal;  // (a column's cells fall into different banks)
+  __shared__ uint32_t table[kSpatialSamples * M];
+  __shared__ uint32_t local[kLines * kStride];
+  __shared__ int scratch[kFrontGridBlock / 64 + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int kWaves = kFrontGridBlock / 64;
+  spatial_quantiles<M>(left, npad, rows, table);
+  if (blockIdx.x == 0)
+    for (int e = threadIdx.x; e < kSpatialSamples * M; e += kFrontGridBlock) tables[e] = table[e];
+  for (int i0 = blockIdx.x * kFrontGridBlock * per; i0 < rows; i0 += gridDim.x * kFrontGridBlock * per) {
+    for (int c = threadIdx.x; c < kLines * kStride; c += kFrontGridBlock) local[c] = ~0u;
+    float x[kFrontRowsPerThread][M];
+    int number[kFrontRowsPerThread], cell[kFrontRowsPerThread], near[kFrontRowsPerThread];
+    uint32_t value[kFrontRowsPerThread];
+    bool keep[kFrontRowsPerThread];
 #pragma unroll
-    for (int k = 0; k < M; ++k) {
-      x[k] = left[(int64_t)k * npad + i];
-      nan |= x[k] != x[k];
+    for (int r = 0; r < kFrontRowsPerThread; ++r) {
+      const int i = i0 + r * kFrontGridBlock + threadIdx.x;
+      keep[r] = r < per && i < rows;
+      number[r] = keep[r] ? left_of[i] : 0;
+#pragma unroll
+      for (int k = 0; k < M; ++k) x[r][k] = keep[r] ? left[(int64_t)k * npad + i] : 0.0f;
     }
-    if (nan) continue;
-    const int c = front_cell<M>(x, table, bits);
-    const uint32_t v = ordered_key(x[M - 1]);
-    // (what a plain load sees may be old, which costs an addition too many and no more)
-    if (v < grid[c]) atomicMin(&grid[c], v);
+    __syncthreads();  // (the cells are clear)
+#pragma unroll
+    for (int r = 0; r < kFrontRowsPerThread; ++r) {
+      bool nan = false;
+#pragma unroll
+      for (int k = 0; k < M; ++k) nan |= x[r][k] != x[r][k];
+      cell[r] = front_cell<M>(x[r], table, bits);
+      near[r] = M == 2 ? cell[r] >> (bits - 6) : (cell[r] >> (2 * bits - 6)) * kStride + ((cell[r] & ((1 << bits) - 1)) >> (bits - 6));
+      value[r] = keep[r] && !nan ? ordered_key(x[r][M - 1]) : ~0u;  // (a row with a NaN beats none and is beaten by none)
+      if (value[r] != ~0u) atomicMin(&local[near[r]], value[r]);
+    }
+    __syncthreads();
+    // every cell: the smallest of the cells before it along the line, then of those in the lines before it
+    for (int line = wave; line < kLines; line += kWaves)
+      local[line * kStride + lane] = lanes_before(lanes_prefix_min(local[line * kStride + lane]));
+    __syncthreads();
+    if constexpr (M == 3) {
+      for (int column = wave; column < kFrontLocal; column += kWaves)
+        local[lane * kStride + column] = lanes_before(lanes_prefix_min(local[lane * kStride + column]));
+      __syncthreads();
+    }
+    uint64_t kept[kFrontRowsPerThread];
+    int mine = 0;
+#pragma unroll
+    for (int r = 0; r < kFrontRowsPerThread; ++r) {
+      if (value[r] != ~0u && local[near[r]] <= value[r]) {
+        keep[r] = false;
+        mask[number[r]] = 0;
+        value[r] = ~0u;
+      }
+      // (what a plain load sees may be old, which costs an addition too many and no more)
+      if (value[r] < grid[cell[r] << spread]) atomicMin(&grid[cell[r] << spread], value[r]);
+      kept[r] = __builtin_amdgcn_ballot_w64(keep[r]);
+      mine += __popcll(kept[r]);
+    }
+    if (lane == 0) scratch[wave] = mine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int all = 0;
+      for (int v = 0; v < kWaves; ++v) all += scratch[v];
+      scratch[kWaves] = atomicAdd(&count->rows_between, all);
+    }
+    __syncthreads();
+    int at = scratch[kWaves];
+    for (int v = 0; v < wave; ++v) at += scratch[v];
+#pragma unroll
+    for (int r = 0; r < kFrontRowsPerThread; ++r) {
+      if (keep[r]) {
+        const int p = at + __popcll(kept[r] & ((1ull << lane) - 1ull));
+#pragma unroll
+        for (int k = 0; k < M; ++k) to[(int64_t)k * npad + p] = x[r][k];
+        to_of[p] = number[r];
+      }
+      at += __popcll(kept[r]);
+    }
+    __syncthreads();  // (cells and counts are used again)
   }
 }
 
-// Row b of `in` (kFrontGrid cells) to column b of `out`: out[c][b] = min of in[b][0 .. c - 1].
-__global__ __launch_bounds__(kFrontGrid) void front_grid_prefix_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                                       int out_stride, const FrontCount* __restrict__ count,
+// Row b of `in` (kFrontGrid cells, 2^spread words apart) to column b of `out`: out[c][b] = min of in[b][0 .. c - 1].
+__global__ __launch_bounds__(kFrontGrid) void front_grid_prefix_kernel(const uint32_t* __restrict__ in, int spread,
+                                                                       uint32_t* __restrict__ out, int out_stride, const FrontCount* __restrict__ count,
                                                                        int64_t ws_step) {
   to_population(ws_step, in, out, count);
   if (count->rows <= kFrontGridLeast) return;
   __shared__ uint32_t last[kFrontGrid / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t v = in[(int64_t)blockIdx.x * kFrontGrid + threadIdx.x];
+  uint32_t v = in[((int64_t)blockIdx.x * kFrontGrid + threadIdx.x) << spread];
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
     const uint32_t o = __shfl_up(v, off);
@@ -679,17 +770,18 @@ __global__ __launch_bounds__(kFrontGridThreads) void front_grid_small_kernel(con
 template <int M>
 __global__ __launch_bounds__(256) void front_grid_filter_kernel(const float* __restrict__ left, const int* __restrict__ left_of,
                                                                 int npad, int bits, FrontCount* __restrict__ count,
-                                                                const uint32_t* __restrict__ below, float* __restrict__ to,
+                                                                const uint32_t* __restrict__ tables, const uint32_t* __restrict__ below, float* __restrict__ to,
                                                                 int* __restrict__ to_of, uint8_t* __restrict__ mask, int population,
                                                                 int bucket_bits, int* __restrict__ to_bucket,
                                                                 int* __restrict__ hist, int64_t ws_step) {
   mask += (int64_t)blockIdx.z * population;
-  to_population(ws_step, left, left_of, count, below, to, to_of, to_bucket, hist);
-  const int rows = count->rows;
-  if (rows <= kFrontGridLeast) return;
+  to_population(ws_step, left, left_of, count, tables, below, to, to_of, to_bucket, hist);
+  if (count->rows <= kFrontGridLeast) return;
+  const int rows = count->rows_between;
   __shared__ uint32_t table[kSpatialSamples * M];
   __shared__ int scratch[5];
-  spatial_quantiles<M>(left, npad, rows, table);  // (the first M - 1 are those of the grid)
+  for (int e = threadIdx.x; e < kSpatialSamples * M; e += 256) table[e] = tables[e];
+  __syncthreads();
   for (int i0 = blockIdx.x * 256 * kFrontRowsPerThread; i0 < rows; i0 += gridDim.x * 256 * kFrontRowsPerThread) {
     float x[kFrontRowsPerThread][M];
     int number[kFrontRowsPerThread], bucket[kFrontRowsPerThread];
@@ -757,21 +849,17 @@ __device__ inline bool half_leaf_dominates(const float* __restrict__ xs, int npa
 // Step 3.  Grid (row blocks of 256, kFrontPairsParts): a wave takes 64 of the rows left against one part of them, which
 // streams past as scalar operands 32 at a time.  Brute force, but at the rate of the vector unit: 10 000 rows of three
 // objectives on one front take 13 us this way, 300 as long waves over all slots below.
-// (to / to_of: the rows left by step 2; null where that step does not exist)
+// (grid_step: step 2 exists)
 constexpr int kFrontPairsParts = 64;
 template <int M>
 __global__ __launch_bounds__(256) void front_pairs_kernel(const float* __restrict__ left, const int* __restrict__ left_of,
-                                                          const float* __restrict__ to, const int* __restrict__ to_of,
                                                           int npad, uint8_t* __restrict__ mask, int population,
-                                                          const FrontCount* __restrict__ count, int64_t ws_step) {
+                                                          const FrontCount* __restrict__ count, int grid_step, int64_t ws_step) {
   mask += (int64_t)blockIdx.z * population;
-  to_population(ws_step, left, left_of, to, to_of, count);
+  to_population(ws_step, left, left_of, count);
   int rows = count->rows;
-  const bool second = rows > kFrontGridLeast && to != nullptr;
-  if (second) rows = count->rows_grid;
+  if (rows > kFrontGridLeast && grid_step != 0) rows = count->rows_grid;
   if (rows > kFrontPairsRows) return;
-  const float* __restrict__ src = second ? to : left;
-  const int* __restrict__ src_of = second ? to_of : left_of;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int j0 = (blockIdx.x * 4 + wave) * 64;
@@ -784,13 +872,13 @@ __global__ __launch_bounds__(256) void front_pairs_kernel(const float* __restric
   const bool all_finite = count->nonfinite == 0;
   float x[M];
 #pragma unroll
-  for (int k = 0; k < M; ++k) x[k] = src[(int64_t)k * npad + j];  // (npad is a multiple of 128: there is such a place)
+  for (int k = 0; k < M; ++k) x[k] = left[(int64_t)k * npad + j];  // (npad is a multiple of 128: there is such a place)
   bool beaten = false;
   for (int ib = i0; ib < i1; ib += 32) {
-    beaten |= half_leaf_dominates<M>(src, npad, ib, i1, x, all_finite);
+    beaten |= half_leaf_dominates<M>(left, npad, ib, i1, x, all_finite);
     if (__builtin_amdgcn_ballot_w64(!beaten && j < rows) == 0ull) break;
   }
-  if (beaten && j < rows) mask[src_of[j]] = 0;
+  if (beaten && j < rows) mask[left_of[j]] = 0;
 }
 
 // Step 4, on the rows left in spatial order (slot_row: the row left that a slot holds).  A workgroup of four waves takes the
