@@ -1345,12 +1345,12 @@ static int stage_crowd_finish(const Ws& w, const int* list, bool want_order, int
 // The copy of a result of 4-byte elements out of the workspace, as the last kernel of an entry point: the result, or
 // `poison` in every element when a device-side wait of the call ran out.
 static int copy_out(const Ctrl* ctrl, void* dst, const void* src, int64_t n, uint32_t poison, hipStream_t s, int batch = 1,
-                    int64_t ws_step = 0) {
+                    int64_t ws_step = 0, int* call_err = nullptr) {
   int64_t blocks = (n + 1023) / 1024;
   if (blocks > 1024) blocks = 1024;
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL(copy_or_poison_kernel, dim3((unsigned)blocks, 1, batch), dim3(256), 0, s, ctrl, static_cast<const uint32_t*>(src),
-                     static_cast<uint32_t*>(dst), n, poison, ws_step);
+                     static_cast<uint32_t*>(dst), n, poison, ws_step, call_err);
   EVX_LAUNCH_CHECK();
   return 0;
 }
@@ -1999,8 +1999,10 @@ static bool make_sort_layout(int64_t n, SortLayout* L) {
 }
 
 // key_cap: see argsort_step_kernel (device memory or null; only the sort of more than kMidArgsortRows keys looks at it).
+// call_err: the error word of the call that this step is a part of (or null).  The sort waits on a control block of its own:
+// without that word, kernels that go by the call's would follow an order of -1.
 static int argsort_step(const void* key, int kind, int64_t stride, int64_t n, const int32_t* prev_order, int32_t* order_out,
-                        void* ws, size_t ws_bytes, void* stream, const int* key_cap = nullptr) {
+                        void* ws, size_t ws_bytes, void* stream, const int* key_cap = nullptr, int* call_err = nullptr) {
   SortLayout L;
   if (key == nullptr || order_out == nullptr || kind < 0 || kind > 2) return kErrBadArg;
   if (!make_sort_layout(n, &L)) return kErrBadArg;
@@ -2050,7 +2052,7 @@ static int argsort_step(const void* key, int kind, int64_t stride, int64_t n, co
                      stride, L.n, prev_order, reinterpret_cast<Ctrl*>(base + L.ctrl), b, order_out, opt().spin_limit, key_cap);
   EVX_LAUNCH_CHECK();
   // (an order of -1 everywhere when one of the sort's grid barriers ran out)
-  return copy_out(reinterpret_cast<const Ctrl*>(base + L.ctrl), order_out, nullptr, n, kPoisonIndex, s);
+  return copy_out(reinterpret_cast<const Ctrl*>(base + L.ctrl), order_out, nullptr, n, kPoisonIndex, s, 1, 0, call_err);
 }
 
 // One stable argsort step of int32 keys for each of `batch` populations in one launch (n <= kMidArgsortRows, the
@@ -2396,7 +2398,7 @@ static int stage_rank_two(const Ws& w, const Fitness& src, int64_t stop_count, b
   } else {
     uint8_t* wb = w.base + L.wide;
     if (int e = argsort_step(w.at<int>(L.rank), kKeyInt32, 1, L.n, nullptr, w.at<int>(L.perm), wb + WL.sort_ws, WL.sort_bytes, s,
-                             &w.ctrl()->reserved[kTwoRounds]))
+                             &w.ctrl()->reserved[kTwoRounds], &w.ctrl()->err))
       return e;
   }
   hipLaunchKernelGGL(two_bounds_kernel, dim3(grid, 1, w.batch), dim3(256), 0, s, w.at<int>(L.perm), w.at<int>(L.rank), L.n,

@@ -1,0 +1,26 @@
+"""What the kernels read and write, on the CPU: the sources built with the address sanitizer (``emulated.py``), every region
+of the workspace with a guarded gap behind it, every result against the C checker."""
+
+import pytest
+
+from tests import emulated
+
+pytestmark = pytest.mark.skipif(emulated.CXX is None, reason="no clang++")
+
+
+@pytest.mark.parametrize("specs", [
+    ["select:1500:3:uniform:::2", "select:1500:3:simplex:::3", "select:700:5:nan", "select:3001:3:grid:::2", "twopart:2500:5:shell"],
+    ["select:4097:3:shell:::2", "select:9000:5:simplex:::2", "select:5000:2:layers", "rank:6001:5:uniform", "until:3000:5:inf"],
+    ["select:33000:2:shell:::2", "select:33000:2:layers", "select:40001:3:simplex:::3"],
+    ["batch:1100:3:shell:7", "batch:1500:5:simplex:5::2", "batch:300:3:uniform:9", "batch:5000:2:uniform:3"],
+    ["select64:3000:3:uniform", "select64:9001:5:simplex", "crowd:1400:2:uniform", "crowd:5000:3:grid", "mask:20000:3:shell", "mask:70000:2:uniform"],
+])
+def test_every_access_lies_in_its_region(specs):
+    out = emulated.run(specs)
+    assert out.count("ok ") == len(specs)
+
+
+def test_nothing_follows_an_order_whose_sort_ran_out_of_time():
+    # (the ranks of more than 32 768 rows of two objectives are sorted by workgroups that wait for each other, on a control
+    # block of the sort's own; the kernels behind it go by the call's: they took its order of -1 for rows)
+    assert "ok " in emulated.run(["select:33000:2:uniform::::poisoned"], EMU_GIVE_UP="argsort_step_kernel")
