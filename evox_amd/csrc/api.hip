@@ -21,6 +21,7 @@
 #include "peel_lds.hpp"
 #include "prefix.hpp"
 #include "radix.hpp"
+#include "records.hpp"
 #include "runs.hpp"
 #include "slots.hpp"
 #include "spatial.hpp"
@@ -32,9 +33,6 @@
 namespace evx {
 
 constexpr int kMaxGrid = 4096;  // slots of the grid barrier
-constexpr int kRecordsMaxRows = 65534;       // largest population whose record units hold three 16-bit slots
-constexpr int kRecordsMaxRowsWide = 262144;  // largest population peeled with the record protocol at all (two
-                                             // 24-bit slots per unit; 128 blocks of 8 waves own 256 rows per wave)
 
 struct Options {
   int peel_blocks_per_cu = 2;
@@ -821,13 +819,8 @@ static int stage_peel(const Ws& w, int64_t stop_count, bool want_perm, hipStream
   int blocks = 0, use_witness = 0;
   if (int e = peel_pass_plan(L, &blocks, &use_witness)) return e;
   if (use_witness && opt().peel_records && L.n <= kRecordsMaxRowsWide) {
-    // all-to-all records: 1 lister + a power of two of sweeping blocks, all resident at once
-    // by size: 64 blocks up to 32768 rows, 128 above (measured at 20000 rows: 221 us per selection with 64
-    // blocks, 225 with 128, 228 with 32, 238 with 192; between 1200 and 6000 rows the count hardly matters), 160 above
-    // five times that, where more waves for the rescans outweigh the longer exchange (128 / 160 blocks, us per selection:
-    // 60 000 x 3 477 / 550, 150 000 x 4 882 / 898, 200 003 x 3 1494 / 1398)
-    const int by_size = L.n <= 32768 ? 64 : L.n <= 163840 ? 128 : 160;
-    const int sweepers = cus >= 64 ? (opt().peel_record_blocks ? opt().peel_record_blocks : by_size) : 16;
+    // all-to-all records: 1 lister + the sweeping blocks, all resident at once
+    const int sweepers = cus >= 64 ? (opt().peel_record_blocks ? opt().peel_record_blocks : record_sweepers(L.n, L.m)) : 16;
     const int wpb = kRecThreads / 64;
     const int list_capacity = wpb * ((L.n + sweepers * wpb - 1) / (sweepers * wpb));
     const size_t rec_lds = bitmap + 24 * (size_t)list_capacity;  // queue (8 + 4 + 4) and ranked pairs (2 x 4) per row

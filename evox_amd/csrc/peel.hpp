@@ -23,6 +23,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "records.hpp"
 
 // Hooks for development builds; they compile to nothing in the library.
 #ifndef EVX_TRACE
@@ -927,14 +928,8 @@ __global__ __launch_bounds__(kPeelThreads) void peel_kernel(const uint64_t* __re
 // each front in original-index space from the records, lists it into perm and recycles bitmaps;
 // `listed` keeps the sweepers from lapping it.  All waits are bounded.
 constexpr int kRecThreads = 512;
-constexpr int kRecUnits = 1024;  // units of one generation = sweepers x units per record
 constexpr int kRecRing = 8;      // == kFrontBuffers: a generation's record slot and bitmap buffer recycle together
 constexpr int kRecLoads = kRecUnits / kRecThreads;
-// Populations of 65 535 rows and more (the wide layout: two slots per unit) have fronts of thousands of rows, and a
-// workgroup whose rows of a front do not fit its record sends everybody to the bitmaps in memory for that pass
-// (200 000 x 3: 2000 rows a front, 128 sweepers with room for 15 each).  Their generations hold four times the
-// units: room for 63 rows per workgroup.
-constexpr int kRecUnitsWide = 4 * kRecUnits;
 constexpr uint32_t kRecOverflowNarrow = 0x8000u;  // in the count field: the rows are in the bitmaps, not in the record
 static_assert(kRecRing == kFrontBuffers, "records and bitmaps are recycled by the same counter");
 
@@ -1035,8 +1030,7 @@ __global__ __launch_bounds__(kRecThreads) void peel_records_kernel(
   if (coherent_load(&ctrl->err) != 0) return;
   constexpr int kRecUnits = WIDE ? evx::kRecUnitsWide : evx::kRecUnits;  // (units of a generation, in this kernel)
   constexpr int kRecLoads = kRecUnits / kRecThreads;
-  int units = 1;  // per record: the largest power of two that gives every sweeper a record
-  while (units * 2 * sweepers <= kRecUnits) units *= 2;
+  const int units = record_units(sweepers, kRecUnits);  // per record
   const int tid = threadIdx.x;
 
   if (blockIdx.x == 0) {
