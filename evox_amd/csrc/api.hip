@@ -914,6 +914,11 @@ static bool crowd_mid_sort(const Layout& L) { return opt().mid_argsort != 0 && L
 // once from it, and these from any other.
 static bool crowd_mid_split(const Layout& L) { return opt().mid_argsort != 0 && L.n > kMidArgsortRows; }
 
+// No front of the population is too large for crowd_small_front: the first of the ordering launches does it all.
+static bool crowd_always_small(const Layout& L) {
+  return L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives;
+}
+
 // Grid of crowd_gather_kernel, crowd_sort_kernel and crowd_finish_kernel (finish.hpp): the radix grid when a front of this
 // population can exceed kRadixMinCandidates rows (they then synchronise across blocks), else one block
 // per 256 candidates and objective.
@@ -1218,7 +1223,8 @@ static size_t crowd_lds_bytes(const Layout& L, int fused) {
   return lds;
 }
 
-// The first two of the launches that order a front from sorted runs (finish.hpp).
+// The first two of the launches that order a front from sorted runs (finish.hpp); the first alone where no front is too
+// large for it.
 static int launch_crowd_runs(const Ws& w, const CrowdArgs& a, int tail_flag, hipStream_t s) {
   const Layout& L = w.L;
   const int most = L.n < kRunMaxRows ? L.n : kRunMaxRows;
@@ -1235,6 +1241,7 @@ static int launch_crowd_runs(const Ws& w, const CrowdArgs& a, int tail_flag, hip
   else
     hipLaunchKernelGGL(crowd_runs_kernel<false>, dim3(grid), dim3(kRunRows), runs_lds, s, a, tail_flag, small_blocks);
   EVX_LAUNCH_CHECK();
+  if (a.mid_sort == 1 && a.fused != 0 && crowd_always_small(L)) return 0;
   const size_t lds = run_rank_lds_bytes(most);
   const void* const terms_kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_terms_kernel<true>) : reinterpret_cast<const void*>(crowd_terms_kernel<false>);
   if (int e = grant_dynamic_lds(terms_kernel, lds)) return e;
@@ -1316,8 +1323,7 @@ static int stage_crowd_finish(const Ws& w, const int* list, bool want_order, int
   const int tail_flag = after_peel_tail ? 1 : 0;
   CrowdArgs a = crowd_args(w, list, false, fused);
   if (without_runs && a.mid_sort == 2) a.mid_sort = 0;
-  if (gather == nullptr && fused != 0 && L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives)
-    return 0;  // (no front of this population is too large for crowd_small_front: nothing is left to do)
+  if (gather == nullptr && fused != 0 && crowd_always_small(L)) return 0;  // (nothing is left to do)
   if (crowd_mid_sort(L)) return launch_crowd_pick(w, a, want_order, gather, tail_flag, s);
   if (gather != nullptr) return kErrBadArg;
   if (a.mid_sort == 2)
@@ -2573,8 +2579,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   }
   if (!one_ordering_launch) {
     if (int e = stage_crowd_sort(w, w.at<int>(L.perm), true, 2, s, peel_orders, without_runs)) return e;
-    const bool never_large = L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives;
-    if (crowd_mid_sort(L) && !never_large) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, &g);
+    if (crowd_mid_sort(L) && !crowd_always_small(L)) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, &g);
     if (int e = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, nullptr, without_runs)) return e;
     if (peel_orders)
       launch_gather(true);

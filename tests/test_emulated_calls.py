@@ -24,3 +24,10 @@ def test_nothing_follows_an_order_whose_sort_ran_out_of_time():
     # (the ranks of more than 32 768 rows of two objectives are sorted by workgroups that wait for each other, on a control
     # block of the sort's own; the kernels behind it go by the call's: they took its order of -1 for rows)
     assert "ok " in emulated.run(["select:33000:2:uniform::::poisoned"], EMU_GIVE_UP="argsort_step_kernel")
+
+
+@pytest.mark.parametrize("spec,searched", [("crowd:1365:3:uniform", False), ("crowd:1366:3:uniform", True), ("crowd:1100:2:grid", False)])
+def test_small_fronts_are_done_in_the_first_ordering_launch(spec, searched):
+    # (1365 x 3 values fit the workgroups that order a small front whatever the mask selects: one launch, nothing behind it)
+    out = emulated.run([spec], EMU_TRACE="1")
+    assert ("crowd_terms_kernel" in out) == searched and "crowd_runs_kernel" in out and "ok " in out
