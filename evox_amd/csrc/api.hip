@@ -914,11 +914,6 @@ static bool crowd_mid_sort(const Layout& L) { return opt().mid_argsort != 0 && L
 // once from it, and these from any other.
 static bool crowd_mid_split(const Layout& L) { return opt().mid_argsort != 0 && L.n > kMidArgsortRows; }
 
-// No front of the population is too large for crowd_small_front: the first of the ordering launches does it all.
-static bool crowd_always_small(const Layout& L) {
-  return L.n <= kFusedFrontRows && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives;
-}
-
 // Grid of crowd_gather_kernel, crowd_sort_kernel and crowd_finish_kernel (finish.hpp): the radix grid when a front of this
 // population can exceed kRadixMinCandidates rows (they then synchronise across blocks), else one block
 // per 256 candidates and objective.
@@ -1164,6 +1159,23 @@ static int dispatch_dominance_prefix(const Ws& w, hipStream_t s, int phase) {
   }
 }
 
+// Workgroups of kRunRows threads that order a small front of one population together (crowd_small_front): all of them are
+// resident at once, a sixteenth of their threads candidates in a round.
+static int crowd_small_blocks(const Ws& w) { return shared_grid(kFusedFrontRows * 16 / kRunRows, device_cus(), w.batch); }
+// The largest front that goes that way where the sorted runs stand behind it.  Several populations share the device: a
+// round of the workgroups that one of them gets, since every further round costs as much as the runs do -- 40 populations of
+// 1400 x 4 around a sphere, last fronts of some 900 rows, us: 275 with up to 1024 rows there, 111 with up to 192.
+static int crowd_small_rows(const Ws& w) {
+  if (w.batch == 1) return kFusedFrontRows;
+  const int round = crowd_small_blocks(w) * (kRunRows / 16);
+  return round < kFusedSoloRows ? kFusedSoloRows : round;
+}
+// No front of the population is too large for crowd_small_front: the first of the ordering launches does it all.
+static bool crowd_always_small(const Ws& w) {
+  const Layout& L = w.L;
+  return L.n <= (crowd_mid_sort(L) ? crowd_small_rows(w) : kFusedFrontRows) && (int64_t)L.n * L.m <= kFusedFrontValues && L.m <= kFusedFrontObjectives;
+}
+
 // Per-objective ordering of the candidates list[ctrl.worst_start ... + ctrl.nv).
 // fused: 0 = the two kernels as stages of their own; 1 / 2 = a small front gets its distances (2: and the selection
 // order) inside crowd_sort_kernel, and crowd_finish_kernel, given the same value, leaves it alone.
@@ -1184,6 +1196,7 @@ static CrowdArgs crowd_args(const Ws& w, const int* list, bool use_orders, int f
   a.use_orders = use_orders ? 1 : 0;
   a.fused = fused;
   a.mid_sort = crowd_mid_sort(L) ? 1 : (crowd_mid_split(L) ? 2 : 0);
+  a.small_rows = crowd_small_rows(w);
   a.dist = w.at<float>(L.dist);
   a.dkey = w.at<uint32_t>(L.dkey);
   a.order = w.at<int>(L.order);
@@ -1229,8 +1242,7 @@ static int launch_crowd_runs(const Ws& w, const CrowdArgs& a, int tail_flag, hip
   const Layout& L = w.L;
   const int most = L.n < kRunMaxRows ? L.n : kRunMaxRows;
   const size_t runs_lds = a.mid_sort == 1 && a.fused != 0 ? kFusedFrontLdsBytes : sizeof(uint32_t) * 2 * kRunRows;
-  // (a small front: up to 64 workgroups of it, which wait for each other, are resident at once)
-  const int small_blocks = shared_grid(kFusedFrontRows * 16 / kRunRows, device_cus(), w.batch);
+  const int small_blocks = crowd_small_blocks(w);
   int grid = (most + kRunRows - 1) / kRunRows * L.m;
   if (grid < small_blocks) grid = small_blocks;
   if (grid > 65536) grid = 65536;
@@ -1241,7 +1253,7 @@ static int launch_crowd_runs(const Ws& w, const CrowdArgs& a, int tail_flag, hip
   else
     hipLaunchKernelGGL(crowd_runs_kernel<false>, dim3(grid), dim3(kRunRows), runs_lds, s, a, tail_flag, small_blocks);
   EVX_LAUNCH_CHECK();
-  if (a.mid_sort == 1 && a.fused != 0 && crowd_always_small(L)) return 0;
+  if (a.mid_sort == 1 && a.fused != 0 && crowd_always_small(w)) return 0;
   const size_t lds = run_rank_lds_bytes(most);
   const void* const terms_kernel = w.batch > 1 ? reinterpret_cast<const void*>(crowd_terms_kernel<true>) : reinterpret_cast<const void*>(crowd_terms_kernel<false>);
   if (int e = grant_dynamic_lds(terms_kernel, lds)) return e;
@@ -1323,7 +1335,7 @@ static int stage_crowd_finish(const Ws& w, const int* list, bool want_order, int
   const int tail_flag = after_peel_tail ? 1 : 0;
   CrowdArgs a = crowd_args(w, list, false, fused);
   if (without_runs && a.mid_sort == 2) a.mid_sort = 0;
-  if (gather == nullptr && fused != 0 && crowd_always_small(L)) return 0;  // (nothing is left to do)
+  if (gather == nullptr && fused != 0 && crowd_always_small(w)) return 0;  // (nothing is left to do)
   if (crowd_mid_sort(L)) return launch_crowd_pick(w, a, want_order, gather, tail_flag, s);
   if (gather != nullptr) return kErrBadArg;
   if (a.mid_sort == 2)
@@ -2579,7 +2591,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   }
   if (!one_ordering_launch) {
     if (int e = stage_crowd_sort(w, w.at<int>(L.perm), true, 2, s, peel_orders, without_runs)) return e;
-    if (crowd_mid_sort(L) && !crowd_always_small(L)) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, &g);
+    if (crowd_mid_sort(L) && !crowd_always_small(w)) return stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, &g);
     if (int e = stage_crowd_finish(w, w.at<int>(L.perm), true, 2, s, peel_orders, nullptr, without_runs)) return e;
     if (peel_orders)
       launch_gather(true);

@@ -205,6 +205,7 @@ struct CrowdArgs {
   // has it all in one launch: the LDS sorter mid_argsort_slice); 2 = a larger population: the sorted runs take a front of
   // kMidSortMinCandidates + 1 to kMidArgsortRows rows, and the other launches leave it alone.
   int mid_sort;
+  int small_rows;  // with the sorted runs: the largest front that crowd_small_front takes
   float* dist;
   uint32_t* dkey;
   int* order;
@@ -226,8 +227,11 @@ __device__ inline bool crowd_mid_applies(const CrowdArgs& a, int nv) {
 }
 // Whether the kernels with the sorted runs order the front.  A front that crowd_small_front takes is not theirs.
 static_assert(kRunMaxRows == kMidArgsortRows, "the runs of a front must fit the LDS of a workgroup");
+__device__ inline bool crowd_small_takes(const CrowdArgs& a, int nv) {
+  return a.fused != 0 && fused_front_applies(nv, a.m) && nv <= a.small_rows;
+}
 __device__ inline bool crowd_runs_take(const CrowdArgs& a, int nv) {
-  if (a.fused != 0 && fused_front_applies(nv, a.m)) return false;
+  if (crowd_small_takes(a, nv)) return false;
   return a.mid_sort == 1 || (a.mid_sort == 2 && nv > kMidSortMinCandidates && nv <= kMidArgsortRows);
 }
 
@@ -572,7 +576,7 @@ __global__ __launch_bounds__(kRunRows) void crowd_runs_kernel(CrowdArgs a, int a
   if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
   if (coherent_load(&a.ctrl->err) != 0) return;
   const int nv = a.ctrl->nv, m = a.m;
-  if (a.mid_sort == 1 && a.fused != 0 && fused_front_applies(nv, m)) {
+  if (a.mid_sort == 1 && crowd_small_takes(a, nv)) {
     crowd_small_front(a.xs, a.npad, a.list_base, a.ctrl, m, a.dist, a.dkey, a.order, a.spin_limit, a.fused, small_blocks, finish_lds, scratch);
     return;
   }
