@@ -1,6 +1,6 @@
 // C ABI of libevox_hip.so (declared in include/evox_hip.h): argument checks, workspace layout
 // and kernel launches.  Nothing here allocates device memory or waits for the device, except
-// evox_hip_read_status(); the selection entry points keep 64 bytes of pinned host memory per device (outcome_slot).
+// evox_hip_read_status(); the selection entry points keep 320 bytes of pinned host memory per device (outcome_slot).
 #include <string.h>
 
 #include <atomic>
@@ -16,6 +16,7 @@
 #include "dominance.hpp"
 #include "finish.hpp"
 #include "hv.hpp"
+#include "launch_words.hpp"
 #include "order.hpp"
 #include "peel.hpp"
 #include "peel_lds.hpp"
@@ -206,15 +207,13 @@ static int device_cus() {
   return v;
 }
 
-// What the last selections on this device found, for the choice of launches of the next one: sixteen words of pinned
-// host memory per device, which the last kernel of a selection writes (1: the peel kernel ordered the last front, 2: it
-// left it to the ordering kernels) and the host reads at its next call of that shape without waiting for anything --
-// a stale or missing word costs a few microseconds, never a result.  Allocated at the first selection on a device
-// that may allocate (not during a stream capture); null until then and for callers that may not.
-// salt: 0 for the selections of 4-byte fitness, 1 for those whose last front is ordered by the kernels of wide.hpp
-// (there the word says whether that front was small, 1, or large, 2), 2 for whether front 0 alone held what was kept
-// (GatherArgs::front0_note).
-static int* outcome_slot(int64_t n, int64_t m, bool may_allocate, hipStream_t s, int salt = 0) {
+// What the last selections on this device found, for the choice of launches of the next one: some words of pinned host
+// memory per device (launch_words.hpp), which the last kernel of a selection writes and the host reads at its next call of
+// that shape without waiting for anything -- a stale or missing word costs a few microseconds, never a result.  Allocated
+// at the first selection on a device that may allocate (not during a stream capture); null until then and for callers
+// that may not.
+static int* outcome_slot(LaunchWord meaning, int64_t n, int64_t m, bool may_allocate, hipStream_t s) {
+  constexpr size_t bytes = sizeof(int) * kWordsPerMeaning * kLaunchWords;
   static std::atomic<int*> words[64];
   static std::atomic<bool> failed[64];
   static std::mutex mu;
@@ -232,17 +231,17 @@ static int* outcome_slot(int64_t n, int64_t m, bool may_allocate, hipStream_t s,
     base = words[dev].load(std::memory_order_acquire);
     if (base == nullptr) {
       void* p = nullptr;
-      if (hipHostMalloc(&p, 64, hipHostMallocDefault) != hipSuccess || p == nullptr) {
+      if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess || p == nullptr) {
         (void)hipGetLastError();
         failed[dev].store(true, std::memory_order_relaxed);
         return nullptr;
       }
-      memset(p, 0, 64);
+      memset(p, 0, bytes);
       base = static_cast<int*>(p);
       words[dev].store(base, std::memory_order_release);
     }
   }
-  return base + (int)(((uint64_t)n * 31u + (uint64_t)m + (uint64_t)salt * 7u) & 15u);
+  return base + launch_word(meaning, n, m);
 }
 
 #define EVX_LAUNCH_CHECK()                          \
@@ -2498,7 +2497,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   // 70 000 x 3 on a plane 304 -> 288 us).
   bool without_runs = false;
   if (batch == 1 && crowd_mid_split(L) && opt().launch_memory) {
-    g.outcome = outcome_slot(n, m, may_allocate, s, 3);
+    g.outcome = outcome_slot(kWordRuns, n, m, may_allocate, s);
     const int small = L.m <= kFusedFrontObjectives ? (kFusedFrontValues / L.m < kFusedFrontRows ? kFusedFrontValues / L.m : kFusedFrontRows) : 0;
     g.outcome_from = small > kMidSortMinCandidates ? small : kMidSortMinCandidates;
     g.outcome_to = kMidArgsortRows;
@@ -2524,7 +2523,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   // kept: the stage 0.98 -> 0.80 ms; a wrong guess costs a second launch, 0.92 ms, once).
   int64_t count_first = 0;
   if (batch == 1 && opt().launch_memory && opt().prefix_count_first && prefix_dominance_applies(L) && !opt().peel_stepped) {
-    g.front0_note = outcome_slot(n, m, may_allocate, s, 2);
+    g.front0_note = outcome_slot(kWordFront0, n, m, may_allocate, s);
     g.front0_size = w.at<int>(L.fsize);
     g.front0_enough = (int)topk;
     if (g.front0_note != nullptr && __atomic_load_n(g.front0_note, __ATOMIC_RELAXED) == 3) count_first = topk;
@@ -2540,7 +2539,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   }
   g.order_from_peel = peel_always_orders ? 1 : 0;
   if (!crowd_mid_split(L))
-    g.outcome = batch == 1 && peel_orders && !peel_always_orders && opt().launch_memory ? outcome_slot(n, m, may_allocate, s) : nullptr;
+    g.outcome = batch == 1 && peel_orders && !peel_always_orders && opt().launch_memory ? outcome_slot(kWordLastFront, n, m, may_allocate, s) : nullptr;
   const int last_outcome = g.outcome != nullptr && g.outcome_to == 0 ? __atomic_load_n(g.outcome, __ATOMIC_RELAXED) : 0;
   // Where the peel kernel may have ordered the last front, the kernels that would order it look at Ctrl.tail_done and
   // return at once.  A launch that does nothing still costs 2 to 4.7 us, so with up to three objectives -- last
@@ -2559,7 +2558,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
     WideLayout WL;
     if (!make_wide_layout(n, m, &WL) || WL.total > L.wide_bytes) return kErrWorkspace;
     uint8_t* wb = w.base + L.wide;
-    int* const wide_outcome = opt().launch_memory ? outcome_slot(n, m, may_allocate, s, 1) : nullptr;
+    int* const wide_outcome = opt().launch_memory ? outcome_slot(kWordWide, n, m, may_allocate, s) : nullptr;
     if (wide_direct_applies(n, wide_outcome)) {
       if (int e = wide_select_direct(WL, wb, w.at<float>(L.xs), kWideFloat32, 1, L.npad, w.at<int>(L.rank), w.at<float>(L.dist), 1,
                                      w.at<int>(L.order), s, wide_outcome))
@@ -2816,7 +2815,7 @@ int evox_hip_nd_environmental_selection_wide(const void* x, int64_t x_row_bytes,
   void* dist = base + L.dist;
   int* order_a = reinterpret_cast<int*>(base + L.order_a);
   int* order_b = reinterpret_cast<int*>(base + L.order_b);
-  int* const outcome = opt().launch_memory ? outcome_slot(n, m, true, s, 1) : nullptr;
+  int* const outcome = opt().launch_memory ? outcome_slot(kWordWide, n, m, true, s) : nullptr;
   if (wide_direct_applies(n, outcome)) {
     if (int e = wide_select_direct(L, base, costs, kind, sr, sc, rank, dist, out_kind, order_a, s, outcome)) return e;
   } else {
@@ -2846,7 +2845,7 @@ int evox_hip_many_nd_environmental_selection_wide(const void* x, int64_t x_row_b
   const int64_t step = (int64_t)align_up(L.total);
   const int64_t dist_bytes = out_kind == 0 ? 8 : 4;
   hipStream_t s = (hipStream_t)stream;
-  int* const outcome = opt().launch_memory ? outcome_slot(n, m, true, s, 1) : nullptr;
+  int* const outcome = opt().launch_memory ? outcome_slot(kWordWide, n, m, true, s) : nullptr;
   const int64_t x_out_step = topk * x_row_bytes, f_out_step = topk * f_row_bytes;
   const bool together = batch > 1 && wide_direct_applies(n, outcome) && (n <= kSmallArgsortRows || opt().mid_argsort) &&
                         ws_bytes >= (size_t)step * (size_t)batch && batch <= 65535;

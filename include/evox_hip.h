@@ -11,7 +11,7 @@
  *   - What the library keeps between calls, per process: the tunables; per device, small host-side tables of what it
  *     has asked the runtime once (compute units, resident workgroups, LDS grants); the scratch buffer of the entry
  *     point named above (EVOX_HIP_STATIC_SCRATCH_BYTES of device memory on every GPU that the process touches,
- *     whether or not that entry point is ever called: it is part of the device image); and 64 bytes of pinned host
+ *     whether or not that entry point is ever called: it is part of the device image); and 320 bytes of pinned host
  *     memory per device, allocated at the first selection, in which the last kernel of a selection notes whether the
  *     peel kernel ordered the last front (for a selection of 8-byte fitness: whether its last front held more than
  *     8192 rows; for a large population whose matrix comes from the per-objective orders: whether front 0 held
@@ -404,7 +404,7 @@ int evox_hip_read_status(const void* workspace, void* stream, int32_t* host_out8
  * (0 = by size, or 8 .. 255 sweeping workgroups of that kernel), "peel_tail" (1 = that kernel also orders a small last front), "tail_merged"
  * (1 = after such a peel the two ordering stages and the gather share one launch, up to three objectives), "launch_memory" (1 = ... unless
  * the last selection of that shape on the device had a last front that the peel kernel left to the ordering kernels, which a word of
- * pinned host memory tells: the library allocates 64 bytes of it per device at the first selection; 0 = never looked at),
+ * pinned host memory tells: the library allocates 320 bytes of it per device at the first selection; 0 = never looked at),
  * "peel_blocks_per_cu" (default 2), "peel_witness" (1 = witness pass, 0 = popcount sweep), "peel_records" (1 = record
  * protocol, 0 = master barrier and front bitmaps), "peel_record_blocks" (0 = by size, or 16 .. 255), "spin_limit" (the bound of every device-side wait: a value above 65535 is a time in units of 10 ns on the device's constant clock, default 4000000 = 40 ms; a value up to 65535 counts failed polls, for tests that force a wait to give up), "two_small_min_rows" (default 128: from this many rows on, a population of two objectives that goes to a one-workgroup kernel takes the one without a dominance matrix, which also raises evox_hip_batched_max_rows(2) to 4096; 0 = never), "two_min_rows" (default 4097: smallest population of two objectives that is ranked without a dominance matrix -- rows sorted by (f1, f2, index), every front the strict prefix minima of f2 among the rows that remain; 0 = never) and "two_min_rows_partial" (default 4097: the same where the ranking may stop at a front, as in a selection; there the peeling ends once the fronts so far hold the rows asked for), "peel_stepped" (0 = the fronts are peeled by one persistent kernel where its grid can be resident at once, 1 = always by one launch per front and the last front by kernels that never wait for each other: slower, needs no co-residency, and waits for the stream between groups of sixteen launches), "dominance_tile_words" (0 = by size: 2 or 4; or 2, 4, 8, 16), "dominance_folded" (1 = only the blocks at or below the diagonal are launched; 0 = the whole rectangle), "mid_argsort" (1 = an argsort step of 8193 to 32768 positions, and a last front of 1025 to 32768 rows, are ordered by workgroups that sort in LDS without waiting for each other; 0 = the radix sort and ranking by counting), "small_sort" (1 = one-kernel slot sort up to 4096 rows),
  * "prefix_min_rows" (default 65536: smallest finite population of three objectives whose matrix is built from the per-objective orders -- a quarter more rows with two, fewer with more: 28672 at eight, 10240 at sixteen; 0 = never),
