@@ -2539,7 +2539,8 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
   }
   g.order_from_peel = peel_always_orders ? 1 : 0;
   if (!crowd_mid_split(L))
-    g.outcome = batch == 1 && peel_orders && !peel_always_orders && opt().launch_memory ? outcome_slot(kWordLastFront, n, m, may_allocate, s) : nullptr;
+    g.outcome = peel_orders && !peel_always_orders && opt().launch_memory
+                    ? outcome_slot(batch > 1 ? kWordBatch : kWordLastFront, n, m, may_allocate, s) : nullptr;
   const int last_outcome = g.outcome != nullptr && g.outcome_to == 0 ? __atomic_load_n(g.outcome, __ATOMIC_RELAXED) : 0;
   // Where the peel kernel may have ordered the last front, the kernels that would order it look at Ctrl.tail_done and
   // return at once.  A launch that does nothing still costs 2 to 4.7 us, so with up to three objectives -- last

@@ -172,9 +172,10 @@ __device__ __forceinline__ void to_population(GatherArgs& g) {
   if (g.out_order != nullptr) g.out_order += b * g.topk;
 }
 
-// What the host's choice of launches at its next call goes by (it reads the words without waiting for anything).
+// What the host's choice of launches at its next call goes by (it reads the words without waiting for anything; of several
+// populations the first one tells).
 __device__ __forceinline__ void gather_notes(const GatherArgs& a, int block) {
-  if (a.outcome != nullptr && block == 0 && threadIdx.x == 0)
+  if (a.outcome != nullptr && block == 0 && blockIdx.z == 0 && threadIdx.x == 0)
     __hip_atomic_store(a.outcome, (a.outcome_to > 0 ? a.ctrl->nv > a.outcome_from && a.ctrl->nv <= a.outcome_to : a.ctrl->tail_done != 0) ? 1 : 2,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (a.front0_note != nullptr && block == 0 && threadIdx.x == 0) {

@@ -31,3 +31,19 @@ def test_small_fronts_are_done_in_the_first_ordering_launch(spec, searched):
     # (1365 x 3 values fit the workgroups that order a small front whatever the mask selects: one launch, nothing behind it)
     out = emulated.run([spec], EMU_TRACE="1")
     assert ("crowd_terms_kernel" in out) == searched and "crowd_runs_kernel" in out and "ok " in out
+
+
+def test_populations_of_a_launch_on_either_side_of_the_small_front():
+    # (64 compute units for six populations: ten workgroups each order a last front of up to 320 rows together, larger ones go
+    # through the sorted runs; uniform fitness stays below, rows around a sphere and on a plane lie above; every call meets
+    # the word that the one before it has left)
+    specs = ["batch:1300:5:uniform:6::2", "batch:1300:5:shell:6::2", "batch:1300:5:simplex:6::2", "batch:1300:5:uniform:6", "batch:1300:3:shell:6::2",
+             "batch:1300:3:simplex:6::2", "batch:1300:3:uniform:6"]
+    assert emulated.run(specs, EMU_CUS="64").count("ok ") == len(specs)
+
+
+def test_populations_whose_peel_orders_their_last_fronts_take_one_launch_for_what_is_left():
+    out = emulated.run(["batch:1300:5:uniform:3::2"], EMU_TRACE="1", EMU_CUS="256")
+    first, second = out.split("rep 1")
+    assert "crowd_terms_kernel" in first and "crowd_gather_kernel" not in first
+    assert "crowd_terms_kernel" not in second and "crowd_gather_kernel" in second
