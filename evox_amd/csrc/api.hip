@@ -71,7 +71,8 @@ struct Options {
                          // them in LDS (0: from the radix sort whose workgroups wait for each other)
   int order_stream_capacity = 16384;  // entries that such a workgroup sorts at once (tests make it small: shares in pieces)
   int prefix_count_first = 1;  // a selection whose last two of this shape found all they keep in front 0 has the order-based
-                               // kernel count dominators first and build the matrix only if front 0 falls short; 0 = never
+                               // kernel count dominators first and build the matrix only if front 0 falls short; 0 = never, 2 = always
+  int64_t prefix_nearby = 1;  // those counts in spatial order: 1 = by size (nearby_totals_apply), 0 = never, else from this many rows on
 };
 static Options g_opt;
 // The tunables that calls made from this thread use: those handed to evox_hip_options_use, else the process-wide ones.
@@ -943,6 +944,20 @@ static int shared_grid(int grid, int resident, int batch) {
 }
 
 constexpr int kNearbyMaxObjectives = 15;  // (the order of the slots is one more)
+// From how many rows on the totals alone are counted in spatial order (their order costs 60 us, and what it saves hangs on
+// the share of the pairs of tile and group that is left).  Whole selections whose front 0 holds what is kept, us, slot
+// order / spatial order, all rows on a plane or (s) around a sphere with a part of front 0 kept:
+//   x 3: 90 112 341 / 321, 100 000 (s) 277 / 291, 125 000 (s) 325 / 333, 131 072 481 / 383, (s) 390 / 334, 200 000 (s) 719 / 568;
+//   x 4: 80 000 307 / 314, 90 112 339 / 327, 100 000 (s) 344 / 327, 200 000 899 / 614;
+//   x 5: 57 344 288 / 294, 62 000 (s) 286 / 292, 65 536 303 / 301, (s) 304 / 300;
+//   x 6: 57 344 (s) 302 / 307, 60 000 317 / 310;  x 8: 57 344 (s) 346 / 350, 60 000 380 / 360, 200 000 (s) 1176 / 743;
+//   x 10: 57 344 (s) 371 / 381, 60 000 (s) 411 / 399;  x 11: 57 344 (s) 423 / 396;  x 15: 40 000 381 / 405, 57 344 (s) 543 / 501.
+static int64_t nearby_least_rows(int m) { return m <= 3 ? 131072 : m == 4 ? 90112 : m == 5 ? 65536 : m <= 10 ? 60000 : 57344; }
+static bool nearby_totals_apply(int n, int m) {
+  const int64_t rule = opt().prefix_nearby;
+  if (rule == 0 || m < 3 || m > kNearbyMaxObjectives) return false;  // (two objectives are ranked without totals)
+  return n >= (rule == 1 ? nearby_least_rows(m) : rule);
+}
 template <int M>
 static int launch_nearby_totals(const Ws& w, hipStream_t s);
 
@@ -976,11 +991,8 @@ static int launch_dominance_prefix(const Ws& w, hipStream_t s, int phase) {
     return 0;
   };
   // (200 000 x 3: 957 -> 769 us, x 4: 972 -> 797; 100 000 x 3: 319 -> 317; 65536 x 3: 184 -> 220: half as many workgroups)
-  // The totals alone in spatial order or in slot order, whole selections in us where front 0 holds what is kept, slot /
-  // spatial: x 3 70 000 298 / 302, 100 000 366 / 355;  x 5 50 000 274 / 293, 60 000 311 / 309, 150 000 630 / 520;  x 8 50 000
-  // 322 / 331, 60 000 401 / 369, 200 000 1176 / 743;  x 12 60 000 495 / 440;  x 15 40 000 381 / 405.
-  if (M <= kNearbyMaxObjectives && phase == 1 && L.n >= (M <= 4 ? 90112 : 57344)) {
-    if constexpr (M <= kNearbyMaxObjectives)
+  if (phase == 1 && nearby_totals_apply(L.n, M)) {
+    if constexpr (M >= 3 && M <= kNearbyMaxObjectives)
       if (int e = launch_nearby_totals<M>(w, s)) return e;
   } else if (TT == 2 && opt().prefix_double_tile > 0 && L.n >= opt().prefix_double_tile) {
     if (int e = launch(dominance_prefix_kernel<M, WW, TT>, TT)) return e;
@@ -1554,8 +1566,10 @@ static int set_named(Options& o, const char* name, int64_t value) {
     o.order_stream = (int)value;
   } else if (!strcmp(name, "order_stream_capacity") && value >= 1 && value <= kOrderStreamCapacity) {
     o.order_stream_capacity = (int)value;
-  } else if (!strcmp(name, "prefix_count_first") && (value == 0 || value == 1)) {
+  } else if (!strcmp(name, "prefix_count_first") && value >= 0 && value <= 2) {
     o.prefix_count_first = (int)value;
+  } else if (!strcmp(name, "prefix_nearby") && value >= 0) {
+    o.prefix_nearby = value;
   } else {
     return kErrBadArg;
   }
@@ -2526,7 +2540,7 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
     g.front0_note = outcome_slot(kWordFront0, n, m, may_allocate, s);
     g.front0_size = w.at<int>(L.fsize);
     g.front0_enough = (int)topk;
-    if (g.front0_note != nullptr && __atomic_load_n(g.front0_note, __ATOMIC_RELAXED) == 3) count_first = topk;
+    if (opt().prefix_count_first == 2 || (g.front0_note != nullptr && __atomic_load_n(g.front0_note, __ATOMIC_RELAXED) == 3)) count_first = topk;
   }
   if (int e = stage_dominance(w, kDomAuto, s, count_first)) return e;
   bool peel_orders = false;  // the peel kernel orders a small last front itself (it says so in Ctrl.tail_done)

@@ -411,7 +411,8 @@ int evox_hip_read_status(const void* workspace, void* stream, int32_t* host_out8
  * "prefix_bands" (default 1), "prefix_double_tile" (default 131072 rows, 0 = never), "prefix_mode" (default 3; 1 and 2 build only half of that kernel's output, for measurements),
  * "batched_stage" (default 1: the one-workgroup kernel reads the dominators of populations of at most 256 rows and eight objectives from a copy of the fitness in LDS when the launch holds no more populations than the device has compute units; 0 = by scalar loads from memory always),
  * "order_stream" (default 1: for more than 32768 rows those orders come from workgroups that read their objective's keys once and sort a share of the order in LDS, without waiting for each other, while shares of 3200 rows need no more workgroups than the device has compute units -- up to 102400 rows of eight objectives; 0 = from the radix sort, whose workgroups wait for each other twelve times), "order_stream_capacity" (default 16384, 1 .. 16384: entries that such a workgroup sorts at once; a larger share is taken in pieces -- tests make it small),
- * "prefix_count_first" (default 1: a selection of such a population whose last two of the same shape on the device found all the rows they keep in front 0 -- told by a word of the pinned host memory of "launch_memory" -- has that kernel count the dominators of every row first and build the matrix, in a second launch, only if front 0 falls short this time; 0 = always both at once).
+ * "prefix_count_first" (default 1: a selection of such a population whose last two of the same shape on the device found all the rows they keep in front 0 -- told by a word of the pinned host memory of "launch_memory" -- has that kernel count the dominators of every row first and build the matrix, in a second launch, only if front 0 falls short this time; 0 = always both at once, 2 = always counts first),
+ * "prefix_nearby" (default 1: those counts are made in spatial order from a number of rows on that falls with the objectives -- 131072 at three, 57344 at eleven to fifteen; 0 = never, any other value = from that many rows on).
  * Returns EVOX_HIP_E_BAD_ARG for an unknown name or a value out of range. */
 int evox_hip_set_option(const char* name, int64_t value);
 

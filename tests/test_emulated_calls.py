@@ -47,3 +47,22 @@ def test_populations_whose_peel_orders_their_last_fronts_take_one_launch_for_wha
     first, second = out.split("rep 1")
     assert "crowd_terms_kernel" in first and "crowd_gather_kernel" not in first
     assert "crowd_terms_kernel" not in second and "crowd_gather_kernel" in second
+
+
+_COUNT_FIRST = ["-o", "prefix_count_first=2", "-o", "prefix_min_rows=16384"]
+
+
+@pytest.mark.parametrize("m", [3, 5])
+def test_totals_in_spatial_order(m):
+    # (in the second call front 0 falls short: the matrix is built where the totals' scratch memory lay)
+    specs = [f"select:{n}:{m}:{data}::{k}" for n, data, k in ((33000, "simplex", 9000), (33001, "shell", 6000), (33025, "equal", 100))]
+    out = emulated.run(_COUNT_FIRST + ["-o", "prefix_nearby=2"] + specs, EMU_TRACE="1")
+    assert out.count("ok ") == len(specs) and out.count("nearby_pairs_kernel") == len(specs)
+    out = emulated.run(_COUNT_FIRST + ["-o", "prefix_nearby=0"] + specs[:1], EMU_TRACE="1")
+    assert "ok " in out and "nearby" not in out
+
+
+@pytest.mark.parametrize("n,spatial", [(57344, False), (65536, True)])
+def test_totals_in_spatial_order_from_the_size_on_at_which_they_are_the_faster(n, spatial):
+    out = emulated.run(["-o", "prefix_count_first=2", f"select:{n}:5:simplex::20000"], EMU_TRACE="1")
+    assert "ok " in out and ("nearby_pairs_kernel" in out) == spatial

@@ -1,13 +1,17 @@
 """Selections of large populations that keep less than front 0 holds: from the third call of a shape on the dominators are
-counted in spatial order, without a matrix.  Against the same selection with the matrix: objectives on either side of the
-tile sizes, populations on either side of the rule, equal rows, equal keys, values on a grid, all rows alike, a NaN, and a
-population whose front 0 falls short after others whose did not."""
+counted in spatial order, without a matrix.  Against the same selection with the matrix, and with the tunables that force
+the counts first and in spatial order whatever the launch memory says against the C checker: objectives on either side of
+the tile sizes, populations on either side of the rule, equal rows, equal keys, values on a grid, all rows alike, a NaN, and
+a population whose front 0 falls short after others whose did not."""
 
+import numpy as np
 import pytest
 import torch
 
 from evox_amd import runtime
 from evox_amd.operators.selection import nd_environmental_selection
+from oracle import c_oracle
+from tests.cases import as_np
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
@@ -35,7 +39,7 @@ def _same(a, b):
     return torch.equal(torch.nan_to_num(a.float(), nan=-7.0), torch.nan_to_num(b.float(), nan=-7.0))
 
 
-@pytest.mark.parametrize("n,m", [(57343, 5), (57344, 5), (90113, 3), (90200, 4), (60001, 8), (58000, 9), (60000, 10), (57345, 15), (57344, 16)])
+@pytest.mark.parametrize("n,m", [(65535, 5), (65536, 5), (131073, 3), (90200, 4), (60001, 8), (59999, 9), (60000, 10), (57345, 15), (57344, 16)])
 def test_totals_in_spatial_order(n, m):
     runtime.release_workspaces()
     x = torch.arange(n, dtype=torch.int32, device=DEV)[:, None]
@@ -50,4 +54,67 @@ def test_totals_in_spatial_order(n, m):
         with runtime.options(prefix_count_first=0):
             want = nd_environmental_selection(x, f, k)
         assert all(_same(a, b) for a, b in zip(got, want)), (call, kind)
+    runtime.release_workspaces()
+
+
+FORCED = dict(prefix_count_first=2, prefix_nearby=2, prefix_min_rows=16384)
+
+
+def _check(got, want, name):
+    order, rank, dist, _ = want
+    xs, _, rs, ds = (as_np(t) for t in got)
+    assert np.array_equal(xs[:, 0].astype(np.int64), order), name
+    assert np.array_equal(rs, rank[order]), name
+    wd = dist[order]
+    assert np.array_equal(np.isinf(ds), np.isinf(wd)), name
+    assert np.array_equal(np.isnan(ds), np.isnan(wd)), name
+    fin = np.isfinite(wd)
+    np.testing.assert_allclose(ds[fin], wd[fin], rtol=1e-4)
+
+
+@pytest.mark.parametrize("n,m", [(32769, 3), (33000, 4), (33024, 5), (36001, 8), (33001, 9), (33000, 10), (32771, 15)])
+@pytest.mark.parametrize("spatial", [True, False])
+def test_totals_against_the_checker(n, m, spatial):
+    x = torch.arange(n, dtype=torch.int32, device=DEV)[:, None]
+    for call, kind in enumerate(["shell", "grid", "alike", "uniform", "nan"]):
+        f = _population("shell" if kind == "nan" else kind, n, m, 7 * n + m + call)
+        if kind == "nan":
+            f[5, 1] = float("nan")
+        k = n // 40 if kind == "shell" else n // 4
+        with runtime.options(**dict(FORCED, prefix_nearby=2 if spatial else 0)):
+            got = nd_environmental_selection(x, f, k)
+            assert runtime.last_status()["error"] == 0
+        _check(got, c_oracle.select(as_np(f), k), kind)
+    runtime.release_workspaces()
+
+
+def test_a_captured_graph_of_spatial_totals_builds_the_matrix_when_a_replay_needs_it():
+    n, m, k = 36000, 8, 5000
+    g = torch.Generator("cpu").manual_seed(410)
+    wide = torch.rand(n, m, generator=g)
+    deep = torch.rand(n, m, generator=g) + (torch.arange(n) % 64)[:, None].float()
+    want = {"wide": c_oracle.select(as_np(wide), k), "deep": c_oracle.select(as_np(deep), k)}
+    assert int((want["wide"][1] == 0).sum()) >= k > int((want["deep"][1] == 0).sum())
+    x = torch.arange(n, dtype=torch.int32, device=DEV)[:, None]
+    f_static = wide.to(DEV).clone()
+    with runtime.options(**FORCED):
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            nd_environmental_selection(x, f_static, k)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = nd_environmental_selection(x, f_static, k)
+    for name in ("wide", "deep", "deep", "wide", "deep"):
+        print("replay:", name, flush=True)
+        f_static.copy_((wide if name == "wide" else deep).to(DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        nd_environmental_selection(x, wide.to(DEV), k)  # eager work between the replays
+        torch.cuda.synchronize()
+        _check(got, want[name], name)
+    del graph
     runtime.release_workspaces()
