@@ -89,6 +89,11 @@ def _translate(name, text):
         b = text.index(': "memory");', a) + len(': "memory");')
         where = re.search(r': "v"\((.*?)\)\s*: "memory"', text[a:b], re.S)[1]
         text = text[:a] + f"emu_load_pair(r0, {where}); emu_load_pair(r1, {where} + 2);" + text[b:]
+    if name == "two_small.hpp":  # (a wave clears its counters and counts its items row by row in lockstep, without a barrier)
+        text = _replaced(text, "cnt[wave * 256 + lane + 64 * i] = 0u;\n", "cnt[wave * 256 + lane + 64 * i] = 0u;\n  (void)emu_ballot(true);\n")
+        text = _replaced(text, "reinterpret_cast<uint4*>(table)[2 * lane + 1] = zero;\n",
+                         "reinterpret_cast<uint4*>(table)[2 * lane + 1] = zero;\n    (void)emu_ballot(true);\n")
+        text = _replaced(text, "if (e - lane >= count) continue;", "if (e - lane >= count) continue; (void)emu_ballot(true);")
     if name == "api.hip":
         text = _replaced(text, "static size_t align_up(size_t v) { return (v + 255) / 256 * 256; }",
                          "static size_t align_up(size_t v) { if (!emu_gaps_on) return (v + 255) / 256 * 256; "

@@ -1,7 +1,8 @@
-#include <unistd.h>
 // calls [-o name=value]... kind:n:m:data[:populations][:rows kept][:repeats][:poisoned] ...
 // Calls of the library on the emulated device, each against the C checker.  The workspace starts out filled with a pattern
 // and is used by one call after the other, as a program does.  poisoned: a wait of the call runs out, its results say so.
+#include <unistd.h>
+
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -45,7 +46,7 @@ static uint8_t* workspace(size_t need) {
   return ws;
 }
 static double now() { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
-#define DIE(...) do { fprintf(stderr, __VA_ARGS__); fprintf(stderr, "\n"); exit(1); } while (0)
+#define DIE(...) do { fprintf(stderr, __VA_ARGS__); fprintf(stderr, "\n"); fflush(stdout); _exit(1); } while (0)
 int main(int argc, char** argv) {
   for (int a = 1; a < argc; ++a) {
     std::string s = argv[a];
