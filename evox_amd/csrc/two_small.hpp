@@ -7,17 +7,29 @@
 // or equal and that are not copies of it, so front r is the set of strict prefix minima of f2 among the rows that
 // fronts 0 .. r-1 have left (two.hpp does the same across workgroups for large populations).  Two objectives mean
 // many thin fronts (C2: 20 fronts of 100 rows), which cost the matrix kernels an exchange between workgroups each;
-// here a front is one prefix minimum over registers, sixteen wave results through LDS and one barrier.
+// here a front is one prefix minimum over the registers of four waves, which hand it on from wave to wave.
 //
-// Everything is a stable LSD radix sort of (32-bit key, 16-bit payload) pairs in LDS, eight bits a pass:
-//   * the order of (f1, f2, index): four passes on the key of f1 (ordered_key, common.hpp) where no two rows share an
-//     f1, else four on the key of f2 and four on that of f1;
-//   * the listing of the fronts by (rank, index): one or two passes on the ranks;
-//   * the last front: its rows by each objective for the crowding distances and by the distance for the index-stable
-//     top-k -- by counting while it has at most 1024 rows, by the radix sort above.
-// A pass ranks the items of a wave among those of equal digit with eight ballots a row of 64 items (stable, no
-// atomics), keeps a counter per (digit, wave) and scans the 4096 counters once.
+// The orders:
+//   * (f1, f2, index): by buckets (two_small_place): a monotone map of f1 to 4096 buckets, LDS counters, and every row
+//     compared with the rows of its own bucket in full -- one pass, whatever ties there are, as long as no bucket is
+//     crowded; else a stable LSD radix sort of (32-bit key, 16-bit payload) pairs, eight bits a pass, on f2 and then f1;
+//   * the listing of the fronts by (rank, index): one or two passes of that sort on the ranks;
+//   * the last front by either objective: its rows already stand in the order of f1, which backwards is that of f2;
+//   * its order by the distance, for the index-stable top-k: by counting while it is small, by buckets, else by the sort.
+// A pass of the sort ranks the items of a wave among those of equal digit through a table of lane masks (stable), keeps
+// a counter per (digit, wave) and scans the 4096 counters once.
+//
+// What bounds it: chains of dependent instructions and LDS round trips inside one workgroup; of 2000 uniform rows the
+// rounds of the peeling 20 us of 34, the order of (f1, f2) 5.5, the listing 3, the gather 3.  us per selection of half the
+// rows (30 values each), in a loop of calls, with a hash table for shared f1, four or eight passes of the sort for the
+// first order, sixteen waves with a barrier per front and the last front by counting or three sorts -> like this:
+//   rows                        200          1024         2000         4096
+//   uniform                     24.4 -> 15   38 -> 26     63.5 -> 37   112 -> 62
+//   twenty fronts, shared f1    26.4 -> 15.6 34.6 -> 22   45 -> 28.3   71 -> 48
+//   one front                   22.8 -> 14.8 88 -> 19.4   59.5 -> 26   99 -> 43
 #pragma once
+
+#include <type_traits>
 
 #include "batched.hpp"
 #include "peel.hpp"
@@ -33,7 +45,11 @@ namespace evx {
 constexpr int kTwoSmallThreads = 1024;
 constexpr int kTwoSmallRows = 4096;
 constexpr int kTwoSmallPer = kTwoSmallRows / kTwoSmallThreads;  // items of a thread in every pass
-constexpr int kTwoSmallCounting = 1024;  // last fronts of at most this many rows are ordered by counting
+constexpr int kTwoSmallBuckets = 4096;   // of two_small_place: four counters per thread
+constexpr uint32_t kTwoSmallCrowd = 64;  // rows of a bucket up to which every row of it looks at every other one
+constexpr int kTwoSmallCounting = 192;   // last fronts of at most this many rows are ordered by counting, larger ones by buckets
+constexpr int kTwoSmallWaves = 4;        // waves that peel: one per SIMD of the compute unit
+constexpr int kTwoSmallRing = 64;        // rounds that a wave may be ahead of the next one
 constexpr uint16_t kTwoSmallUnset = 0xFFFFu;
 // dynamic LDS: keys and payloads of the sort twice over, its counters, the keys of both objectives by row, ranks,
 // the three orders, the distances
@@ -95,6 +111,7 @@ __device__ inline uint32_t max_before_wave(const uint32_t* sixteen, int wave) {
 //      four times the vector instructions);
 //   2. the 4096 counters are scanned in the order (digit, wave), four per thread;
 //   3. the items go to their places.
+template <bool PARTIAL>  // leave out the items whose key is kTwoSmallUnset; the others end up side by side
 __device__ inline void two_small_pass(const uint32_t* key_in, const uint16_t* pay_in, uint32_t* key_out, uint16_t* pay_out,
                                       int count, int shift, uint32_t* cnt, uint32_t* part, uint32_t* lanes_a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -132,7 +149,7 @@ __device__ inline void two_small_pass(const uint32_t* key_in, const uint16_t* pa
     for (int r = 0; r < kTwoSmallPer; ++r) {
       const int e = first + r * 64;
       if (e - lane >= count) continue;  // (wave-uniform: a row without items)
-      if (e < count) {
+      if (e < count && !(PARTIAL && key[r] == kTwoSmallUnset)) {
         const uint32_t d = (key[r] >> shift) & 255u;
         atomicOr(&table[d], 1ull << lane);
         const uint64_t same = table[d];
@@ -174,7 +191,7 @@ __device__ inline void two_small_pass(const uint32_t* key_in, const uint16_t* pa
   if (wave_has_items) {
 #pragma unroll
     for (int r = 0; r < kTwoSmallPer; ++r) {
-      if (first + r * 64 < count) {
+      if (first + r * 64 < count && !(PARTIAL && key[r] == kTwoSmallUnset)) {
         const uint32_t d = (key[r] >> shift) & 255u;
         const int to = (int)cnt[wave * 256 + d] + rin[r];
         key_out[to] = key[r];
@@ -192,9 +209,10 @@ __device__ inline void two_small_pass(const uint32_t* key_in, const uint16_t* pa
 // that take few values, such as counts or multiples of a step, leave the low bits of their float32 images alike.
 __device__ inline void two_small_sort(uint32_t*& key_a, uint16_t*& pay_a, uint32_t*& key_b, uint16_t*& pay_b, int count, int passes,
                                       uint32_t* cnt, uint32_t* part, uint32_t* lanes_a, uint32_t vary = 0xFFFFFFFFu) {
+#pragma unroll 1  // (code that runs once waits for memory at every line of it)
   for (int p = 0; p < passes; ++p) {
     if (((vary >> (8 * p)) & 255u) == 0u) continue;  // (the same in every thread)
-    two_small_pass(key_a, pay_a, key_b, pay_b, count, 8 * p, cnt, part, lanes_a);
+    two_small_pass<false>(key_a, pay_a, key_b, pay_b, count, 8 * p, cnt, part, lanes_a);
     uint32_t* tk = key_a;
     key_a = key_b;
     key_b = tk;
@@ -204,27 +222,215 @@ __device__ inline void two_small_sort(uint32_t*& key_a, uint16_t*& pay_a, uint32
   }
 }
 
+// The smallest and the largest of the workgroup's values (smallest > largest: no thread had any).  lo16, hi16: sixteen words each.
+// Ends with every thread past a barrier; the caller puts another one before lo16 and hi16 are written again.
+__device__ inline void two_small_range(uint32_t& lo, uint32_t& hi, uint32_t* lo16, uint32_t* hi16) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t wave_lo = wave_prefix_min(lo), wave_hi = ~wave_prefix_min(~hi);
+  if (lane == 63) {
+    lo16[wave] = wave_lo;
+    hi16[wave] = wave_hi;
+  }
+  __syncthreads();
+  lo = min_before_wave(lo16, kTwoSmallThreads / 64);
+  hi = max_before_wave(hi16, kTwoSmallThreads / 64);
+}
+
+// Places of `count` items (item tid + 1024 r of thread tid; id below 4096, all different) in the ascending order of
+// (comp, id).  bucket: a map of comp to 0 .. kTwoSmallBuckets - 1 that never decreases as comp grows.  False, with
+// nothing but cnt and part touched, when a bucket holds more than kTwoSmallCrowd items.  twins: some item of this thread shares its comp
+// with another one.  cnt: kTwoSmallBuckets words; part: 16 words; comps, ids: count entries each.  Bound by LDS: an
+// atomic, a scan of four counters per thread and as many reads per item as its bucket has members.
+__device__ inline bool two_small_place(const uint64_t (&comp)[kTwoSmallPer], const uint32_t (&id)[kTwoSmallPer],
+                                       const uint32_t (&bucket)[kTwoSmallPer], int count, uint32_t* cnt, uint32_t* part,
+                                       uint64_t* comps, uint16_t* ids, int (&place)[kTwoSmallPer], bool& twins) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  uint32_t arrived[kTwoSmallPer];
+#pragma unroll
+  for (int r = 0; r < kTwoSmallPer; ++r)
+    arrived[r] = tid + kTwoSmallThreads * r < count ? atomicAdd(&cnt[bucket[r]], 1u) : 0u;
+  __syncthreads();
+  const uint4 mine = reinterpret_cast<const uint4*>(cnt)[tid];
+  const uint32_t sum = mine.x + mine.y + mine.z + mine.w;
+  const uint32_t incl = wave_prefix_sum(sum);
+  if (lane == 63) part[wave] = incl;
+  const bool crowded = max(max(mine.x, mine.y), max(mine.z, mine.w)) > kTwoSmallCrowd;
+  if (__syncthreads_or(crowded)) return false;
+  const uint32_t run = incl - sum + sum_before_wave(part, wave);
+  reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(run, run + mine.x, run + mine.x + mine.y, run + mine.x + mine.y + mine.z);
+  __syncthreads();
+  uint32_t first[kTwoSmallPer], end[kTwoSmallPer];
+#pragma unroll
+  for (int r = 0; r < kTwoSmallPer; ++r) {
+    first[r] = end[r] = 0u;
+    if (tid + kTwoSmallThreads * r < count) {
+      first[r] = cnt[bucket[r]];
+      end[r] = bucket[r] + 1u < (uint32_t)kTwoSmallBuckets ? cnt[bucket[r] + 1u] : (uint32_t)count;
+      comps[first[r] + arrived[r]] = comp[r];
+      ids[first[r] + arrived[r]] = (uint16_t)id[r];
+    }
+  }
+  __syncthreads();
+  twins = false;
+#pragma unroll
+  for (int r = 0; r < kTwoSmallPer; ++r) {
+    int before = 0;
+    for (uint32_t q = first[r]; q < end[r]; q += 4) {  // (four members' reads in flight together)
+      uint64_t other[4];
+      uint32_t other_id[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t at = min(q + (uint32_t)u, end[r] - 1u);
+        other[u] = comps[at];
+        other_id[u] = q + (uint32_t)u < end[r] ? (uint32_t)ids[at] : id[r];  // (the item itself counts for nothing)
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool another = other_id[u] != id[r];
+        before += another && (other[u] < comp[r] || (other[u] == comp[r] && other_id[u] < id[r])) ? 1 : 0;
+        twins |= another && other[u] == comp[r];
+      }
+    }
+    place[r] = (int)first[r] + before;
+  }
+  return true;
+}
+
+// ---- The peeling.  Wave w < waves holds positions 64 PER w .. 64 PER (w + 1) - 1 of the (f1, f2, index) order, PER
+// consecutive ones per lane; val holds f2 (kTwoNone for what is out of the sweep).  In round r a wave needs the smallest
+// f2 of front r among the positions before its own, and tells the next wave the smallest up to its end: the waves go
+// through the rounds one after the other, none waits for a later one but to keep kTwoSmallRing rounds of messages.  A
+// message also carries how many rows the rounds before it have ranked, so the last wave sees the end a round late and
+// raises `ended`; rounds that earlier waves went through by then count for nothing (their ranks lie above the last front's).
+// Four waves, one per SIMD, because a round is bound by instruction issue: sixteen waves of a quarter of the positions
+// spend sixteen issue slots on each of the seven steps of the prefix minimum.  Sixteen positions per lane above 2048 rows, eight
+// below (2000 uniform rows: 20 us with four waves of eight, 22 with two of sixteen), four up to 256 (one wave, no messages).
+struct TwoSmallPeel {
+  unsigned long long ring[kTwoSmallWaves - 1][kTwoSmallRing];  // round + 1 << 48 | rows ranked << 32 | smallest f2
+  int progress[kTwoSmallWaves];                                 // rounds whose message wave w has taken
+  int ended;                                                    // 1 + the round of the last front, 0: not known yet
+  int total, nv;                                                // rows ranked up to the last front, rows in it
+};
+
+template <int PER, bool COPIES>  // COPIES: some row has copies, counted at the first one's position (the other instance reads no count)
+__device__ __forceinline__ void two_small_rounds(const uint32_t* val, const uint32_t* copies, uint16_t* rank_at, int n, int waves,
+                                                 int ranked_already, int stop, TwoSmallPeel* st) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // (known to be uniform: the branches below are scalar)
+  const bool first_wave = wave == 0, last_wave = wave == waves - 1;
+  auto word = [](const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+  const int at = (wave * 64 + lane) * PER;
+  uint32_t v[PER];
+  int ranked[PER], group[PER];  // group: a row and its copies
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    v[e] = at + e < n ? val[at + e] : kTwoNone;
+    group[e] = COPIES && at + e < n ? 1 + (int)copies[at + e] : 1;
+    ranked[e] = kTwoSmallUnset;
+  }
+  auto message = [&](int round) {
+    return first_wave ? 0ull : __hip_atomic_load(&st->ring[wave - 1][round % kTwoSmallRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  unsigned long long in = message(0);
+  int own = 0, before_last = 0;  // rows ranked by this wave so far; (last wave) by all waves before the last round
+  for (int round = 0;; ++round) {
+    int over = last_wave ? 0 : word(&st->ended);  // (asked for early)
+    uint32_t before[PER];  // smallest of the lane's own earlier positions (so that no step below waits for the one before it)
+    before[0] = kTwoNone;
+#pragma unroll
+    for (int e = 1; e < PER; ++e) before[e] = min(before[e - 1], v[e - 1]);
+    const uint32_t incl = wave_prefix_min(min(before[PER - 1], v[PER - 1]));
+    uint32_t running = (uint32_t)__builtin_amdgcn_update_dpp((int)kTwoNone, (int)incl, 0x138, 0xf, 0xf, false);  // wave_shr:1
+    uint32_t lowest = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    int total = own;
+    over = __builtin_amdgcn_readfirstlane(over);
+    if (!first_wave) {
+      // (the wave before never waits for this one's round; it leaves without a message only once `ended` is set)
+      uint32_t in_lo, in_hi;
+      for (;;) {
+        in_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)in);
+        in_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(in >> 32));
+        if ((in_hi >> 16) == (uint32_t)round + 1u || over != 0) break;
+        in = message(round);
+        const int now_over = last_wave ? 0 : word(&st->ended);
+        over |= __builtin_amdgcn_readfirstlane(now_over);
+      }
+      in = message(round + 1);  // (the next one: it may be there when this round is over)
+      running = min(running, in_lo);
+      lowest = min(lowest, in_lo);
+      total += (int)(in_hi & 0xFFFFu);
+      if (lane == 0) __hip_atomic_store(&st->progress[wave], round + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (!last_wave) {
+      if (round >= kTwoSmallRing && round % (kTwoSmallRing / 2) == 0) {
+        // room for the next half ring: the next wave has taken what lies there
+        int taken;
+        do {
+          const int p = word(&st->progress[wave + 1]), now_over = word(&st->ended);
+          taken = __builtin_amdgcn_readfirstlane(p);
+          over |= __builtin_amdgcn_readfirstlane(now_over);
+        } while (taken < round - kTwoSmallRing / 2 && over == 0);
+      }
+      if (over != 0) break;
+      if (lane == 0)
+        __hip_atomic_store(&st->ring[wave][round % kTwoSmallRing],
+                           ((unsigned long long)(((uint32_t)round + 1u) << 16 | (uint32_t)total) << 32) | lowest, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else if (round > 0) {
+      total += ranked_already;  // (rows with a NaN: front 0)
+      if (total >= stop) {      // reached at the latest when every row is ranked
+        if (lane == 0) {
+          st->total = total;
+          st->nv = total - before_last;
+          __hip_atomic_store(&st->ended, round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        break;
+      }
+      before_last = total;
+    }
+    int add = 0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const uint32_t mine = v[e];
+      const bool now = mine < min(running, before[e]);  // (a row out of the sweep holds kTwoNone, which is below nothing)
+      ranked[e] = now ? round : ranked[e];
+      v[e] = now ? kTwoNone : mine;
+      if constexpr (COPIES)
+        add += now ? group[e] : 0;
+      else
+        add += __popcll(__builtin_amdgcn_ballot_w64(now));
+    }
+    own += COPIES ? wave_sum(add) : add;
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e)
+    if (at + e < n) rank_at[at + e] = (uint16_t)ranked[e];
+}
+
 // Grid: one workgroup of kTwoSmallThreads per population; dynamic LDS kTwoSmallLdsBytes.  a.m == 2, a.n <= kTwoSmallRows.
 __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t two_small_lds[];
-  __shared__ __attribute__((aligned(16))) uint32_t wave_min[2][16];
+  __shared__ TwoSmallPeel peel[1];
   __shared__ __attribute__((aligned(16))) uint32_t part[16];
-  __shared__ uint32_t round_count[3];
-  __shared__ uint32_t vary_bits[2];  // bits in which the keys of f1 / of f2 differ from those of row 0
-  __shared__ __attribute__((aligned(16))) uint32_t wave_first[16];
-  uint32_t* key_a = reinterpret_cast<uint32_t*>(two_small_lds);
+  __shared__ __attribute__((aligned(16))) uint32_t lo16[16];
+  __shared__ __attribute__((aligned(16))) uint32_t hi16[16];
+  __shared__ uint32_t vary_bits[2];  // (radix path) bits in which the keys of f1 / of f2 differ from those of row 0
+  __shared__ int nan_rows_lds[1];
+  uint32_t* key_a = reinterpret_cast<uint32_t*>(two_small_lds);  // the sort's buffers
   uint32_t* key_b = key_a + kTwoSmallRows;
   uint16_t* pay_a = reinterpret_cast<uint16_t*>(key_b + kTwoSmallRows);
   uint16_t* pay_b = pay_a + kTwoSmallRows;
   uint32_t* cnt = reinterpret_cast<uint32_t*>(pay_b + kTwoSmallRows);
-  uint32_t* k1 = cnt + kTwoSmallRows;  // ordered keys of the objectives by row
+  uint32_t* k1 = cnt + kTwoSmallRows;  // ordered keys of the objectives by position of the (f1, f2, index) order
   uint32_t* k2 = k1 + kTwoSmallRows;
-  float* dist = reinterpret_cast<float*>(k2 + kTwoSmallRows);  // by position of the output; before that:
+  float* dist = reinterpret_cast<float*>(k2 + kTwoSmallRows);  // of the last front's rows, by row; before that:
   uint32_t* lanes_a = reinterpret_cast<uint32_t*>(dist);       // the lane masks of the sort's first eight waves
-  uint16_t* rank16 = reinterpret_cast<uint16_t*>(dist + kTwoSmallRows);  // by row
-  uint16_t* lexi = rank16 + kTwoSmallRows;   // row at every position of the (f1, f2, index) order
-  uint16_t* perm = lexi + kTwoSmallRows;     // rows by (rank, index)
-  uint16_t* order = perm + kTwoSmallRows;    // the selection order
+  uint16_t* rank16 = reinterpret_cast<uint16_t*>(dist + kTwoSmallRows);  // ranks by position
+  uint16_t* lexi = rank16 + kTwoSmallRows;     // row at every position
+  uint16_t* first_at = lexi + kTwoSmallRows;   // position of the first copy of the row at every position (where there are copies)
+  uint16_t* other16 = first_at + kTwoSmallRows;
 
   const int n = a.n;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -232,44 +438,80 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
   auto fitness_at = [&](int i, int k) {
     return f[(int64_t)i * a.f_stride_row + (int64_t)k * a.f_stride_col + (i >= a.n_first ? a.f_second : 0)];
   };
+  constexpr uint32_t kNanKey = 0xFFFFFFFFu;  // (ordered_key)
 
   EVX_BATCH_TRACE(0);
-  // ---- keys, and the order of (f1, f2, index).  Where no two rows share their f1 -- the rule for objectives that are
-  // computed, not counted -- the rows by (f1, index) are that order: four passes; else the rows by (f2, index) and
-  // then, stably, by f1: eight.  Whether two rows share an f1 is asked of a hash table (8192 words in the buffers that
-  // the sort does not use yet: open addressing, a row that meets its own key in the table has found a twin).
-  bool twin = false;
+  // ---- keys, and the order of (f1, f2, index)
+  bool has_copies = false;
   {
-    uint32_t* const seen = key_b;  // key_b, pay_a, pay_b: 32 KB in a row
-    constexpr uint32_t kEmpty = 0xFFFFFFFFu;
-    for (int i = tid; i < 2 * kTwoSmallRows / 4; i += kTwoSmallThreads)
-      reinterpret_cast<uint4*>(seen)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
-    int nan_f1 = 0;
-    uint32_t mine1[kTwoSmallPer], mine2[kTwoSmallPer];
-    if (tid < 2) vary_bits[tid] = 0u;
+    uint32_t a1[kTwoSmallPer], a2[kTwoSmallPer], id[kTwoSmallPer], bucket[kTwoSmallPer];
+    uint64_t comp[kTwoSmallPer];
+    int place[kTwoSmallPer];
+    uint32_t lo = 0xFFFFFFFFu, hi = 0u;  // of the finite values of f1
+    const uint32_t key_inf = ordered_key(INFINITY), key_neg_inf = ordered_key(-INFINITY);
 #pragma unroll
     for (int r = 0; r < kTwoSmallPer; ++r) {
       const int i = tid + kTwoSmallThreads * r;
-      mine1[r] = kEmpty;
-      mine2[r] = kEmpty;
+      a1[r] = a2[r] = 0u;
       if (i < n) {
-        const uint32_t a1 = ordered_key(fitness_at(i, 0)), a2 = ordered_key(fitness_at(i, 1));
-        k1[i] = a1;
-        k2[i] = a2;
-        mine1[r] = a1;
-        mine2[r] = a2;
-        nan_f1 += a1 == kEmpty ? 1 : 0;  // (the key of a NaN is the table's mark for a free word: counted instead)
+        a1[r] = ordered_key(fitness_at(i, 0));
+        a2[r] = ordered_key(fitness_at(i, 1));
+      }
+      id[r] = (uint32_t)i;
+      comp[r] = ((uint64_t)a1[r] << 32) | a2[r];
+      if (i < n && a1[r] > key_neg_inf && a1[r] < key_inf) {
+        lo = min(lo, a1[r]);
+        hi = max(hi, a1[r]);
       }
     }
-    __syncthreads();
-    {
-      const uint32_t ref1 = k1[0], ref2 = k2[0];
+    if (tid == 0) {
+      nan_rows_lds[0] = 0;
+      peel->ended = 0;
+    }
+    if (tid < kTwoSmallWaves) peel->progress[tid] = 0;
+    if (tid < (kTwoSmallWaves - 1) * kTwoSmallRing) (&peel->ring[0][0])[tid] = 0ull;
+    two_small_range(lo, hi, lo16, hi16);
+    // Buckets of equal width in the value of f1 first, then in its image (values over many binades): no row of f1 may lie
+    // in a lower bucket than one with a smaller f1, which holds however the differences and products round; a width of
+    // zero or one that overflows puts all finite values into one bucket, a NaN always lies in the last.
+    bool ordered = false;
+#pragma unroll 1
+    for (int attempt = 0; attempt < 2 && !ordered; ++attempt) {
+      const float v0 = cost_of_key(lo), width = cost_of_key(hi) - v0;
+      const float image_scale = lo < hi ? (float)(kTwoSmallBuckets - 3) / (float)(hi - lo) : 0.0f;
+      const float value_scale = lo < hi && width > 0.0f ? (float)(kTwoSmallBuckets - 1) / width : 0.0f;
+#pragma unroll
+      for (int r = 0; r < kTwoSmallPer; ++r) {
+        if (attempt == 0) {
+          const float t = (cost_of_key(a1[r]) - v0) * value_scale;
+          bucket[r] = a1[r] == kNanKey || t >= (float)(kTwoSmallBuckets - 1) ? kTwoSmallBuckets - 1 : t > 0.0f ? (uint32_t)t : 0u;
+        } else {
+          bucket[r] = a1[r] < lo ? 0u : a1[r] > hi ? kTwoSmallBuckets - 1 : 1u + min((uint32_t)((float)(a1[r] - lo) * image_scale), (uint32_t)kTwoSmallBuckets - 3u);
+        }
+      }
+      ordered = two_small_place(comp, id, bucket, n, cnt, part, reinterpret_cast<uint64_t*>(key_a), pay_a, place, has_copies);
+    }
+    EVX_BATCH_TRACE(1);
+    if (!ordered) {  // (the same in every thread) many rows share an f1
+      __syncthreads();
+      if (tid < 2) vary_bits[tid] = 0u;
+#pragma unroll
+      for (int r = 0; r < kTwoSmallPer; ++r) {
+        const int i = tid + kTwoSmallThreads * r;
+        if (i < n) {
+          k1[i] = a1[r];
+          k2[i] = a2[r];
+          key_a[i] = a2[r];
+          pay_a[i] = (uint16_t)i;
+        }
+      }
+      __syncthreads();
       uint32_t v1 = 0u, v2 = 0u;
 #pragma unroll
       for (int r = 0; r < kTwoSmallPer; ++r) {
         if (tid + kTwoSmallThreads * r < n) {
-          v1 |= mine1[r] ^ ref1;
-          v2 |= mine2[r] ^ ref2;
+          v1 |= a1[r] ^ k1[0];
+          v2 |= a2[r] ^ k2[0];
         }
       }
 #pragma unroll
@@ -281,356 +523,346 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
         if (v1) atomicOr(&vary_bits[0], v1);
         if (v2) atomicOr(&vary_bits[1], v2);
       }
+      __syncthreads();
+      two_small_sort(key_a, pay_a, key_b, pay_b, n, 4, cnt, part, lanes_a, vary_bits[1]);
+      for (int s = tid; s < n; s += kTwoSmallThreads) key_a[s] = k1[pay_a[s]];
+      __syncthreads();
+      two_small_sort(key_a, pay_a, key_b, pay_b, n, 4, cnt, part, lanes_a, vary_bits[0]);
+      // by position: every thread takes what it moves out of the arrays by row before any of it is written
+#pragma unroll
+      for (int r = 0; r < kTwoSmallPer; ++r) {
+        const int s = tid + kTwoSmallThreads * r;
+        if (s < n) {
+          id[r] = pay_a[s];
+          a1[r] = k1[id[r]];
+          a2[r] = k2[id[r]];
+          place[r] = s;
+        }
+      }
+      key_a = reinterpret_cast<uint32_t*>(two_small_lds);
+      key_b = key_a + kTwoSmallRows;
+      pay_a = reinterpret_cast<uint16_t*>(key_b + kTwoSmallRows);
+      pay_b = pay_a + kTwoSmallRows;
+      has_copies = true;  // (asked below)
+      __syncthreads();
     }
+    int nan_rows = 0;
 #pragma unroll
     for (int r = 0; r < kTwoSmallPer; ++r) {
-      if (mine1[r] == kEmpty) continue;
-      uint32_t at = (mine1[r] * 2654435761u) >> 19;  // 13 bits
-      for (int probe = 0; probe < 2 * kTwoSmallRows; ++probe) {
-        const uint32_t old = atomicCAS(&seen[at], kEmpty, mine1[r]);
-        if (old == kEmpty) break;
-        if (old == mine1[r]) {
-          twin = true;
-          break;
-        }
-        at = (at + 1u) & (2u * kTwoSmallRows - 1u);
+      if (tid + kTwoSmallThreads * r < n) {
+        k1[place[r]] = a1[r];
+        k2[place[r]] = a2[r];
+        lexi[place[r]] = (uint16_t)id[r];
+        nan_rows += a1[r] == kNanKey || a2[r] == kNanKey ? 1 : 0;
       }
     }
-    nan_f1 = wave_sum(nan_f1);
-    if (lane == 0) part[wave] = (uint32_t)nan_f1;
-    twin = __syncthreads_or(twin) != 0;
-    twin |= sum_before_wave(part, 16) > 1u;
+    if (nan_rows != 0) atomicAdd(&nan_rows_lds[0], nan_rows);
+    has_copies = __syncthreads_or(has_copies) != 0;
   }
-  for (int i = tid; i < n; i += kTwoSmallThreads) {
-    key_a[i] = twin ? k2[i] : k1[i];
-    pay_a[i] = (uint16_t)i;
-  }
-  __syncthreads();
-  EVX_BATCH_TRACE(1);
-  two_small_sort(key_a, pay_a, key_b, pay_b, n, 4, cnt, part, lanes_a, vary_bits[twin ? 1 : 0]);
   EVX_BATCH_TRACE(2);
-  if (twin) {
-    for (int s = tid; s < n; s += kTwoSmallThreads) key_a[s] = k1[pay_a[s]];
-    __syncthreads();
-    two_small_sort(key_a, pay_a, key_b, pay_b, n, 4, cnt, part, lanes_a, vary_bits[0]);
-  }
-  for (int s = tid; s < n; s += kTwoSmallThreads) lexi[s] = pay_a[s];
-  __syncthreads();
-  EVX_BATCH_TRACE(3);
+  const int nan_rows = nan_rows_lds[0];
 
-  // ---- the peeling.  A thread holds four consecutive positions of the order.  Out of the sweep: rows with a NaN
-  // (nothing compares with them: front 0) and the copies of a row (they take the rank of the first copy, which
-  // counts for all of them).  During the peeling the buffers of the sort hold: key_b = copies per first row,
-  // pay_b = rank by position.
-  uint32_t* copies = key_b;
-  uint16_t* rank_at = pay_b;
-  uint32_t v[kTwoSmallPer];
-  int first_of[kTwoSmallPer];   // position of the first copy (the position itself for a first row)
-  bool is_nan[kTwoSmallPer], is_copy[kTwoSmallPer];
-  uint32_t last_first = 0u;     // 1 + the last position of this thread that is not a copy, 0 = none
-  int nan_rows = 0;
+  // ---- out of the sweep: rows with a NaN (nothing compares with them: front 0) and the copies of a row (they take
+  // the rank of the first copy, which counts for all of them)
+  uint32_t* copies = cnt;           // per position of a first row
+  uint32_t* val = k2;
+  if (nan_rows != 0 || has_copies) {
+    val = key_a;
+    uint32_t last_first = 0u;  // 1 + the last position of this thread that is not a copy, 0 = none
+    bool is_copy[kTwoSmallPer];
 #pragma unroll
-  for (int e = 0; e < kTwoSmallPer; ++e) {
-    const int s = kTwoSmallPer * tid + e;
-    v[e] = kTwoNone;
-    is_nan[e] = false;
-    is_copy[e] = false;
-    first_of[e] = s;
-    if (s < n) {
-      const int row = lexi[s];
-      const uint32_t a1 = k1[row], a2 = k2[row];
-      is_nan[e] = a1 == 0xFFFFFFFFu || a2 == 0xFFFFFFFFu;
-      if (!is_nan[e] && s > 0) {
-        const int before = lexi[s - 1];
-        is_copy[e] = k1[before] == a1 && k2[before] == a2;
+    for (int e = 0; e < kTwoSmallPer; ++e) {
+      const int s = kTwoSmallPer * tid + e;
+      is_copy[e] = false;
+      if (s < n) {
+        const uint32_t a1 = k1[s], a2 = k2[s];
+        const bool is_nan = a1 == kNanKey || a2 == kNanKey;
+        is_copy[e] = !is_nan && s > 0 && k1[s - 1] == a1 && k2[s - 1] == a2;
+        val[s] = is_nan || is_copy[e] ? kTwoNone : a2;
+        if (!is_copy[e]) last_first = (uint32_t)s + 1u;
+        copies[s] = 0u;
       }
-      if (!is_nan[e] && !is_copy[e]) v[e] = a2;
-      if (!is_copy[e]) last_first = (uint32_t)s + 1u;
-      nan_rows += is_nan[e] ? 1 : 0;
-      copies[s] = 0u;
     }
-  }
-  {
     // the first copy of a copy: the last position before it that is not one (a prefix maximum)
     const uint32_t incl = ~wave_prefix_min(~last_first);
     const uint32_t excl = ~(uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFFu, (int)~incl, 0x138, 0xf, 0xf, false);  // wave_shr:1
-    if (lane == 63) wave_first[wave] = incl;
-    if (tid < 3) round_count[tid] = 0u;
+    if (lane == 63) hi16[wave] = incl;
     __syncthreads();
-    uint32_t carry = max(excl, max_before_wave(wave_first, wave));
+    uint32_t carry = max(excl, max_before_wave(hi16, wave));
 #pragma unroll
     for (int e = 0; e < kTwoSmallPer; ++e) {
       const int s = kTwoSmallPer * tid + e;
       if (s < n) {
         if (!is_copy[e]) carry = (uint32_t)s + 1u;
-        first_of[e] = (int)carry - 1;  // (a copy always has a first row before it)
-        if (is_copy[e]) atomicAdd(&copies[first_of[e]], 1u);
+        first_at[s] = (uint16_t)(carry - 1u);  // (a copy always has a first row before it)
+        if (is_copy[e]) atomicAdd(&copies[carry - 1u], 1u);
       }
     }
-    nan_rows = (int)wave_sum(nan_rows);
-    if (lane == 0 && nan_rows != 0) atomicAdd(&round_count[0], (uint32_t)nan_rows);
+    __syncthreads();
   }
+  EVX_BATCH_TRACE(3);
   const int stop = a.stop_count;
-  EVX_BATCH_TRACE(4);
-  int group[kTwoSmallPer];       // a first row and its copies
-  uint16_t ranked[kTwoSmallPer];  // (in registers: a round must not wait for LDS more often than it has to)
-#pragma unroll
-  for (int e = 0; e < kTwoSmallPer; ++e) {
-    group[e] = 1;
-    ranked[e] = is_nan[e] ? (uint16_t)0 : kTwoSmallUnset;
+  {
+    const int per = n <= 64 * 4 ? 4 : n <= 64 * kTwoSmallWaves * 8 ? 8 : 16;
+    const int waves = (n + 64 * per - 1) / (64 * per);
+    auto rounds = [&](auto positions) {
+      if (has_copies)
+        two_small_rounds<decltype(positions)::value, true>(val, copies, rank16, n, waves, nan_rows, stop, peel);
+      else
+        two_small_rounds<decltype(positions)::value, false>(val, copies, rank16, n, waves, nan_rows, stop, peel);
+    };
+    if (wave < waves) {
+      if (per == 4)
+        rounds(std::integral_constant<int, 4>());
+      else if (per == 8)
+        rounds(std::integral_constant<int, 8>());
+      else
+        rounds(std::integral_constant<int, 16>());
+    }
+    __syncthreads();
   }
-  int total = 0, worst = 0, nv = 0;
-  // A wave all of whose rows are ranked (or that never had any) only keeps the barriers and the count of the rounds
-  // company: sixteen waves share the compute unit's four vector units, and what one of them does not issue the others
-  // issue sooner.
-  bool wave_live = true;     // (wave-uniform)
-  bool wave_copies = false;  // some first row of this wave has copies: the rows of a round are then added, not counted
-  for (int round = 0;; ++round) {
-    uint32_t running = kTwoNone;
-    if (wave_live) {
-      uint32_t tmin = kTwoNone;
-#pragma unroll
-      for (int e = 0; e < kTwoSmallPer; ++e) tmin = min(tmin, v[e]);
-      const uint32_t incl = wave_prefix_min(tmin);
-      running = (uint32_t)__builtin_amdgcn_update_dpp((int)kTwoNone, (int)incl, 0x138, 0xf, 0xf, false);  // wave_shr:1
-      if (lane == 63) wave_min[round & 1][wave] = incl;
-    } else if (lane == 63) {
-      wave_min[round & 1][wave] = kTwoNone;  // (not earlier: the round before may still be reading the other word)
-    }
-    if (round == 2) EVX_PASS_TRACE(11);
-    __syncthreads();  // (the first one also completes the copies' counts)
-    if (round == 2) EVX_PASS_TRACE(12);
-    if (round == 0) {
-      bool any = false;
-#pragma unroll
-      for (int e = 0; e < kTwoSmallPer; ++e)
-        if (kTwoSmallPer * tid + e < n) {
-          group[e] = 1 + (int)copies[kTwoSmallPer * tid + e];
-          any |= group[e] > 1;
-        }
-      wave_copies = __builtin_amdgcn_ballot_w64(any) != 0ull;
-    }
-    // (the counter of the next round: last read after the barrier before this one)
-    if (tid == 0) round_count[(round + 1) % 3] = 0u;
-    if (round > 0) {
-      const int size = (int)round_count[(round - 1) % 3];
-      total += size;
-      if (size == 0 || total >= stop) {
-        worst = round - 1;
-        nv = size;
-        break;
-      }
-    }
-    if (!wave_live) continue;
-    running = min(running, min_before_wave(wave_min[round & 1], wave));
-    if (round == 2) EVX_PASS_TRACE(13);
-    int add = 0;
-    bool left = false;
-    bool now[kTwoSmallPer];
-#pragma unroll
-    for (int e = 0; e < kTwoSmallPer; ++e) {
-      const uint32_t mine = v[e];
-      now[e] = mine < running;  // (a row out of the sweep holds kTwoNone, which is below nothing)
-      running = min(running, mine);
-      if (now[e]) {
-        ranked[e] = (uint16_t)round;
-        v[e] = kTwoNone;
-      }
-      left |= v[e] != kTwoNone;
-    }
-    if (round == 2) EVX_PASS_TRACE(14);
-    if (wave_copies) {
-#pragma unroll
-      for (int e = 0; e < kTwoSmallPer; ++e) add += now[e] ? group[e] : 0;
-      add = wave_sum(add);
-    } else {
-#pragma unroll
-      for (int e = 0; e < kTwoSmallPer; ++e) add += __popcll(__builtin_amdgcn_ballot_w64(now[e]));
-    }
-    if (lane == 0 && add != 0) atomicAdd(&round_count[round % 3], (uint32_t)add);
-    wave_live = __builtin_amdgcn_ballot_w64(left) != 0ull;
-    if (round == 2) EVX_PASS_TRACE(15);
-  }
+  const int worst = peel->ended - 1, total = peel->total, nv = peel->nv;
   const int worst_start = total - nv;
-  EVX_BATCH_TRACE(5);
-#pragma unroll
-  for (int e = 0; e < kTwoSmallPer; ++e)
-    if (kTwoSmallPer * tid + e < n) rank_at[kTwoSmallPer * tid + e] = ranked[e];
-  __syncthreads();
-  // ranks by row: the copies take that of their first row
+  EVX_BATCH_TRACE(4);
+
+  // ---- ranks by row into the sort's first buffer, and the rows of the last front put together in the order of (f1, f2, index)
+  const bool selecting = a.out_f != nullptr;
+  const bool by_value = !(worst == 0 && nan_rows != 0);  // (a last front with NaN rows is ordered by sorting below)
+  int members = 0;
+  uint32_t rank_of[kTwoSmallPer], m1[kTwoSmallPer], m2[kTwoSmallPer], m_row[kTwoSmallPer], m_first[kTwoSmallPer];
 #pragma unroll
   for (int e = 0; e < kTwoSmallPer; ++e) {
     const int s = kTwoSmallPer * tid + e;
-    if (s < n) rank16[lexi[s]] = rank_at[first_of[e]];
-  }
-  __syncthreads();
-  if (a.rank_all)
-    for (int i = tid; i < n; i += kTwoSmallThreads)
-      a.rank_all[(int64_t)blockIdx.x * n + i] = rank16[i] == kTwoSmallUnset ? kRankUnset : (int)rank16[i];
-  if (a.out_f == nullptr) return;  // rank-only mode
-
-  EVX_BATCH_TRACE(6);
-  // ---- the rows by (rank, index): the rows are in index order, the sort is stable (the rows not ranked come last)
-  key_a = reinterpret_cast<uint32_t*>(two_small_lds);
-  key_b = key_a + kTwoSmallRows;
-  pay_a = reinterpret_cast<uint16_t*>(key_b + kTwoSmallRows);
-  pay_b = pay_a + kTwoSmallRows;
-  for (int i = tid; i < n; i += kTwoSmallThreads) {
-    key_a[i] = rank16[i];
-    pay_a[i] = (uint16_t)i;
-  }
-  __syncthreads();
-  two_small_sort(key_a, pay_a, key_b, pay_b, n, worst < 255 ? 1 : 2, cnt, part, lanes_a);
-  for (int p = tid; p < n; p += kTwoSmallThreads) perm[p] = pay_a[p];
-  __syncthreads();
-
-  // ---- crowding distances of the last front (candidate q = perm[worst_start + q], in index order) and the order
-  // by (distance descending, index): non_dominate.py:209-231 with the mask rank == worst, :253
-  const int need = stop - worst_start;
-  EVX_BATCH_TRACE(7);
-  auto better_fronts = [&]() {  // (the distances share their LDS with the sort: only once the last sort is over)
-    for (int p = tid; p < stop; p += kTwoSmallThreads) {
-      dist[p] = -INFINITY;
-      if (p < worst_start) order[p] = perm[p];
+    rank_of[e] = kTwoSmallUnset;
+    if (s < n) {
+      m1[e] = k1[s];
+      m2[e] = k2[s];
+      m_row[e] = lexi[s];
+      m_first[e] = has_copies ? (uint32_t)first_at[s] : (uint32_t)s;
+      rank_of[e] = nan_rows != 0 && (m1[e] == kNanKey || m2[e] == kNanKey) ? 0u : (uint32_t)rank16[m_first[e]];
+      if (rank_of[e] > (uint32_t)worst) rank_of[e] = kTwoSmallUnset;  // (not ranked, or in a round after the last front's)
+      members += rank_of[e] == (uint32_t)worst ? 1 : 0;
     }
-    __syncthreads();
-  };
-  if (nv <= kTwoSmallCounting) {
-    better_fronts();
-    // by counting: thread q is candidate q; tile and below lie in the sort's buffers
-    uint64_t* tile = reinterpret_cast<uint64_t*>(two_small_lds);                   // nv + 4 entries
-    float* scost = reinterpret_cast<float*>(tile + (kTwoSmallCounting + 4));       // by position
-    int* below = reinterpret_cast<int*>(scost + kTwoSmallCounting);
-    const bool cand = tid < nv;
-    const int row = cand ? perm[worst_start + tid] : 0;
-    bool boundary = false;
-    float acc = 0.0f;
+  }
+  const uint32_t members_incl = wave_prefix_sum((uint32_t)members);
+  if (lane == 63) part[wave] = members_incl;
+  if (a.rank_all) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const uint32_t ck = cand ? (k == 0 ? k1[row] : k2[row]) : 0u;
-      __syncthreads();
-      if (tid < nv + 4) tile[tid] = cand ? ((uint64_t)ck << 32) | (uint32_t)tid : ~0ull;
-      if (tid < 4 && nv + tid >= kTwoSmallThreads) tile[nv + tid] = ~0ull;
-      const int p = position_by_counting(tile, below, nv, tid, kTwoSmallThreads);
-      if (cand) scost[p] = cost_of_key(ck);
-      __syncthreads();
-      if (cand) {
-        if (p == 0 || p == nv - 1) {
-          boundary = true;
-        } else {
-          const float term = (scost[p + 1] - scost[p - 1]) / (scost[nv - 1] - scost[0]);
-          acc = k == 0 ? term : acc + term;
+    for (int e = 0; e < kTwoSmallPer; ++e)
+      if (kTwoSmallPer * tid + e < n)
+        a.rank_all[(int64_t)blockIdx.x * n + m_row[e]] = rank_of[e] == kTwoSmallUnset ? kRankUnset : (int)rank_of[e];
+  }
+  if (!selecting) return;  // rank-only mode
+  __syncthreads();         // (also: every read of key_a as `val` is over, and every read of k1, k2, lexi and first_at)
+  {
+    uint32_t to = members_incl - (uint32_t)members + sum_before_wave(part, wave);
+#pragma unroll
+    for (int e = 0; e < kTwoSmallPer; ++e) {
+      const int s = kTwoSmallPer * tid + e;
+      if (s < n) {
+        key_a[m_row[e]] = rank_of[e];
+        pay_a[m_row[e]] = (uint16_t)m_row[e];
+        if (rank_of[e] == (uint32_t)worst) {
+          k1[to] = m1[e];
+          k2[to] = m2[e];
+          lexi[to] = (uint16_t)m_row[e];
+          if (has_copies) {  // how many copies stand before this one, and how many there are
+            first_at[to] = (uint16_t)((uint32_t)s - m_first[e]);
+            other16[to] = (uint16_t)(1u + copies[m_first[e]]);
+          }
+          ++to;
         }
       }
     }
-    const float d = boundary ? INFINITY : acc;
     __syncthreads();
-    if (tid < nv + 4) tile[tid] = cand ? ((uint64_t)ordered_key(-d) << 32) | (uint32_t)tid : ~0ull;
-    if (tid < 4 && nv + tid >= kTwoSmallThreads) tile[nv + tid] = ~0ull;
-    const int p = position_by_counting(tile, below, nv, tid, kTwoSmallThreads);
-    if (cand && p < need) {
-      order[worst_start + p] = (uint16_t)row;
-      dist[worst_start + p] = d;
-    }
-  } else {
-    // by the radix sort: a thread has candidates q = tid + 1024 r; scost (by position) and pos (by candidate) lie
-    // in the counters' neighbours k-independent: scost in `dist`'s tail is not free, so they take the copy buffers
-    float acc[kTwoSmallPer];
-    bool boundary[kTwoSmallPer];
+  }
+  EVX_BATCH_TRACE(5);
+
+  // ---- distances of the last front: crowding_distance with the mask rank == worst, non_dominate.py:209-231.  Its rows,
+  // leaving copies aside, stand in the ascending order of f1 and in the descending one of f2 (of two rows that share
+  // either, one dominates the other); copies stand by index, in both orders.
+  const int need = stop - worst_start;
+  uint32_t d_row[kTwoSmallPer];
+  float d_of[kTwoSmallPer];
+  if (by_value) {
+    const float span1 = cost_of_key(k1[nv - 1]) - cost_of_key(k1[0]);
+    const float span2 = cost_of_key(k2[0]) - cost_of_key(k2[nv - 1]);
 #pragma unroll
     for (int r = 0; r < kTwoSmallPer; ++r) {
-      acc[r] = 0.0f;
-      boundary[r] = false;
-    }
-    for (int k = 0; k < 2; ++k) {
-      key_a = reinterpret_cast<uint32_t*>(two_small_lds);
-      key_b = key_a + kTwoSmallRows;
-      pay_a = reinterpret_cast<uint16_t*>(key_b + kTwoSmallRows);
-      pay_b = pay_a + kTwoSmallRows;
-      for (int q = tid; q < nv; q += kTwoSmallThreads) {
-        const int row = perm[worst_start + q];
-        key_a[q] = k == 0 ? k1[row] : k2[row];
-        pay_a[q] = (uint16_t)q;
+      const int p = tid + kTwoSmallThreads * r;
+      d_row[r] = 0u;
+      d_of[r] = 0.0f;
+      if (p < nv) {
+        const int before = has_copies ? first_at[p] : 0, group = has_copies ? other16[p] : 1;
+        const int q = nv - (p - before) - group + before;  // position in the order of f2
+        d_row[r] = lexi[p];
+        if (p == 0 || p == nv - 1 || q == 0 || q == nv - 1) {
+          d_of[r] = INFINITY;
+        } else {
+          d_of[r] = (cost_of_key(k1[p + 1]) - cost_of_key(k1[p - 1])) / span1;
+          d_of[r] += (cost_of_key(k2[nv - 2 - q]) - cost_of_key(k2[nv - q])) / span2;
+        }
       }
-      __syncthreads();
-      two_small_sort(key_a, pay_a, key_b, pay_b, nv, 4, cnt, part, lanes_a);  // four passes: the result is where it started
-      // position of every candidate: into the other payload buffer
-      for (int p = tid; p < nv; p += kTwoSmallThreads) pay_b[pay_a[p]] = (uint16_t)p;
-      __syncthreads();
-      const float span = cost_of_key(key_a[nv - 1]) - cost_of_key(key_a[0]);
+    }
+    __syncthreads();  // (cnt, as `copies`, and k1, k2 are free from here on)
+  }
+
+  // ---- the ranked rows by (rank, index): the rows are in index order, a pass of the sort is stable
+  two_small_pass<true>(key_a, pay_a, key_b, pay_b, n, 0, cnt, part, lanes_a);
+  uint32_t* listed_rank = key_b;  // rank and row at every position of the listing
+  uint16_t* listed = pay_b;
+  if (worst >= 255) {
+    two_small_pass<false>(key_b, pay_b, key_a, pay_a, total, 8, cnt, part, lanes_a);
+    listed_rank = key_a;
+    listed = pay_a;
+  }
+  uint32_t* const free32 = worst >= 255 ? key_b : key_a;  // the buffers of the sort that hold nothing now
+  uint16_t* const free16 = worst >= 255 ? pay_b : pay_a;
+  uint64_t* const comps = reinterpret_cast<uint64_t*>(k1);  // (k1 and k2)
+  EVX_BATCH_TRACE(6);
+
+  // ---- the order of the last front by (distance descending, index), non_dominate.py:253, into the listing: nobody reads
+  // its rows there any more except where they are taken from it first
+  if (by_value && nv <= kTwoSmallCounting) {
+    uint64_t* tile = comps;  // nv + 4 entries
+    int* below = reinterpret_cast<int*>(cnt);
+    const bool cand = tid < nv;
+    if (tid < nv + 4) tile[tid] = cand ? ((uint64_t)ordered_key(-d_of[0]) << 32) | d_row[0] : ~0ull;
+    const int p = position_by_counting(tile, below, nv, tid, kTwoSmallThreads);
+    if (cand) dist[d_row[0]] = d_of[0];
+    if (cand && p < need) listed[worst_start + p] = (uint16_t)d_row[0];
+  } else {
+    bool placed = false;
+    if (by_value) {
+      uint64_t comp[kTwoSmallPer];
+      uint32_t bucket[kTwoSmallPer];
+      int place[kTwoSmallPer];
+      uint32_t lo = 0xFFFFFFFFu, hi = 0u;  // keys of the finite distances
+      const uint32_t key_neg_inf = ordered_key(-INFINITY);
 #pragma unroll
       for (int r = 0; r < kTwoSmallPer; ++r) {
-        const int q = tid + kTwoSmallThreads * r;
-        if (q < nv) {
-          const int p = pay_b[q];
-          if (p == 0 || p == nv - 1) {
-            boundary[r] = true;
-          } else {
-            const float term = (cost_of_key(key_a[p + 1]) - cost_of_key(key_a[p - 1])) / span;
-            acc[r] = k == 0 ? term : acc[r] + term;
+        const uint32_t key = ordered_key(-d_of[r]);
+        comp[r] = key;
+        if (tid + kTwoSmallThreads * r < nv && key != key_neg_inf && key != kNanKey) {
+          lo = min(lo, key);
+          hi = max(hi, key);
+        }
+      }
+      two_small_range(lo, hi, lo16, hi16);
+      const float scale = lo < hi ? (float)(kTwoSmallBuckets - 3) / (float)(hi - lo) : 0.0f;
+#pragma unroll
+      for (int r = 0; r < kTwoSmallPer; ++r) {
+        const uint32_t key = (uint32_t)comp[r];
+        bucket[r] = key < lo ? 0u : key > hi ? kTwoSmallBuckets - 1 : 1u + min((uint32_t)((float)(key - lo) * scale), (uint32_t)kTwoSmallBuckets - 3u);
+      }
+      bool twins;
+      placed = two_small_place(comp, d_row, bucket, nv, cnt, part, comps, lexi, place, twins);
+      if (placed) {
+#pragma unroll
+        for (int r = 0; r < kTwoSmallPer; ++r) {
+          if (tid + kTwoSmallThreads * r < nv) {
+            dist[d_row[r]] = d_of[r];
+            if (place[r] < need) listed[worst_start + place[r]] = (uint16_t)d_row[r];
           }
         }
       }
+    }
+    if (!placed) {
+      // by the radix sort, candidate q = listed[worst_start + q] (in index order): many equal distances, or rows with a NaN.
+      // d_by_row shares nothing with the sort's lane masks, which lie in k1 here.
+      uint32_t* sk_a = free32;
+      uint32_t* sk_b = k2;
+      uint16_t* sp_a = free16;
+      uint16_t* sp_b = first_at;
+      uint32_t* const masks = k1;
       __syncthreads();
-    }
-    key_a = reinterpret_cast<uint32_t*>(two_small_lds);
-    key_b = key_a + kTwoSmallRows;
-    pay_a = reinterpret_cast<uint16_t*>(key_b + kTwoSmallRows);
-    pay_b = pay_a + kTwoSmallRows;
-    float* d_of = reinterpret_cast<float*>(cnt + kTwoSmallRows);  // (= k1: no longer needed once the keys below are built)
-    float d_mine[kTwoSmallPer];
+      if (by_value) {
 #pragma unroll
-    for (int r = 0; r < kTwoSmallPer; ++r) d_mine[r] = boundary[r] ? INFINITY : acc[r];
-    __syncthreads();
+        for (int r = 0; r < kTwoSmallPer; ++r)
+          if (tid + kTwoSmallThreads * r < nv) dist[d_row[r]] = d_of[r];
+      } else {
+        float acc[kTwoSmallPer];
+        bool boundary[kTwoSmallPer];
 #pragma unroll
-    for (int r = 0; r < kTwoSmallPer; ++r) {
-      const int q = tid + kTwoSmallThreads * r;
-      if (q < nv) {
-        key_a[q] = ordered_key(-d_mine[r]);
-        pay_a[q] = (uint16_t)q;
-        d_of[q] = d_mine[r];
+        for (int r = 0; r < kTwoSmallPer; ++r) {
+          acc[r] = 0.0f;
+          boundary[r] = false;
+        }
+#pragma unroll 1
+        for (int k = 0; k < 2; ++k) {
+          sk_a = free32;
+          sk_b = k2;
+          sp_a = free16;
+          sp_b = first_at;
+          for (int q = tid; q < nv; q += kTwoSmallThreads) {
+            sk_a[q] = ordered_key(fitness_at(listed[worst_start + q], k));
+            sp_a[q] = (uint16_t)q;
+          }
+          __syncthreads();
+          two_small_sort(sk_a, sp_a, sk_b, sp_b, nv, 4, cnt, part, masks);
+          for (int p = tid; p < nv; p += kTwoSmallThreads) other16[sp_a[p]] = (uint16_t)p;  // position of every candidate
+          __syncthreads();
+          const float span = cost_of_key(sk_a[nv - 1]) - cost_of_key(sk_a[0]);
+#pragma unroll
+          for (int r = 0; r < kTwoSmallPer; ++r) {
+            const int q = tid + kTwoSmallThreads * r;
+            if (q < nv) {
+              const int p = other16[q];
+              if (p == 0 || p == nv - 1) {
+                boundary[r] = true;
+              } else {
+                const float term = (cost_of_key(sk_a[p + 1]) - cost_of_key(sk_a[p - 1])) / span;
+                acc[r] = k == 0 ? term : acc[r] + term;
+              }
+            }
+          }
+          __syncthreads();
+        }
+#pragma unroll
+        for (int r = 0; r < kTwoSmallPer; ++r) {
+          const int q = tid + kTwoSmallThreads * r;
+          if (q < nv) dist[listed[worst_start + q]] = boundary[r] ? INFINITY : acc[r];
+        }
       }
-    }
-    __syncthreads();
-    two_small_sort(key_a, pay_a, key_b, pay_b, nv, 4, cnt, part, lanes_a);
-    better_fronts();
-    for (int p = tid; p < need; p += kTwoSmallThreads) {
-      const int q = pay_a[p];
-      order[worst_start + p] = perm[worst_start + q];
-      dist[worst_start + p] = d_of[q];
+      __syncthreads();
+      sk_a = free32;
+      sk_b = k2;
+      sp_a = free16;
+      sp_b = first_at;
+      for (int q = tid; q < nv; q += kTwoSmallThreads) {
+        const int row = listed[worst_start + q];
+        sk_a[q] = ordered_key(-dist[row]);
+        sp_a[q] = (uint16_t)row;
+      }
+      __syncthreads();
+      two_small_sort(sk_a, sp_a, sk_b, sp_b, nv, 4, cnt, part, masks);
+      for (int p = tid; p < need; p += kTwoSmallThreads) listed[worst_start + p] = sp_a[p];
     }
   }
   __syncthreads();
-  EVX_BATCH_TRACE(8);
+  EVX_BATCH_TRACE(7);
 
   // ---- the selected rows
   const int topk = stop;
   const int64_t ob = (int64_t)blockIdx.x * topk;
   for (int p = tid; p < topk; p += kTwoSmallThreads) {
-    const int src = order[p];
-    a.out_rank[ob + p] = (int)rank16[src];
-    a.out_dist[ob + p] = dist[p];
-    a.out_f[(ob + p) * 2] = fitness_at(src, 0);
-    a.out_f[(ob + p) * 2 + 1] = fitness_at(src, 1);
+    const int src = listed[p];
+    const float f1 = fitness_at(src, 0), f2 = fitness_at(src, 1);
+    a.out_rank[ob + p] = p < worst_start ? (int)listed_rank[p] : worst;
+    a.out_dist[ob + p] = p < worst_start ? -INFINITY : dist[src];
+    a.out_f[(ob + p) * 2] = f1;
+    a.out_f[(ob + p) * 2 + 1] = f2;
   }
+  EVX_BATCH_TRACE(8);
   if (a.x != nullptr) {
     const uint8_t* __restrict__ xb = a.x + (int64_t)blockIdx.x * a.x_stride_b;
     uint8_t* __restrict__ dst = a.out_x + ob * a.x_row_bytes;
-    const int64_t row_units = a.x_row_bytes / a.x_unit;
-    const int64_t units = row_units * topk;
-    if (a.x_unit >= 4 && units < (1ll << 31)) {
-      if (a.x_unit == 16)
-        gather_units<uint4>(xb, dst, order, a.x_row_stride, (uint32_t)row_units, (uint32_t)units, tid, kTwoSmallThreads, a.n_first,
-                            a.x_second);
-      else
-        gather_units<uint32_t>(xb, dst, order, a.x_row_stride, (uint32_t)row_units, (uint32_t)units, tid, kTwoSmallThreads,
-                               a.n_first, a.x_second);
-    } else {
+    if (!gather_whole_units(a, xb, dst, listed, topk, tid, kTwoSmallThreads)) {
       for (int p = wave; p < topk; p += kTwoSmallThreads / 64) {
-        const int src = order[p];
+        const int src = listed[p];
         const uint8_t* __restrict__ sp = xb + (int64_t)src * a.x_row_stride + (src >= a.n_first ? a.x_second : 0);
         uint8_t* __restrict__ dp = dst + (int64_t)p * a.x_row_bytes;
-        if (a.x_unit == 4) {
+        if (a.x_unit >= 4) {
           for (int64_t b = lane * 4; b < a.x_row_bytes; b += 64 * 4)
             *reinterpret_cast<uint32_t*>(dp + b) = *reinterpret_cast<const uint32_t*>(sp + b);
         } else {

@@ -120,3 +120,36 @@ def test_limits_and_the_switch():
     f = torch.rand(4097, 2).to(DEV)
     assert not runtime.small_population_kernel_fits(4097, 2, 1)
     assert np.array_equal(as_np(non_dominate_rank(f)), as_np(er.ranks_by_peeling(f.cpu())))
+
+
+def _crowded(kind, n, seed):
+    """Populations on either side of the choices inside the kernel: how f1 is spread decides between buckets of equal width,
+    buckets of its image and the radix sort; the last front's distances between counting, buckets and the sort."""
+    g = torch.Generator("cpu").manual_seed(seed)
+    f = torch.rand(n, 2, generator=g)
+    if kind == "decades":  # f1 over forty decades and both signs
+        f[:, 0] = torch.pow(10.0, 40.0 * f[:, 0] - 20.0) * torch.where(f[:, 1] < 0.5, -1.0, 1.0)
+    elif kind == "few":  # hundreds of rows share an f1
+        f[:, 0] = (f[:, 0] * 6).floor()
+    elif kind == "spaced":  # one front, all inner distances equal
+        f[:, 0] = torch.randperm(n, generator=g).float()
+        f[:, 1] = float(n) - f[:, 0]
+    elif kind == "twice":  # one front, every row there twice (and some NaN rows of the same front)
+        f[:, 0] = torch.randperm(n, generator=g).div(2, rounding_mode="floor").float()
+        f[:, 1] = -f[:, 0].sqrt()
+    elif kind == "nan front":
+        f[:, 1] = 1.0 - f[:, 0]
+        f[:: 7, 0] = float("nan")
+    elif kind == "outlier":  # an infinity and a huge value beside values close together
+        f[0, 0], f[1, 0] = float("inf"), 3.0e38
+        f[2, 0] = -float("inf")
+    return f, torch.arange(n, dtype=torch.float32)[:, None].repeat(1, 2)
+
+
+@pytest.mark.parametrize("kind", ["uniform", "decades", "few", "spaced", "twice", "nan front", "outlier"])
+@pytest.mark.parametrize("n", [129, 192, 193, 256, 257, 2048, 2049])
+def test_around_the_choices_inside_the_kernel(kind, n):
+    f, x = _crowded(kind, n, 7 * n)
+    assert np.array_equal(as_np(non_dominate_rank(f.to(DEV))), as_np(er.ranks_by_peeling(f)))
+    for topk in (n // 2, n):
+        _same_selection(nd_environmental_selection(x.to(DEV), f.to(DEV), topk), er.environmental_selection(x, f, topk), (kind, n, topk))
