@@ -29,6 +29,7 @@
 #include "stepped.hpp"
 #include "two.hpp"
 #include "two_small.hpp"
+#include "few.hpp"
 #include "wide.hpp"
 
 namespace evx {
@@ -46,6 +47,8 @@ struct Options {
                             // and the last front is ordered likewise; 0: only where the persistent grids cannot be resident
   int64_t two_small_min_rows = 128;  // populations of two objectives and at least this many rows (at most 4096) that go to a
                                    // one-workgroup kernel take the one without a matrix (two_small.hpp); 0 = never
+  int64_t few_max_rows = kFewRows;  // populations of three to eight objectives and at most this many rows that reach the entry points
+                                    // with a workspace: matrix by the whole device, the rest by one workgroup (few.hpp); 0 = never
   int64_t two_min_rows = 4097;  // populations of two objectives and at least this many rows are ranked without a matrix (two.hpp); 0 = never
   int64_t two_min_rows_partial = 4097;  // ... when the ranking may stop at the front that holds a given row (measured, us per
                                         // selection of half the rows, without / with a matrix: 5000 rows 110 / 178, 20 000 rows
@@ -1443,7 +1446,31 @@ static int64_t batched_rows_limit(int64_t m) {
   return m == 2 && opt().two_small_min_rows > 0 ? kTwoSmallRows : kBatchedMaxRows;
 }
 
+// Few populations of at most 256 rows and three to eight objectives: sixteen waves each (few.hpp).
+template <int M>
+static int launch_few_whole_m(const BatchedArgs& a, int batch, hipStream_t s) {
+  const int groups = (a.n + 63) / 64;
+  const int nt = groups * 2 * groups * 64 < kFewRows ? groups * 2 * groups * 64 : kFewRows;  // (a wave per group and half word)
+  const size_t lds = few_whole_lds_bytes(nt, a.n, M);
+  if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(few_whole_kernel<M>), lds)) return e;
+  hipLaunchKernelGGL(few_whole_kernel<M>, dim3(batch), dim3(nt), lds, s, a);
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+static int launch_few_whole(const BatchedArgs& a, int batch, hipStream_t s) {
+  switch (a.m) {
+    case 3: return launch_few_whole_m<3>(a, batch, s);
+    case 4: return launch_few_whole_m<4>(a, batch, s);
+    case 5: return launch_few_whole_m<5>(a, batch, s);
+    case 6: return launch_few_whole_m<6>(a, batch, s);
+    case 7: return launch_few_whole_m<7>(a, batch, s);
+    default: return launch_few_whole_m<8>(a, batch, s);
+  }
+}
+
 static int launch_batched(const BatchedArgs& a, int64_t batch, hipStream_t s) {
+  if (a.m >= 3 && a.m <= kFewObjectives && a.n <= kFewWholeRows && batch <= device_cus() && opt().few_max_rows > 0)
+    return launch_few_whole(a, (int)batch, s);
   if (a.m == 2 && opt().two_small_min_rows > 0 && (a.n >= opt().two_small_min_rows || a.n > kBatchedMaxRows))
     return launch_two_small(a, batch, s);
   switch (a.m) {
@@ -1471,6 +1498,9 @@ static int launch_batched(const BatchedArgs& a, int64_t batch, hipStream_t s) {
 
 using namespace evx;
 
+constexpr int kFewBatch = 64;  // populations that share those launches at most
+static bool few_applies(const Layout& L, const Fitness& fit, int batch);
+static int stage_few(const Ws& w, const Fitness& fit, BatchedArgs a, hipStream_t s);
 static bool two_applies(const Layout& L, int64_t stop_count);
 static int many_two_share(const Layout& L, int64_t batch, int64_t stop_count);
 static int stage_rank_two(const Ws& w, const Fitness& src, int64_t stop_count, bool fill_dist, int* rank_until, hipStream_t s);
@@ -1531,6 +1561,8 @@ static int set_named(Options& o, const char* name, int64_t value) {
     o.launch_memory = (int)value;
   } else if (!strcmp(name, "peel_stepped") && (value == 0 || value == 1)) {
     o.peel_stepped = (int)value;
+  } else if (!strcmp(name, "few_max_rows") && value >= 0 && value <= kFewRows) {
+    o.few_max_rows = value;
   } else if (!strcmp(name, "two_small_min_rows") && value >= 0) {
     o.two_small_min_rows = value;
   } else if (!strcmp(name, "two_min_rows") && value >= 0) {
@@ -1669,6 +1701,12 @@ static int rank_rows(const Fitness& fit, int64_t n, int64_t m, int64_t stop_coun
     if (ws_step < (int64_t)w.L.total || (ws_step & 255) != 0 || ws_bytes < (size_t)ws_step * (size_t)batch) return kErrWorkspace;
     w.batch = batch;
     w.step = ws_step;
+  }
+  if (few_applies(w.L, fit, batch)) {
+    BatchedArgs a = {};
+    a.stop_count = (int)stop_count;
+    a.rank_all = rank_out;
+    return stage_few(w, fit, a, s);
   }
   if (batch == 1 ? two_applies(w.L, stop_count) : many_two_share(w.L, batch, stop_count) >= batch) {
     int* until = stop_count < n ? w.at<int>(w.L.order) : (int*)nullptr;
@@ -2434,6 +2472,47 @@ static int stage_rank_two(const Ws& w, const Fitness& src, int64_t stop_count, b
   return 0;
 }
 
+// Populations that two launches take (few.hpp): all whose rows fit the threads of one workgroup (against the pipeline, us
+// per selection of half the rows: 300 x 3 37 -> 17, 1000 x 3 45 -> 21, 1000 x 5 47 -> 31, 1000 x 8 82 -> 47; all ranks of 1000 x 3
+// 64 -> 23), unless a tunable asks for a kernel of the pipeline.  The two parts of a population must have equal strides.
+static bool few_applies(const Layout& L, const Fitness& fit, int batch) {
+  if (L.n > opt().few_max_rows || L.m < 3 || L.m > kFewObjectives || batch > kFewBatch) return false;
+  const Options usual;
+  if (opt().peel_stepped || !opt().peel_lds || !opt().peel_records || !opt().peel_witness || !opt().peel_tail || !opt().tail_merged ||
+      !opt().small_sort || !opt().dominance_folded || opt().dominance_tile_words || opt().peel_lds_blocks || opt().peel_record_blocks ||
+      opt().spin_limit != usual.spin_limit)
+    return false;
+  return fit.n_first >= L.n || (fit.sr == fit.sr2 && fit.sc == fit.sc2 && ((fit.f2 - fit.f) * (int64_t)sizeof(float) == (const char*)fit.f2 - (const char*)fit.f));
+}
+static int stage_few(const Ws& w, const Fitness& fit, BatchedArgs a, hipStream_t s) {
+  const Layout& L = w.L;
+  a.f = fit.f;
+  a.f_stride_b = fit.step;
+  a.f_stride_row = fit.sr;
+  a.f_stride_col = fit.sc;
+  a.n = L.n;
+  a.m = L.m;
+  a.n_first = (int)(fit.n_first < L.n ? fit.n_first : L.n);
+  a.f_second = fit.n_first < L.n ? (fit.f2 - fit.f) - fit.n_first * fit.sr : 0;
+  const int nt = (int)round_up(L.n, 64);
+  const dim3 grid(nt / 64, (nt + 127) / 128, w.batch);
+  uint64_t* const words = w.at<uint64_t>(L.dom);
+  switch (L.m) {
+    case 3: hipLaunchKernelGGL(few_dominance_kernel<3>, grid, dim3(256), 0, s, a, words, w.step); break;
+    case 4: hipLaunchKernelGGL(few_dominance_kernel<4>, grid, dim3(256), 0, s, a, words, w.step); break;
+    case 5: hipLaunchKernelGGL(few_dominance_kernel<5>, grid, dim3(256), 0, s, a, words, w.step); break;
+    case 6: hipLaunchKernelGGL(few_dominance_kernel<6>, grid, dim3(256), 0, s, a, words, w.step); break;
+    case 7: hipLaunchKernelGGL(few_dominance_kernel<7>, grid, dim3(256), 0, s, a, words, w.step); break;
+    default: hipLaunchKernelGGL(few_dominance_kernel<8>, grid, dim3(256), 0, s, a, words, w.step); break;
+  }
+  EVX_LAUNCH_CHECK();
+  const size_t lds = few_finish_lds_bytes(nt, L.n, L.m);
+  if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(few_finish_kernel), lds)) return e;
+  hipLaunchKernelGGL(few_finish_kernel, dim3(w.batch), dim3(nt), lds, s, a, words, w.ctrl(), w.step);
+  EVX_LAUNCH_CHECK();
+  return 0;
+}
+
 // Shared body of the two selection entry points: the population is one part or two.
 static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_bytes, const void* x2,
                        int64_t x2_row_stride_bytes, const Fitness& fit, int64_t n, int64_t m, int64_t topk, void* out_x,
@@ -2461,6 +2540,21 @@ static int select_rows(const void* x, int64_t x_row_bytes, int64_t x_row_stride_
                            (uintptr_t)x_row_bytes | (uintptr_t)x_row_stride_bytes | (uintptr_t)x2_row_stride_bytes |
                            (uintptr_t)x_step_bytes | (uintptr_t)x2_step_bytes;
     unit = (bits % 16 == 0) ? 16 : (bits % 4 == 0) ? 4 : 1;
+  }
+  if (out_order == nullptr && few_applies(L, fit, batch) && (x == x2 || x_row_stride_bytes == x2_row_stride_bytes) && x_step_bytes == x2_step_bytes) {
+    BatchedArgs a = {};
+    a.stop_count = (int)topk;
+    a.x = static_cast<const uint8_t*>(x);
+    a.x_stride_b = x_step_bytes;
+    a.x_row_stride = x_row_stride_bytes;
+    a.x_row_bytes = x_row_bytes;
+    a.x_unit = unit;
+    if (fit.n_first < n) a.x_second = (static_cast<const uint8_t*>(x2) - static_cast<const uint8_t*>(x)) - fit.n_first * x_row_stride_bytes;
+    a.out_x = static_cast<uint8_t*>(out_x);
+    a.out_f = out_f;
+    a.out_rank = out_rank;
+    a.out_dist = out_dist;
+    return stage_few(w, fit, a, s);
   }
   GatherArgs g = {};
   g.order = w.at<int>(L.order);

@@ -224,7 +224,7 @@ __device__ inline void two_small_sort(uint32_t*& key_a, uint16_t*& pay_a, uint32
 
 // The smallest and the largest of the workgroup's values (smallest > largest: no thread had any).  lo16, hi16: sixteen words each.
 // Ends with every thread past a barrier; the caller puts another one before lo16 and hi16 are written again.
-__device__ inline void two_small_range(uint32_t& lo, uint32_t& hi, uint32_t* lo16, uint32_t* hi16) {
+__device__ inline void two_small_range(uint32_t& lo, uint32_t& hi, uint32_t* lo16, uint32_t* hi16, int nt) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wave_lo = wave_prefix_min(lo), wave_hi = ~wave_prefix_min(~hi);
   if (lane == 63) {
@@ -232,25 +232,39 @@ __device__ inline void two_small_range(uint32_t& lo, uint32_t& hi, uint32_t* lo1
     hi16[wave] = wave_hi;
   }
   __syncthreads();
-  lo = min_before_wave(lo16, kTwoSmallThreads / 64);
-  hi = max_before_wave(hi16, kTwoSmallThreads / 64);
+  lo = min_before_wave(lo16, nt / 64);
+  hi = max_before_wave(hi16, nt / 64);
 }
 
-// Places of `count` items (item tid + 1024 r of thread tid; id below 4096, all different) in the ascending order of
-// (comp, id).  bucket: a map of comp to 0 .. kTwoSmallBuckets - 1 that never decreases as comp grows.  False, with
+// Buckets 0 .. buckets - 1 for keys (ordered_key) whose finite ones lie between lo and hi: none lower than that of a smaller key,
+// however the differences and products round.  By value: of equal width, everything but NaN in the first one where the width is
+// zero or overflows.  By image: of equal width in the key (values over many binades), infinities in buckets of their own.
+__device__ inline uint32_t bucket_by_value(uint32_t key, uint32_t lo, uint32_t hi, int buckets) {
+  const float v0 = cost_of_key(lo), width = cost_of_key(hi) - v0;
+  const float scale = lo < hi && width > 0.0f ? (float)(buckets - 1) / width : 0.0f;
+  const float t = (cost_of_key(key) - v0) * scale;
+  return key == 0xFFFFFFFFu || t >= (float)(buckets - 1) ? (uint32_t)buckets - 1u : t > 0.0f ? (uint32_t)t : 0u;
+}
+__device__ inline uint32_t bucket_by_image(uint32_t key, uint32_t lo, uint32_t hi, int buckets) {
+  const float scale = lo < hi ? (float)(buckets - 3) / (float)(hi - lo) : 0.0f;
+  return key < lo ? 0u : key > hi ? (uint32_t)buckets - 1u : 1u + min((uint32_t)((float)(key - lo) * scale), (uint32_t)buckets - 3u);
+}
+
+// Places of `count` items (item tid + nt r of thread tid of the nt in the workgroup; id below 65536, all different) in the ascending order of
+// (comp, id).  bucket: a map of comp to 0 .. 4 nt - 1 that never decreases as comp grows.  False, with
 // nothing but cnt and part touched, when a bucket holds more than kTwoSmallCrowd items.  twins: some item of this thread shares its comp
-// with another one.  cnt: kTwoSmallBuckets words; part: 16 words; comps, ids: count entries each.  Bound by LDS: an
+// with another one.  cnt: 4 nt words; part: 16 words; comps, ids: count entries each.  Bound by LDS: an
 // atomic, a scan of four counters per thread and as many reads per item as its bucket has members.
-__device__ inline bool two_small_place(const uint64_t (&comp)[kTwoSmallPer], const uint32_t (&id)[kTwoSmallPer],
-                                       const uint32_t (&bucket)[kTwoSmallPer], int count, uint32_t* cnt, uint32_t* part,
-                                       uint64_t* comps, uint16_t* ids, int (&place)[kTwoSmallPer], bool& twins) {
+template <int PER>
+__device__ inline bool two_small_place(const uint64_t (&comp)[PER], const uint32_t (&id)[PER], const uint32_t (&bucket)[PER], int count,
+                                       int nt, uint32_t* cnt, uint32_t* part, uint64_t* comps, uint16_t* ids, int (&place)[PER], bool& twins) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(0u, 0u, 0u, 0u);
   __syncthreads();
-  uint32_t arrived[kTwoSmallPer];
+  uint32_t arrived[PER];
 #pragma unroll
-  for (int r = 0; r < kTwoSmallPer; ++r)
-    arrived[r] = tid + kTwoSmallThreads * r < count ? atomicAdd(&cnt[bucket[r]], 1u) : 0u;
+  for (int r = 0; r < PER; ++r)
+    arrived[r] = tid + nt * r < count ? atomicAdd(&cnt[bucket[r]], 1u) : 0u;
   __syncthreads();
   const uint4 mine = reinterpret_cast<const uint4*>(cnt)[tid];
   const uint32_t sum = mine.x + mine.y + mine.z + mine.w;
@@ -261,13 +275,13 @@ __device__ inline bool two_small_place(const uint64_t (&comp)[kTwoSmallPer], con
   const uint32_t run = incl - sum + sum_before_wave(part, wave);
   reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(run, run + mine.x, run + mine.x + mine.y, run + mine.x + mine.y + mine.z);
   __syncthreads();
-  uint32_t first[kTwoSmallPer], end[kTwoSmallPer];
+  uint32_t first[PER], end[PER];
 #pragma unroll
-  for (int r = 0; r < kTwoSmallPer; ++r) {
+  for (int r = 0; r < PER; ++r) {
     first[r] = end[r] = 0u;
-    if (tid + kTwoSmallThreads * r < count) {
+    if (tid + nt * r < count) {
       first[r] = cnt[bucket[r]];
-      end[r] = bucket[r] + 1u < (uint32_t)kTwoSmallBuckets ? cnt[bucket[r] + 1u] : (uint32_t)count;
+      end[r] = bucket[r] + 1u < 4u * (uint32_t)nt ? cnt[bucket[r] + 1u] : (uint32_t)count;
       comps[first[r] + arrived[r]] = comp[r];
       ids[first[r] + arrived[r]] = (uint16_t)id[r];
     }
@@ -275,7 +289,7 @@ __device__ inline bool two_small_place(const uint64_t (&comp)[kTwoSmallPer], con
   __syncthreads();
   twins = false;
 #pragma unroll
-  for (int r = 0; r < kTwoSmallPer; ++r) {
+  for (int r = 0; r < PER; ++r) {
     int before = 0;
     for (uint32_t q = first[r]; q < end[r]; q += 4) {  // (four members' reads in flight together)
       uint64_t other[4];
@@ -470,26 +484,14 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
     }
     if (tid < kTwoSmallWaves) peel->progress[tid] = 0;
     if (tid < (kTwoSmallWaves - 1) * kTwoSmallRing) (&peel->ring[0][0])[tid] = 0ull;
-    two_small_range(lo, hi, lo16, hi16);
-    // Buckets of equal width in the value of f1 first, then in its image (values over many binades): no row of f1 may lie
-    // in a lower bucket than one with a smaller f1, which holds however the differences and products round; a width of
-    // zero or one that overflows puts all finite values into one bucket, a NaN always lies in the last.
-    bool ordered = false;
+    two_small_range(lo, hi, lo16, hi16, kTwoSmallThreads);
+    bool ordered = false;  // by buckets of equal width in the value of f1, else in its image
 #pragma unroll 1
     for (int attempt = 0; attempt < 2 && !ordered; ++attempt) {
-      const float v0 = cost_of_key(lo), width = cost_of_key(hi) - v0;
-      const float image_scale = lo < hi ? (float)(kTwoSmallBuckets - 3) / (float)(hi - lo) : 0.0f;
-      const float value_scale = lo < hi && width > 0.0f ? (float)(kTwoSmallBuckets - 1) / width : 0.0f;
 #pragma unroll
-      for (int r = 0; r < kTwoSmallPer; ++r) {
-        if (attempt == 0) {
-          const float t = (cost_of_key(a1[r]) - v0) * value_scale;
-          bucket[r] = a1[r] == kNanKey || t >= (float)(kTwoSmallBuckets - 1) ? kTwoSmallBuckets - 1 : t > 0.0f ? (uint32_t)t : 0u;
-        } else {
-          bucket[r] = a1[r] < lo ? 0u : a1[r] > hi ? kTwoSmallBuckets - 1 : 1u + min((uint32_t)((float)(a1[r] - lo) * image_scale), (uint32_t)kTwoSmallBuckets - 3u);
-        }
-      }
-      ordered = two_small_place(comp, id, bucket, n, cnt, part, reinterpret_cast<uint64_t*>(key_a), pay_a, place, has_copies);
+      for (int r = 0; r < kTwoSmallPer; ++r)
+        bucket[r] = attempt == 0 ? bucket_by_value(a1[r], lo, hi, kTwoSmallBuckets) : bucket_by_image(a1[r], lo, hi, kTwoSmallBuckets);
+      ordered = two_small_place<kTwoSmallPer>(comp, id, bucket, n, kTwoSmallThreads, cnt, part, reinterpret_cast<uint64_t*>(key_a), pay_a, place, has_copies);
     }
     EVX_BATCH_TRACE(1);
     if (!ordered) {  // (the same in every thread) many rows share an f1
@@ -748,15 +750,11 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
           hi = max(hi, key);
         }
       }
-      two_small_range(lo, hi, lo16, hi16);
-      const float scale = lo < hi ? (float)(kTwoSmallBuckets - 3) / (float)(hi - lo) : 0.0f;
+      two_small_range(lo, hi, lo16, hi16, kTwoSmallThreads);
 #pragma unroll
-      for (int r = 0; r < kTwoSmallPer; ++r) {
-        const uint32_t key = (uint32_t)comp[r];
-        bucket[r] = key < lo ? 0u : key > hi ? kTwoSmallBuckets - 1 : 1u + min((uint32_t)((float)(key - lo) * scale), (uint32_t)kTwoSmallBuckets - 3u);
-      }
+      for (int r = 0; r < kTwoSmallPer; ++r) bucket[r] = bucket_by_image((uint32_t)comp[r], lo, hi, kTwoSmallBuckets);
       bool twins;
-      placed = two_small_place(comp, d_row, bucket, nv, cnt, part, comps, lexi, place, twins);
+      placed = two_small_place<kTwoSmallPer>(comp, d_row, bucket, nv, kTwoSmallThreads, cnt, part, comps, lexi, place, twins);
       if (placed) {
 #pragma unroll
         for (int r = 0; r < kTwoSmallPer; ++r) {

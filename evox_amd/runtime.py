@@ -15,14 +15,15 @@ _last: Optional[Tuple[torch.Tensor, int]] = None  # (workspace, stream handle) o
 
 CHECK_STATUS = os.environ.get("EVOX_AMD_CHECK_STATUS", "0") not in ("", "0")
 
-# Populations of at most evox_hip_batched_max_rows(m) rows can run in the one-workgroup-per-population
-# kernel, larger ones need the bit-matrix pipeline.  None = choose by size: a lone population is faster in
-# the pipeline, which spreads it over the whole device, from a size on that shrinks as the objectives grow
-# (measured, one-workgroup kernel against pipeline, in us: 3 objectives 48/75 at 704 rows and 86/81 at 960;
-# 5 objectives 60/71 at 704, 94/80 at 960; 8 objectives 65/68 at 256, 85/76 at 384; 16 objectives 67/77 at 128,
-# 119/101 at 256); two or three populations up to twice that size, and four or more always, take the
-# one-workgroup kernel, which runs them side by side.  True / False force the choice where it is possible
-# (tests use that to drive small inputs through both).
+# Populations of at most evox_hip_batched_max_rows(m) rows can run in the one-workgroup-per-population kernels, larger
+# ones need a workspace.  None = choose by size.  Three to eight objectives: a lone population of more than 256 rows is
+# faster in the two launches whose first one spreads the matrix over the whole device (selection of half the rows,
+# us, one workgroup against two launches: 256 x 3 14 / 17 -- both bound by the host there --, 300 x 3 23 / 17, 500 x 3
+# 29 / 17, 1000 x 3 96 / 21, 256 x 8 33 / 30, 300 x 8 83 / 31); up to 32 populations are from 513 rows on (512 x 3: 28 / 29,
+# 700 x 3: 46 / 29, 1000 x 3: 104 / 29 to 33; 64 of 700: 46 / 47).  Other numbers of objectives: a lone population is faster in the
+# pipeline from a size on that shrinks as the objectives grow (16 objectives 67 / 77 at 128 rows, 119 / 101 at 256), two or
+# three from twice that size on, four or more never.  True / False force the choice where it is possible (tests use that to drive small
+# inputs through both).
 use_small_population_kernel = None
 
 
@@ -55,6 +56,8 @@ def small_population_kernel_fits(n: int, m: int, batch: int) -> bool:
         return False
     if use_small_population_kernel is True:
         return True
+    if 3 <= m <= 8:
+        return n <= 256 or (batch > 1 and (n <= 512 or batch > 32))
     if batch >= 4:
         return True
     return n <= _lone_population_limit(m) * (1 if batch == 1 else 2)
