@@ -20,8 +20,14 @@ def cal_hv(fit: torch.Tensor, ref: torch.Tensor, pop_size, n_sample: int) -> tor
     """Same contract as the reference's ``cal_hv``: ``fit`` (N, M), ``ref`` (M,) reference point, ``pop_size``
     the number of points to be kept, ``n_sample`` uniform samples drawn with ``torch.rand`` on ``fit.device``
     between the per-objective minimum and ``ref`` (a seeded generator gives the reference's samples)."""
-    if type(pop_size) is int and pop_size > 0 and ops.hv_whole_call_fits(fit, ref, n_sample):
-        return ops.hype_contributions(fit, ref, pop_size, torch.rand(n_sample, fit.size(1), device=fit.device))
+    if type(pop_size) is int and pop_size > 0 and ops.plain_eager():
+        with ops.quiet():
+            fits = ops.hv_whole_call_fits(fit, ref, n_sample)
+            m, device = (fit.size(1), fit.device) if fits else (0, None)
+        if fits:
+            u = torch.rand(n_sample, m, device=device)
+            with ops.quiet():
+                return ops.hype_contributions(fit, ref, pop_size, u)
     n, m = fit.size()
     alpha = hv_alpha(n, pop_size, fit.device)
     f_min = torch.min(fit, dim=0).values

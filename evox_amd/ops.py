@@ -24,6 +24,24 @@ from . import _lib, runtime
 _current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
+class _Here:
+    """The device guard of a call on the current device: nothing to change, nothing to put back."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *_):
+        return None
+
+
+_HERE = _Here()
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, which costs 3 us, where the device is not the current one."""
+    return _HERE if device.index is not None and device.index == _current_device() else torch.cuda.device(device)
+
+
 def _batched_first(info, dims, tensors):
     """The tensors of a vmap rule with the mapped dimension in front; those that are not mapped are expanded."""
     out = []
@@ -69,7 +87,7 @@ def _order_preserving_f32(t: torch.Tensor, what: str) -> torch.Tensor:
         # the rest in one kernel: a value opens a new rank when it differs from the one before it, the ranks go back to
         # the rows that the values came from
         dense = torch.empty(flat.size(0), flat.size(2), flat.size(1), dtype=torch.float32, device=t.device)
-        with torch.cuda.device(t.device):
+        with _on(t.device):
             _lib.call("evox_hip_dense_rank_rows", values.data_ptr(), 0 if flat.dtype == torch.float64 else 1, index.data_ptr(),
                       flat.size(0), flat.size(2), flat.size(1), dense.data_ptr(), runtime.stream_handle(t.device))
         return dense.reshape(t.shape)
@@ -130,7 +148,7 @@ def nd_rank(f: torch.Tensor) -> torch.Tensor:
         return out
     if m == 0:
         return out.zero_()
-    with torch.cuda.device(f.device):
+    with _on(f.device):
         flat_f = f32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         if runtime.small_population_kernel_fits(n, m, flat_f.size(0)):
@@ -183,7 +201,7 @@ def nd_rank_until(f: torch.Tensor, count: int) -> torch.Tensor:
     out = torch.empty(f32.shape[:-1], dtype=torch.int32, device=f.device)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(f.device):
+    with _on(f.device):
         _rank_many(f32.reshape(-1, n, m), out.view(-1, n), count)
     return out
 
@@ -213,7 +231,7 @@ def nd_first_front(f: torch.Tensor) -> torch.Tensor:
         return out
     if m == 0:
         return out.fill_(True)
-    with torch.cuda.device(f.device):
+    with _on(f.device):
         flat_f = f32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         stream = runtime.stream_handle(f.device)
@@ -260,7 +278,7 @@ def crowding(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Tensor:
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with torch.cuda.device(costs.device):
+    with _on(costs.device):
         flat_c = c32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
@@ -329,7 +347,7 @@ def crowding_wide(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Te
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with torch.cuda.device(costs.device):
+    with _on(costs.device):
         flat_c = wide.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
@@ -391,7 +409,7 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
         return out_x, out_f, out_rank, out_dist
     if out_rank.numel() == topk and n <= _WIDE_WHOLE_MAX:
         # one population: the whole selection in one call of the library
-        with torch.cuda.device(f.device):
+        with _on(f.device):
             wb = wide.reshape(n, m)
             rows_f = f.reshape(n, m).contiguous()
             rows_x = x.reshape(n, -1).contiguous()
@@ -412,7 +430,7 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
     # the ranks, as far as the front that holds the topk-th row, from the ranking kernels on a float32 image of the
     # fitness that keeps every comparison (the rows behind that front are marked unset)
     rank = nd_rank_until(f, topk)
-    with torch.cuda.device(f.device):
+    with _on(f.device):
         flat_w = wide.reshape(-1, n, m)
         flat_f = f.reshape(-1, n, m).contiguous()
         flat_x = x.reshape(flat_w.size(0), n, -1).contiguous()
@@ -526,7 +544,7 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
     out_dist = torch.empty(*batch, topk, dtype=torch.float32, device=f.device)
     if out_rank.numel() == 0:
         return out_x, out_f.to(f.dtype), out_rank, out_dist
-    with torch.cuda.device(f.device):
+    with _on(f.device):
         flat_f = f32.reshape(-1, n, m)
         flat_x = x.reshape(flat_f.size(0), n, -1)
         if flat_x.stride(-1) != 1 and flat_x.size(-1) > 1:
@@ -633,7 +651,7 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
     out_f = torch.empty(topk, m, dtype=torch.float32, device=f_a.device)
     out_rank = torch.empty(topk, dtype=torch.int32, device=f_a.device)
     out_dist = torch.empty(topk, dtype=torch.float32, device=f_a.device)
-    with torch.cuda.device(f_a.device):
+    with _on(f_a.device):
         width = 1
         for d in tail:
             width *= d
@@ -698,7 +716,7 @@ def stable_argsort_step(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         if prev.dtype != torch.int32 or prev.shape != (n,):
             raise ValueError("prev must be an int32 order of the same length as the key")
         prev = prev.contiguous()
-    with torch.cuda.device(key.device):
+    with _on(key.device):
         ws = runtime.sort_workspace(n, key.device)
         stream = runtime.stream_handle(key.device)
         _lib.call("evox_hip_stable_argsort_step", key.data_ptr(), kind, key.stride(0), n,
@@ -737,7 +755,7 @@ def stable_argsort_rows(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         prev = prev.contiguous()
     if key.stride(0) < 0 or key.stride(1) < 0:
         key = key.contiguous()
-    with torch.cuda.device(key.device):
+    with _on(key.device):
         ws = runtime.sort_workspace(n, key.device)
         stream = runtime.stream_handle(key.device)
         _lib.call("evox_hip_stable_argsort_step_batched", key.data_ptr(), kind, key.stride(0), key.stride(1), batch, n,
@@ -782,7 +800,7 @@ def hv_contributions(fit: torch.Tensor, samples: torch.Tensor, alpha: torch.Tens
     out = torch.zeros(n, dtype=torch.float32, device=fit.device)
     if n == 0 or n_sample == 0 or m == 0:
         return out
-    with torch.cuda.device(fit.device):
+    with _on(fit.device):
         fit_t = _as_f32(fit, "fitness").t().contiguous()
         samples_t = _as_f32(samples, "samples").t().contiguous()
         alpha32 = _as_f32(alpha, "alpha").contiguous()
@@ -821,7 +839,7 @@ def hv_covered_count(points: torch.Tensor, samples: torch.Tensor) -> torch.Tenso
         return out
     if m == 0:  # an empty conjunction holds: every sample is covered (torch.all over an empty dimension)
         return out + n_sample
-    with torch.cuda.device(points.device):
+    with _on(points.device):
         points_t = _as_f32(points, "points").t().contiguous()
         samples_t = _as_f32(samples, "samples").t().contiguous()
         need = int(_lib.lib().evox_hip_hv_covered_workspace_bytes(n_sample))
@@ -847,6 +865,12 @@ torch.library.register_vmap(hv_covered_count, _hv_covered_count_vmap)
 _HV_OBJECTIVES = 16  # most objectives of the whole-call hypervolume kernels
 
 
+# Looking at a tensor's attributes under a function mode (a default device set with ``torch.device(...)`` is one) goes through
+# Python each time: the whole-call functions below look at them, and make their buffers, with the modes off -- 20 us of a
+# call of the metric.  Only where plain_eager() holds: a tracer does not get here.
+quiet = torch._C.DisableTorchFunction
+
+
 def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> bool:
     """Whether a whole hypervolume estimate runs in the library (hv_estimate, hype_contributions): plain float32 tensors
     under a float32 default, no derivative asked for and nothing looking at the call; every other call goes through the
@@ -866,7 +890,7 @@ def _hv_whole_call(bytes_query: str, entry: str, points: torch.Tensor, ref: torc
     u = u.contiguous()
     n_sample = u.size(0)
     need = int(getattr(_lib.lib(), bytes_query)(n, m, n_sample))
-    with torch.cuda.device(points.device):
+    with _on(points.device):
         ws = torch.empty(need, dtype=torch.uint8, device=points.device)
         _lib.call(entry, points.data_ptr(), points.stride(0), points.stride(1), n, m, ref.data_ptr(), ref.stride(0), *extra, u.data_ptr(),
                   n_sample, out.data_ptr(), ws.data_ptr(), need, runtime.stream_handle(points.device))
@@ -897,7 +921,7 @@ def tournament_pick(parents: torch.Tensor, fitness: torch.Tensor) -> torch.Tenso
     fit = _order_preserving_f32(fitness, "fitness") if fitness.numel() > 0 else fitness.float()
     par = parents.contiguous()
     out = torch.empty(par.size(0), dtype=torch.int64, device=parents.device)
-    with torch.cuda.device(parents.device):
+    with _on(parents.device):
         _lib.call("evox_hip_tournament_pick", par.data_ptr(), par.size(0), par.size(1), fit.data_ptr(), fit.size(0), fit.size(1),
                   fit.stride(0), fit.stride(1), out.data_ptr(), runtime.stream_handle(parents.device))
     return out
@@ -958,7 +982,7 @@ def tournament_pick_keys_direct(parents: torch.Tensor, keys: List[torch.Tensor])
     pointers = (ctypes.c_void_p * count)(*[t.data_ptr() for t in keys])
     kinds = (ctypes.c_int32 * count)(*[0 if t.dtype is torch.float32 else 1 for t in keys])
     strides = (ctypes.c_int64 * count)(*[t.stride(0) for t in keys])
-    with torch.cuda.device(parents.device):
+    with _on(parents.device):
         _lib.call("evox_hip_tournament_pick_keys", par.data_ptr(), par.size(0), par.size(1), keys[0].size(0), count,
                   ctypes.addressof(pointers), ctypes.addressof(kinds), ctypes.addressof(strides), out.data_ptr(),
                   runtime.stream_handle(parents.device))

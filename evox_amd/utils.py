@@ -53,6 +53,15 @@ def lexsort(keys: Sequence[torch.Tensor], dim: int = -1) -> torch.Tensor:
     if keys[0].numel() == 0:
         keys[0].size(dim)  # an IndexError for a dimension the keys do not have
         return torch.empty(shape, dtype=torch.int64, device=keys[0].device)
+    if keys[0].dim() == 1 and dim in (-1, 0):  # nothing to move; the function behind the operator where nothing looks at the call
+        step = ops.stable_argsort_step
+        if ops.plain_eager() and not any(type(k) is not torch.Tensor or k.requires_grad or k.is_neg() or k.is_conj() for k in keys):
+            step = getattr(step, "_init_fn", step)
+        order = None
+        for key in keys:
+            for part, kind in _key_parts(key):
+                order = step(part, kind, order)
+        return order.to(torch.int64)
     moved = [k.movedim(dim, -1) for k in keys]
     n = moved[0].shape[-1]
     rows = [m.reshape(-1, n) for m in moved]
