@@ -465,14 +465,11 @@ def batched_line(args, dev):
 
     kernel_us = event_time_us(launch, max(5, min(args.steps, 30)), inner=8)
     pairs = float(batch) * n * n
-    # every row is tested against all rows of its population (no slot order inside a workgroup):
-    # m subtractions, (m - 1) ORs three at a time, clamp, shift-in per pair
-    executed = (m + m // 2 + 2) * pairs
-    rates = valu_issue_rates(dev)
-    roofline = {"kernel": "batched_kernel", "bound": "valu", "achieved": executed / kernel_us / 1e3,
-                "peak": VALU_FP32_PEAK_GOPS, "unit": "Gop/s", "frac": executed / kernel_us / 1e3 / VALU_FP32_PEAK_GOPS,
-                "traffic": None, "kernel_us": kernel_us, "measured_issue_rates_Gops": rates,
-                "frac_of_measured_rate": executed / kernel_us / 1e3 / rates["arithmetic_form_unit_m3"]}
+    # the rows of the populations and the fitness read once, the selected ones written once
+    moved = float(batch) * (n * m * 4 + w.topk * (2 * x.size(2) * 4 + m * 4 + 8))
+    roofline = {"kernel": "sets_kernel", "bound": "hbm", "achieved": moved / kernel_us / 1e3, "peak": 8000.0, "unit": "GB/s",
+                "frac": moved / kernel_us / 1e3 / 8000.0, "traffic": moved, "kernel_us": kernel_us,
+                "note": "no pairs are compared: orders of the objectives, prefix sets in LDS"}
     out = {
         "metric": "dominance comparisons/sec through nd_environmental_selection (N^2 ordered pairs per population and step)",
         "value": pairs / (ms_per_step * 1e-3), "unit": "comparisons/s", "n_gpus": 1, "steps": args.steps,

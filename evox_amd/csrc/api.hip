@@ -30,6 +30,7 @@
 #include "two.hpp"
 #include "two_small.hpp"
 #include "few.hpp"
+#include "sets.hpp"
 #include "wide.hpp"
 
 namespace evx {
@@ -49,6 +50,8 @@ struct Options {
                                    // one-workgroup kernel take the one without a matrix (two_small.hpp); 0 = never
   int64_t few_max_rows = kFewRows;  // populations of three to eight objectives and at most this many rows that reach the entry points
                                     // with a workspace: matrix by the whole device, the rest by one workgroup (few.hpp); 0 = never
+  int64_t sets_min_rows = 257;  // populations of three to eight objectives and at least this many rows that go to a one-workgroup
+                                // kernel take the one that compares no pairs (sets.hpp); more than kSetsRows = never
   int64_t two_min_rows = 4097;  // populations of two objectives and at least this many rows are ranked without a matrix (two.hpp); 0 = never
   int64_t two_min_rows_partial = 4097;  // ... when the ranking may stop at the front that holds a given row (measured, us per
                                         // selection of half the rows, without / with a matrix: 5000 rows 110 / 178, 20 000 rows
@@ -1468,7 +1471,48 @@ static int launch_few_whole(const BatchedArgs& a, int batch, hipStream_t s) {
   }
 }
 
+// Populations of three to eight objectives: one workgroup each, dominators from the orders of the objectives (sets.hpp).
+template <int M>
+static int launch_sets_m(const BatchedArgs& a, int64_t batch, hipStream_t s) {
+  const int rows = (int)round_up(a.n, 64);
+  const bool narrow = rows <= kSetsNarrowRows;
+  const size_t lds = sets_lds_bytes(rows, M);
+  const void* const kernel = narrow ? reinterpret_cast<const void*>(sets_kernel<M, 8>) : reinterpret_cast<const void*>(sets_kernel<M, 16>);
+  if (int e = grant_dynamic_lds(kernel, lds)) return e;
+  for (int64_t b0 = 0; b0 < batch; b0 += 0x40000000ll) {
+    BatchedArgs part = a;
+    const int64_t nb = batch - b0 < 0x40000000ll ? batch - b0 : 0x40000000ll;
+    part.f += b0 * a.f_stride_b;
+    if (part.rank_all) part.rank_all += b0 * a.n;
+    if (part.x) part.x += b0 * a.x_stride_b;
+    if (part.out_x) part.out_x += b0 * a.stop_count * a.x_row_bytes;
+    if (part.out_f) part.out_f += b0 * a.stop_count * a.m;
+    if (part.out_rank) part.out_rank += b0 * a.stop_count;
+    if (part.out_dist) part.out_dist += b0 * a.stop_count;
+    if (narrow)
+      hipLaunchKernelGGL((sets_kernel<M, 8>), dim3((unsigned)nb), dim3(rows), lds, s, part);
+    else
+      hipLaunchKernelGGL((sets_kernel<M, 16>), dim3((unsigned)nb), dim3(rows), lds, s, part);
+    EVX_LAUNCH_CHECK();
+  }
+  return 0;
+}
+static int launch_sets(const BatchedArgs& a, int64_t batch, hipStream_t s) {
+  switch (a.m) {
+    case 3: return launch_sets_m<3>(a, batch, s);
+    case 4: return launch_sets_m<4>(a, batch, s);
+    case 5: return launch_sets_m<5>(a, batch, s);
+    case 6: return launch_sets_m<6>(a, batch, s);
+    case 7: return launch_sets_m<7>(a, batch, s);
+    default: return launch_sets_m<8>(a, batch, s);
+  }
+}
+
 static int launch_batched(const BatchedArgs& a, int64_t batch, hipStream_t s) {
+  // (1024 populations, us, all pairs against the orders of the objectives: 256 x 3 uniform 27 / 27, values of four levels 28 / 33, 192 x 3
+  // 20 to 23 / 23 and 21 / 39; from 257 rows on no slower on any data: 257 x 3 46 / 31 and 48 / 37, 512 x 3 64 / 44, 390 x 5 146 / 52, 390 x 8 210 / 93,
+  // with four levels 123 / 124)
+  if (a.m >= 3 && a.m <= kSetsObjectives && a.n >= opt().sets_min_rows && a.n <= kSetsRows) return launch_sets(a, batch, s);
   if (a.m >= 3 && a.m <= kFewObjectives && a.n <= kFewWholeRows && batch <= device_cus() && opt().few_max_rows > 0)
     return launch_few_whole(a, (int)batch, s);
   if (a.m == 2 && opt().two_small_min_rows > 0 && (a.n >= opt().two_small_min_rows || a.n > kBatchedMaxRows))
@@ -1563,6 +1607,8 @@ static int set_named(Options& o, const char* name, int64_t value) {
     o.peel_stepped = (int)value;
   } else if (!strcmp(name, "few_max_rows") && value >= 0 && value <= kFewRows) {
     o.few_max_rows = value;
+  } else if (!strcmp(name, "sets_min_rows") && value >= 1) {
+    o.sets_min_rows = value;
   } else if (!strcmp(name, "two_small_min_rows") && value >= 0) {
     o.two_small_min_rows = value;
   } else if (!strcmp(name, "two_min_rows") && value >= 0) {

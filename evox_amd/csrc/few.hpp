@@ -133,6 +133,100 @@ __device__ inline int few_position(uint32_t key, int nv, int nt, uint32_t* cnt, 
   return position_by_counting(comps, reinterpret_cast<int*>(cnt), nv, q, nt);
 }
 
+// The fronts of a population (non_dominate.py:29-59): a row joins when none of its dominators is unranked.  Thread j holds the words of
+// row j (words from the population's own on are zero).  front: zeroed, behind a barrier.  order: the rows by (rank, index), up to the
+// front that reaches a.stop_count; rows behind it keep kRankUnset.  A front is WORDS ANDs of 64 bits, one barrier, and a fold of the
+// front's words.
+struct FewFronts {
+  int rank;                     // of this thread's row (-1: no row)
+  int worst, worst_start, nv;  // the last front: its rank, the rows before it, its rows
+};
+template <int WORDS>
+__device__ __forceinline__ FewFronts few_peel(const BatchedArgs& a, uint64_t (&row)[WORDS], uint64_t (*front)[kFewWords], uint16_t* order,
+                                              Ctrl* __restrict__ ctrl) {
+  const int j = threadIdx.x, lane = j & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(j >> 6);
+  int rank = j < a.n ? kRankUnset : -1;
+  int level = 0, ranked = 0, nv = 0;
+  for (;; ++level) {
+    uint64_t* const cur = front[level & 1];
+    uint64_t left = 0ull;
+#pragma unroll
+    for (int w = 0; w < WORDS; ++w) left |= row[w];
+    const bool now = rank == kRankUnset && left == 0ull;
+    if (now) rank = level;
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(now);
+    if (lane == 0) cur[wave] = mine;
+    __syncthreads();
+    // rows of the front, and those of the waves before this one: a word per lane, four steps inside a row of sixteen lanes
+    int held = __popcll(cur[lane & (kFewWords - 1)]);
+    held += __builtin_amdgcn_update_dpp(0, held, 0x111, 0xf, 0xf, true);  // row_shr:1
+    held += __builtin_amdgcn_update_dpp(0, held, 0x112, 0xf, 0xf, true);  // row_shr:2
+    held += __builtin_amdgcn_update_dpp(0, held, 0x114, 0xf, 0xf, true);  // row_shr:4
+    held += __builtin_amdgcn_update_dpp(0, held, 0x118, 0xf, 0xf, true);  // row_shr:8
+    const int size = __builtin_amdgcn_readlane(held, kFewWords - 1);
+    const int before = wave == 0 ? 0 : __builtin_amdgcn_readlane(held, wave - 1);
+    if (now) order[ranked + before + __popcll(mine & ((1ull << lane) - 1ull))] = (uint16_t)j;
+    if (size == 0 || ranked + size >= a.stop_count) {
+      nv = size;
+      break;
+    }
+    ranked += size;
+#pragma unroll
+    for (int w = 0; w < WORDS; w += 2) {
+      const ulonglong2 gone = *reinterpret_cast<const ulonglong2*>(cur + w);
+      row[w] &= ~gone.x;
+      row[w + 1] &= ~gone.y;
+    }
+  }
+  if (j == 0 && ctrl != nullptr) {
+    ctrl->err = 0;
+    ctrl->nfronts = level + 1;
+    ctrl->worst = level;
+    ctrl->worst_start = ranked;
+    ctrl->nv = nv;
+    ctrl->need = a.stop_count - ranked;
+    ctrl->passes = level;
+    ctrl->tail_done = 1;
+  }
+  return {rank, level, ranked, nv};
+}
+
+// The selected rows, in the order of `order`: everything that LDS holds by row (fit by objective, `rows` apart), and x from memory.
+__device__ __forceinline__ void few_gather(const BatchedArgs& a, const uint16_t* order, const uint16_t* rank_lds, const float* dist,
+                                           const float* fit, int rows) {
+  const int j = threadIdx.x, lane = j & 63, nt = blockDim.x, m = a.m;
+  const int wave = __builtin_amdgcn_readfirstlane(j >> 6);
+  const int topk = a.stop_count;
+  const int64_t ob = (int64_t)blockIdx.x * topk;
+  for (int p = j; p < topk; p += nt) {
+    const int src = order[p];
+    a.out_rank[ob + p] = rank_lds[src];
+    a.out_dist[ob + p] = dist[src];
+  }
+  for (int e = j; e < topk * m; e += nt) {
+    const int p = e / m, k = e - p * m;
+    a.out_f[ob * m + e] = fit[(size_t)k * rows + order[p]];
+  }
+  if (a.x != nullptr) {
+    const uint8_t* __restrict__ xb = a.x + (int64_t)blockIdx.x * a.x_stride_b;
+    uint8_t* __restrict__ dst = a.out_x + ob * a.x_row_bytes;
+    if (!gather_whole_units(a, xb, dst, order, topk, j, nt)) {
+      for (int p = wave; p < topk; p += nt >> 6) {
+        const int src = order[p];
+        const uint8_t* __restrict__ sp = xb + (int64_t)src * a.x_row_stride + (src >= a.n_first ? a.x_second : 0);
+        uint8_t* __restrict__ dp = dst + (int64_t)p * a.x_row_bytes;
+        if (a.x_unit >= 4) {
+          for (int64_t b = lane * 4; b < a.x_row_bytes; b += 64 * 4)
+            *reinterpret_cast<uint32_t*>(dp + b) = *reinterpret_cast<const uint32_t*>(sp + b);
+        } else {
+          for (int64_t b = lane; b < a.x_row_bytes; b += 64) dp[b] = sp[b];
+        }
+      }
+    }
+  }
+}
+
 // Everything behind the matrix, by one workgroup of nt >= n threads: thread j < n holds row j, the others help where candidates
 // are placed and rows gathered.  WORDS: words of a row at most.  mine: row j's fitness is at fit_of(k).  words: as above.
 template <int WORDS, class FitOf>
@@ -161,54 +255,8 @@ __device__ __forceinline__ void few_finish(const BatchedArgs& a, const uint64_t*
   __syncthreads();
   EVX_BATCH_TRACE(1);
 
-  // ---- peeling: a row joins the front when none of its dominators is unranked (non_dominate.py:29-59)
-  uint64_t alive[WORDS];
-#pragma unroll
-  for (int w = 0; w < WORDS; ++w) alive[w] = ~0ull;
-  int rank = valid ? kRankUnset : -1;
-  int level = 0, ranked = 0, nv = 0;
-  for (;; ++level) {
-    uint64_t* const cur = front[level & 1];
-    uint64_t left = 0ull;
-#pragma unroll
-    for (int w = 0; w < WORDS; ++w) left |= row[w] & alive[w];
-    const bool now = rank == kRankUnset && left == 0ull;
-    if (now) rank = level;
-    const uint64_t mine = __builtin_amdgcn_ballot_w64(now);
-    if (lane == 0) cur[wave] = mine;
-    __syncthreads();
-    // rows of the front, and those of the waves before this one: a word per lane, four steps inside a row of sixteen lanes
-    int held = __popcll(cur[lane & (kFewWords - 1)]);
-    held += __builtin_amdgcn_update_dpp(0, held, 0x111, 0xf, 0xf, true);  // row_shr:1
-    held += __builtin_amdgcn_update_dpp(0, held, 0x112, 0xf, 0xf, true);  // row_shr:2
-    held += __builtin_amdgcn_update_dpp(0, held, 0x114, 0xf, 0xf, true);  // row_shr:4
-    held += __builtin_amdgcn_update_dpp(0, held, 0x118, 0xf, 0xf, true);  // row_shr:8
-    const int size = __builtin_amdgcn_readlane(held, kFewWords - 1);
-    const int before = wave == 0 ? 0 : __builtin_amdgcn_readlane(held, wave - 1);
-    if (now) order[ranked + before + __popcll(mine & ((1ull << lane) - 1ull))] = (uint16_t)j;
-    if (size == 0 || ranked + size >= a.stop_count) {
-      nv = size;
-      break;
-    }
-    ranked += size;
-#pragma unroll
-    for (int w = 0; w < WORDS; w += 2) {
-      const ulonglong2 gone = *reinterpret_cast<const ulonglong2*>(cur + w);
-      alive[w] &= ~gone.x;
-      alive[w + 1] &= ~gone.y;
-    }
-  }
-  const int worst_start = ranked, worst = level;
-  if (j == 0 && ctrl != nullptr) {
-    ctrl->err = 0;
-    ctrl->nfronts = worst + 1;
-    ctrl->worst = worst;
-    ctrl->worst_start = worst_start;
-    ctrl->nv = nv;
-    ctrl->need = a.stop_count - worst_start;
-    ctrl->passes = worst;
-    ctrl->tail_done = 1;
-  }
+  const FewFronts got = few_peel<WORDS>(a, row, front, order, ctrl);
+  const int rank = got.rank, worst_start = got.worst_start, nv = got.nv;
   if (a.rank_all && valid) a.rank_all[(int64_t)blockIdx.x * n + j] = rank;
   if (a.out_f == nullptr) return;  // rank-only mode
   if (valid) {
@@ -250,35 +298,7 @@ __device__ __forceinline__ void few_finish(const BatchedArgs& a, const uint64_t*
   __syncthreads();
 
   EVX_BATCH_TRACE(4);
-  // ---- the selected rows
-  const int topk = a.stop_count;
-  const int64_t ob = (int64_t)blockIdx.x * topk;
-  for (int p = j; p < topk; p += nt) {
-    const int src = order[p];
-    a.out_rank[ob + p] = rank_lds[src];
-    a.out_dist[ob + p] = dist[src];
-  }
-  for (int e = j; e < topk * m; e += nt) {
-    const int p = e / m, k = e - p * m;
-    a.out_f[ob * m + e] = fit[(size_t)k * rows + order[p]];
-  }
-  if (a.x != nullptr) {
-    const uint8_t* __restrict__ xb = a.x + (int64_t)blockIdx.x * a.x_stride_b;
-    uint8_t* __restrict__ dst = a.out_x + ob * a.x_row_bytes;
-    if (!gather_whole_units(a, xb, dst, order, topk, j, nt)) {
-      for (int p = wave; p < topk; p += nt >> 6) {
-        const int src = order[p];
-        const uint8_t* __restrict__ sp = xb + (int64_t)src * a.x_row_stride + (src >= a.n_first ? a.x_second : 0);
-        uint8_t* __restrict__ dp = dst + (int64_t)p * a.x_row_bytes;
-        if (a.x_unit >= 4) {
-          for (int64_t b = lane * 4; b < a.x_row_bytes; b += 64 * 4)
-            *reinterpret_cast<uint32_t*>(dp + b) = *reinterpret_cast<const uint32_t*>(sp + b);
-        } else {
-          for (int64_t b = lane; b < a.x_row_bytes; b += 64) dp[b] = sp[b];
-        }
-      }
-    }
-  }
+  few_gather(a, order, rank_lds, dist, fit, rows);
   EVX_BATCH_TRACE(5);
 }
 

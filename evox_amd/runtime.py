@@ -16,11 +16,11 @@ _last: Optional[Tuple[torch.Tensor, int]] = None  # (workspace, stream handle) o
 CHECK_STATUS = os.environ.get("EVOX_AMD_CHECK_STATUS", "0") not in ("", "0")
 
 # Populations of at most evox_hip_batched_max_rows(m) rows can run in the one-workgroup-per-population kernels, larger
-# ones need a workspace.  None = choose by size.  Three to eight objectives: a lone population of more than 256 rows is
-# faster in the two launches whose first one spreads the matrix over the whole device (selection of half the rows,
-# us, one workgroup against two launches: 256 x 3 14 / 17 -- both bound by the host there --, 300 x 3 23 / 17, 500 x 3
-# 29 / 17, 1000 x 3 96 / 21, 256 x 8 33 / 30, 300 x 8 83 / 31); up to 32 populations are from 513 rows on (512 x 3: 28 / 29,
-# 700 x 3: 46 / 29, 1000 x 3: 104 / 29 to 33; 64 of 700: 46 / 47).  Other numbers of objectives: a lone population is faster in the
+# ones need a workspace.  None = choose by size.  Three to eight objectives: up to 256 rows always; above, a few populations are
+# faster in the two launches whose first one spreads the matrix over the whole device (selection of half the rows, us, two launches
+# against one workgroup each: one of 300 x 3 12.5 / 16, one of 1000 x 3 21 / 28, one of 1000 x 8 47 / 60, 16 of 512 x 3 17.5 / 18.8, 16 of 1000 x 8
+# 59 / 62, 32 of 512 x 3 18.9 / 18.9, 32 of 512 x 5 25 / 28, 32 of 1000 x 3 32 / 30, 32 of 1000 x 8 70 / 61, 64 of 300 x 3 33 / 17, 64 of 1000 x 8
+# 138 / 62), more are not.  Other numbers of objectives: a lone population is faster in the
 # pipeline from a size on that shrinks as the objectives grow (16 objectives 67 / 77 at 128 rows, 119 / 101 at 256), two or
 # three from twice that size on, four or more never.  True / False force the choice where it is possible (tests use that to drive small
 # inputs through both).
@@ -57,7 +57,7 @@ def small_population_kernel_fits(n: int, m: int, batch: int) -> bool:
     if use_small_population_kernel is True:
         return True
     if 3 <= m <= 8:
-        return n <= 256 or (batch > 1 and (n <= 512 or batch > 32))
+        return n <= 256 or batch >= 32
     if batch >= 4:
         return True
     return n <= _lone_population_limit(m) * (1 if batch == 1 else 2)

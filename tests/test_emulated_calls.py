@@ -14,6 +14,8 @@ pytestmark = pytest.mark.skipif(emulated.CXX is None, reason="no clang++")
     ["select:33000:2:shell:::2", "select:33000:2:layers", "select:40001:3:simplex:::3"],
     ["batch:1100:3:shell:7", "batch:1500:5:simplex:5::2", "batch:300:3:uniform:9", "batch:5000:2:uniform:3"],
     ["batch:1100:2:shell:3::2", "batch:4000:2:layers:2", "batch:3001:2:equal:2", "batch:130:2:nan:5", "batch:2047:2:chain:2"],
+    ["batch:300:3:uniform:2", "batch:500:3:grid:2", "batch:512:3:simplex:2", "batch:512:3:equal", "batch:257:3:nan:3", "batch:500:5:chain:2",
+     "batch:400:5:inf:2", "batch:513:3:uniform", "batch:1000:5:grid", "batch:1024:3:shell", "batch:777:3:equal", "batch:900:5:nan"],
     ["select64:3000:3:uniform", "select64:9001:5:simplex", "crowd:1400:2:uniform", "crowd:5000:3:grid", "mask:20000:3:shell", "mask:70000:2:uniform"],
 ])
 def test_every_access_lies_in_its_region(specs):
