@@ -219,26 +219,35 @@ __global__ __launch_bounds__(64 * WORDS) __attribute__((amdgpu_waves_per_eu(WORD
         const bool writes = kSetsSegment * segment < rows;
         const int words = min(rows / 32 - panel * 16, 16);
         for (int word = kWide ? wave : j >> 5; word < words; word += kWide ? waves : 2 * waves) {  // (wave-uniform)
-          uint32_t held[kSetsSegment];
-          uint32_t run = 0u;
+          const uint4* const from = reinterpret_cast<const uint4*>(by_value + kSetsSegment * segment);
+          uint32_t pairs[8];
           if (writes) {
-            const uint4* const from = reinterpret_cast<const uint4*>(by_value + kSetsSegment * segment);
             const uint4 low = from[0], high = from[1];
-            const uint32_t pairs[8] = {low.x, low.y, low.z, low.w, high.x, high.y, high.z, high.w};
+            pairs[0] = low.x; pairs[1] = low.y; pairs[2] = low.z; pairs[3] = low.w;
+            pairs[4] = high.x; pairs[5] = high.y; pairs[6] = high.z; pairs[7] = high.w;
+          } else {
 #pragma unroll
-            for (int t = 0; t < kSetsSegment; ++t) {
-              const uint32_t at = ((pairs[t >> 1] >> (16 * (t & 1))) & 0xFFFFu) - 32u * (uint32_t)(panel * 16 + word);
-              run |= at < 32u ? 1u << at : 0u;
-              held[t] = run;
-            }
+            for (int t = 0; t < 8; ++t) pairs[t] = ~0u;  // (row 65535: in no word)
           }
+          const uint32_t base = 32u * (uint32_t)(panel * 16 + word);
+          auto bit_of = [&](int t) {
+            const uint32_t at = ((t & 1) ? pairs[t >> 1] >> 16 : pairs[t >> 1] & 0xFFFFu) - base;
+            return at < 32u ? 1u << at : 0u;
+          };
+          // (once for the total, once more for the entries: sixteen words held in between would not fit the registers)
+          uint32_t run = 0u;
+#pragma unroll
+          for (int t = 0; t < kSetsSegment; ++t) run |= bit_of(t);
           const uint32_t incl = sets_prefix_or<kWide>(run);
-          uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x138, 0xf, 0xf, false);  // wave_shr:1
-          if (segment == 0) before = 0u;
+          run = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x138, 0xf, 0xf, false);  // wave_shr:1
+          if (segment == 0) run = 0u;
           if (writes) {
             uint32_t* const to = table + (size_t)kSetsSegment * segment * kSetsEntry + 4 * segment + word;
 #pragma unroll
-            for (int t = 0; t < kSetsSegment; ++t) to[t * kSetsEntry] = held[t] | before;
+            for (int t = 0; t < kSetsSegment; ++t) {
+              run |= bit_of(t);
+              to[t * kSetsEntry] = run;
+            }
           }
         }
         __syncthreads();
