@@ -64,8 +64,8 @@ struct Options {
   int dominance_folded = 1;      // tiles of two words: only the blocks at or below the diagonal are launched
   int mid_argsort = 1;  // an argsort step of 8193 .. kMidArgsortRows positions in one kernel without waits (0: the radix sort)
   int small_sort = 1;  // populations up to kSmallSortRows rows are put in slot order by one kernel (0: bucket sort)
-  int64_t prefix_min_rows = 65536;  // finite populations of at least this many rows and 3 objectives (a quarter more
-                                    // with 2, fewer with more: 28672 at 8, 10240 at 16 -- prefix_least_rows) get
+  int64_t prefix_min_rows = 65536;  // finite populations of at least 20/32 of this many rows and 3 objectives (40/32
+                                    // with 2, fewer with more: 32769 at 4, 28672 at 8, 10240 at 16 -- prefix_least_rows) get
                                     // their matrix from the per-objective orders (prefix.hpp); 0 = never
   int64_t prefix_double_tile = 131072;  // order-based matrix, up to four objectives: from this many rows on a workgroup
                                         // takes both tiles of a 128-byte line; 0 = never
@@ -73,7 +73,7 @@ struct Options {
   int prefix_bands = 1;  // stretches of the order-based matrix: 1 = bands of rows counted from row 0, 0 = from each tile's diagonal
   int batched_stage = 1;  // the one-workgroup kernel reads its dominators from a copy of the fitness in LDS when the populations
                           // have at most 256 rows and are no more than the device has compute units (0: by scalar loads always)
-  int order_stream = 1;  // the per-objective orders of more than 32768 rows come from workgroups that sort shares of
+  int order_stream = 1;  // the per-objective orders of more than 32768 rows come from workgroups that place shares of
                          // them in LDS (0: from the radix sort whose workgroups wait for each other)
   int order_stream_capacity = 16384;  // entries that such a workgroup sorts at once (tests make it small: shares in pieces)
   int prefix_count_first = 1;  // a selection whose last two of this shape found all they keep in front 0 has the order-based
@@ -478,14 +478,17 @@ static int stage_prepare(const Ws& w, const Fitness& src, bool with_sort, hipStr
 //   33 000 335 / 325, 50 000 584 / 386;  x 9: 20 000 251 / 305, 26 000 342 / 323;  x 10: 20 000 269 / 315, 26 000 363 / 329;
 //   x 12: 16 000 261 / 308, 20 000 312 / 307;  x 14: 16 000 301 / 327, 20 000 363 / 327;  x 16: 12 000 253 / 330,
 //   16 000 342 / 344, 20 000 424 / 352;  x 2 (65 536 rows): 227 / 239, (100 000) 558 / 370.
-// As thirty-seconds of the tunable (65 536 rows for three objectives):
+// With the orders from shares that are placed by buckets (prefix.hpp, above kMidArgsortRows rows; they also order the last front):
+//   x 3: 33 000 264 / 287 (one front: 284 / 214), 41 000 309 / 309 (shell 242 / 223), 52 000 385 / 344;  x 4: 33 000 215 / 212 (shell 205 / 177);
+//   x 5: 33 000 218 / 205 (one front 324 / 223), 42 000 283 / 230;  x 6: 33 000 228 / 197;  x 7: 33 000 260 / 200 (one front 377 / 245).
+// As thirty-seconds of the tunable (20 of them are 40 960 rows; four to seven objectives begin where those orders do):
 // Up to kMidArgsortRows rows the orders come from workgroups that sort in LDS and cost 60 to 90 us less:
 //   x 8: 26 000 254 / 261, 32 768 322 / 295;  x 9: 16 000 212 / 224, 20 000 252 / 236;  x 10: 16 000 222 / 231,
 //   20 000 268 / 245;  x 12: 12 000 198 / 210, 16 000 257 / 225;  x 16: 9000 220 / 215, 12 000 259 / 237.
 static int64_t prefix_least_rows(int m) {
-  int parts = m <= 2 ? 40 : m == 3 ? 32 : m <= 5 ? 22 : m == 6 ? 20 : m == 7 ? 18 : m == 8 ? 16 : m <= 10 ? 12 : m <= 12 ? 10 : m <= 14 ? 9 : 8;
+  int parts = m <= 2 ? 40 : m == 3 ? 20 : m <= 8 ? 16 : m <= 10 ? 12 : m <= 12 ? 10 : m <= 14 ? 9 : 8;
   if (opt().mid_argsort && m >= 8) parts = m == 8 ? 14 : m <= 10 ? 9 : m <= 12 ? 7 : m <= 14 ? 6 : 5;
-  return opt().prefix_min_rows / 32 * parts + (opt().prefix_min_rows % 32 != 0 ? 1 : 0);
+  return opt().prefix_min_rows / 32 * parts + (opt().prefix_min_rows % 32 != 0 || (m >= 4 && m <= 7) ? 1 : 0);
 }
 static bool prefix_dominance_applies(const Layout& L) {
   if (opt().prefix_min_rows <= 0 || L.m < 2 || L.m > kPrefixMaxObjectives) return false;
@@ -1113,25 +1116,26 @@ static int stage_dominance_prefix(const Ws& w, bool orders_only, hipStream_t s, 
     EVX_LAUNCH_CHECK();
     return orders_only ? 0 : dispatch_dominance_prefix(w, s, phase);
   }
-  // shares of one objective's order that the streaming kernel would cut: as many as give every compute unit a
-  // workgroup, if shares of kOrderStreamShare rows need no more than that
-  const int stream_parts = device_cus() / L.m;
+  // shares of one objective's order: as many as give every compute unit a workgroup, while they fit one (whole selections, us, shares /
+  // radix sort below: 200 000 x 8 693 / 780, 250 000 x 8 826 / 910, 120 000 x 16 1100 / 1236)
+  const int stream_parts = device_cus() / L.m < kOrderStreamMaxParts ? device_cus() / L.m : kOrderStreamMaxParts;
   if (opt().order_stream && L.n > kOrderStreamSample && L.n <= kOrderStreamMaxRows && (L.npad & 3) == 0 && stream_parts >= 1 &&
       stream_parts <= kOrderStreamSample && (int64_t)stream_parts * kOrderStreamShare >= L.n) {
-    // larger populations likewise, by workgroups that read their objective's keys once and sort their share of the
-    // order in LDS -- while those shares stay small: 40 000 x 8 the orders in 52 instead of 127 us, 65 536 x 3 57 / 90,
-    // 100 000 x 8 105 / 144, 200 000 x 3 120 / 147; 200 000 x 8 (shares of 6250 rows) 201 / 185: the radix sort below
-    const size_t stream_lds = sizeof(double) * kOrderStreamCapacity;
-    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(objective_order_stream_kernel), stream_lds)) return e;
+    // larger populations likewise: the rows grouped by share of an objective's order, then the shares placed in LDS
+    if (int e = grant_dynamic_lds(reinterpret_cast<const void*>(objective_order_stream_kernel), kOrderStreamLdsBytes)) return e;
     const int parts = stream_parts;
-    hipLaunchKernelGGL(objective_order_stream_kernel, dim3(L.m * parts), dim3(kOrderStreamThreads), stream_lds, s, w.at<float>(L.xs),
-                       L.npad, L.n, L.m, parts, opt().order_stream_capacity, w.at<SortParam>(L.sortparam), w.ctrl(),
-                       w.at<int>(L.total0), w.at<int>(L.witness0), radix_buffers(w));
+    const int per = (L.n + parts - 1) / parts;
+    // (the matrix is written behind these launches)
+    unsigned long long* const bounds = w.at<unsigned long long>(L.dom);
+    uint32_t* const offsets = w.at<uint32_t>(L.dom) + order_bounds_words(L.m, parts);
+    const RadixBuffers buf = radix_buffers(w);
+    hipLaunchKernelGGL(objective_shares_kernel, dim3(L.m * parts), dim3(kOrderStreamThreads),
+                       8 * (size_t)kOrderStreamSample + 4 * (size_t)kOrderStreamBuckets, s, w.at<float>(L.xs), L.npad, L.n, L.m, parts, per,
+                       w.at<SortParam>(L.sortparam), w.ctrl(), w.at<int>(L.total0), w.at<int>(L.witness0), buf.kstride, buf.pairs[1], offsets, bounds);
     EVX_LAUNCH_CHECK();
-    int64_t blocks = ((int64_t)L.n * L.m + 255) / 256;
-    if (blocks > device_cus() * 8) blocks = device_cus() * 8;
-    hipLaunchKernelGGL(objective_positions_kernel, dim3((unsigned)blocks), dim3(256), 0, s, L.n, L.m, w.at<int>(L.slot_of),
-                       w.at<SortParam>(L.sortparam), w.ctrl(), w.at<int>(L.pos), w.at<int>(L.scost), radix_buffers(w));
+    hipLaunchKernelGGL(objective_order_stream_kernel, dim3(L.m * parts), dim3(kOrderStreamThreads), kOrderStreamLdsBytes, s, w.at<float>(L.xs),
+                       L.npad, L.n, L.m, parts, per, opt().order_stream_capacity, w.at<int>(L.slot_of), w.at<SortParam>(L.sortparam), w.ctrl(),
+                       offsets, bounds, w.at<int>(L.pos), w.at<int>(L.scost), buf);
     EVX_LAUNCH_CHECK();
     return orders_only ? 0 : dispatch_dominance_prefix(w, s, phase);
   }

@@ -9,8 +9,9 @@
 // objective; a row of a larger slot has a larger key sum and is never in the intersection).  Infinities and
 // NaN are left to the pairwise kernel (a NaN has no place in the order).
 //
-//  1. objective_order_kernel: one segmented radix sort orders the slots by every objective (radix.hpp) and
-//     leaves pos[k][slot] and upper[k][slot].
+//  1. The slots in the order of every objective, pos[k][slot] and upper[k][slot]: by workgroups that sort in LDS
+//     (objective_order_lds_kernel, objective_order_stream_kernel), for the largest populations by one segmented radix sort
+//     (objective_order_kernel).
 //  2. dominance_prefix_kernel: a workgroup takes a tile of 512 dominator slots (8 matrix words, 64 bytes of
 //     every row; 256 slots above ten objectives, where the tables of 512 no longer fit the LDS) and a stretch
 //     of rows below it.  Restricted to one word of the tile, the prefix of objective k that belongs to row j is
@@ -29,6 +30,7 @@
 #include "order.hpp"
 #include "peel.hpp"
 #include "radix.hpp"
+#include "two.hpp"
 
 namespace evx {
 
@@ -154,68 +156,319 @@ __global__ __launch_bounds__(kMidArgsortThreads) void objective_order_lds_kernel
   }
 }
 
-// The same orders for larger populations, still without a wait between workgroups: the workgroups share the
-// objectives out, `parts` to each, and a workgroup produces a run of consecutive positions of its objective's order.
+// The same orders for larger populations, still without a wait between workgroups, in two launches: the rows are cut into `parts`
+// shares of every objective's order, and a workgroup places the rows of one share.
 // Rows are composites (key << 20 | original index: distinct, below 2^52).  Every workgroup of an objective sorts the
-// same kOrderStreamSample composites (rows n i / sample) and takes the composites between two of them as its share,
-// which makes `parts` shares of about n / parts rows whatever the values are, equal ones included; it then reads the
-// objective's keys once, counts the composites below its share (where its run starts) and collects those inside it in
-// LDS, sorts them there (the bitonic network of radix.hpp over doubles 2^52 + composite, which order like the
-// composites) and writes the run.  A share that does not fit `capacity` entries -- rows arranged so that the sample
-// misses where they crowd -- is taken in pieces: the largest stretch of composites from the share's start that fits is
-// found by bisection over the composites, a pass over the keys per step, as often as it takes.
-// Where the time goes (200 000 x 8 in 32 shares of 6250 rows, 154 us): the sort of the sample 23 us, the pass over the
-// keys 34 + 20 for storing what it collects, the sort of the share 77 (padded to 8192; 35 when padded to 4096) -- the
-// network's passes are what this costs, which is why the host takes this kernel only while shares of at most
-// kOrderStreamShare rows leave it no more workgroups than the device has compute units.
-// Grid: m * parts workgroups of kOrderStreamThreads.  Dynamic LDS: 8 * kOrderStreamCapacity bytes.  n <= 2^20.
+// same kOrderStreamSample composites (rows n i / sample); the composites between two of them are a share, which makes `parts` shares of
+// about n / parts rows whatever the values are, equal ones included.
+//  1. objective_shares_kernel: a workgroup takes `per` consecutive rows and groups them by their share, by bisection in the sample; where
+//     the groups begin is left in offsets[objective][chunk][share].
+//  2. objective_order_stream_kernel: a workgroup collects its share's groups in LDS, places them and writes its run of the order, and
+//     positions and bounds by slot.  A share that does not fit `capacity` entries -- rows arranged so that the sample
+//     misses where they crowd -- is taken in pieces instead, each collected in a pass over all keys: the largest stretch of composites from
+//     the share's start that fits is found by bisection over the composites, a pass per step, as often as it takes.
+// Placing is by buckets (of equal width in the value, then in the composite: shares of one
+// value), every entry among those of its bucket; the network of radix.hpp only sorts what crowds in both.
+// A workgroup that read all keys of its objective for its share, and sorted that by the network, took 78 us of vector issue for the
+// reading alone at 200 000 rows (96 us, 20 more for positions and bounds in a launch of their own; 160 us and more by the radix sort
+// above); now 12 + 40 us at 200 003 x 3 and 12 + 52 at 200 000 x 8: 7 the sample, 8 to 10 fetching the groups (chains of two reads), 9 to 13 the
+// placing, 12 to 18 the scattered positions and bounds.
+// Grid: m * parts workgroups of kOrderStreamThreads each.  Dynamic LDS: kOrderStreamLdsBytes.  n <= 2^20.
 constexpr int kOrderStreamThreads = 1024;
 constexpr int kOrderStreamCapacity = 16384;
+constexpr int kOrderStreamPer = kOrderStreamCapacity / kOrderStreamThreads;
+constexpr int kOrderStreamBuckets = 4 * kOrderStreamThreads;
+constexpr uint32_t kOrderStreamCrowd = 48;  // entries of a bucket up to which every one looks at every other one
 constexpr int kOrderStreamSample = 2048;
 constexpr int kOrderStreamMaxRows = 1 << 20;
-constexpr int kOrderStreamShare = 3200;  // rows of a share, at most, that the host aims at: sorted as 4096 entries
+constexpr int kOrderStreamShare = 8192;  // rows of a share, at most, that the host aims at
+constexpr int kOrderChunkPer = kOrderStreamShare / kOrderStreamThreads;  // rows of a thread in the first launch
+constexpr int kOrderStreamMaxParts = 128;
+// Words of the offsets and of the shares' bounds (two each), the first launch's other result.
+__host__ __device__ inline size_t order_offsets_words(int m, int parts) { return (size_t)m * (size_t)parts * (size_t)(parts + 1); }
+__host__ __device__ inline size_t order_bounds_words(int m, int parts) { return 2 * (size_t)m * (size_t)(parts + 1); }
+constexpr size_t kOrderStreamLdsBytes = 8 * (size_t)kOrderStreamCapacity + 4 * (size_t)kOrderStreamBuckets;
 
-__global__ __launch_bounds__(kOrderStreamThreads) void objective_order_stream_kernel(const float* __restrict__ xs, int npad, int n, int m,
-                                                                                     int parts, int capacity,
-                                                                                     const SortParam* __restrict__ param,
-                                                                                     const Ctrl* __restrict__ ctrl,
-                                                                                     int* __restrict__ total0, int* __restrict__ witness0,
-                                                                                     RadixBuffers buf) {
-  extern __shared__ __attribute__((aligned(16))) double order_stream_comp[];
-  __shared__ int taken;           // composites of the present pass that lie in its range
-  __shared__ int below_of[16];    // per wave: composites below the range
+// Places of `count` composites (entry tid + kOrderStreamThreads r of comp is `mine[r]`) in ascending order, by buckets; afterwards
+// comp[place] holds them in that order.  False, with comp as it was, when they crowd.  cnt: kOrderStreamBuckets words; part, lo16, hi16: sixteen
+// words each.  Every thread calls it, past a barrier behind the last write of comp; ends with one.
+template <int PER>
+__device__ inline bool order_stream_place(unsigned long long* comp, int count, uint32_t* cnt, uint32_t* part, uint32_t* lo16, uint32_t* hi16) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kWaves = kOrderStreamThreads / 64;
+  constexpr unsigned long long kMask = (1ull << 52) - 1ull;
+  unsigned long long mine[PER];
+  uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    const int e = tid + kOrderStreamThreads * r;
+    mine[r] = 0ull;
+    if (e < count) {
+      mine[r] = comp[bitonic_slot(e)] & kMask;
+      const uint32_t key = (uint32_t)(mine[r] >> 20);
+      lo = min(lo, key);
+      hi = max(hi, key);
+    }
+  }
+  const uint32_t wave_lo = wave_prefix_min(lo), wave_hi = ~wave_prefix_min(~hi);
+  if (lane == 63) {
+    lo16[wave] = wave_lo;
+    hi16[wave] = wave_hi;
+  }
+  __syncthreads();
+  for (int w = 0; w < kWaves; ++w) {
+    lo = min(lo, lo16[w]);
+    hi = max(hi, hi16[w]);
+  }
+  // (by value: finite values only; by composite: the rows of one value by their index)
+  const float v0 = cost_of_key(lo), width = cost_of_key(hi) - v0;
+  const bool by_value = lo < hi && width > 0.0f && width <= 3.4028234663852886e38f;
+  const float scale = by_value ? (float)(kOrderStreamBuckets - 1) / width : 0.0f;
+  const unsigned long long from = (unsigned long long)lo << 20, span = ((unsigned long long)hi << 20 | 0xFFFFFull) - from;
+  const float scale_all = (float)(kOrderStreamBuckets - 1) / (float)span;
+#pragma unroll 1
+  for (int attempt = by_value ? 0 : 1; attempt < 2; ++attempt) {
+    auto bucket_of_entry = [&](unsigned long long c) {
+      const float t = attempt == 0 ? (cost_of_key((uint32_t)(c >> 20)) - v0) * scale : (float)(c - from) * scale_all;
+      return min((uint32_t)t, (uint32_t)kOrderStreamBuckets - 1u);
+    };
+    reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    uint32_t arrived[(PER + 1) / 2];  // (two to a word)
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+      const uint32_t at = tid + kOrderStreamThreads * r < count ? atomicAdd(&cnt[bucket_of_entry(mine[r])], 1u) : 0u;
+      if (r & 1)
+        arrived[r >> 1] |= at << 16;
+      else
+        arrived[r >> 1] = at;
+    }
+    __syncthreads();
+    const uint4 held = reinterpret_cast<const uint4*>(cnt)[tid];
+    const uint32_t sum = held.x + held.y + held.z + held.w;
+    uint32_t incl = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t up = __shfl_up(incl, off);
+      if (lane >= off) incl += up;
+    }
+    if (lane == 63) part[wave] = incl;
+    if (__syncthreads_or(max(max(held.x, held.y), max(held.z, held.w)) > kOrderStreamCrowd)) continue;
+    uint32_t run = incl - sum;
+    for (int w = 0; w < wave; ++w) run += part[w];
+    reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(run, run + held.x, run + held.x + held.y, run + held.x + held.y + held.z);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; ++r)
+      if (tid + kOrderStreamThreads * r < count) comp[cnt[bucket_of_entry(mine[r])] + ((arrived[r >> 1] >> (16 * (r & 1))) & 0xFFFFu)] = mine[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+      if (tid + kOrderStreamThreads * r < count) {
+        const uint32_t bucket = bucket_of_entry(mine[r]);
+        const uint32_t first = cnt[bucket], end = bucket + 1u < (uint32_t)kOrderStreamBuckets ? cnt[bucket + 1u] : (uint32_t)count;
+        uint32_t before = 0u;
+        for (uint32_t q = first; q < end; q += 4) {  // (four members' reads in flight together)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) before += comp[min(q + (uint32_t)u, end - 1u)] < mine[r] && q + (uint32_t)u < end ? 1u : 0u;
+        }
+        const uint32_t place = first + before;
+        if (r & 1)
+          arrived[r >> 1] = (arrived[r >> 1] & 0xFFFFu) | place << 16;
+        else
+          arrived[r >> 1] = (arrived[r >> 1] & 0xFFFF0000u) | place;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; ++r)
+      if (tid + kOrderStreamThreads * r < count) comp[(arrived[r >> 1] >> (16 * (r & 1))) & 0xFFFFu] = mine[r];
+    __syncthreads();
+    return true;
+  }
+  return false;
+}
+
+constexpr unsigned long long kOrderBias = 0x4330000000000000ull;  // the bits of 2^52 as a double
+constexpr unsigned long long kOrderEnd = 1ull << 52;               // above every composite
+
+// per = ceil(n / parts) <= kOrderStreamShare.  grouped[k * kstride + row's place]: the composites of a chunk by share.
+__global__ __launch_bounds__(kOrderStreamThreads) void objective_shares_kernel(const float* __restrict__ xs, int npad, int n, int m, int parts,
+                                                                               int per, const SortParam* __restrict__ param,
+                                                                               const Ctrl* __restrict__ ctrl, int* __restrict__ total0,
+                                                                               int* __restrict__ witness0, int kstride,
+                                                                               unsigned long long* __restrict__ grouped,
+                                                                               uint32_t* __restrict__ offsets,
+                                                                               unsigned long long* __restrict__ bounds) {
+  extern __shared__ __attribute__((aligned(16))) double order_shares_lds[];
+  __shared__ uint32_t part16[16];
+  __shared__ uint32_t lo16[16];
+  __shared__ uint32_t hi16[16];
+  __shared__ unsigned long long bound_lds[kOrderStreamMaxParts + 1];
+  __shared__ uint32_t group[kOrderStreamMaxParts];
   if (param->nonfinite != 0 || ctrl->err != 0) return;
   for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
     total0[j] = 0;
     witness0[j] = -1;
   }
+  double* const comp = order_shares_lds;
+  unsigned long long* const composites = reinterpret_cast<unsigned long long*>(order_shares_lds);
+  uint32_t* const cnt = reinterpret_cast<uint32_t*>(order_shares_lds + kOrderStreamSample);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int k = (int)blockIdx.x % m, chunk = (int)blockIdx.x / m;
+  const float* __restrict__ col = xs + (int64_t)k * npad;
+  const int e0 = min(chunk * per, n), e1 = min(e0 + per, n);
+  uint32_t key[kOrderChunkPer];
+#pragma unroll
+  for (int r = 0; r < kOrderChunkPer; ++r) {  // (asked for ahead of the sample's sort)
+    const int e = e0 + tid + kOrderStreamThreads * r;
+    key[r] = e < e1 ? ordered_key(col[e]) : 0u;
+  }
+  for (int i = tid; i < kOrderStreamSample; i += kOrderStreamThreads) {
+    const int e = (int)(((int64_t)i * n) / kOrderStreamSample);
+    comp[bitonic_slot(i)] =
+        __longlong_as_double((long long)(kOrderBias | (unsigned long long)ordered_key(col[e]) << 20 | (unsigned long long)(unsigned)e));
+  }
+  if (tid < kOrderStreamMaxParts) group[tid] = 0u;
+  __syncthreads();
+  const bool placed = order_stream_place<kOrderStreamSample / kOrderStreamThreads>(composites, kOrderStreamSample, cnt, part16, lo16, hi16);
+  if (!placed) bitonic_sort_lds(comp, kOrderStreamSample);
+  if (tid <= parts) {
+    const int i = (int)(((int64_t)tid * kOrderStreamSample) / parts);
+    const unsigned long long b = tid == 0 ? 0ull : tid == parts ? kOrderEnd : composites[placed ? i : bitonic_slot(i)] & (kOrderEnd - 1ull);
+    bound_lds[tid] = b;
+    if (chunk == 0) bounds[k * (parts + 1) + tid] = b;
+  }
+  __syncthreads();
+  uint32_t where[kOrderChunkPer];  // share << 16 | place in its group
+#pragma unroll
+  for (int r = 0; r < kOrderChunkPer; ++r) {
+    const int e = e0 + tid + kOrderStreamThreads * r;
+    where[r] = 0u;
+    if (e < e1) {
+      const unsigned long long c = (unsigned long long)key[r] << 20 | (unsigned long long)(unsigned)e;
+      int from = 0, until = parts;  // bound_lds[from] <= c < bound_lds[until]
+      while (until - from > 1) {
+        const int mid = (from + until) >> 1;
+        if (bound_lds[mid] <= c)
+          from = mid;
+        else
+          until = mid;
+      }
+      where[r] = (uint32_t)from << 16 | atomicAdd(&group[from], 1u);
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    uint32_t before = 0u;
+#pragma unroll
+    for (int half = 0; half < kOrderStreamMaxParts / 64; ++half) {
+      const uint32_t mine = group[64 * half + lane];
+      uint32_t incl = mine;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+      }
+      group[64 * half + lane] = before + incl - mine;
+      before += __shfl(incl, 63);
+    }
+  }
+  __syncthreads();
+  unsigned long long* __restrict__ const out = grouped + (int64_t)k * kstride + e0;
+#pragma unroll
+  for (int r = 0; r < kOrderChunkPer; ++r) {
+    const int e = e0 + tid + kOrderStreamThreads * r;
+    if (e < e1) out[group[where[r] >> 16] + (where[r] & 0xFFFFu)] = (unsigned long long)key[r] << 20 | (unsigned long long)(unsigned)e;
+  }
+  uint32_t* __restrict__ const off = offsets + ((int64_t)k * parts + chunk) * (parts + 1);
+  if (tid <= parts) off[tid] = tid < parts ? group[tid] : (uint32_t)(e1 - e0);
+}
+
+__global__ __launch_bounds__(kOrderStreamThreads) void objective_order_stream_kernel(const float* __restrict__ xs, int npad, int n, int m,
+                                                                                     int parts, int per, int capacity,
+                                                                                     const int* __restrict__ slot_of,
+                                                                                     SortParam* __restrict__ param,
+                                                                                     const Ctrl* __restrict__ ctrl,
+                                                                                     const uint32_t* __restrict__ offsets,
+                                                                                     const unsigned long long* __restrict__ bounds,
+                                                                                     int* __restrict__ pos, int* __restrict__ upper,
+                                                                                     RadixBuffers buf) {
+  extern __shared__ __attribute__((aligned(16))) double order_stream_comp[];
+  __shared__ int taken;           // composites of the present pass that lie in its range
+  __shared__ int below_of[16];    // per wave: composites below the range
+  __shared__ int upto_of[16];     // per wave: values up to that of the range's end
+  __shared__ uint32_t part16[16];
+  __shared__ uint32_t lo16[16];
+  __shared__ uint32_t hi16[16];
+  __shared__ int group_first[kOrderStreamMaxParts];  // of a chunk's rows of this share: the first one in the chunk, their number, their place here
+  __shared__ int group_rows[kOrderStreamMaxParts];
+  __shared__ int group_at[kOrderStreamMaxParts];
+  __shared__ int share_rows;
+  __shared__ int share_below;
+  if (param->nonfinite != 0 || ctrl->err != 0) return;
   double* const comp = order_stream_comp;
+  unsigned long long* const composites = reinterpret_cast<unsigned long long*>(order_stream_comp);
+  uint32_t* const cnt = reinterpret_cast<uint32_t*>(order_stream_comp + kOrderStreamCapacity);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int k = (int)blockIdx.x % m, part = (int)blockIdx.x / m;
-  if (part >= parts) return;
+  if (blockIdx.x == 0 && tid == 0) param->orders_valid = 1;
   const float* __restrict__ col = xs + (int64_t)k * npad;
+  const unsigned long long* __restrict__ grouped = buf.pairs[1] + (int64_t)k * buf.kstride;
   unsigned long long* __restrict__ sorted = buf.pairs[0] + (int64_t)k * buf.kstride;
-  constexpr unsigned long long kBias = 0x4330000000000000ull;  // the bits of 2^52 as a double
-  constexpr unsigned long long kEnd = 1ull << 52;               // above every composite
-  auto composite = [&](int e) { return ((unsigned long long)ordered_key(col[e]) << 20) | (unsigned long long)(unsigned)e; };
+  int* __restrict__ const pos_k = pos + (int64_t)k * buf.kstride;
+  int* __restrict__ const upper_k = upper + (int64_t)k * buf.kstride;
+  constexpr unsigned long long kBias = kOrderBias, kEnd = kOrderEnd;
+  auto as_entry = [&](unsigned long long c) { return __longlong_as_double((long long)(kBias | c)); };
 
-  // ---- the share: between two members of the sorted sample
-  for (int i = tid; i < kOrderStreamSample; i += kOrderStreamThreads)
-    comp[bitonic_slot(i)] = __longlong_as_double((long long)(kBias | composite((int)(((int64_t)i * n) / kOrderStreamSample))));
-  __syncthreads();
-  bitonic_sort_lds(comp, kOrderStreamSample);
-  auto sample_at = [&](int i) { return (unsigned long long)__double_as_longlong(comp[bitonic_slot(i)]) & (kEnd - 1ull); };
-  unsigned long long lo = part == 0 ? 0ull : sample_at((int)(((int64_t)part * kOrderStreamSample) / parts));
-  const unsigned long long end = part == parts - 1 ? kEnd : sample_at((int)(((int64_t)(part + 1) * kOrderStreamSample) / parts));
-  __syncthreads();  // (the sample is overwritten from here on)
+  // ---- the share: between two members of the sorted sample, a group of every chunk
+  unsigned long long lo = bounds[k * (parts + 1) + part];
+  const unsigned long long end = bounds[k * (parts + 1) + part + 1];
+  auto groups_of = [&](int share) {  // (called by every thread, past the last use of the lists; ends with a barrier)
+    if (wave == 0) {
+      int rows = 0, below = 0;
+#pragma unroll
+      for (int half = 0; half < kOrderStreamMaxParts / 64; ++half) {
+        const int c = 64 * half + lane;
+        const uint32_t* const off = offsets + ((int64_t)k * parts + min(c, parts - 1)) * (parts + 1) + share;
+        const int first = c < parts ? (int)off[0] : 0, here = c < parts ? (int)off[1] - first : 0;
+        int incl = here, firsts = first;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int up = __shfl_up(incl, o), up_first = __shfl_up(firsts, o);
+          if (lane >= o) {
+            incl += up;
+            firsts += up_first;
+          }
+        }
+        group_first[c] = first;
+        group_rows[c] = here;
+        group_at[c] = rows + incl - here;
+        rows += __shfl(incl, 63);
+        below += __shfl(firsts, 63);
+      }
+      if (lane == 0) {
+        share_rows = rows;
+        share_below = below;
+      }
+    }
+    __syncthreads();
+  };
+  groups_of(part);
 
   // One pass over the objective's keys: the composites in [from, to) are counted (the return value) and, with `collect`,
-  // the first `capacity` of them stored; *below = the composites smaller than `from`.
-  auto pass = [&](unsigned long long from, unsigned long long to, bool collect, int* below) {
+  // the first `capacity` of them stored; *below = the composites smaller than `from`, *upto = the rows whose value is at most that
+  // of `to`.  Most keys are told by two comparisons of floats (all are finite), the others by their composites.
+  constexpr uint32_t kLowest = 0x00800000u, kHighest = 0xFF7FFFFFu;  // the keys of the finite values
+  auto value_of = [&](uint32_t key) {  // (a bound of a bisection need not be the key of a value)
+    return key < kLowest ? -INFINITY : key > kHighest ? INFINITY : cost_of_key(key);
+  };
+  auto pass = [&](unsigned long long from, unsigned long long to, bool collect, int* below, int* upto) {
     if (tid == 0) taken = 0;
     __syncthreads();
     const unsigned long long span = to - from;
-    int under = 0;  // (wave-uniform)
+    const float from_value = value_of((uint32_t)(from >> 20)), to_value = to == kEnd ? INFINITY : value_of((uint32_t)(to >> 20));
+    int under = 0, most = 0;  // (wave-uniform)
     // (a wave takes 256 keys a step and fetches the keys of kAhead steps before it looks at the first of them)
     constexpr int kAhead = 8;
     for (int g0 = 256 * wave; g0 < n; g0 += kAhead * 4 * kOrderStreamThreads) {  // (wave-uniform)
@@ -223,7 +476,7 @@ __global__ __launch_bounds__(kOrderStreamThreads) void objective_order_stream_ke
 #pragma unroll
       for (int a = 0; a < kAhead; ++a) {
         const int e0 = g0 + a * 4 * kOrderStreamThreads + 4 * lane;
-        q[a] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        q[a] = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);  // (beyond every value; in no range, whose last value is `to`'s or the largest one)
         if (e0 + 3 < n) {
           q[a] = *reinterpret_cast<const float4*>(col + e0);
         } else if (e0 < n) {
@@ -238,80 +491,153 @@ __global__ __launch_bounds__(kOrderStreamThreads) void objective_order_stream_ke
         if (b0 >= n) break;  // (wave-uniform)
         const int e0 = b0 + 4 * lane;
         const float v[4] = {q[a].x, q[a].y, q[a].z, q[a].w};
-        unsigned long long c[4];
-        uint64_t in[4];
-        int here = 0;
+        uint64_t near[4];
+        uint64_t any = 0ull;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          c[u] = ((unsigned long long)ordered_key(v[u]) << 20) | (unsigned long long)(unsigned)(e0 + u);
-          const bool live = e0 + u < n;
-          in[u] = __builtin_amdgcn_ballot_w64(live && c[u] - from < span);
-          under += __popcll(__builtin_amdgcn_ballot_w64(live && c[u] < from));
-          here += __popcll(in[u]);
+          const uint64_t less = __builtin_amdgcn_ballot_w64(v[u] < from_value);
+          const uint64_t least = __builtin_amdgcn_ballot_w64(v[u] <= to_value);
+          near[u] = least & ~less;
+          under += __popcll(less);
+          most += __popcll(least);
+          any |= near[u];
         }
-        if (here != 0) {  // (wave-uniform)
-          int at = 0;
-          if (lane == 0) at = atomicAdd(&taken, here);
-          at = __builtin_amdgcn_readfirstlane(at);
-          if (collect) {
+        if (any != 0ull) {  // (wave-uniform)
+          unsigned long long c[4];
+          uint64_t in[4];
+          int here = 0;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int mine = at + __popcll(in[u] & ((1ull << lane) - 1ull));
-              if (((in[u] >> lane) & 1ull) != 0ull && mine < capacity)
-                comp[bitonic_slot(mine)] = __longlong_as_double((long long)(kBias | c[u]));
-              at += __popcll(in[u]);
+          for (int u = 0; u < 4; ++u) {
+            c[u] = ((unsigned long long)ordered_key(v[u]) << 20) | (unsigned long long)(unsigned)(e0 + u);
+            const bool live = (near[u] >> lane & 1ull) != 0ull && e0 + u < n;
+            in[u] = __builtin_amdgcn_ballot_w64(live && c[u] - from < span);
+            under += __popcll(__builtin_amdgcn_ballot_w64(live && c[u] < from));
+            here += __popcll(in[u]);
+          }
+          if (here != 0) {  // (wave-uniform)
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&taken, here);
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (collect) {
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                const int mine = at + __popcll(in[u] & ((1ull << lane) - 1ull));
+                if (((in[u] >> lane) & 1ull) != 0ull && mine < capacity) comp[bitonic_slot(mine)] = as_entry(c[u]);
+                at += __popcll(in[u]);
+              }
             }
           }
         }
       }
     }
-    if (lane == 0) below_of[wave] = under;
+    if (lane == 0) {
+      below_of[wave] = under;
+      upto_of[wave] = most;
+    }
     __syncthreads();
     if (below != nullptr) {
-      int sum = 0;
+      int sum = 0, sum_upto = 0;
 #pragma unroll
-      for (int w = 0; w < kOrderStreamThreads / 64; ++w) sum += below_of[w];
+      for (int w = 0; w < kOrderStreamThreads / 64; ++w) {
+        sum += below_of[w];
+        sum_upto += upto_of[w];
+      }
       *below = sum;
+      *upto = sum_upto;
     }
     const int count = taken;
     __syncthreads();  // (everybody has read the counters before the next pass clears them)
     return count;
   };
 
-  int run_start = 0;
-  bool first = true;
-  while (lo < end) {  // (the same in every thread)
+  const bool whole = share_rows <= capacity;  // (the same in every thread, as all that steers the loop)
+  while (lo < end) {
     unsigned long long hi = end;
-    int below = 0;
-    int count = pass(lo, hi, true, &below);
-    if (first) run_start = below;
-    first = false;
-    if (count > capacity) {
+    int below = share_below, upto = 0, count = share_rows;
+    if (whole) {
+      // thirty-two lanes to a group
+      for (int c = tid >> 5; c < parts; c += kOrderStreamThreads / 32) {
+        const unsigned long long* __restrict__ const from = grouped + (int64_t)c * per + group_first[c];
+        for (int i = tid & 31; i < group_rows[c]; i += 32) comp[bitonic_slot(group_at[c] + i)] = as_entry(from[i]);
+      }
+      __syncthreads();
+    } else {
+      count = pass(lo, hi, true, &below, &upto);
       // [lo, fits) holds at most one composite; [lo, over) too many
       unsigned long long fits = lo + 1ull, over = hi;
-      while (over - fits > 1ull) {
-        const unsigned long long mid = fits + (over - fits) / 2ull;
-        if (pass(lo, mid, false, nullptr) <= capacity)
-          fits = mid;
-        else
-          over = mid;
+      if (count > capacity) {
+        while (over - fits > 1ull) {
+          const unsigned long long mid = fits + (over - fits) / 2ull;
+          if (pass(lo, mid, false, nullptr, nullptr) <= capacity)
+            fits = mid;
+          else
+            over = mid;
+        }
+        hi = fits;
+        count = pass(lo, hi, true, &below, &upto);
       }
-      hi = fits;
-      count = pass(lo, hi, true, nullptr);
     }
     if (count > 0) {
-      int padded = kRowsBitonicMin;
-      while (padded < count) padded <<= 1;
-      for (int e = count + tid; e < padded; e += kOrderStreamThreads) comp[bitonic_slot(e)] = (double)INFINITY;
-      __syncthreads();
-      bitonic_sort_lds(comp, padded);
+      bool placed;
+      if (count <= 4 * kOrderStreamThreads)
+        placed = order_stream_place<4>(composites, count, cnt, part16, lo16, hi16);
+      else if (count <= 8 * kOrderStreamThreads)
+        placed = order_stream_place<8>(composites, count, cnt, part16, lo16, hi16);
+      else
+        placed = order_stream_place<kOrderStreamPer>(composites, count, cnt, part16, lo16, hi16);
+      if (!placed) {
+        int padded = kRowsBitonicMin;
+        while (padded < count) padded <<= 1;
+        for (int e = count + tid; e < padded; e += kOrderStreamThreads) comp[bitonic_slot(e)] = (double)INFINITY;
+        __syncthreads();
+        bitonic_sort_lds(comp, padded);
+      }
+      auto entry_at = [&](int e) { return composites[placed ? e : bitonic_slot(e)] & (kEnd - 1ull); };
+      const uint32_t hi_key = (uint32_t)(hi >> 20);
+      if (whole && hi < kEnd && (uint32_t)(entry_at(count - 1) >> 20) == hi_key) {
+        // (rows of the last value lie in the next shares too, up to the last share that begins no later than that value ends)
+        const unsigned long long* const bound = bounds + k * (parts + 1);
+        int share = part + 1, behind = parts;  // bound[share] is of that value, bound[behind] of a larger one
+        while (behind - share > 1) {
+          const int mid = (share + behind) >> 1;
+          if ((uint32_t)(bound[mid] >> 20) == hi_key)
+            share = mid;
+          else
+            behind = mid;
+        }
+        __syncthreads();
+        if (tid == 0) taken = 0;
+        groups_of(share);
+        int equal = 0;
+        for (int c = tid >> 5; c < parts; c += kOrderStreamThreads / 32)
+          for (int i = tid & 31; i < group_rows[c]; i += 32) equal += (uint32_t)(grouped[(int64_t)c * per + group_first[c] + i] >> 20) == hi_key ? 1 : 0;
+        if (equal != 0) atomicAdd(&taken, equal);
+        __syncthreads();
+        upto = share_below + taken;
+      }
       for (int e = tid; e < count; e += kOrderStreamThreads) {
-        const unsigned long long c = (unsigned long long)__double_as_longlong(comp[bitonic_slot(e)]) & (kEnd - 1ull);
-        sorted[run_start + e] = ((c >> 20) << 32) | (c & 0xFFFFFull);
+        const unsigned long long c = entry_at(e);
+        const uint32_t key = (uint32_t)(c >> 20);
+        const int slot = slot_of[(int)(c & 0xFFFFFull)];
+        sorted[below + e] = ((unsigned long long)key << 32) | (c & 0xFFFFFull);
+        // the rows of its value or a smaller one: up to the first entry of a larger value, or beyond this range where `hi` cuts its value
+        int last = e + 1;
+        if (last < count && (uint32_t)(entry_at(last) >> 20) == key) {
+          int from = e + 2, until = count;
+          while (from < until) {
+            const int mid = (from + until) >> 1;
+            if ((uint32_t)(entry_at(mid) >> 20) > key)
+              until = mid;
+            else
+              from = mid + 1;
+          }
+          last = from;
+        }
+        pos_k[slot] = below + e;
+        upper_k[slot] = hi < kEnd && key == hi_key ? upto : below + last;
       }
       __syncthreads();
     }
-    run_start += count;
     lo = hi;
   }
 }

@@ -52,6 +52,14 @@ def test_populations_whose_peel_orders_their_last_fronts_take_one_launch_for_wha
     assert "crowd_terms_kernel" not in second and "crowd_gather_kernel" in second
 
 
+def test_objective_orders_from_shares():
+    # (smaller than the sizes at which they take this path by themselves; the shares of the last one do not fit)
+    specs = ["-o", "prefix_min_rows=16384", "-o", "mid_argsort=0", "select:17001:3:grid", "select:17000:3:layers", "rank:17000:5:simplex",
+             "-o", "order_stream_capacity=1000", "select:17003:5:shell"]
+    out = emulated.run(specs, EMU_TRACE="1")
+    assert out.count("ok ") == 4 and out.count("objective_shares_kernel") == 4
+
+
 _COUNT_FIRST = ["-o", "prefix_count_first=2", "-o", "prefix_min_rows=16384"]
 
 
