@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kMidArgsortThreads) void objective_order_lds_kernel
 //     positions and bounds by slot.  A share that does not fit `capacity` entries -- rows arranged so that the sample
 //     misses where they crowd -- is taken in pieces instead, each collected in a pass over all keys: the largest stretch of composites from
 //     the share's start that fits is found by bisection over the composites, a pass per step, as often as it takes.
-// Placing is by buckets (of equal width in the value, then in the composite: shares of one
+// Placing is by buckets (of equal width in the value; where they crowd, of the index for the rows of the share's first and last
 // value), every entry among those of its bucket; the network of radix.hpp only sorts what crowds in both.
 // A workgroup that read all keys of its objective for its share, and sorted that by the network, took 78 us of vector issue for the
 // reading alone at 200 000 rows (96 us, 20 more for positions and bounds in a launch of their own; 160 us and more by the radix sort
@@ -220,17 +220,49 @@ __device__ inline bool order_stream_place(unsigned long long* comp, int count, u
     lo = min(lo, lo16[w]);
     hi = max(hi, hi16[w]);
   }
-  // (by value: finite values only; by composite: the rows of one value by their index)
+  // (by value: finite values only; by ends: the rows of the smallest and of the largest value by their index, a quarter of the buckets each,
+  // the others by value in between -- shares of one value or two)
   const float v0 = cost_of_key(lo), width = cost_of_key(hi) - v0;
   const bool by_value = lo < hi && width > 0.0f && width <= 3.4028234663852886e38f;
   const float scale = by_value ? (float)(kOrderStreamBuckets - 1) / width : 0.0f;
-  const unsigned long long from = (unsigned long long)lo << 20, span = ((unsigned long long)hi << 20 | 0xFFFFFull) - from;
-  const float scale_all = (float)(kOrderStreamBuckets - 1) / (float)span;
+  uint32_t first_lo = 0u, first_hi = 0u;
+  float scale_lo = 0.0f, scale_hi = 0.0f;
 #pragma unroll 1
   for (int attempt = by_value ? 0 : 1; attempt < 2; ++attempt) {
-    auto bucket_of_entry = [&](unsigned long long c) {
-      const float t = attempt == 0 ? (cost_of_key((uint32_t)(c >> 20)) - v0) * scale : (float)(c - from) * scale_all;
-      return min((uint32_t)t, (uint32_t)kOrderStreamBuckets - 1u);
+    if (attempt == 1) {
+      // the smallest and the largest index with either value
+      uint32_t at[4] = {~0u, ~0u, ~0u, ~0u};
+#pragma unroll
+      for (int r = 0; r < PER; ++r) {
+        if (tid + kOrderStreamThreads * r < count) {
+          const uint32_t key = (uint32_t)(mine[r] >> 20), index = (uint32_t)(mine[r] & 0xFFFFFull);
+          if (key == lo) at[0] = min(at[0], index), at[1] = min(at[1], ~index);
+          if (key == hi) at[2] = min(at[2], index), at[3] = min(at[3], ~index);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t of_wave = wave_prefix_min(at[i]);
+        if (lane == 63) cnt[16 * i + wave] = of_wave;
+      }
+      __syncthreads();
+      for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) at[i] = min(at[i], cnt[16 * i + w]);
+      __syncthreads();
+      first_lo = at[0];
+      first_hi = at[2];
+      scale_lo = (float)(kOrderStreamBuckets / 4 - 1) / (float)(~at[1] - at[0] + 1u);
+      scale_hi = (float)(kOrderStreamBuckets / 4 - 1) / (float)(~at[3] - at[2] + 1u);
+    }
+    auto bucket_of_entry = [&](unsigned long long c) -> uint32_t {
+      const uint32_t key = (uint32_t)(c >> 20), index = (uint32_t)(c & 0xFFFFFull);
+      const uint32_t t = by_value ? min((uint32_t)((cost_of_key(key) - v0) * scale), (uint32_t)kOrderStreamBuckets - 1u) : 0u;
+      if (attempt == 0) return t;
+      constexpr uint32_t kQuarter = (uint32_t)kOrderStreamBuckets / 4u;
+      if (key == lo) return min((uint32_t)((float)(index - first_lo) * scale_lo), kQuarter - 1u);
+      if (key == hi) return 3u * kQuarter + min((uint32_t)((float)(index - first_hi) * scale_hi), kQuarter - 1u);
+      return kQuarter + t / 2u;
     };
     reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
