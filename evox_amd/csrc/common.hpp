@@ -185,6 +185,18 @@ struct Ctrl {
   unsigned long long arrive[1];  // one slot per block (allocated to the grid size)
 };
 constexpr int kReleaseCopies = 32;
+
+// Whether an earlier kernel of the call, or another workgroup of this launch, has given up: the same answer for the whole
+// workgroup.  (A look of every wave's own is not: where the word is set between the looks of two waves, the ones that stay go on
+// with LDS that the others were to fill, wait for what they were to write, or index with it.)  Every thread calls it; word: LDS that
+// nobody else uses before its last barrier.
+__device__ inline bool call_failed(const Ctrl* ctrl, int* word) {
+  if (threadIdx.x == 0) *word = coherent_load(&ctrl->err);
+  __syncthreads();
+  const bool failed = *word != 0;
+  __syncthreads();
+  return failed;
+}
 constexpr unsigned long long kReleaseGiveUp = ~0ull;
 
 }  // namespace evx

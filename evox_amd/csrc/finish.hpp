@@ -253,7 +253,7 @@ __device__ inline void crowd_sort_body(const CrowdArgs& a, unsigned gen0, int ep
   float* __restrict__ dist = a.dist;
   uint32_t* __restrict__ dkey = a.dkey;
   int* __restrict__ order = a.order;
-  if (coherent_load(&ctrl->err) != 0) return;
+  if (call_failed(ctrl, scratch)) return;
   const int nv = ctrl->nv;
   if (a.mid_sort == 2 && crowd_runs_take(a, nv)) return;  // another launch's front
   if (fused != 0 && fused_front_applies(nv, m)) {  // a small front: distances (and order) right here
@@ -455,7 +455,7 @@ __device__ inline void crowd_finish_body(const CrowdArgs& a, int want_order, uns
   float* __restrict__ dist = a.dist;
   uint32_t* __restrict__ dkey = a.dkey;
   int* __restrict__ order = a.order;
-  if (coherent_load(&ctrl->err) != 0) return;
+  if (call_failed(ctrl, scratch)) return;
   const int nv = ctrl->nv;
   if (a.mid_sort == 2 && crowd_runs_take(a, nv)) return;  // another launch's front
   if (fused != 0 && fused_front_applies(nv, m)) return;  // crowd_sort_kernel has done it all
@@ -574,13 +574,13 @@ __global__ __launch_bounds__(kRunRows) void crowd_runs_kernel(CrowdArgs a, int a
   __shared__ int scratch[1];
   if constexpr (MANY) to_population(a);
   if (after_peel_tail != 0 && a.ctrl->tail_done != 0) return;
-  if (coherent_load(&a.ctrl->err) != 0) return;
   const int nv = a.ctrl->nv, m = a.m;
-  if (a.mid_sort == 1 && crowd_small_takes(a, nv)) {
+  if (a.mid_sort == 1 && crowd_small_takes(a, nv)) {  // (the workgroups of such a launch wait for each other)
+    if (call_failed(a.ctrl, scratch)) return;
     crowd_small_front(a.xs, a.npad, a.list_base, a.ctrl, m, a.dist, a.dkey, a.order, a.spin_limit, a.fused, small_blocks, finish_lds, scratch);
     return;
   }
-  if (!crowd_runs_take(a, nv)) return;
+  if (coherent_load(&a.ctrl->err) != 0 || !crowd_runs_take(a, nv)) return;
   const int* __restrict__ list = a.list_base + a.ctrl->worst_start;
   const int runs = runs_of(nv);
   for (int item = blockIdx.x; item < runs * m; item += gridDim.x) {
@@ -783,12 +783,12 @@ __global__ __launch_bounds__(T) void crowd_gather_kernel(CrowdArgs a, GatherArgs
     to_population(g);
   }
   Ctrl* ctrl = a.ctrl;
-  if (coherent_load(&ctrl->err) != 0) {
-    gather_body(g, blockIdx.x, gridDim.x, 0);
+  if (ctrl->tail_done != 0) {  // (no workgroup of this launch waits then; after a failed wait of an earlier one nothing is gathered)
+    gather_body(g, blockIdx.x, gridDim.x, ctrl->worst_start);
     return;
   }
-  if (ctrl->tail_done != 0) {
-    gather_body(g, blockIdx.x, gridDim.x, ctrl->worst_start);
+  if (call_failed(ctrl, scratch)) {
+    gather_body(g, blockIdx.x, gridDim.x, 0);
     return;
   }
   const unsigned gen0 = radix_generation_base(ctrl);

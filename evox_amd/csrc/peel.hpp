@@ -732,7 +732,7 @@ __global__ __launch_bounds__(kPeelThreads) void peel_kernel(const uint64_t* __re
   extern __shared__ uint64_t front_lds[];  // nwords words (nwords is even: rows are padded to 128),
                                            // followed by nwords more (unranked rows) in witness mode
   __shared__ int scratch[kPeelThreads];
-  if (coherent_load(&ctrl->err) != 0) return;  // an earlier kernel of this call gave up
+  if (call_failed(ctrl, scratch)) return;
 
   if (blockIdx.x == 0) {
     // ---- master: nothing but the barrier
@@ -1027,7 +1027,7 @@ __global__ __launch_bounds__(kRecThreads) void peel_records_kernel(
                                          // (result bits, row, result word) and the (slot, original index) pairs
                                          // of the rows just ranked
   __shared__ int sh[32];
-  if (coherent_load(&ctrl->err) != 0) return;
+  if (call_failed(ctrl, sh)) return;
   constexpr int kRecUnits = WIDE ? evx::kRecUnitsWide : evx::kRecUnits;  // (units of a generation, in this kernel)
   constexpr int kRecLoads = kRecUnits / kRecThreads;
   const int units = record_units(sweepers, kRecUnits);  // per record

@@ -251,7 +251,8 @@ __global__ __launch_bounds__(kLdsPeelThreads) void peel_lds_kernel(
     to_population(ws_step, dom, orig_of, rank, dist_fill, fronts_slot, fronts_orig, fsize, perm, fstart, ctrl, records);
     to_population(ws_step, tail.xs_sorted, tail.dist, tail.order, tail.buffer);
   }
-  if (coherent_load(&ctrl->err) != 0) return;
+  // (the error word as call_failed has it, without its barriers: thread 0 looks, and the workgroup goes by that behind its first one)
+  if (threadIdx.x == 0) sh[40] = coherent_load(&ctrl->err);
   int units = 2;  // per record: the largest power of two up to 32 that gives every sweeper a record
   while (units * 2 * sweepers <= kRecUnits && units < 32) units *= 2;
   const int tid = threadIdx.x;
@@ -268,6 +269,8 @@ __global__ __launch_bounds__(kLdsPeelThreads) void peel_lds_kernel(
     int* word_base = reinterpret_cast<int*>(front_lds + nwords);
     uint16_t* orig_lds = reinterpret_cast<uint16_t*>(word_base + nwords);
     for (int j = tid; j < n; j += blockDim.x) orig_lds[j] = (uint16_t)orig_of[j];
+    __syncthreads();
+    if (sh[40] != 0) return;
     int ranked = 0;
     bool prev_overflow = false;
     // The two units that this thread reads are loaded a level ahead, before the listing of the present level: while
@@ -404,6 +407,7 @@ __global__ __launch_bounds__(kLdsPeelThreads) void peel_lds_kernel(
     if (lane == 63) sh[8 + wave] = incl;
     if (tid < 8) sh[tid] = 0;
     __syncthreads();
+    if (sh[40] != 0) return;
     int before = 0;
     for (int v = 0; v < wave; ++v) before += sh[8 + v];
     if (tid < rows_cap) row_off[tid] = before + incl - rw;

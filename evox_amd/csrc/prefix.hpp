@@ -82,7 +82,7 @@ __global__ __launch_bounds__(kRadixThreads) void objective_order_kernel(const fl
   __shared__ int base[256];
   __shared__ int scratch[kRadixThreads];
   if (param->nonfinite != 0) return;
-  if (coherent_load(&ctrl->err) != 0) return;
+  if (call_failed(ctrl, scratch)) return;
   const unsigned gen0 = radix_generation_base(ctrl);
   if (blockIdx.x == 0) {
     radix_master(ctrl, gen0, 12, spin_limit, scratch);

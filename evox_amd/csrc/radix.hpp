@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kRadixThreads) void argsort_step_kernel(const void*
   extern __shared__ int radix_lds[];
   __shared__ int base[256];
   __shared__ int scratch[kRadixThreads];
-  if (coherent_load(&ctrl->err) != 0) return;
+  if (call_failed(ctrl, scratch)) return;
   const unsigned gen0 = radix_generation_base(ctrl);
   const bool capped = key_cap != nullptr && kind == kKeyInt32;
   const uint32_t cap = capped ? (uint32_t)*key_cap : 0xFFFFFFFFu;

@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kTwoThreads) void two_peel_kernel(const float* __re
   __shared__ __attribute__((aligned(16))) uint32_t in_lds[2][4];
   __shared__ int ranked_lds[2];    // rows this workgroup ranked in a round, by the parity of the round
   __shared__ int unranked_lds[kTwoWaves];
-  if (coherent_load(&ctrl->err) != 0) return;
+  if (call_failed(ctrl, ranked_lds)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = blockIdx.x;

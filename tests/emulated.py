@@ -82,6 +82,7 @@ def _translate(name, text):
     text = re.sub(r"__attribute__\(\(amdgpu_waves_per_eu\(.*?\)\)\) void", "void", text)
     if "zero_words[" in text or "words[i] = 0u" in text:  # (one loop clears several regions and what lies between them)
         text = re.sub(r"(\w+)\[(\w)\] = 0u;", r"{ if (!__asan_address_is_poisoned(&\1[\2])) \1[\2] = 0u; }", text)
+    text = re.sub(r"coherent_load\(&((?:a\.)?ctrl->err)\)", r"emu_error_word(&\1, kErrBarrierTimeout)", text)
     if name == "calibrate.hpp":
         text = re.sub(r"asm volatile\(.*?\);", ";", text, flags=re.S)
     if name == "peel_lds.hpp":

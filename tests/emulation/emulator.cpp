@@ -7,7 +7,9 @@
 // which lets the lanes still inside a loop finish it before those behind it go on.
 //
 // EMU_CUS: compute units of the device (256).  EMU_TRACE: print every launch.  EMU_GIVE_UP: waits inside launches of the
-// kernel of this name run out at their first look at the clock.
+// kernel of this name run out at their first look at the clock.  EMU_ERROR_BEHIND=name:launch:block:look: in that
+// launch (1, 2, ...) of those with this in their names, another workgroup sets the error word right behind that look (1, 2, ...) that
+// the first wave of that workgroup takes at it; a wave of the workgroup that sees it at the same point ends the run.
 #include <hip/hip_runtime.h>
 
 #include <sched.h>
@@ -72,12 +74,16 @@ struct Worker {
   Fiber* now = nullptr;
   char* stacks = nullptr;
   size_t n_stacks = 0;
-  unsigned loads = 0;
+  unsigned loads = 0, barriers = 0;  // (barriers: that the workgroup has passed)
   bool spinning;
 };
 static thread_local Worker* W;
 static const bool g_trace = getenv("EMU_TRACE") != nullptr;
 static bool g_give_up;
+static int g_look;          // the look at the error word behind which it is set; 0: none
+static unsigned g_look_block;
+static unsigned g_look_barriers;
+static int g_looks_of[1024];  // looks that the lanes of that workgroup have taken
 constexpr size_t kStack = 64 * 1024;
 
 static void to_main() {
@@ -134,6 +140,7 @@ static void run_block(Worker& w, int threads) {
     w.stacks = (char*)mmap(nullptr, threads * kStack, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     w.n_stacks = threads;
   }
+  w.barriers = 0;
   const int waves = (threads + 63) / 64;
   w.f.resize(threads);
   w.vals.resize((size_t)waves * 64);
@@ -205,6 +212,7 @@ static void run_block(Worker& w, int threads) {
       every &= (int)f.v;
     }
     if (all_wait && waiting) {
+      ++w.barriers;
       for (auto& f : w.f)
         if (f.st == kBlock) {
           f.any = any;
@@ -275,6 +283,15 @@ void run(const char* name, dim3 g, dim3 b, size_t lds, const std::function<void(
   }
   const char* give_up = getenv("EMU_GIVE_UP");
   g_give_up = give_up != nullptr && strcmp(give_up, name) == 0;
+  char behind[100] = "";
+  int launch = 0, look = 0;
+  g_look = 0;
+  if (const char* e = getenv("EMU_ERROR_BEHIND"); e && sscanf(e, "%99[^:]:%d:%u:%d", behind, &launch, &g_look_block, &look) == 4 && strstr(name, behind)) {
+    static int launches;
+    if (++launches == launch) g_look = look;
+    memset(g_looks_of, 0, sizeof(g_looks_of));
+    g_look_barriers = ~0u;
+  }
   std::unique_lock<std::mutex> l(mu);
   gdim = g;
   bdim = b;
@@ -302,6 +319,23 @@ long long wall_clock64() {
   static std::atomic<long long> leap{0};
   if (emu::g_give_up) return (leap += 1ll << 40) | 1;
   return (std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch()).count() / 100000) | 1;
+}
+
+int emu_error_word(const int* p, int failed) {
+  if (emu::g_look == 0 || blockIdx.x != emu::g_look_block) return emu_aload(p);
+  const int v = __atomic_load_n(p, __ATOMIC_SEQ_CST);  // (no lane lets the others go on here: the first wave looks first)
+  const int look = ++emu::g_looks_of[threadIdx.x];
+  if (threadIdx.x == 0 && look == emu::g_look) {
+    fprintf(stderr, "another workgroup gives up\n");
+    emu_astore(const_cast<int*>(p), failed);
+    emu::g_look_barriers = emu::W->barriers;
+  } else if (threadIdx.x < 64) {
+    return look == emu::g_look ? 0 : v;  // (the lanes of a wave look together)
+  } else if (v != 0 && look <= emu::g_look && emu::W->barriers == emu::g_look_barriers) {
+    fprintf(stderr, "emulator: the waves of a workgroup see different error words\n");
+    abort();
+  }
+  return v;
 }
 
 using emu::block_op;

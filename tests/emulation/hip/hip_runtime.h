@@ -113,6 +113,7 @@ template <class T, class U> inline T atomicMin(T* p, U v) { T o = __atomic_load_
 template <class T, class U, class V> inline T atomicCAS(T* p, U a, V b) { T o = (T)a; __atomic_compare_exchange_n(p, &o, (T)b, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST); return o; }
 template <class T> __attribute__((noinline)) T emu_aload(const T* p) { emu::load_yield(); T v; __atomic_load(const_cast<T*>(p), &v, __ATOMIC_SEQ_CST); return v; }
 #define __hip_atomic_load(p, o, s) emu_aload(p)
+int emu_error_word(const int* p, int failed);  // a look at the error word of a call; `failed`: what says that a wait ran out
 // A 16-byte load of two 8-byte units, each of which arrives as a whole.
 template <class V> inline void emu_load_pair(V& r, const unsigned long long* p) {
   const unsigned long long a = emu_aload(p), b = emu_aload(p + 1);

@@ -29,6 +29,24 @@ def test_nothing_follows_an_order_whose_sort_ran_out_of_time():
     assert "ok " in emulated.run(["select:33000:2:uniform::::poisoned"], EMU_GIVE_UP="argsort_step_kernel")
 
 
+@pytest.mark.parametrize("options,spec,look", [
+    ("", "select:33000:2:uniform", "argsort_step_kernel:1:2:1"),
+    ("", "select:33000:2:uniform", "two_peel_kernel:1:4:1"),
+    ("peel_lds=0 peel_records=0", "select:1500:3:uniform", "peel_kernel:1:5:1"),
+    ("peel_lds=0", "select:1500:3:uniform", "peel_records_kernel:1:5:1"),
+    ("", "select:1500:3:uniform", "kernel:3:5:1"),  # peel_lds_kernel
+    ("peel_lds=0", "select:1500:3:uniform", "crowd_runs_kernel:1:0:1"),
+    ("", "select:1500:3:simplex", "crowd_gather_kernel:1:0:1"),
+    ("", "select:1500:3:simplex", "crowd_gather_kernel:1:0:2"),  # crowd_sort_body, crowd_finish_body
+    ("", "select:1500:3:simplex", "crowd_gather_kernel:1:0:3"),
+])
+def test_a_workgroup_leaves_as_a_whole(options, spec, look):
+    # (another workgroup's wait runs out while this one starts: between the looks that two of its waves take at the error word)
+    set_to = ["spin_limit=20000"] + options.split()
+    out = emulated.run([a for o in set_to for a in ("-o", o)] + [spec + "::::poisoned"], EMU_ERROR_BEHIND=look)
+    assert "ok " in out and "another workgroup gives up" in out
+
+
 @pytest.mark.parametrize("spec,searched", [("crowd:1365:3:uniform", False), ("crowd:1366:3:uniform", True), ("crowd:1100:2:grid", False)])
 def test_small_fronts_are_done_in_the_first_ordering_launch(spec, searched):
     # (1365 x 3 values fit the workgroups that order a small front whatever the mask selects: one launch, nothing behind it)
