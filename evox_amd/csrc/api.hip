@@ -994,7 +994,7 @@ static int launch_dominance_prefix(const Ws& w, hipStream_t s, int phase) {
     hipLaunchKernelGGL(kernel, dim3(tiles, stretches), dim3(kPrefixThreads), lds, s, w.at<int>(L.pos), w.at<int>(L.scost),
                        w.at<uint32_t>(L.kid_sorted), w.at<uint64_t>(L.dom), L.n, L.kstride, L.wstride, L.nwords, shift, buckets,
                        chunk, bands, phase == 0 ? opt().prefix_mode : phase, w.at<int>(L.total0), w.at<int>(L.witness0),
-                       w.at<SortParam>(L.sortparam), phase == 2 ? w.at<int>(L.fsize) : (const int*)nullptr, (int)w.matrix_unless,
+                       w.at<SortParam>(L.sortparam), w.ctrl(), phase == 2 ? w.at<int>(L.fsize) : (const int*)nullptr, (int)w.matrix_unless,
                        NearbyWork{});
     EVX_LAUNCH_CHECK();
     return 0;
@@ -1076,7 +1076,7 @@ static int launch_nearby_totals(const Ws& w, hipStream_t s) {
   const NearbyWork work = {w.at<int>(box), w.at<uint16_t>(near_list), w.at<int>(near_count), w.at<int2>(full), w.at<int2>(rest), w.at<int>(queue), cap};
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(kPrefixThreads), lds, s, w.at<int>(pos_at), w.at<int>(upper_at), (const uint32_t*)nullptr,
                      (uint64_t*)nullptr, L.n, stride, (int64_t)0, groups, 0, kPrefixBuckets, 0, 0, 1, w.at<int>(L.total0), w.at<int>(L.witness0),
-                     param, &w.ctrl()->err, 0, work);
+                     param, w.ctrl(), (const int*)nullptr, 0, work);
   EVX_LAUNCH_CHECK();
   return 0;
 }

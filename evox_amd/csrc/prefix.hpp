@@ -926,7 +926,7 @@ __device__ __forceinline__ uint64_t wave_scan_halves(uint64_t v, Op op) {  // (n
 // every row of the stretch and adds their popcount to total0[row]; witness0[row] = the highest non-empty word so far
 // (both start from objective_order_kernel's 0 and -1).  Sets param->totals_valid.  mode: bit 0 = the row totals,
 // bit 1 = the matrix.  NEARBY: the totals alone, of rows in spatial order, by workgroups that take parts of
-// the work until none is left (unless_front0: the error word).  unless_front0 (null: always run): the size of front 0, known from a launch with mode 1 and the
+// the work until none is left.  unless_front0 (null: always run): the size of front 0, known from a launch with mode 1 and the
 // count stage; when it holds `enough` rows nobody will read the matrix, and the launch (mode 2) does nothing.
 struct NearbyWork {
   const int* box;         // [tile][objective]: smallest and largest position
@@ -943,14 +943,15 @@ __global__ __launch_bounds__(kPrefixThreads) void dominance_prefix_kernel(const 
                                                                           int64_t wstride, int nwords, int shift, int buckets,
                                                                           int chunk, int bands, int mode, int* __restrict__ total0,
                                                                           int* __restrict__ witness0, SortParam* __restrict__ param,
-                                                                          const int* __restrict__ unless_front0, int enough, NearbyWork work) {
+                                                                          const Ctrl* __restrict__ ctrl, const int* __restrict__ unless_front0, int enough,
+                                                                          NearbyWork work) {
   static_assert(!NEARBY || TT == 1, "a tile of rows in spatial order");
   constexpr int TS = 64 * WW, T = kPrefixThreads;
   constexpr int TPL = 16 / (WW * TT);  // workgroups that share a 128-byte line of the matrix
   constexpr int MPL = TS / 64;  // members of the tile per lane when a wave walks through them
   extern __shared__ uint64_t prefix_lds[];
-  if (param->nonfinite != 0) return;
-  if (unless_front0 != nullptr && (NEARBY ? *unless_front0 != 0 : *unless_front0 >= enough)) return;
+  if (param->nonfinite != 0 || ctrl->err != 0) return;  // (after a failed wait nobody has written the positions, which index the tables)
+  if (unless_front0 != nullptr && *unless_front0 >= enough) return;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) param->totals_valid = 1;  // for the count stage
   __shared__ uint16_t nearby[NEARBY ? kPrefixNearbyGroups : 1];
   __shared__ int nearby_item;

@@ -29,9 +29,17 @@ def test_nothing_follows_an_order_whose_sort_ran_out_of_time():
     assert "ok " in emulated.run(["select:33000:2:uniform::::poisoned"], EMU_GIVE_UP="argsort_step_kernel")
 
 
+@pytest.mark.parametrize("options,spec", [("mid_argsort=0", "select:17001:3:uniform::"), ("prefix_count_first=2 prefix_nearby=2", "select:33000:3:simplex::9000")])
+def test_no_matrix_follows_orders_whose_sort_ran_out_of_time(options, spec):
+    # (it is built from positions that nobody has written then)
+    set_to = ["prefix_min_rows=16384", "order_stream=0"] + options.split()
+    assert "ok " in emulated.run([a for o in set_to for a in ("-o", o)] + [spec + "::poisoned"], EMU_GIVE_UP="objective_order_kernel")
+
+
 @pytest.mark.parametrize("options,spec,look", [
     ("", "select:33000:2:uniform", "argsort_step_kernel:1:2:1"),
     ("", "select:33000:2:uniform", "two_peel_kernel:1:4:1"),
+    ("prefix_min_rows=16384 mid_argsort=0 order_stream=0", "select:17001:3:uniform", "objective_order_kernel:1:2:1"),
     ("peel_lds=0 peel_records=0", "select:1500:3:uniform", "peel_kernel:1:5:1"),
     ("peel_lds=0", "select:1500:3:uniform", "peel_records_kernel:1:5:1"),
     ("", "select:1500:3:uniform", "kernel:3:5:1"),  # peel_lds_kernel
