@@ -110,7 +110,8 @@ def _passes(batch: int, per_launch: int):
 
 
 def _rank_many(flat_f: torch.Tensor, flat_out: torch.Tensor, count: int) -> None:
-    """Ranks of (B, N, M) float32 fitness as far as the front that holds the count-th row, into (B, N) int32."""
+    """Ranks of (B, N, M) float32 fitness as far as the front that holds the count-th row, into (B, N) int32; called with
+    the stream's lock."""
     batch, n, m = flat_f.shape
     if batch == 1:
         ws = runtime.workspace(n, m, flat_f.device)
@@ -156,7 +157,8 @@ def nd_rank(f: torch.Tensor) -> torch.Tensor:
                       flat_f.stride(1), flat_f.stride(2), flat_out.data_ptr(), runtime.stream_handle(f.device))
             runtime.note_small_kernel_call()
         else:
-            _rank_many(flat_f, flat_out, n)
+            with runtime.turn(f.device):
+                _rank_many(flat_f, flat_out, n)
     return out
 
 
@@ -201,7 +203,7 @@ def nd_rank_until(f: torch.Tensor, count: int) -> torch.Tensor:
     out = torch.empty(f32.shape[:-1], dtype=torch.int32, device=f.device)
     if out.numel() == 0:
         return out
-    with _on(f.device):
+    with _on(f.device), runtime.turn(f.device):
         _rank_many(f32.reshape(-1, n, m), out.view(-1, n), count)
     return out
 
@@ -231,7 +233,7 @@ def nd_first_front(f: torch.Tensor) -> torch.Tensor:
         return out
     if m == 0:
         return out.fill_(True)
-    with _on(f.device):
+    with _on(f.device), runtime.turn(f.device):
         flat_f = f32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         stream = runtime.stream_handle(f.device)
@@ -278,7 +280,7 @@ def crowding(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Tensor:
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with _on(costs.device):
+    with _on(costs.device), runtime.turn(costs.device):
         flat_c = c32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
@@ -347,7 +349,7 @@ def crowding_wide(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Te
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with _on(costs.device):
+    with _on(costs.device), runtime.turn(costs.device):
         flat_c = wide.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
@@ -409,7 +411,7 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
         return out_x, out_f, out_rank, out_dist
     if out_rank.numel() == topk and n <= _WIDE_WHOLE_MAX:
         # one population: the whole selection in one call of the library
-        with _on(f.device):
+        with _on(f.device), runtime.turn(f.device):
             wb = wide.reshape(n, m)
             rows_f = f.reshape(n, m).contiguous()
             rows_x = x.reshape(n, -1).contiguous()
@@ -430,7 +432,7 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
     # the ranks, as far as the front that holds the topk-th row, from the ranking kernels on a float32 image of the
     # fitness that keeps every comparison (the rows behind that front are marked unset)
     rank = nd_rank_until(f, topk)
-    with _on(f.device):
+    with _on(f.device), runtime.turn(f.device):
         flat_w = wide.reshape(-1, n, m)
         flat_f = f.reshape(-1, n, m).contiguous()
         flat_x = x.reshape(flat_w.size(0), n, -1).contiguous()
@@ -525,15 +527,16 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
                       out_x.data_ptr() if has_x else None, out_f.data_ptr(), out_rank.data_ptr(), out_dist.data_ptr(), stream)
             runtime.note_small_kernel_call()
         else:
-            ws = runtime.workspace(n, m, f.device)
+            with runtime.turn(f.device):
+                ws = runtime.workspace(n, m, f.device)
 
-            def issue():
-                _lib.call("evox_hip_nd_environmental_selection", x.data_ptr() if has_x else None, row_bytes, row_bytes,
-                          f.data_ptr(), n, m, f.stride(0), f.stride(1), topk, out_x.data_ptr() if has_x else None,
-                          out_f.data_ptr(), out_rank.data_ptr(), out_dist.data_ptr(), None, ws.data_ptr(), ws.numel(), stream)
-                runtime.note_call(ws, stream)
+                def issue():
+                    _lib.call("evox_hip_nd_environmental_selection", x.data_ptr() if has_x else None, row_bytes, row_bytes,
+                              f.data_ptr(), n, m, f.stride(0), f.stride(1), topk, out_x.data_ptr() if has_x else None,
+                              out_f.data_ptr(), out_rank.data_ptr(), out_dist.data_ptr(), None, ws.data_ptr(), ws.numel(), stream)
+                    runtime.note_call(ws, stream)
 
-            runtime.checked(issue)
+                runtime.checked(issue)
         return out_x, out_f, out_rank, out_dist
     f32 = _as_f32(f, "fitness")
     batch = f.shape[:bd]
@@ -576,7 +579,8 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
                           fo_r[b0].data_ptr(), fo_d[b0].data_ptr(), ws.data_ptr(), ws.numel(), stream)
                 runtime.note_call(ws, stream, min(per_launch, nb), step)
 
-        runtime.checked(issue)
+        with runtime.turn(f.device):
+            runtime.checked(issue)
     return out_x, out_f.to(f.dtype), out_rank, out_dist
 
 
@@ -663,9 +667,10 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
         es = xa.element_size()
         row_bytes = xa.size(1) * es
         has_x = row_bytes > 0
-        ws = runtime.workspace(n, m, f_a.device)
         stream = runtime.stream_handle(f_a.device)
+
         def issue():
+            ws = runtime.workspace(n, m, f_a.device)
             _lib.call("evox_hip_nd_environmental_selection_two_part", xa.data_ptr() if has_x else None, xa.stride(0) * es,
                       xb.data_ptr() if has_x else None, xb.stride(0) * es, row_bytes, fa32.data_ptr(), n_a, fa32.stride(0),
                       fa32.stride(1), fb32.data_ptr(), n_b, fb32.stride(0), fb32.stride(1), m, topk,
@@ -673,7 +678,8 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
                       ws.data_ptr(), ws.numel(), stream)
             runtime.note_call(ws, stream)
 
-        runtime.checked(issue)
+        with runtime.turn(f_a.device):
+            runtime.checked(issue)
     return out_x, out_f.to(f_a.dtype), out_rank, out_dist
 
 
@@ -716,7 +722,7 @@ def stable_argsort_step(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         if prev.dtype != torch.int32 or prev.shape != (n,):
             raise ValueError("prev must be an int32 order of the same length as the key")
         prev = prev.contiguous()
-    with _on(key.device):
+    with _on(key.device), runtime.turn(key.device):
         ws = runtime.sort_workspace(n, key.device)
         stream = runtime.stream_handle(key.device)
         _lib.call("evox_hip_stable_argsort_step", key.data_ptr(), kind, key.stride(0), n,
@@ -755,7 +761,7 @@ def stable_argsort_rows(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         prev = prev.contiguous()
     if key.stride(0) < 0 or key.stride(1) < 0:
         key = key.contiguous()
-    with _on(key.device):
+    with _on(key.device), runtime.turn(key.device):
         ws = runtime.sort_workspace(n, key.device)
         stream = runtime.stream_handle(key.device)
         _lib.call("evox_hip_stable_argsort_step_batched", key.data_ptr(), kind, key.stride(0), key.stride(1), batch, n,

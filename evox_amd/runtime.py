@@ -11,7 +11,7 @@ import torch
 from . import _lib
 
 _workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
-_last: Optional[Tuple[torch.Tensor, int]] = None  # (workspace, stream handle) of the latest call
+_last: Optional[Tuple[torch.Tensor, int, int, int]] = None  # (workspace, stream handle, copies, their step) of the latest call
 
 CHECK_STATUS = os.environ.get("EVOX_AMD_CHECK_STATUS", "0") not in ("", "0")
 
@@ -84,12 +84,41 @@ def stream_handle(device: torch.device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
+def _place(device: torch.device) -> Tuple[int, int]:
+    return (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
+
+
+_turns: Dict[Tuple[int, int], "threading.RLock"] = {}  # (never cleared: a thread may hold one)
+
+
+def turn(device: torch.device):
+    """The lock of the current stream of ``device``.  Calls on a stream share its workspace, each from the first of its
+    launches to the last, and the library lets go of the interpreter while it enqueues them: a thread holds the lock from
+    before it takes the workspace until the library has returned, so that no other thread's launches come in between."""
+    place = _place(device)
+    lock = _turns.get(place)
+    return lock if lock is not None else _turns.setdefault(place, threading.RLock())
+
+
+def _buffer(need: int, device: torch.device) -> torch.Tensor:
+    """The buffer of the current stream of ``device``, made anew where it holds less than ``need`` bytes."""
+    place = _place(device)
+    ws = _workspaces.get(place)
+    if ws is None or ws.numel() < need:
+        _workspaces.pop(place, None)
+        ws = None
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        assert ws.data_ptr() % 256 == 0
+        _workspaces[place] = ws
+    return ws
+
+
 _workspace_need = {}  # (rows, objectives, with the matrix) -> bytes (asked of the library once per shape)
 
 
 def workspace(n: int, m: int, device: torch.device, with_matrix: bool = True) -> torch.Tensor:
     """A uint8 tensor of at least evox_hip_workspace_bytes(n, m) bytes, cached per (device, stream):
-    calls on one stream are ordered, so they can share it.  ``with_matrix=False`` asks only for the
+    calls on one stream are ordered, so they can share it (``turn``).  ``with_matrix=False`` asks only for the
     bytes that the entry points without a dominance matrix need."""
     need = _workspace_need.get((n, m, with_matrix))
     if need is None:
@@ -99,15 +128,7 @@ def workspace(n: int, m: int, device: torch.device, with_matrix: bool = True) ->
             raise ValueError(f"unsupported population shape n={n}, m={m}")
         if len(_workspace_need) < 4096:
             _workspace_need[(n, m, with_matrix)] = need
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        _workspaces.pop(key, None)
-        ws = None
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        assert ws.data_ptr() % 256 == 0
-        _workspaces[key] = ws
-    return ws
+    return _buffer(need, device)
 
 
 def sort_workspace(n: int, device: torch.device) -> torch.Tensor:
@@ -116,14 +137,7 @@ def sort_workspace(n: int, device: torch.device) -> torch.Tensor:
     need = int(_lib.lib().evox_hip_argsort_workspace_bytes(n))
     if need == 0:
         raise ValueError(f"unsupported sort length n={n}")
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        _workspaces.pop(key, None)
-        ws = None
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    return _buffer(need, device)
 
 
 def wide_workspace(n: int, m: int, device: torch.device, copies: int = 1) -> torch.Tensor:
@@ -134,29 +148,14 @@ def wide_workspace(n: int, m: int, device: torch.device, copies: int = 1) -> tor
         raise ValueError(f"unsupported population shape n={n}, m={m}")
     if copies > 1:
         need = ((need + 255) // 256 * 256) * copies
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        _workspaces.pop(key, None)
-        ws = None
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    return _buffer(need, device)
 
 
 def sized_workspace(need: int, device: torch.device) -> torch.Tensor:
     """The per-(device, stream) buffer of `workspace`, at least `need` bytes."""
     if need <= 0:
         raise ValueError("unsupported population shape")
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        _workspaces.pop(key, None)
-        ws = None
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        assert ws.data_ptr() % 256 == 0
-        _workspaces[key] = ws
-    return ws
+    return _buffer(need, device)
 
 
 def many_workspace(batch: int, n: int, m: int, stop_count: int, device: torch.device):
@@ -168,15 +167,7 @@ def many_workspace(batch: int, n: int, m: int, stop_count: int, device: torch.de
     per_launch = int(lib.evox_hip_many_populations_per_launch(batch, n, m, stop_count))
     if need == 0 or per_launch < 1:
         raise ValueError(f"unsupported population shape n={n}, m={m}")
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        _workspaces.pop(key, None)
-        ws = None
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        assert ws.data_ptr() % 256 == 0
-        _workspaces[key] = ws
-    return ws, per_launch, need // per_launch
+    return _buffer(need, device), per_launch, need // per_launch
 
 
 def release_workspaces() -> None:
@@ -188,7 +179,7 @@ def note_call(ws: torch.Tensor, stream: int, copies: int = 1, step: int = 0) -> 
     global _last
     _last = (ws, stream, copies, step)
     if CHECK_STATUS:
-        last_status()
+        _status(ws, stream, copies, step)  # (not that of _last: another thread may have noted a call of its own)
 
 
 # With status checking on, a ranking or selection whose device-side wait ran out (the persistent kernels need all
@@ -217,9 +208,11 @@ def note_small_kernel_call() -> None:
 def last_status() -> dict:
     """Waits for the latest call and returns its control block; raises if the device reported an error.
     Calls served by the small-population kernel have no control block: {"error": 0}."""
-    if _last is None:
-        return {"error": 0}
-    ws, stream, copies, step = _last
+    last = _last
+    return {"error": 0} if last is None else _status(*last)
+
+
+def _status(ws: torch.Tensor, stream: int, copies: int, step: int) -> dict:
     out = (ctypes.c_int32 * 8)()
     for b in reversed(range(copies)):  # (the control block reported is that of the first copy)
         code = _lib.lib().evox_hip_read_status(ws.data_ptr() + b * step, stream, out)

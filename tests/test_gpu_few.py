@@ -84,3 +84,34 @@ def test_several_populations(b, n, m):
     for i in range(b):
         _same([t[i] for t in got], er.environmental_selection(xs[i], fs[i], n // 2), (b, i))
     assert runtime.last_status()["error"] == 0
+
+
+def test_host_threads_on_one_stream():
+    """Threads whose calls take several launches each on the workspace of the default stream: every result is its own population's."""
+    import threading
+
+    populations = [_population("uniform", n, m, n)[0] for n, m in ((300, 3), (700, 5), (1000, 3), (2500, 3))]
+    want = [as_np(er.ranks_by_peeling(f)) for f in populations]
+    on_device = [f.to(DEV) for f in populations]
+    results, errors = [], []
+
+    def work(first):
+        try:
+            mine = []
+            for rep in range(100):
+                i = (first + rep) % len(on_device)
+                mine.append((i, non_dominate_rank(on_device[i])))
+            results.append(mine)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(first,)) for first in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for mine in results:
+        for i, rank in mine:
+            assert np.array_equal(as_np(rank), want[i]), i
