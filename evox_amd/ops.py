@@ -109,13 +109,13 @@ def _passes(batch: int, per_launch: int):
     return [(b0, min(per_launch, batch - b0)) for b0 in range(0, batch, per_launch)]
 
 
-def _rank_many(flat_f: torch.Tensor, flat_out: torch.Tensor, count: int) -> None:
+def _rank_many(here: runtime.Place, flat_f: torch.Tensor, flat_out: torch.Tensor, count: int) -> None:
     """Ranks of (B, N, M) float32 fitness as far as the front that holds the count-th row, into (B, N) int32; called with
     the stream's lock."""
     batch, n, m = flat_f.shape
+    stream = here.handle
     if batch == 1:
-        ws = runtime.workspace(n, m, flat_f.device)
-        stream = runtime.stream_handle(flat_f.device)
+        ws = runtime.workspace(n, m, here)
 
         def issue_one():
             _lib.call("evox_hip_non_dominate_rank_until", flat_f.data_ptr(), n, m, flat_f.stride(1), flat_f.stride(2), count,
@@ -124,10 +124,9 @@ def _rank_many(flat_f: torch.Tensor, flat_out: torch.Tensor, count: int) -> None
 
         runtime.checked(issue_one)
         return
-    stream = runtime.stream_handle(flat_f.device)
 
     def issue():
-        ws, per_launch, step = runtime.many_workspace(batch, n, m, count, flat_f.device)
+        ws, per_launch, step = runtime.many_workspace(batch, n, m, count, here)
         for b0, nb in _passes(batch, per_launch):
             _lib.call("evox_hip_many_non_dominate_rank_until", flat_f[b0].data_ptr(), nb, n, m, flat_f.stride(0), flat_f.stride(1),
                       flat_f.stride(2), count, flat_out[b0].data_ptr(), ws.data_ptr(), ws.numel(), stream)
@@ -157,8 +156,9 @@ def nd_rank(f: torch.Tensor) -> torch.Tensor:
                       flat_f.stride(1), flat_f.stride(2), flat_out.data_ptr(), runtime.stream_handle(f.device))
             runtime.note_small_kernel_call()
         else:
-            with runtime.turn(f.device):
-                _rank_many(flat_f, flat_out, n)
+            here = runtime.place(f.device)
+            with here.turn:
+                _rank_many(here, flat_f, flat_out, n)
     return out
 
 
@@ -203,8 +203,8 @@ def nd_rank_until(f: torch.Tensor, count: int) -> torch.Tensor:
     out = torch.empty(f32.shape[:-1], dtype=torch.int32, device=f.device)
     if out.numel() == 0:
         return out
-    with _on(f.device), runtime.turn(f.device):
-        _rank_many(f32.reshape(-1, n, m), out.view(-1, n), count)
+    with _on(f.device), (here := runtime.place(f.device)).turn:
+        _rank_many(here, f32.reshape(-1, n, m), out.view(-1, n), count)
     return out
 
 
@@ -233,16 +233,16 @@ def nd_first_front(f: torch.Tensor) -> torch.Tensor:
         return out
     if m == 0:
         return out.fill_(True)
-    with _on(f.device), runtime.turn(f.device):
+    with _on(f.device), (here := runtime.place(f.device)).turn:
         flat_f = f32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
-        stream = runtime.stream_handle(f.device)
+        stream = here.handle
         if flat_f.size(0) == 1:
-            ws = runtime.workspace(n, m, f.device, with_matrix=False)
+            ws = runtime.workspace(n, m, here, with_matrix=False)
             _lib.call("evox_hip_first_front_mask", flat_f.data_ptr(), n, m, flat_f.stride(1), flat_f.stride(2), flat_out.data_ptr(),
                       ws.data_ptr(), ws.numel(), stream)
         else:
-            ws = runtime.sized_workspace(int(_lib.lib().evox_hip_many_first_front_workspace_bytes(flat_f.size(0), n, m)), f.device)
+            ws = runtime.sized_workspace(int(_lib.lib().evox_hip_many_first_front_workspace_bytes(flat_f.size(0), n, m)), here)
             _lib.call("evox_hip_many_first_front_mask", flat_f.data_ptr(), flat_f.size(0), n, m, flat_f.stride(0), flat_f.stride(1),
                       flat_f.stride(2), flat_out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         runtime.note_call(ws, stream)
@@ -280,18 +280,18 @@ def crowding(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Tensor:
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with _on(costs.device), runtime.turn(costs.device):
+    with _on(costs.device), (here := runtime.place(costs.device)).turn:
         flat_c = c32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
-        stream = runtime.stream_handle(costs.device)
+        stream = here.handle
         if flat_c.size(0) == 1:
-            ws = runtime.workspace(n, m, costs.device)
+            ws = runtime.workspace(n, m, here)
             _lib.call("evox_hip_crowding_distance", flat_c.data_ptr(), n, m, flat_c.stride(1), flat_c.stride(2),
                       None if flat_mask is None else flat_mask.data_ptr(), 0 if flat_mask is None else flat_mask.stride(1),
                       flat_out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         else:
-            ws = runtime.sized_workspace(int(_lib.lib().evox_hip_many_crowding_workspace_bytes(flat_c.size(0), n, m)), costs.device)
+            ws = runtime.sized_workspace(int(_lib.lib().evox_hip_many_crowding_workspace_bytes(flat_c.size(0), n, m)), here)
             _lib.call("evox_hip_many_crowding_distance", flat_c.data_ptr(), flat_c.size(0), n, m, flat_c.stride(0), flat_c.stride(1),
                       flat_c.stride(2), None if flat_mask is None else flat_mask.data_ptr(),
                       0 if flat_mask is None else flat_mask.stride(0), 0 if flat_mask is None else flat_mask.stride(1),
@@ -349,12 +349,12 @@ def crowding_wide(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Te
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with _on(costs.device), runtime.turn(costs.device):
+    with _on(costs.device), (here := runtime.place(costs.device)).turn:
         flat_c = wide.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
-        stream = runtime.stream_handle(costs.device)
-        ws = runtime.wide_workspace(n, m, costs.device)
+        stream = here.handle
+        ws = runtime.wide_workspace(n, m, here)
         for b in range(flat_c.size(0)):
             c = flat_c[b]
             mk = None if flat_mask is None else flat_mask[b]
@@ -411,14 +411,14 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
         return out_x, out_f, out_rank, out_dist
     if out_rank.numel() == topk and n <= _WIDE_WHOLE_MAX:
         # one population: the whole selection in one call of the library
-        with _on(f.device), runtime.turn(f.device):
+        with _on(f.device), (here := runtime.place(f.device)).turn:
             wb = wide.reshape(n, m)
             rows_f = f.reshape(n, m).contiguous()
             rows_x = x.reshape(n, -1).contiguous()
             row_bytes, f_row_bytes = rows_x.size(-1) * rows_x.element_size(), m * rows_f.element_size()
             has_x = row_bytes > 0
-            ws = runtime.workspace(n, m, f.device)
-            stream = runtime.stream_handle(f.device)
+            ws = runtime.workspace(n, m, here)
+            stream = here.handle
 
             def issue():
                 _lib.call("evox_hip_nd_environmental_selection_wide_whole", rows_x.data_ptr() if has_x else None, row_bytes, row_bytes,
@@ -432,7 +432,7 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
     # the ranks, as far as the front that holds the topk-th row, from the ranking kernels on a float32 image of the
     # fitness that keeps every comparison (the rows behind that front are marked unset)
     rank = nd_rank_until(f, topk)
-    with _on(f.device), runtime.turn(f.device):
+    with _on(f.device), (here := runtime.place(f.device)).turn:
         flat_w = wide.reshape(-1, n, m)
         flat_f = f.reshape(-1, n, m).contiguous()
         flat_x = x.reshape(flat_w.size(0), n, -1).contiguous()
@@ -442,10 +442,10 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
         has_x = row_bytes > 0
         fo_x = out_x.view(flat_w.size(0), topk, -1)
         fo_f, fo_r, fo_d = out_f.view(-1, topk, m), out_rank.view(-1, topk), out_dist.view(-1, topk)
-        stream = runtime.stream_handle(f.device)
+        stream = here.handle
         count = flat_w.size(0)
         if count == 1:
-            ws = runtime.wide_workspace(n, m, f.device)
+            ws = runtime.wide_workspace(n, m, here)
             wb = flat_w[0]
             _lib.call("evox_hip_nd_environmental_selection_wide", flat_x.data_ptr() if has_x else None, row_bytes, row_bytes,
                       flat_f.data_ptr(), f_row_bytes, f_row_bytes, wb.data_ptr(), kind, n, m, wb.stride(0), wb.stride(1),
@@ -459,7 +459,7 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
             flat_rank = flat_rank.contiguous()
             for b0 in range(0, count, per_call):
                 nb = min(per_call, count - b0)
-                ws = runtime.wide_workspace(n, m, f.device, nb)
+                ws = runtime.wide_workspace(n, m, here, nb)
                 wb = flat_w[b0:b0 + nb]
                 _lib.call("evox_hip_many_nd_environmental_selection_wide", flat_x[b0].data_ptr() if has_x else None, row_bytes, row_bytes,
                           n * row_bytes, flat_f[b0].data_ptr(), f_row_bytes, f_row_bytes, n * f_row_bytes, wb.data_ptr(), kind, nb, n, m,
@@ -520,15 +520,17 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
         es = x.element_size()
         row_bytes = (x.numel() // n) * es
         has_x = row_bytes > 0
-        stream = runtime.stream_handle(f.device)
         if runtime.small_population_kernel_fits(n, m, 1):
             _lib.call("evox_hip_batched_nd_environmental_selection", x.data_ptr() if has_x else None, row_bytes, row_bytes,
                       n * row_bytes, f.data_ptr(), 1, n, m, n * f.stride(0), f.stride(0), f.stride(1), topk,
-                      out_x.data_ptr() if has_x else None, out_f.data_ptr(), out_rank.data_ptr(), out_dist.data_ptr(), stream)
+                      out_x.data_ptr() if has_x else None, out_f.data_ptr(), out_rank.data_ptr(), out_dist.data_ptr(),
+                      runtime.stream_handle(f.device))
             runtime.note_small_kernel_call()
         else:
-            with runtime.turn(f.device):
-                ws = runtime.workspace(n, m, f.device)
+            here = runtime.place(f.device)
+            stream = here.handle
+            with here.turn:
+                ws = runtime.workspace(n, m, here)
 
                 def issue():
                     _lib.call("evox_hip_nd_environmental_selection", x.data_ptr() if has_x else None, row_bytes, row_bytes,
@@ -569,9 +571,10 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
             return out_x, out_f.to(f.dtype), out_rank, out_dist
         batch_count = flat_f.size(0)
         es = flat_x.element_size()
+        here = runtime.place(f.device)
 
         def issue():
-            ws, per_launch, step = runtime.many_workspace(batch_count, n, m, topk, f.device)
+            ws, per_launch, step = runtime.many_workspace(batch_count, n, m, topk, here)
             for b0, nb in _passes(batch_count, per_launch):
                 _lib.call("evox_hip_many_nd_environmental_selection", flat_x[b0].data_ptr() if has_x else None, row_bytes,
                           flat_x.stride(1) * es, flat_x.stride(0) * es, flat_f[b0].data_ptr(), nb, n, m, flat_f.stride(0),
@@ -579,7 +582,7 @@ def nd_select(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.Tensor
                           fo_r[b0].data_ptr(), fo_d[b0].data_ptr(), ws.data_ptr(), ws.numel(), stream)
                 runtime.note_call(ws, stream, min(per_launch, nb), step)
 
-        with runtime.turn(f.device):
+        with here.turn:
             runtime.checked(issue)
     return out_x, out_f.to(f.dtype), out_rank, out_dist
 
@@ -667,10 +670,11 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
         es = xa.element_size()
         row_bytes = xa.size(1) * es
         has_x = row_bytes > 0
-        stream = runtime.stream_handle(f_a.device)
+        here = runtime.place(f_a.device)
+        stream = here.handle
 
         def issue():
-            ws = runtime.workspace(n, m, f_a.device)
+            ws = runtime.workspace(n, m, here)
             _lib.call("evox_hip_nd_environmental_selection_two_part", xa.data_ptr() if has_x else None, xa.stride(0) * es,
                       xb.data_ptr() if has_x else None, xb.stride(0) * es, row_bytes, fa32.data_ptr(), n_a, fa32.stride(0),
                       fa32.stride(1), fb32.data_ptr(), n_b, fb32.stride(0), fb32.stride(1), m, topk,
@@ -678,7 +682,7 @@ def nd_select_two_part(x_a: torch.Tensor, f_a: torch.Tensor, x_b: torch.Tensor, 
                       ws.data_ptr(), ws.numel(), stream)
             runtime.note_call(ws, stream)
 
-        with runtime.turn(f_a.device):
+        with here.turn:
             runtime.checked(issue)
     return out_x, out_f.to(f_a.dtype), out_rank, out_dist
 
@@ -722,9 +726,9 @@ def stable_argsort_step(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         if prev.dtype != torch.int32 or prev.shape != (n,):
             raise ValueError("prev must be an int32 order of the same length as the key")
         prev = prev.contiguous()
-    with _on(key.device), runtime.turn(key.device):
-        ws = runtime.sort_workspace(n, key.device)
-        stream = runtime.stream_handle(key.device)
+    with _on(key.device), (here := runtime.place(key.device)).turn:
+        ws = runtime.sort_workspace(n, here)
+        stream = here.handle
         _lib.call("evox_hip_stable_argsort_step", key.data_ptr(), kind, key.stride(0), n,
                   None if prev is None else prev.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         # only the radix sort of long keys waits on the device and keeps a control block
@@ -761,9 +765,9 @@ def stable_argsort_rows(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         prev = prev.contiguous()
     if key.stride(0) < 0 or key.stride(1) < 0:
         key = key.contiguous()
-    with _on(key.device), runtime.turn(key.device):
-        ws = runtime.sort_workspace(n, key.device)
-        stream = runtime.stream_handle(key.device)
+    with _on(key.device), (here := runtime.place(key.device)).turn:
+        ws = runtime.sort_workspace(n, here)
+        stream = here.handle
         _lib.call("evox_hip_stable_argsort_step_batched", key.data_ptr(), kind, key.stride(0), key.stride(1), batch, n,
                   None if prev is None else prev.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         if _argsort_waits(n) and (batch < 2 or n > _ROWS_ARGSORT_MAX):

@@ -10,7 +10,6 @@ import torch
 
 from . import _lib
 
-_workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
 _last: Optional[Tuple[torch.Tensor, int, int, int]] = None  # (workspace, stream handle, copies, their step) of the latest call
 
 CHECK_STATUS = os.environ.get("EVOX_AMD_CHECK_STATUS", "0") not in ("", "0")
@@ -84,42 +83,57 @@ def stream_handle(device: torch.device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
-def _place(device: torch.device) -> Tuple[int, int]:
-    return (device.index if device.index is not None else torch.cuda.current_device(), stream_handle(device))
+class Place:
+    """A stream of a device: its handle, the workspace that calls on it share, and the lock under which they use it.
+
+    A call works on the workspace from the first of its launches to the last, and the library lets go of the interpreter while
+    it enqueues them: a thread holds ``turn`` from before it takes the workspace until the library has returned, so that no
+    other thread's launches come in between."""
+
+    __slots__ = ("device", "handle", "turn", "kept")
+
+    def __init__(self, device: torch.device, handle: int):
+        self.device, self.handle, self.turn, self.kept = device, handle, threading.RLock(), None
+
+    def buffer(self, need: int) -> torch.Tensor:
+        """At least ``need`` bytes: the stream's buffer, made anew where it holds less.  A call that is being captured gets one of
+        its own, from the graph's memory: a replay works on it whatever later calls do to the stream's buffer (a larger one
+        replaces it, and other streams' calls may run beside the replay)."""
+        if _capturing():
+            return torch.empty(need, dtype=torch.uint8, device=self.device)
+        ws = self.kept
+        if ws is None or ws.numel() < need:
+            self.kept = ws = None
+            ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+            assert ws.data_ptr() % 256 == 0
+            self.kept = ws
+        return ws
 
 
-_turns: Dict[Tuple[int, int], "threading.RLock"] = {}  # (never cleared: a thread may hold one)
+_capturing = torch.cuda.is_current_stream_capturing
+_places: Dict[Tuple[int, int], Place] = {}
 
 
-def turn(device: torch.device):
-    """The lock of the current stream of ``device``.  Calls on a stream share its workspace, each from the first of its
-    launches to the last, and the library lets go of the interpreter while it enqueues them: a thread holds the lock from
-    before it takes the workspace until the library has returned, so that no other thread's launches come in between."""
-    place = _place(device)
-    lock = _turns.get(place)
-    return lock if lock is not None else _turns.setdefault(place, threading.RLock())
+def place(device: torch.device) -> Place:
+    """The current stream of ``device``."""
+    handle = stream_handle(device)
+    index = device.index
+    key = (index if index is not None else torch.cuda.current_device(), handle)
+    here = _places.get(key)
+    return here if here is not None else _places.setdefault(key, Place(device, handle))
 
 
-def _buffer(need: int, device: torch.device) -> torch.Tensor:
-    """The buffer of the current stream of ``device``, made anew where it holds less than ``need`` bytes."""
-    place = _place(device)
-    ws = _workspaces.get(place)
-    if ws is None or ws.numel() < need:
-        _workspaces.pop(place, None)
-        ws = None
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        assert ws.data_ptr() % 256 == 0
-        _workspaces[place] = ws
-    return ws
+def _buffer(need: int, where) -> torch.Tensor:
+    return (where if type(where) is Place else place(where)).buffer(need)
 
 
-_workspace_need = {}  # (rows, objectives, with the matrix) -> bytes (asked of the library once per shape)
+_workspace_need = {}  # (rows, objectives, with the matrix), or the length of a sort -> bytes (asked of the library once per shape)
 
 
-def workspace(n: int, m: int, device: torch.device, with_matrix: bool = True) -> torch.Tensor:
-    """A uint8 tensor of at least evox_hip_workspace_bytes(n, m) bytes, cached per (device, stream):
-    calls on one stream are ordered, so they can share it (``turn``).  ``with_matrix=False`` asks only for the
-    bytes that the entry points without a dominance matrix need."""
+def workspace(n: int, m: int, where, with_matrix: bool = True) -> torch.Tensor:
+    """A uint8 tensor of at least evox_hip_workspace_bytes(n, m) bytes, cached per (device, stream) -- ``where`` is a ``Place``,
+    or a device for its current stream: calls on one stream are ordered, so they can share it.  ``with_matrix=False`` asks
+    only for the bytes that the entry points without a dominance matrix need."""
     need = _workspace_need.get((n, m, with_matrix))
     if need is None:
         query = _lib.lib().evox_hip_workspace_bytes if with_matrix else _lib.lib().evox_hip_first_front_workspace_bytes
@@ -128,19 +142,23 @@ def workspace(n: int, m: int, device: torch.device, with_matrix: bool = True) ->
             raise ValueError(f"unsupported population shape n={n}, m={m}")
         if len(_workspace_need) < 4096:
             _workspace_need[(n, m, with_matrix)] = need
-    return _buffer(need, device)
+    return _buffer(need, where)
 
 
-def sort_workspace(n: int, device: torch.device) -> torch.Tensor:
+def sort_workspace(n: int, where) -> torch.Tensor:
     """Workspace of the standalone stable argsort; shares the per-(device, stream) buffer of `workspace`
     (every call initialises the parts it uses)."""
-    need = int(_lib.lib().evox_hip_argsort_workspace_bytes(n))
-    if need == 0:
-        raise ValueError(f"unsupported sort length n={n}")
-    return _buffer(need, device)
+    need = _workspace_need.get(n)
+    if need is None:
+        need = int(_lib.lib().evox_hip_argsort_workspace_bytes(n))
+        if need == 0:
+            raise ValueError(f"unsupported sort length n={n}")
+        if len(_workspace_need) < 4096:
+            _workspace_need[n] = need
+    return _buffer(need, where)
 
 
-def wide_workspace(n: int, m: int, device: torch.device, copies: int = 1) -> torch.Tensor:
+def wide_workspace(n: int, m: int, where, copies: int = 1) -> torch.Tensor:
     """Workspace of the entry points for 8-byte fitness (`copies` of it, each rounded up to 256 bytes, for as many
     populations in the same launches); shares the per-(device, stream) buffer of `workspace`."""
     need = int(_lib.lib().evox_hip_wide_workspace_bytes(n, m))
@@ -148,17 +166,17 @@ def wide_workspace(n: int, m: int, device: torch.device, copies: int = 1) -> tor
         raise ValueError(f"unsupported population shape n={n}, m={m}")
     if copies > 1:
         need = ((need + 255) // 256 * 256) * copies
-    return _buffer(need, device)
+    return _buffer(need, where)
 
 
-def sized_workspace(need: int, device: torch.device) -> torch.Tensor:
+def sized_workspace(need: int, where) -> torch.Tensor:
     """The per-(device, stream) buffer of `workspace`, at least `need` bytes."""
     if need <= 0:
         raise ValueError("unsupported population shape")
-    return _buffer(need, device)
+    return _buffer(need, where)
 
 
-def many_workspace(batch: int, n: int, m: int, stop_count: int, device: torch.device):
+def many_workspace(batch: int, n: int, m: int, stop_count: int, where):
     """Workspace of the entry points that take many populations of one shape: (tensor, populations per launch, bytes
     from one population's copy of the workspace to the next); shares the per-(device, stream) buffer of `workspace`.
     Asked anew at every call: the answer depends on the tunables in use."""
@@ -167,11 +185,12 @@ def many_workspace(batch: int, n: int, m: int, stop_count: int, device: torch.de
     per_launch = int(lib.evox_hip_many_populations_per_launch(batch, n, m, stop_count))
     if need == 0 or per_launch < 1:
         raise ValueError(f"unsupported population shape n={n}, m={m}")
-    return _buffer(need, device), per_launch, need // per_launch
+    return _buffer(need, where), per_launch, need // per_launch
 
 
 def release_workspaces() -> None:
-    _workspaces.clear()
+    for here in list(_places.values()):
+        here.kept = None
 
 
 def note_call(ws: torch.Tensor, stream: int, copies: int = 1, step: int = 0) -> None:

@@ -115,3 +115,33 @@ def test_host_threads_on_one_stream():
     for mine in results:
         for i, rank in mine:
             assert np.array_equal(as_np(rank), want[i]), i
+
+
+@pytest.mark.parametrize("n,m", [(300, 3), (1000, 8), (2500, 3)])
+def test_a_captured_call_keeps_its_workspace(n, m):
+    """Captured on a stream whose buffer a larger call then replaces: replays neither read nor write what the allocator has
+    given away since."""
+    f = torch.rand(n, m, generator=torch.Generator("cpu").manual_seed(n))
+    static = f.to(DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        non_dominate_rank(static)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = non_dominate_rank(static)
+    with torch.cuda.stream(side):
+        non_dominate_rank(torch.rand(9000, m, device=DEV))
+        taken = [torch.full((1 << shift,), 7, dtype=torch.uint8, device=DEV) for shift in range(9, 25) for _ in range(3)]
+    torch.cuda.synchronize()
+    for seed in range(4):
+        f = torch.rand(n, m, generator=torch.Generator("cpu").manual_seed(seed))
+        static.copy_(f)
+        graph.replay()
+        eager = non_dominate_rank(f.to(DEV))
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and np.array_equal(as_np(eager), as_np(er.ranks_by_peeling(f))), seed
+    assert all(bool((t == 7).all()) for t in taken)
+    del graph
+    runtime.release_workspaces()

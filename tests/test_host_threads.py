@@ -1,6 +1,6 @@
 """Host threads that call on one stream: a call's launches are enqueued without another thread's in between, since calls on a
-stream share its workspace and the library lets go of the interpreter while it enqueues.  On the CPU, with the library's entry
-points replaced by ones that take a while."""
+stream share its workspace and the library lets go of the interpreter while it enqueues.  And a captured call's workspace, which
+is the graph's own.  On the CPU, with the library's entry points replaced by ones that take a while."""
 
 import contextlib
 import threading
@@ -58,7 +58,7 @@ def device_on_the_cpu(monkeypatch):
     monkeypatch.setattr(runtime, "require_gpu_tensor", lambda t, what: None)
     monkeypatch.setattr(runtime, "stream_handle", lambda device: 7)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(runtime, "_capturing", lambda: False)
     empty = torch.empty
 
     def aligned(*size, **kw):  # (as the allocator of a GPU gives it)
@@ -68,7 +68,7 @@ def device_on_the_cpu(monkeypatch):
         return whole[-whole.data_ptr() % 256:][:size[0]]
 
     monkeypatch.setattr(torch, "empty", aligned)
-    for cache in ("_workspaces", "_workspace_need", "_batched_max_rows"):
+    for cache in ("_places", "_workspace_need", "_batched_max_rows"):
         monkeypatch.setattr(runtime, cache, {})
     yield overlaps
 
@@ -91,3 +91,16 @@ def test_calls_of_two_threads_on_a_stream_take_turns(name, device_on_the_cpu):
         t.join()
     assert not errors, errors
     assert device_on_the_cpu == []
+
+
+def test_a_captured_call_keeps_no_buffer_that_later_calls_replace(device_on_the_cpu, monkeypatch):
+    """A replay works on the memory that the call was captured with: the stream's buffer, which a larger call replaces, would go
+    back to the allocator under it."""
+    device = torch.device("cpu")
+    here = runtime.place(device)
+    eager = runtime.workspace(300, 3, here)
+    monkeypatch.setattr(runtime, "_capturing", lambda: True)
+    captured = runtime.workspace(300, 3, here)
+    assert captured.data_ptr() != eager.data_ptr() and here.kept is eager
+    monkeypatch.setattr(runtime, "_capturing", lambda: False)
+    assert runtime.workspace(300, 3, here) is eager
