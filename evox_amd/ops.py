@@ -9,12 +9,14 @@ front; the operators themselves accept any number of leading batch dimensions, s
 need no extra registrations.
 """
 
+import contextlib
 import ctypes
 from typing import List, Optional, Tuple
 
 import torch
 
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import _lib, runtime
@@ -875,10 +877,17 @@ torch.library.register_vmap(hv_covered_count, _hv_covered_count_vmap)
 _HV_OBJECTIVES = 16  # most objectives of the whole-call hypervolume kernels
 
 
-# Looking at a tensor's attributes under a function mode (a default device set with ``torch.device(...)`` is one) goes through
-# Python each time: the whole-call functions below look at them, and make their buffers, with the modes off -- 20 us of a
-# call of the metric.  Only where plain_eager() holds: a tracer does not get here.
-quiet = torch._C.DisableTorchFunction
+def only_default_device() -> bool:
+    """Whether no torch function mode is on but default devices (``torch.set_default_device``, ``with torch.device(...)``):
+    nothing of the caller's looks at the functions that are called."""
+    return all(type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
+def quiet():
+    """Looking at a tensor's attributes under a function mode goes through Python each time: the whole-call functions below look
+    at them, and make their buffers, with the default devices off -- 20 us of a call of the metric.  Only where plain_eager()
+    holds: a tracer does not get here.  A function mode of the caller's own goes on seeing every call."""
+    return torch._C.DisableTorchFunction() if only_default_device() else contextlib.nullcontext()
 
 
 def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> bool:

@@ -55,7 +55,7 @@ def lexsort(keys: Sequence[torch.Tensor], dim: int = -1) -> torch.Tensor:
         return torch.empty(shape, dtype=torch.int64, device=keys[0].device)
     if keys[0].dim() == 1 and dim in (-1, 0):  # nothing to move; the function behind the operator where nothing looks at the call
         step = ops.stable_argsort_step
-        if ops.plain_eager() and not any(type(k) is not torch.Tensor or k.requires_grad or k.is_neg() or k.is_conj() for k in keys):
+        if ops.plain_eager() and ops.only_default_device() and not any(type(k) is not torch.Tensor or k.requires_grad or k.is_neg() or k.is_conj() for k in keys):
             step = getattr(step, "_init_fn", step)
         order = None
         for key in keys:

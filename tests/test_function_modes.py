@@ -1,0 +1,69 @@
+"""Torch function modes: default devices are taken off where the calls look at tensors, a mode of the caller's own sees what it
+saw before there were ways past the dispatcher."""
+
+import pytest
+import torch
+from torch.overrides import TorchFunctionMode
+
+from evox_amd import ops, utils
+from evox_amd.hype import cal_hv
+from evox_amd.metrics import hv
+
+
+class Seen(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(getattr(func, "__name__", func)))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("device", [False, True])
+def test_a_mode_of_the_callers_sees_the_quiet_calls(device):
+    with torch.device("cpu") if device else Seen():
+        with Seen() as seen, ops.quiet():
+            torch.empty(3)
+    assert "empty" in seen.names
+
+
+def test_a_default_device_is_taken_off():
+    with torch.device("meta"):
+        with ops.quiet():
+            assert torch.empty(3).device.type == "cpu"
+
+
+def test_a_sort_goes_through_the_operator_where_a_mode_looks(monkeypatch):
+    called = []
+
+    class Step:
+        def __call__(self, key, kind, prev):
+            called.append("operator")
+            return torch.argsort(key).int()
+
+        def _init_fn(self, key, kind, prev):
+            called.append("function")
+            return torch.argsort(key).int()
+
+    monkeypatch.setattr(ops, "stable_argsort_step", Step())
+    key = torch.tensor([3.0, 1.0, 2.0])
+    for mode, way in ((Seen(), "operator"), (torch.device("cpu"), "function")):
+        with mode:
+            assert utils.lexsort([key]).tolist() == [1, 2, 0]
+        assert called.pop() == way and not called
+    assert utils.lexsort([key]).tolist() == [1, 2, 0] and called == ["function"]
+
+
+@pytest.mark.gpu
+def test_hypervolumes_under_a_mode_are_the_same():
+    f = torch.rand(200, 3, generator=torch.Generator("cpu").manual_seed(0)).to("cuda")
+    ref = torch.ones(3, device="cuda")
+    for call in (lambda: hv(f, ref, 5000), lambda: cal_hv(f, ref, 100, 5000)):
+        with torch.device("cuda"):
+            torch.manual_seed(1)
+            plain = call()
+            torch.manual_seed(1)
+            with Seen() as seen:
+                watched = call()
+        assert torch.equal(plain, watched) and "rand" in seen.names and "empty" in seen.names
