@@ -103,8 +103,80 @@ __host__ __device__ inline size_t few_finish_lds_bytes(int nt, int n, int m) {
   return (size_t)nt * (4 * 4 + 8) + 32 + rows * (4 * (size_t)m + 4 + 4 + 2 + 2 + 2);
 }
 
+// Place of this thread's candidate (thread q < nv holds candidate q; entry: its key, then q) in the ascending order of the entries,
+// by buckets: as two_small_place, for an item per thread.  bucket: a map of the key to 0 .. 4 nt - 1 that never decreases.  False when
+// more than kTwoSmallCrowd candidates of different keys share one.  Every thread calls it.
+// Candidates of one key that fill a bucket (values of a few levels, copies, distances of zero) are placed by their indices: the few buckets
+// that can be as full are numbered, and a wave counts its candidates of each by a ballot.  1000 rows of one front, all equal, us per selection
+// of half of them, three / eight objectives: by counting 112 / 245, like this 30 / 56; values of four levels, 700 x 8: 65 -> 45, of sixteen, 1000 x 8: 68 -> 53.
+// cnt: 4 nt words; comps: nv entries; ids: nv; part: 16 words.
+constexpr uint32_t kFewCrowd = 40;  // candidates of a bucket up to which each one looks at all
+__device__ inline bool few_place(uint64_t entry, uint32_t bucket, int nv, int nt, uint32_t* cnt, uint64_t* comps, uint16_t* ids, uint32_t* part,
+                                 int& place) {
+  const int q = threadIdx.x, lane = q & 63, wave = q >> 6;
+  const bool cand = q < nv;
+  reinterpret_cast<uint4*>(cnt)[q] = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  const uint32_t arrived = cand ? atomicAdd(&cnt[bucket], 1u) : 0u;
+  __syncthreads();
+  const uint4 mine = reinterpret_cast<const uint4*>(cnt)[q];
+  const uint32_t sum = mine.x + mine.y + mine.z + mine.w;
+  const uint32_t incl = wave_prefix_sum(sum);
+  if (lane == 63) part[wave] = incl;
+  const bool crowds = __syncthreads_or(max(max(mine.x, mine.y), max(mine.z, mine.w)) > kFewCrowd) != 0;
+  const uint32_t run = incl - sum + sum_before_wave(part, wave);
+  reinterpret_cast<uint4*>(cnt)[q] = make_uint4(run, run + mine.x, run + mine.x + mine.y, run + mine.x + mine.y + mine.z);
+  __syncthreads();
+  uint32_t first = 0u, end = 0u;
+  if (cand) {
+    first = cnt[bucket];
+    end = bucket + 1u < 4u * (uint32_t)nt ? cnt[bucket + 1u] : (uint32_t)nv;
+    comps[first + arrived] = entry;
+  }
+  if (q < 4) part[q] = 0u;  // crowds; whether one of them is too large; those of different keys
+  __syncthreads();
+  if (crowds) {
+    const bool big = end - first > kFewCrowd;
+    if (big && arrived == 0u) cnt[bucket] = atomicAdd(&part[0], 1u);  // (its start has been read by all)
+    __syncthreads();
+    const int crowd_count = (int)part[0];  // (at most 1024 / (kFewCrowd + 1))
+    uint32_t number = big ? cnt[bucket] : ~0u;
+    if (big && (uint32_t)(comps[first] >> 32) != (uint32_t)(entry >> 32)) {
+      atomicOr(&part[2 + (number >> 5)], 1u << (number & 31u));
+      if (end - first > kTwoSmallCrowd) part[1] = 1u;
+    }
+    __syncthreads();
+    if (part[1] != 0u) return false;
+    const uint64_t mixed = (uint64_t)part[3] << 32 | part[2];
+    if (big && (mixed >> number & 1ull)) number = ~0u;  // (each one looks at all)
+    const int waves = nt >> 6;
+    uint32_t below = 0u;
+#pragma unroll 1
+    for (int c = 0; c < crowd_count; ++c) {
+      const uint64_t of = __builtin_amdgcn_ballot_w64(number == (uint32_t)c);
+      if (number == (uint32_t)c) below = (uint32_t)__popcll(of & ((1ull << lane) - 1ull));
+      if (lane == 0) ids[c * waves + wave] = (uint16_t)__popcll(of);
+    }
+    __syncthreads();
+    if (number != ~0u) {
+#pragma unroll 4
+      for (int w = 0; w < wave; ++w) below += ids[number * waves + w];
+      place = (int)(first + below);
+      return true;
+    }
+  }
+  uint32_t before = 0u;
+  for (uint32_t at = first; at < end; at += 4) {  // (four members' reads in flight together)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) before += comps[min(at + (uint32_t)u, end - 1u)] < entry && at + (uint32_t)u < end ? 1u : 0u;
+  }
+  place = (int)(first + before);
+  return true;
+}
+
 // Position of this thread's candidate (thread q < nv holds candidate q with `key`) in the ascending order of (key, q): by
-// buckets -- of equal width in the key's value, then in the key --, or by counting where the candidates are few or crowd.
+// buckets -- of equal width in the key's value or in the key, whichever fits its range, then the other --, or by counting where the
+// candidates are few or crowd.
 // lo, hi: smallest and largest key of a finite value, -inf and +inf / NaN outside.  Every thread of the workgroup calls it.
 __device__ inline int few_position(uint32_t key, int nv, int nt, uint32_t* cnt, uint64_t* comps, uint16_t* ids, uint32_t* part, uint32_t* lo16,
                                    uint32_t* hi16) {
@@ -112,23 +184,23 @@ __device__ inline int few_position(uint32_t key, int nv, int nt, uint32_t* cnt, 
   const bool cand = q < nv;
   const int parts = nt / ((nv + 63) & ~63);  // threads that share the comparisons of a candidate
   __syncthreads();  // (comps, cnt and the costs of the call before are free)
+  const uint64_t entry = ((uint64_t)key << 32) | (uint32_t)q;
   if (nv > kFewCounting * parts) {
     const uint32_t key_inf = ordered_key(INFINITY), key_neg_inf = ordered_key(-INFINITY);
     uint32_t lo = 0xFFFFFFFFu, hi = 0u;
     if (cand && key > key_neg_inf && key < key_inf) lo = hi = key;
     two_small_range(lo, hi, lo16, hi16, nt);
-    const uint64_t comp[1] = {key};
-    const uint32_t id[1] = {(uint32_t)q};
+    const bool wide = lo < hi && (lo ^ hi) >> 31 == 0u && lo != 0x80000000u && hi - lo > 24u << 23;  // (values of one sign, none zero, over more than 24 binades)
 #pragma unroll 1
     for (int attempt = 0; attempt < 2; ++attempt) {
-      const uint32_t bucket[1] = {attempt == 0 ? bucket_by_value(key, lo, hi, 4 * nt) : bucket_by_image(key, lo, hi, 4 * nt)};
-      int place[1];
-      bool twins;
-      if (two_small_place<1>(comp, id, bucket, nv, nt, cnt, part, comps, ids, place, twins)) return place[0];
+      int place;
+      if (few_place(entry, (attempt == 0) != wide ? bucket_by_value(key, lo, hi, 4 * nt) : bucket_by_image(key, lo, hi, 4 * nt), nv, nt, cnt, comps,
+                    ids, part, place))
+        return place;
     }
     __syncthreads();
   }
-  if (q < nv + 4) comps[q] = cand ? ((uint64_t)key << 32) | (uint32_t)q : ~0ull;
+  if (q < nv + 4) comps[q] = cand ? entry : ~0ull;
   if (q < 4 && nv + q >= nt) comps[nv + q] = ~0ull;
   return position_by_counting(comps, reinterpret_cast<int*>(cnt), nv, q, nt);
 }
@@ -272,10 +344,21 @@ __device__ __forceinline__ void few_finish(const BatchedArgs& a, const uint64_t*
   const int mine_row = cand ? order[worst_start + j] : 0;
   bool boundary = false;
   float acc = 0.0f;
+  // ... and, behind the objectives, the index-stable top-k on the last front by (-distance, row index) (:253).  (One piece of code for
+  // both: a second copy of the placement costs half a microsecond of fetching it.)
 #pragma unroll 1
-  for (int k = 0; k < m; ++k) {
-    const uint32_t key = cand ? ordered_key(fit[(size_t)k * rows + mine_row]) : 0u;
+  for (int k = 0;; ++k) {
+    const float d = k == m && boundary ? INFINITY : acc;
+    if (k == m) {
+      EVX_BATCH_TRACE(3);
+    }
+    const uint32_t key = cand ? ordered_key(k == m ? -d : fit[(size_t)k * rows + mine_row]) : 0u;
     const int p = few_position(key, nv, nt, cnt, comps, ids, part, lo16, hi16);
+    if (k == m) {
+      if (cand) dist[mine_row] = d;
+      if (cand && p < need) order[worst_start + p] = (uint16_t)mine_row;  // (every candidate has been read from there)
+      break;
+    }
     if (cand) scost[p] = cost_of_key(key);
     __syncthreads();
     if (cand) {
@@ -286,14 +369,6 @@ __device__ __forceinline__ void few_finish(const BatchedArgs& a, const uint64_t*
         acc = k == 0 ? term : acc + term;
       }
     }
-  }
-  const float d = boundary ? INFINITY : acc;
-  EVX_BATCH_TRACE(3);
-  // ---- index-stable top-k on the last front by (-distance, row index) (:253)
-  {
-    const int p = few_position(cand ? ordered_key(-d) : 0u, nv, nt, cnt, comps, ids, part, lo16, hi16);
-    if (cand) dist[mine_row] = d;
-    if (cand && p < need) order[worst_start + p] = (uint16_t)mine_row;  // (every candidate has been read from there)
   }
   __syncthreads();
 

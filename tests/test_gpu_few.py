@@ -86,6 +86,22 @@ def test_several_populations(b, n, m):
     assert runtime.last_status()["error"] == 0
 
 
+@pytest.mark.parametrize("m", [3, 8])
+@pytest.mark.parametrize("n", [65, 200, 256, 257, 512, 700, 1000, 1024])
+@pytest.mark.parametrize("levels", [1, 2, 4, 16, 30])
+def test_last_fronts_of_few_levels(n, m, levels):
+    """Candidates that crowd a bucket of the placement: of one value, of several (levels, with copies at both ends and between)."""
+    g = torch.Generator("cpu").manual_seed(n + m + levels)
+    f = torch.randint(0, levels, (n, m), generator=g).float()
+    f[:, 0] = torch.where(torch.rand(n, generator=g) < 0.1, f[:, 0] * 1e-12 * torch.rand(n, generator=g), f[:, 0])  # (close ones beside)
+    x = torch.arange(n * 2.0).reshape(n, 2)
+    for data in (f, -f, torch.cat([f[: n // 2] * 1e30, f[n // 2:] * 1e-30])):
+        for k in (1, n // 2, n):
+            _same(nd_environmental_selection(x.to(DEV), data.to(DEV), k), er.environmental_selection(x, data, k), (levels, n, m, k))
+            batch = nd_environmental_selection(x.expand(32, n, 2).to(DEV), data.expand(32, n, m).to(DEV), k)  # (without pairs above 256 rows)
+            _same([t[7] for t in batch], er.environmental_selection(x, data, k), (levels, n, m, k, "batch"))
+
+
 def test_host_threads_on_one_stream():
     """Threads whose calls take several launches each on the workspace of the default stream: every result is its own population's."""
     import threading
