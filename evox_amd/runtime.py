@@ -15,11 +15,12 @@ _last: Optional[Tuple[torch.Tensor, int, int, int]] = None  # (workspace, stream
 CHECK_STATUS = os.environ.get("EVOX_AMD_CHECK_STATUS", "0") not in ("", "0")
 
 # Populations of at most evox_hip_batched_max_rows(m) rows can run in the one-workgroup-per-population kernels, larger
-# ones need a workspace.  None = choose by size.  Three to eight objectives: up to 256 rows always; above, a few populations are
-# faster in the two launches whose first one spreads the matrix over the whole device (selection of half the rows, us, two launches
-# against one workgroup each: one of 300 x 3 12.5 / 16, one of 1000 x 3 21 / 28, one of 1000 x 8 47 / 60, 16 of 512 x 3 17.5 / 18.8, 16 of 1000 x 8
-# 59 / 62, 32 of 512 x 3 18.9 / 18.9, 32 of 512 x 5 25 / 28, 32 of 1000 x 3 32 / 30, 32 of 1000 x 8 70 / 61, 64 of 300 x 3 33 / 17, 64 of 1000 x 8
-# 138 / 62), more are not.  Other numbers of objectives: a lone population is faster in the
+# ones need a workspace.  None = choose by size.  Three to eight objectives: up to 256 rows always.  Above, one population is faster in
+# the two launches whose first one spreads the matrix over the whole device (selection of half the rows, us, two launches
+# against one workgroup: 300 x 3 12.5 / 16, 1000 x 3 21 / 28, 1000 x 8 47 / 60); two to 31 only from a size on that shrinks as the objectives
+# grow, since that call costs the host 29 us against 18 (in a loop of calls, 2 to 16 populations: 512 x 3 29 / 19, 777 x 3 29 / 29, 1000 x 3
+# 29 / 32, 512 x 5 29 / 26, 1000 x 5 31 / 41, 300 x 8 32 / 30, 777 x 8 42 / 52); from 32 populations on never (32 of 1000 x 3 32 / 30, of
+# 1000 x 8 70 / 61, 64 of 300 x 3 33 / 17).  Other numbers of objectives: a lone population is faster in the
 # pipeline from a size on that shrinks as the objectives grow (16 objectives 67 / 77 at 128 rows, 119 / 101 at 256), two or
 # three from twice that size on, four or more never.  True / False force the choice where it is possible (tests use that to drive small
 # inputs through both).
@@ -27,13 +28,7 @@ use_small_population_kernel = None
 
 
 def _lone_population_limit(m: int) -> int:
-    if m <= 3:
-        return 896
-    if m <= 5:
-        return 768
-    if m <= 8:
-        return 288
-    return 160
+    return 896 if m <= 2 else 160  # (three to eight objectives have a rule of their own)
 
 
 _batched_max_rows = {}  # objectives -> rows that the one-workgroup kernel takes (asked of the library once)
@@ -56,7 +51,7 @@ def small_population_kernel_fits(n: int, m: int, batch: int) -> bool:
     if use_small_population_kernel is True:
         return True
     if 3 <= m <= 8:
-        return n <= 256 or batch >= 32
+        return n <= 256 or batch >= 32 or (batch >= 2 and n <= (832 if m == 3 else 576 if m <= 5 else 320))
     if batch >= 4:
         return True
     return n <= _lone_population_limit(m) * (1 if batch == 1 else 2)
