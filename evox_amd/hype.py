@@ -21,12 +21,13 @@ def cal_hv(fit: torch.Tensor, ref: torch.Tensor, pop_size, n_sample: int) -> tor
     the number of points to be kept, ``n_sample`` uniform samples drawn with ``torch.rand`` on ``fit.device``
     between the per-objective minimum and ``ref`` (a seeded generator gives the reference's samples)."""
     if type(pop_size) is int and pop_size > 0 and ops.plain_eager():
-        with ops.quiet():
+        quiet = ops.quiet()
+        with quiet():
             fits = ops.hv_whole_call_fits(fit, ref, n_sample)
             m, device = (fit.size(1), fit.device) if fits else (0, None)
         if fits:
             u = torch.rand(n_sample, m, device=device)
-            with ops.quiet():
+            with quiet():
                 return ops.hype_contributions(fit, ref, pop_size, u)
     n, m = fit.size()
     alpha = hv_alpha(n, pop_size, fit.device)

@@ -13,12 +13,13 @@ def hv(objs: torch.Tensor, ref: torch.Tensor, num_sample: int = 100000) -> torch
     reference's samples; the sample-against-points test (hv.py:18) runs in the HIP kernel, without the
     (num_sample, n_points, n_objs) temporaries of the reference."""
     if ops.plain_eager():
-        with ops.quiet():
+        quiet = ops.quiet()
+        with quiet():
             fits = ops.hv_whole_call_fits(objs, ref, num_sample)
             m = objs.size(1) if fits else 0
         if fits:
             u = torch.rand(num_sample, m)  # (on the default device: the modes see this one)
-            with ops.quiet():
+            with quiet():
                 return ops.hv_estimate(objs, ref, u.to(objs.device))
     points = torch.abs(objs - ref)
     bound = torch.max(points, dim=0).values

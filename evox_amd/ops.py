@@ -44,6 +44,27 @@ def _on(device: torch.device):
     return _HERE if device.index is not None and device.index == _current_device() else torch.cuda.device(device)
 
 
+class _Elsewhere:
+    """A stream's lock, on another device than the current one: with its device guard."""
+
+    def __init__(self, here: runtime.Place):
+        self.guard, self.turn = torch.cuda.device(here.device), here.turn
+
+    def __enter__(self):
+        self.guard.__enter__()
+        self.turn.acquire()
+
+    def __exit__(self, *exc):
+        self.turn.release()
+        return self.guard.__exit__(*exc)
+
+
+def _at(here: runtime.Place):
+    """The lock of a stream, with its device the current one."""
+    index = here.device.index
+    return here.turn if index is not None and index == _current_device() else _Elsewhere(here)
+
+
 def _batched_first(info, dims, tensors):
     """The tensors of a vmap rule with the mapped dimension in front; those that are not mapped are expanded."""
     out = []
@@ -205,7 +226,8 @@ def nd_rank_until(f: torch.Tensor, count: int) -> torch.Tensor:
     out = torch.empty(f32.shape[:-1], dtype=torch.int32, device=f.device)
     if out.numel() == 0:
         return out
-    with _on(f.device), (here := runtime.place(f.device)).turn:
+    here = runtime.place(f.device)
+    with _at(here):
         _rank_many(here, f32.reshape(-1, n, m), out.view(-1, n), count)
     return out
 
@@ -235,7 +257,8 @@ def nd_first_front(f: torch.Tensor) -> torch.Tensor:
         return out
     if m == 0:
         return out.fill_(True)
-    with _on(f.device), (here := runtime.place(f.device)).turn:
+    here = runtime.place(f.device)
+    with _at(here):
         flat_f = f32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         stream = here.handle
@@ -282,7 +305,8 @@ def crowding(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Tensor:
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with _on(costs.device), (here := runtime.place(costs.device)).turn:
+    here = runtime.place(costs.device)
+    with _at(here):
         flat_c = c32.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
@@ -351,7 +375,8 @@ def crowding_wide(costs: torch.Tensor, mask: Optional[torch.Tensor]) -> torch.Te
         return out
     if m == 0:
         raise ValueError("costs must have at least one objective")
-    with _on(costs.device), (here := runtime.place(costs.device)).turn:
+    here = runtime.place(costs.device)
+    with _at(here):
         flat_c = wide.reshape(-1, n, m)
         flat_out = out.view(-1, n)
         flat_mask = None if mask is None else mask.reshape(-1, n)
@@ -413,7 +438,8 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
         return out_x, out_f, out_rank, out_dist
     if out_rank.numel() == topk and n <= _WIDE_WHOLE_MAX:
         # one population: the whole selection in one call of the library
-        with _on(f.device), (here := runtime.place(f.device)).turn:
+        here = runtime.place(f.device)
+        with _at(here):
             wb = wide.reshape(n, m)
             rows_f = f.reshape(n, m).contiguous()
             rows_x = x.reshape(n, -1).contiguous()
@@ -434,7 +460,8 @@ def nd_select_wide(x: torch.Tensor, f: torch.Tensor, topk: int) -> Tuple[torch.T
     # the ranks, as far as the front that holds the topk-th row, from the ranking kernels on a float32 image of the
     # fitness that keeps every comparison (the rows behind that front are marked unset)
     rank = nd_rank_until(f, topk)
-    with _on(f.device), (here := runtime.place(f.device)).turn:
+    here = runtime.place(f.device)
+    with _at(here):
         flat_w = wide.reshape(-1, n, m)
         flat_f = f.reshape(-1, n, m).contiguous()
         flat_x = x.reshape(flat_w.size(0), n, -1).contiguous()
@@ -728,7 +755,8 @@ def stable_argsort_step(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         if prev.dtype != torch.int32 or prev.shape != (n,):
             raise ValueError("prev must be an int32 order of the same length as the key")
         prev = prev.contiguous()
-    with _on(key.device), (here := runtime.place(key.device)).turn:
+    here = runtime.place(key.device)
+    with _at(here):
         ws = runtime.sort_workspace(n, here)
         stream = here.handle
         _lib.call("evox_hip_stable_argsort_step", key.data_ptr(), kind, key.stride(0), n,
@@ -767,7 +795,8 @@ def stable_argsort_rows(key: torch.Tensor, kind: int, prev: Optional[torch.Tenso
         prev = prev.contiguous()
     if key.stride(0) < 0 or key.stride(1) < 0:
         key = key.contiguous()
-    with _on(key.device), (here := runtime.place(key.device)).turn:
+    here = runtime.place(key.device)
+    with _at(here):
         ws = runtime.sort_workspace(n, here)
         stream = here.handle
         _lib.call("evox_hip_stable_argsort_step_batched", key.data_ptr(), kind, key.stride(0), key.stride(1), batch, n,
@@ -877,17 +906,23 @@ torch.library.register_vmap(hv_covered_count, _hv_covered_count_vmap)
 _HV_OBJECTIVES = 16  # most objectives of the whole-call hypervolume kernels
 
 
+_modes_on, _mode_at = torch._C._len_torch_function_stack, torch._C._get_function_stack_at
+
+
 def only_default_device() -> bool:
     """Whether no torch function mode is on but default devices (``torch.set_default_device``, ``with torch.device(...)``):
     nothing of the caller's looks at the functions that are called."""
-    return all(type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(torch._C._len_torch_function_stack()))
+    for i in range(_modes_on()):
+        if type(_mode_at(i)) is not DeviceContext:
+            return False
+    return True
 
 
 def quiet():
-    """Looking at a tensor's attributes under a function mode goes through Python each time: the whole-call functions below look
-    at them, and make their buffers, with the default devices off -- 20 us of a call of the metric.  Only where plain_eager()
-    holds: a tracer does not get here.  A function mode of the caller's own goes on seeing every call."""
-    return torch._C.DisableTorchFunction() if only_default_device() else contextlib.nullcontext()
+    """The context in which the whole-call functions below look at tensors and make their buffers: with the default devices
+    off, since looking at an attribute under a function mode goes through Python each time -- 20 us of a call of the metric.  Only
+    where plain_eager() holds: a tracer does not get here.  A function mode of the caller's own goes on seeing every call."""
+    return torch._C.DisableTorchFunction if only_default_device() else contextlib.nullcontext
 
 
 def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> bool:
@@ -904,11 +939,19 @@ def hv_whole_call_fits(points: torch.Tensor, ref: torch.Tensor, n_sample) -> boo
             and not points.is_neg() and not ref.is_neg())
 
 
+_hv_need = {}  # (query, points, objectives, samples, device) -> bytes (asked of the library once per shape)
+
+
 def _hv_whole_call(bytes_query: str, entry: str, points: torch.Tensor, ref: torch.Tensor, extra: tuple, u: torch.Tensor, out: torch.Tensor):
     n, m = points.shape
     u = u.contiguous()
     n_sample = u.size(0)
-    need = int(getattr(_lib.lib(), bytes_query)(n, m, n_sample))
+    shape = (bytes_query, n, m, n_sample, points.device.index)
+    need = _hv_need.get(shape)
+    if need is None:
+        need = int(getattr(_lib.lib(), bytes_query)(n, m, n_sample))
+        if len(_hv_need) < 4096:
+            _hv_need[shape] = need
     with _on(points.device):
         ws = torch.empty(need, dtype=torch.uint8, device=points.device)
         _lib.call(entry, points.data_ptr(), points.stride(0), points.stride(1), n, m, ref.data_ptr(), ref.stride(0), *extra, u.data_ptr(),

@@ -23,14 +23,14 @@ class Seen(TorchFunctionMode):
 @pytest.mark.parametrize("device", [False, True])
 def test_a_mode_of_the_callers_sees_the_quiet_calls(device):
     with torch.device("cpu") if device else Seen():
-        with Seen() as seen, ops.quiet():
+        with Seen() as seen, ops.quiet()():
             torch.empty(3)
     assert "empty" in seen.names
 
 
 def test_a_default_device_is_taken_off():
     with torch.device("meta"):
-        with ops.quiet():
+        with ops.quiet()():
             assert torch.empty(3).device.type == "cpu"
 
 

@@ -54,6 +54,7 @@ def device_on_the_cpu(monkeypatch):
     monkeypatch.setattr(ops._lib, "call", call)
     monkeypatch.setattr(ops._lib, "lib", lambda: Library())
     monkeypatch.setattr(ops, "_on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(ops, "_at", lambda here: here.turn)
     monkeypatch.setattr(ops, "_current_device", lambda: None)
     monkeypatch.setattr(runtime, "require_gpu_tensor", lambda t, what: None)
     monkeypatch.setattr(runtime, "stream_handle", lambda device: 7)
@@ -91,6 +92,34 @@ def test_calls_of_two_threads_on_a_stream_take_turns(name, device_on_the_cpu):
         t.join()
     assert not errors, errors
     assert device_on_the_cpu == []
+
+
+def test_a_call_on_another_device_holds_the_lock_inside_its_guard(monkeypatch):
+    inside = []
+
+    @contextlib.contextmanager
+    def guard(device):
+        inside.append(device)
+        try:
+            yield
+        finally:
+            inside.remove(device)
+
+    monkeypatch.setattr(torch.cuda, "device", guard)
+    here = runtime.Place(torch.device("cuda", 1), 7)
+    monkeypatch.setattr(ops, "_current_device", lambda: 0)
+    with pytest.raises(KeyError):
+        with ops._at(here):
+            assert inside == [here.device]
+            other = threading.Thread(target=lambda: inside.append(here.turn.acquire(blocking=False)))
+            other.start()
+            other.join()
+            assert inside.pop() is False
+            raise KeyError
+    assert not inside and here.turn.acquire(blocking=False)
+    here.turn.release()
+    monkeypatch.setattr(ops, "_current_device", lambda: 1)
+    assert ops._at(here) is here.turn
 
 
 def test_a_captured_call_keeps_no_buffer_that_later_calls_replace(device_on_the_cpu, monkeypatch):
