@@ -12,7 +12,7 @@
 // The orders:
 //   * (f1, f2, index): by buckets (two_small_place): a monotone map of f1 to 4096 buckets, LDS counters, and every row
 //     compared with the rows of its own bucket in full -- one pass, whatever ties there are, as long as no bucket is
-//     crowded; else a stable LSD radix sort of (32-bit key, 16-bit payload) pairs, eight bits a pass, on f2 and then f1;
+//     crowded (none is tried where all f1 are the same, only one where a sample says that few are); else a stable LSD radix sort of (32-bit key, 16-bit payload) pairs, eight bits a pass, on f2 and then f1;
 //   * the listing of the fronts by (rank, index): one or two passes of that sort on the ranks;
 //   * the last front by either objective: its rows already stand in the order of f1, which backwards is that of f2;
 //   * its order by the distance, for the index-stable top-k: by counting while it is small, by buckets, else by the sort.
@@ -27,6 +27,8 @@
 //   uniform                     24.4 -> 15   38 -> 26     63.5 -> 37   112 -> 62
 //   twenty fronts, shared f1    26.4 -> 15.6 34.6 -> 22   45 -> 28.3   71 -> 48
 //   one front                   22.8 -> 14.8 88 -> 19.4   59.5 -> 26   99 -> 43
+//   equal rows                  16 -> 15     77 -> 27     58 -> 35     96 -> 55
+//   four levels                 21 -> 18     29 -> 29     48 -> 41     108 -> 62
 #pragma once
 
 #include <type_traits>
@@ -48,6 +50,7 @@ constexpr int kTwoSmallPer = kTwoSmallRows / kTwoSmallThreads;  // items of a th
 constexpr int kTwoSmallBuckets = 4096;   // of two_small_place: four counters per thread
 constexpr uint32_t kTwoSmallCrowd = 64;  // rows of a bucket up to which every row of it looks at every other one
 constexpr int kTwoSmallCounting = 192;   // last fronts of at most this many rows are ordered by counting, larger ones by buckets
+constexpr int kTwoSmallTied = 512;       // ... up to which they are where many distances are equal: 500 rows, all equal, 28 -> 21 us; 1000 33 -> 38
 constexpr int kTwoSmallWaves = 4;        // waves that peel: one per SIMD of the compute unit
 constexpr int kTwoSmallRing = 64;        // rounds that a wave may be ahead of the next one
 constexpr uint16_t kTwoSmallUnset = 0xFFFFu;
@@ -432,6 +435,7 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
   __shared__ __attribute__((aligned(16))) uint32_t hi16[16];
   __shared__ uint32_t vary_bits[2];  // (radix path) bits in which the keys of f1 / of f2 differ from those of row 0
   __shared__ int nan_rows_lds[1];
+  __shared__ int tied_lds[1];  // many rows of the last front share a distance
   uint32_t* key_a = reinterpret_cast<uint32_t*>(two_small_lds);  // the sort's buffers
   uint32_t* key_b = key_a + kTwoSmallRows;
   uint16_t* pay_a = reinterpret_cast<uint16_t*>(key_b + kTwoSmallRows);
@@ -480,21 +484,34 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
     }
     if (tid == 0) {
       nan_rows_lds[0] = 0;
+      tied_lds[0] = 0;
       peel->ended = 0;
     }
     if (tid < kTwoSmallWaves) peel->progress[tid] = 0;
     if (tid < (kTwoSmallWaves - 1) * kTwoSmallRing) (&peel->ring[0][0])[tid] = 0ull;
     two_small_range(lo, hi, lo16, hi16, kTwoSmallThreads);
-    bool ordered = false;  // by buckets of equal width in the value of f1, else in its image
-#pragma unroll 1
-    for (int attempt = 0; attempt < 2 && !ordered; ++attempt) {
+    // By buckets of equal width in the value of f1, else in its image.  Where one f1 is that of many rows neither will do, and an attempt
+    // that fails takes 3 us (additions to one counter): none is made where all values are the same, and no second one where sixty-four
+    // rows of a sample share their f1 with four of them more often than if some eighty rows of the population did.
+    bool ordered = false;
+    auto place_by = [&](auto bucket_of) {
 #pragma unroll
-      for (int r = 0; r < kTwoSmallPer; ++r)
-        bucket[r] = attempt == 0 ? bucket_by_value(a1[r], lo, hi, kTwoSmallBuckets) : bucket_by_image(a1[r], lo, hi, kTwoSmallBuckets);
-      ordered = two_small_place<kTwoSmallPer>(comp, id, bucket, n, kTwoSmallThreads, cnt, part, reinterpret_cast<uint64_t*>(key_a), pay_a, place, has_copies);
+      for (int r = 0; r < kTwoSmallPer; ++r) bucket[r] = bucket_of(a1[r], lo, hi, kTwoSmallBuckets);
+      return two_small_place<kTwoSmallPer>(comp, id, bucket, n, kTwoSmallThreads, cnt, part, reinterpret_cast<uint64_t*>(key_a), pay_a, place, has_copies);
+    };
+    if (__builtin_expect(lo < hi, 1)) {
+      ordered = place_by([](uint32_t key, uint32_t from, uint32_t to, int buckets) { return bucket_by_value(key, from, to, buckets); });
+      if (__builtin_expect(!ordered, 0)) {
+        const uint32_t key = ordered_key(fitness_at((int)((unsigned)(lane * n) >> 6), 0));  // (by every wave for itself)
+        int same = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) same += __popcll(__builtin_amdgcn_ballot_w64(key == (uint32_t)__builtin_amdgcn_readlane((int)key, 8 + 16 * u)));
+        if (same * n <= 7 * n + 4 * 63 * 80)
+          ordered = place_by([](uint32_t key, uint32_t from, uint32_t to, int buckets) { return bucket_by_image(key, from, to, buckets); });
+      }
     }
     EVX_BATCH_TRACE(1);
-    if (!ordered) {  // (the same in every thread) many rows share an f1
+    if (__builtin_expect(!ordered, 0)) {  // (the same in every thread) many rows share an f1
       __syncthreads();
       if (tid < 2) vary_bits[tid] = 0u;
 #pragma unroll
@@ -568,7 +585,7 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
   // the rank of the first copy, which counts for all of them)
   uint32_t* copies = cnt;           // per position of a first row
   uint32_t* val = k2;
-  if (nan_rows != 0 || has_copies) {
+  if (__builtin_expect(nan_rows != 0 || has_copies, 0)) {
     val = key_a;
     uint32_t last_first = 0u;  // 1 + the last position of this thread that is not a copy, 0 = none
     bool is_copy[kTwoSmallPer];
@@ -706,6 +723,9 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
         }
       }
     }
+    const uint32_t key = ordered_key(d_of[0]);
+    const uint64_t same = __builtin_amdgcn_ballot_w64(tid < nv && key == (uint32_t)__builtin_amdgcn_readlane((int)key, 32));
+    if (lane == 0 && __popcll(same) >= 40) tied_lds[0] = 1;
     __syncthreads();  // (cnt, as `copies`, and k1, k2 are free from here on)
   }
 
@@ -725,7 +745,8 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
 
   // ---- the order of the last front by (distance descending, index), non_dominate.py:253, into the listing: nobody reads
   // its rows there any more except where they are taken from it first
-  if (by_value && nv <= kTwoSmallCounting) {
+  const bool tied = by_value && tied_lds[0] != 0;  // (buckets would be crowded)
+  if (by_value && (nv <= kTwoSmallCounting || __builtin_expect(tied && nv <= kTwoSmallTied, 0))) {
     uint64_t* tile = comps;  // nv + 4 entries
     int* below = reinterpret_cast<int*>(cnt);
     const bool cand = tid < nv;
@@ -735,7 +756,7 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
     if (cand && p < need) listed[worst_start + p] = (uint16_t)d_row[0];
   } else {
     bool placed = false;
-    if (by_value) {
+    if (by_value && __builtin_expect(!tied, 1)) {
       uint64_t comp[kTwoSmallPer];
       uint32_t bucket[kTwoSmallPer];
       int place[kTwoSmallPer];
@@ -765,7 +786,7 @@ __global__ __launch_bounds__(kTwoSmallThreads) void two_small_kernel(BatchedArgs
         }
       }
     }
-    if (!placed) {
+    if (__builtin_expect(!placed, 0)) {
       // by the radix sort, candidate q = listed[worst_start + q] (in index order): many equal distances, or rows with a NaN.
       // d_by_row shares nothing with the sort's lane masks, which lie in k1 here.
       uint32_t* sk_a = free32;

@@ -153,3 +153,28 @@ def test_around_the_choices_inside_the_kernel(kind, n):
     assert np.array_equal(as_np(non_dominate_rank(f.to(DEV))), as_np(er.ranks_by_peeling(f)))
     for topk in (n // 2, n):
         _same_selection(nd_environmental_selection(x.to(DEV), f.to(DEV), topk), er.environmental_selection(x, f, topk), (kind, n, topk))
+
+
+@pytest.mark.parametrize("n", [128, 200, 512, 513, 1024, 1025, 2500])
+@pytest.mark.parametrize("kind", ["one f1", "two f1", "four levels", "one f1 and infinities", "copies of a line"])
+def test_many_rows_of_one_value(kind, n):
+    """One f1 (no buckets are tried), few (no second attempt), and last fronts whose distances are mostly equal, on either side
+    of the sizes up to which they are ordered by counting."""
+    g = torch.Generator("cpu").manual_seed(n + len(kind))
+    f = torch.rand(n, 2, generator=g)
+    if kind == "two f1":
+        f[:, 0] = (f[:, 0] * 2).floor()
+    elif kind == "four levels":
+        f = (f * 4).floor()
+    elif kind == "copies of a line":
+        f[:, 0] = (f[:, 0] * 12).floor()
+        f[:, 1] = 12.0 - f[:, 0]
+    else:
+        f[:, 0] = -0.25
+        if kind != "one f1":
+            f[::7, 0] = float("inf")
+            f[3::11, 0] = -float("inf")
+    x = torch.arange(n, dtype=torch.float32)[:, None].repeat(1, 3)
+    for topk in (n // 2, n):
+        _same_selection(nd_environmental_selection(x.to(DEV), f.to(DEV), topk), er.environmental_selection(x, f, topk), (kind, n, topk))
+    assert np.array_equal(as_np(non_dominate_rank(f.to(DEV))), as_np(er.ranks_by_peeling(f)))
