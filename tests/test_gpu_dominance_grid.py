@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
 
 
-# rows -> row blocks of 128: 1, 2, 3, 4, 5, 40, 41, 79, 157 (the pipeline takes a lone population from 897 rows on;
-# smaller ones reach the kernel with the one-workgroup kernel switched off)
+# rows -> row blocks of 128: 1, 2, 3, 4, 5, 40, 41, 79, 157 (up to 1024 rows the kernel is reached with the one-workgroup kernels and the two
+# launches for few rows switched off)
 # Tiles of four words (more than 24 576 rows, 32 768 from six objectives on): row blocks of 256, 129 and 157 of them.
 @pytest.mark.parametrize("n", [100, 200, 300, 512, 640, 5100, 5200, 10050, 20000, 33000, 40001])
 @pytest.mark.parametrize("m", [2, 3, 5])
@@ -29,7 +29,7 @@ def test_folded_and_full_grid_agree_with_the_checker(n, m):
     runtime.use_small_population_kernel = False
     try:
         for folded in (1, 0):
-            with runtime.options(dominance_folded=folded):
+            with runtime.options(dominance_folded=folded, few_max_rows=0):
                 got = as_np(non_dominate_rank(fd))
                 assert runtime.last_status()["error"] == 0
             assert np.array_equal(got, want), (n, m, folded)

@@ -19,7 +19,8 @@ DEV = torch.device("cuda", 0)
 @pytest.fixture(autouse=True)
 def through_the_pipeline():
     runtime.use_small_population_kernel = False
-    yield
+    with runtime.options(few_max_rows=0):  # (up to 1024 rows of three to eight objectives: two launches of their own otherwise)
+        yield
     runtime.use_small_population_kernel = None
 
 

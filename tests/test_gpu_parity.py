@@ -3,6 +3,7 @@
 Tolerances (from the task statement): ranks bit-exact; crowding distance within 1e-5 relative on
 finite values with infinities and NaN positions exact; selected order exact."""
 
+import contextlib
 import ctypes
 import sys
 
@@ -34,7 +35,9 @@ def population_path(request):
     one-workgroup-per-population kernel, as in production, and with everything forced through the
     bit-matrix pipeline."""
     runtime.use_small_population_kernel = request.param == "small-kernel"
-    yield request.param
+    # (few_max_rows: up to 1024 rows of three to eight objectives the pipeline's entry points would take two launches of their own)
+    with runtime.options(few_max_rows=0) if request.param == "pipeline" else contextlib.nullcontext():
+        yield request.param
     runtime.use_small_population_kernel = None
 
 
