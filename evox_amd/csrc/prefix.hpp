@@ -189,10 +189,111 @@ __host__ __device__ inline size_t order_offsets_words(int m, int parts) { return
 __host__ __device__ inline size_t order_bounds_words(int m, int parts) { return 2 * (size_t)m * (size_t)(parts + 1); }
 constexpr size_t kOrderStreamLdsBytes = 8 * (size_t)kOrderStreamCapacity + 4 * (size_t)kOrderStreamBuckets;
 
+// The rest of order_stream_place<PER, true> once some buckets crowd: cnt holds where the buckets begin, `held` the sizes of the thread's four and
+// `run` where the first of them begins.  False, with comp as it was, if a crowded bucket holds several values.  word: one word.
+template <int PER, typename BUCKET>
+__device__ inline bool order_sample_place(unsigned long long* comp, const unsigned long long (&mine)[PER], int count, uint4 held, uint32_t run,
+                                          uint32_t* cnt, uint32_t* word, BUCKET bucket_of_entry) {
+  constexpr int kWaves = kOrderStreamThreads / 64;
+  constexpr int kEntries = PER * kOrderStreamThreads;
+  constexpr int kMostCrowded = kEntries / (int)(kOrderStreamCrowd + 1u);  // crowded buckets, at most
+  static_assert(PER * kWaves * kMostCrowded <= 2 * kEntries, "the table takes the composites' place");
+  static_assert(kEntries < (1 << 16) && kMostCrowded < (1 << 8), "number << 16 | first place");
+  __shared__ uint32_t key_of[kMostCrowded];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the crowded buckets are numbered from 1 on
+  if (tid == 0) *word = 0u;
+  __syncthreads();
+  const uint32_t size[4] = {held.x, held.y, held.z, held.w};
+  uint32_t first_of = run;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (size[i] > kOrderStreamCrowd) cnt[4 * tid + i] = (atomicAdd(word, 1u) + 1u) << 16 | first_of;
+    first_of += size[i];
+  }
+  __syncthreads();
+  uint32_t bucket[PER], number[PER];
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    const bool live = tid + kOrderStreamThreads * r < count;
+    bucket[r] = live ? bucket_of_entry(mine[r]) : 0u;
+    number[r] = live ? cnt[bucket[r]] >> 16 : 0u;
+    if (number[r] != 0u) key_of[number[r] - 1u] = (uint32_t)(mine[r] >> 20);  // (any member's)
+  }
+  __syncthreads();
+  bool other = false;
+#pragma unroll
+  for (int r = 0; r < PER; ++r) other |= number[r] != 0u && key_of[number[r] - 1u] != (uint32_t)(mine[r] >> 20);
+  if (__syncthreads_or(other)) return false;
+  // members of a wave per crowded bucket, and how many lie in front of each
+  uint32_t* const table = reinterpret_cast<uint32_t*>(comp);
+  for (int i = tid; i < PER * kWaves * kMostCrowded; i += kOrderStreamThreads) table[i] = 0u;
+  __syncthreads();
+  uint32_t place[PER];
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    place[r] = 0u;
+    uint64_t left = __builtin_amdgcn_ballot_w64(number[r] != 0u);
+    while (left != 0ull) {  // (wave-uniform)
+      const int at = __builtin_ctzll(left);
+      const uint32_t of = (uint32_t)__builtin_amdgcn_readlane((int)number[r], at);
+      const uint64_t same = __builtin_amdgcn_ballot_w64(number[r] == of);
+      if (number[r] == of) place[r] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+      if (lane == at) table[(r * kWaves + wave) * kMostCrowded + (int)of - 1] = (uint32_t)__popcll(same);
+      left &= ~same;
+    }
+  }
+  __syncthreads();
+  if (tid < kMostCrowded) {
+    uint32_t before = 0u;
+    for (int w = 0; w < PER * kWaves; ++w) {
+      const uint32_t here = table[w * kMostCrowded + tid];
+      table[w * kMostCrowded + tid] = before;
+      before += here;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < PER; ++r)
+    if (number[r] != 0u) place[r] += (cnt[bucket[r]] & 0xFFFFu) + table[(r * kWaves + wave) * kMostCrowded + (int)number[r] - 1];
+  __syncthreads();
+  // (the others anywhere in their bucket, then by the members below them)
+  uint32_t first[PER], end[PER];
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    first[r] = cnt[bucket[r]] & 0xFFFFu;
+    end[r] = bucket[r] + 1u < (uint32_t)kOrderStreamBuckets ? cnt[bucket[r] + 1u] & 0xFFFFu : (uint32_t)count;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    if (tid + kOrderStreamThreads * r < count) {
+      if (number[r] == 0u) place[r] = atomicAdd(&cnt[bucket[r]], 1u);
+      comp[place[r]] = mine[r];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    if (tid + kOrderStreamThreads * r < count && number[r] == 0u) {
+      place[r] = first[r];
+      for (uint32_t q = first[r]; q < end[r]; ++q) place[r] += comp[q] < mine[r] ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < PER; ++r)
+    if (tid + kOrderStreamThreads * r < count) comp[place[r]] = mine[r];
+  __syncthreads();
+  return true;
+}
+
 // Places of `count` composites (entry tid + kOrderStreamThreads r of comp is `mine[r]`) in ascending order, by buckets; afterwards
 // comp[place] holds them in that order.  False, with comp as it was, when they crowd.  cnt: kOrderStreamBuckets words; part, lo16, hi16: sixteen
 // words each.  Every thread calls it, past a barrier behind the last write of comp; ends with one.
-template <int PER>
+// BY_INDEX: the entries lie in the order of their indices, so that the members of a crowded bucket of one value need only be counted, a wave's
+// by a ballot (half of 60 000 x 4 rows of four levels selected: 387 us where the middle levels of the sample went to the network, now 378; uniform values 302 as before).
+template <int PER, bool BY_INDEX = false>
 __device__ inline bool order_stream_place(unsigned long long* comp, int count, uint32_t* cnt, uint32_t* part, uint32_t* lo16, uint32_t* hi16) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr int kWaves = kOrderStreamThreads / 64;
@@ -285,11 +386,18 @@ __device__ inline bool order_stream_place(unsigned long long* comp, int count, u
       if (lane >= off) incl += up;
     }
     if (lane == 63) part[wave] = incl;
-    if (__syncthreads_or(max(max(held.x, held.y), max(held.z, held.w)) > kOrderStreamCrowd)) continue;
+    const bool crowded = __syncthreads_or(max(max(held.x, held.y), max(held.z, held.w)) > kOrderStreamCrowd) != 0;
+    if (crowded && (!BY_INDEX || attempt == 1)) continue;
     uint32_t run = incl - sum;
     for (int w = 0; w < wave; ++w) run += part[w];
     reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(run, run + held.x, run + held.x + held.y, run + held.x + held.y + held.z);
     __syncthreads();
+    if constexpr (BY_INDEX) {
+      if (__builtin_expect(crowded, 0)) {
+        if (order_sample_place<PER>(comp, mine, count, held, run, cnt, lo16, bucket_of_entry)) return true;
+        continue;
+      }
+    }
 #pragma unroll
     for (int r = 0; r < PER; ++r)
       if (tid + kOrderStreamThreads * r < count) comp[cnt[bucket_of_entry(mine[r])] + ((arrived[r >> 1] >> (16 * (r & 1))) & 0xFFFFu)] = mine[r];
@@ -363,7 +471,7 @@ __global__ __launch_bounds__(kOrderStreamThreads) void objective_shares_kernel(c
   }
   if (tid < kOrderStreamMaxParts) group[tid] = 0u;
   __syncthreads();
-  const bool placed = order_stream_place<kOrderStreamSample / kOrderStreamThreads>(composites, kOrderStreamSample, cnt, part16, lo16, hi16);
+  const bool placed = order_stream_place<kOrderStreamSample / kOrderStreamThreads, true>(composites, kOrderStreamSample, cnt, part16, lo16, hi16);
   if (!placed) bitonic_sort_lds(comp, kOrderStreamSample);
   if (tid <= parts) {
     const int i = (int)(((int64_t)tid * kOrderStreamSample) / parts);
