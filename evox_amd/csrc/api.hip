@@ -481,6 +481,7 @@ static int stage_prepare(const Ws& w, const Fitness& src, bool with_sort, hipStr
 // With the orders from shares that are placed by buckets (prefix.hpp, above kMidArgsortRows rows; they also order the last front):
 //   x 3: 33 000 264 / 287 (one front: 284 / 214), 41 000 309 / 309 (shell 242 / 223), 52 000 385 / 344;  x 4: 33 000 215 / 212 (shell 205 / 177);
 //   x 5: 33 000 218 / 205 (one front 324 / 223), 42 000 283 / 230;  x 6: 33 000 228 / 197;  x 7: 33 000 260 / 200 (one front 377 / 245).
+// (Few levels share the loss and the gain: 41 000 x 3 of four 271 / 277, of eight 290 / 297;  33 000 x 4 of four 266 / 258.)
 // As thirty-seconds of the tunable (20 of them are 40 960 rows; four to seven objectives begin where those orders do):
 // Up to kMidArgsortRows rows the orders come from workgroups that sort in LDS and cost 60 to 90 us less:
 //   x 8: 26 000 254 / 261, 32 768 322 / 295;  x 9: 16 000 212 / 224, 20 000 252 / 236;  x 10: 16 000 222 / 231,
@@ -1514,7 +1515,7 @@ static int launch_sets(const BatchedArgs& a, int64_t batch, hipStream_t s) {
 
 static int launch_batched(const BatchedArgs& a, int64_t batch, hipStream_t s) {
   // (1024 populations, us, all pairs against the orders of the objectives: 256 x 3 uniform 27 / 27, values of four levels 28 / 33, 192 x 3
-  // 20 to 23 / 23 and 21 / 39; from 257 rows on no slower on any data: 257 x 3 46 / 31 and 48 / 37, 512 x 3 64 / 44, 390 x 5 146 / 52, 390 x 8 210 / 93,
+  // 20 to 23 / 23 and 21 / 39; from 257 rows on no slower on any data: 257 x 3 46 / 31 and 48 / 37, 512 x 3 64 / 41, 390 x 5 146 / 54, 390 x 8 210 / 87,
   // with four levels 123 / 124)
   if (a.m >= 3 && a.m <= kSetsObjectives && a.n >= opt().sets_min_rows && a.n <= kSetsRows) return launch_sets(a, batch, s);
   if (a.m >= 3 && a.m <= kFewObjectives && a.n <= kFewWholeRows && batch <= device_cus() && opt().few_max_rows > 0)
@@ -1546,7 +1547,9 @@ static int launch_batched(const BatchedArgs& a, int64_t batch, hipStream_t s) {
 
 using namespace evx;
 
-constexpr int kFewBatch = 64;  // populations that share those launches at most
+// Populations that share those launches at most.  From 32 on the entry points without a workspace are the faster ones (64 x (300 x 3) 17 us
+// against 33; the Python side goes by that), but a caller who is here would get the pipeline instead.
+constexpr int kFewBatch = 64;
 static bool few_applies(const Layout& L, const Fitness& fit, int batch);
 static int stage_few(const Ws& w, const Fitness& fit, BatchedArgs a, hipStream_t s);
 static bool two_applies(const Layout& L, int64_t stop_count);
@@ -2523,7 +2526,7 @@ static int stage_rank_two(const Ws& w, const Fitness& src, int64_t stop_count, b
 }
 
 // Populations that two launches take (few.hpp): all whose rows fit the threads of one workgroup (against the pipeline, us
-// per selection of half the rows: 300 x 3 37 -> 17, 1000 x 3 45 -> 21, 1000 x 5 47 -> 31, 1000 x 8 82 -> 47; all ranks of 1000 x 3
+// per selection of half the rows in a loop of calls; the device alone is done with 300 x 3 in 12.5: 300 x 3 37 -> 17, 1000 x 3 45 -> 21, 1000 x 5 47 -> 31, 1000 x 8 82 -> 47; all ranks of 1000 x 3
 // 64 -> 23), unless a tunable asks for a kernel of the pipeline.  The two parts of a population must have equal strides.
 static bool few_applies(const Layout& L, const Fitness& fit, int batch) {
   if (L.n > opt().few_max_rows || L.m < 3 || L.m > kFewObjectives || batch > kFewBatch) return false;

@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kMidArgsortThreads) void objective_order_lds_kernel
 // value), every entry among those of its bucket; the network of radix.hpp only sorts what crowds in both.
 // A workgroup that read all keys of its objective for its share, and sorted that by the network, took 78 us of vector issue for the
 // reading alone at 200 000 rows (96 us, 20 more for positions and bounds in a launch of their own; 160 us and more by the radix sort
-// above); now 12 + 40 us at 200 003 x 3 and 12 + 52 at 200 000 x 8: 7 the sample, 8 to 10 fetching the groups (chains of two reads), 9 to 13 the
+// above); now 15 + 42 us at 200 003 x 3 and 20 + 57 at 200 000 x 8: 7 the sample, 8 to 10 fetching the groups (chains of two reads), 9 to 13 the
 // placing, 12 to 18 the scattered positions and bounds.
 // Grid: m * parts workgroups of kOrderStreamThreads each.  Dynamic LDS: kOrderStreamLdsBytes.  n <= 2^20.
 constexpr int kOrderStreamThreads = 1024;

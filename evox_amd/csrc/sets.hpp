@@ -18,7 +18,8 @@
 // positions and W / 2 reads of 16 bytes: a table entry of all words of a row, so that a lane reads them in pieces of 16 bytes, four
 // words further on per segment, so that the lanes that write meet different banks.  512 rows of up to five objectives leave room for
 // four workgroups on a compute unit (36 KB of LDS, 64 registers).  Bound by vector issue and LDS in equal parts: of the 41 us of 1024
-// populations of 512 x 3 the orders take 12, the table 5, the fronts and their distances 10, the gather 10 (64 MB).  us per selection of half the rows,
+// populations of 512 x 3 the orders take 12, the table 5, the fronts and their distances 10, the gather 10 (64 MB); the narrow
+// instance still has 7 VGPRs in scratch at three objectives, 10 at four, 22 at five, 27 at eight.  us per selection of half the rows,
 // pairs -> orders: 1024 x (512 x 3) 64 -> 41, 512 x (700 x 3) 67 -> 50, 390 x (1000 x 3) 129 -> 60, 1024 x (390 x 5)
 // 146 -> 54, 1024 x (390 x 8) 210 -> 87.
 #pragma once

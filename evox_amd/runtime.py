@@ -16,7 +16,7 @@ CHECK_STATUS = os.environ.get("EVOX_AMD_CHECK_STATUS", "0") not in ("", "0")
 
 # Populations of at most evox_hip_batched_max_rows(m) rows can run in the one-workgroup-per-population kernels, larger
 # ones need a workspace.  None = choose by size.  Three to eight objectives: up to 256 rows always.  Above, one population is faster in
-# the two launches whose first one spreads the matrix over the whole device (selection of half the rows, us, two launches
+# the two launches whose first one spreads the matrix over the whole device (selection of half the rows, us on the device, two launches
 # against one workgroup: 300 x 3 12.5 / 16, 1000 x 3 21 / 28, 1000 x 8 47 / 60); two to 31 only from a size on that shrinks as the objectives
 # grow, since that call costs the host 29 us against 18 (in a loop of calls, 2 to 16 populations: 512 x 3 29 / 19, 777 x 3 29 / 29, 1000 x 3
 # 29 / 32, 512 x 5 29 / 26, 1000 x 5 31 / 41, 300 x 8 32 / 30, 777 x 8 42 / 52); from 32 populations on never (32 of 1000 x 3 32 / 30, of

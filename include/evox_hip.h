@@ -410,7 +410,8 @@ int evox_hip_read_status(const void* workspace, void* stream, int32_t* host_out8
  * "prefix_min_rows" (default 65536: finite populations of at least 20/32 of this many rows of three objectives have their matrix built from the per-objective orders -- 40/32 with two, fewer with more: 32769 at four, 28672 at eight, 10240 at sixteen; 0 = never),
  * "prefix_bands" (default 1), "prefix_double_tile" (default 131072 rows, 0 = never), "prefix_mode" (default 3; 1 and 2 build only half of that kernel's output, for measurements),
  * "sets_min_rows" (default 257: populations of three to eight objectives and at least this many rows that the one-workgroup entry points take go without a comparison of pairs; 1025 = never),
- * "batched_stage" (default 1: the one-workgroup kernel reads the dominators of populations of at most 256 rows and eight objectives from a copy of the fitness in LDS when the launch holds no more populations than the device has compute units; 0 = by scalar loads from memory always),
+ * "few_max_rows" (default 1024: a population, or up to 64 together, of at most this many rows and three to eight objectives that reaches an entry point with a workspace takes two launches of its own instead of the pipeline -- up to 256 rows and from 32 populations on the entry points without a workspace are the faster ones, 64 x (300 x 3) 17 us against 33; 0 = never, also not the kernel in which sixteen waves share the pairs of up to 256 rows),
+ * "batched_stage" (default 1: the one-workgroup kernel that compares pairs -- by default that of one objective, of two below 128 rows, and of three to eight where "few_max_rows" is 0 -- reads the dominators of populations of at most 256 rows from a copy of the fitness in LDS when the launch holds no more populations than the device has compute units; 0 = by scalar loads from memory always),
  * "order_stream" (default 1: for more than 32768 rows those orders come from workgroups that place a share of the order each in LDS, in two launches, without waiting for each other, while shares of 8192 rows need no more workgroups than the device has compute units -- up to 262144 rows of eight objectives; 0 = from the radix sort, whose workgroups wait for each other twelve times), "order_stream_capacity" (default 16384, 1 .. 16384: entries that such a workgroup sorts at once; a larger share is taken in pieces -- tests make it small),
  * "prefix_count_first" (default 1: a selection of such a population whose last two of the same shape on the device found all the rows they keep in front 0 -- told by a word of the pinned host memory of "launch_memory" -- has that kernel count the dominators of every row first and build the matrix, in a second launch, only if front 0 falls short this time; 0 = always both at once, 2 = always counts first),
  * "prefix_nearby" (default 1: those counts are made in spatial order from a number of rows on that falls with the objectives -- 131072 at three, 57344 at eleven to fifteen; 0 = never, any other value = from that many rows on).
